@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define KCH_ABI_VERSION 19
+#define KCH_ABI_VERSION 20
 
 #define KCH_OK 0
 #define KCH_ERR_INVALID 1     /* bad pointer / shape / argument */
@@ -260,6 +260,15 @@ int kch_csa_ste_bwd(const float* q_idx, const float* w_idx, const float* kc, con
                     float* dq_idx, float* dw_idx, float* dK_idx, float* dZ_idx, float* dBp, int B,
                     int T, int m, int nIh, int cI, float scale, int normalize, void* ws,
                     size_t ws_bytes, void* stream);
+
+/*
+ * The dense dsel of kch_csa_ste_bwd from the selection's slots:
+ * dsel[b,t,idx[b,t,j]] += slot[b,t,j] for every idx >= 0 (idx, slot
+ * [B,T,topk]; dsel [B,T,nb] fp32 holds zeros, or the dense term of
+ * ste_mode='full_softmax', on entry).
+ */
+int kch_csa_ste_scatter(const int* idx, const float* slot, float* dsel, int B, int T, int topk,
+                        int nb, void* stream);
 
 /*
  * Backward of the KDA layer's front end and of the stack's LayerNorm (the

@@ -554,6 +554,18 @@ int kch_csa_ste_bwd(const float* q_idx, const float* w_idx, const float* kc, con
   return hip_status(fn, kch::ste_bwd_dispatch(p, bp, ws, (hipStream_t)stream));
 }
 
+int kch_csa_ste_scatter(const int* idx, const float* slot, float* dsel, int B, int T, int topk, int nb,
+                        void* stream) {
+  const char* fn = "kch_csa_ste_scatter";
+  if (B < 0 || T < 0 || topk < 0 || nb < 0)
+    return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d T=%d topk=%d nb=%d", fn, B, T, topk, nb);
+  if ((long long)B * T * topk >= (1LL << 39) || (long long)B * T * nb >= (1LL << 40))
+    return fail(KCH_ERR_UNSUPPORTED, "%s: too large", fn);
+  if ((long long)B * T * topk == 0) return KCH_OK;
+  if (!idx || !slot || !dsel) return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
+  return hip_status(fn, kch::ste_scatter_launch(idx, slot, dsel, (long long)B * T, topk, nb, (hipStream_t)stream));
+}
+
 int kch_kda_gates_bwd(const void* proj, long long ld_proj, const void* gl, long long ld_gl,
                       const void* dq, const void* dk, const void* dv, const void* dg,
                       const void* dbeta, void* dproj, void* dgl, int B, int T, int H, int HV, int K,

@@ -657,7 +657,6 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
 }
 
 hipError_t sel_bitmap_launch(const int* idx, uint32_t* sel, long long nq, int topk, int nw, hipStream_t s);
-hipError_t hca_bwd_finish_launch(const HcaBwdParams& p, int nchunk, hipStream_t s);
 
 hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
   const int HD = p.c;

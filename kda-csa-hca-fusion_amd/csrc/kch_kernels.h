@@ -131,7 +131,7 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk);
 hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s);
 size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk);
 
-// The STE surrogate's backward for the indexer (hca_backward.hip): fp32,
+// The STE surrogate's backward for the indexer (ste_backward.hip): fp32,
 // cI in {64, 128}, nIh in {1, 2, 4, 8}, nIh * cI <= 512.
 struct SteBwdParams {
   const float* qi;    // [B,T,nIh,cI] indexer queries as given
@@ -150,6 +150,11 @@ struct SteBwdParams {
 size_t ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m);
 // bp: the key compression's inputs and outputs for the block kernel
 hipError_t ste_bwd_dispatch(SteBwdParams p, HcaBwdParams bp, void* ws, hipStream_t stream);
+// dsel[row, idx[row, j]] += slot[row, j] over rows of topk slots, nb columns
+hipError_t ste_scatter_launch(const int* idx, const float* slot, float* dsel, long long rows, int topk, int nb,
+                              hipStream_t s);
+// the block and window kernels on the partials (hca_backward.hip)
+hipError_t hca_bwd_finish_launch(const HcaBwdParams& p, int nchunk, hipStream_t s);
 hipError_t hca_bwd_dispatch(HcaBwdParams p, void* ws, hipStream_t stream);
 
 hipError_t kda_chunk_dispatch(const KdaParams& p, int dtype, hipStream_t stream);

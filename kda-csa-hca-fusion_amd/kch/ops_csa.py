@@ -647,10 +647,12 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
     raw = _compress(fn, Kf, Zf, Bf, m, out_raw=True, key=kc, normalize=bool(normalize_qk))
     if not normalize_qk:
         kc = raw
-    idx64 = idx.long()
     dsel = (torch.zeros(B_, T, nb, device=dev, dtype=f32) if dsel_extra is None
-            else dsel_extra.to(f32).clone()).scatter_add_(
-        -1, idx64.clamp(min=0), slot.to(f32) * (idx64 >= 0).to(f32))
+            else dsel_extra.to(f32).clone(memory_format=torch.contiguous_format))
+    idx32 = idx.to(dtype=torch.int32).contiguous()
+    slot = slot.to(f32).contiguous()
+    _lib.call("kch_csa_ste_scatter", _lib.ptr(idx32), _lib.ptr(slot), _lib.ptr(dsel), B_, T,
+              idx.shape[-1], nb, _lib.stream_of(qf))
     scale = 1.0 if normalize_qk else cI ** -0.5
     dq = torch.empty_like(qf)
     dw = torch.empty_like(wf)

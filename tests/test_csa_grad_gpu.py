@@ -380,3 +380,49 @@ def test_naive_csa_aux_contrastive_raises(dev):
     with pytest.raises(NotImplementedError):
         kch.naive_csa(H, *ps, m=m, topk=2, nh=nh, nIh=nIh, c=c, c_I=cI, dc=dc,
                       ste_mode='aux_contrastive')
+
+
+STE_EDGES = [
+    # B, T, m, topk, nIh, cI, norm: heads per tile, channels, blocks off whole tiles
+    (1, 1, 1, 1, 1, 64, True),         # one query, one block
+    (2, 63, 3, 5, 2, 64, False),       # 21 blocks (no 4-element rows), raw queries and keys
+    (1, 129, 1, 16, 4, 64, True),      # a 129-block row: two key tiles, one block in the last
+    (2, 132, 4, 8, 8, 64, True),       # eight heads: two queries a tile
+    (1, 260, 4, 64, 1, 128, True),     # 16 queries a tile, 65 blocks
+    (1, 576, 2, 24, 4, 128, False),    # several query chunks per key tile
+    (3, 100, 4, 3, 2, 48, True),       # channels padded to 64
+]
+
+
+@pytest.mark.parametrize("B,T,m,topk,nIh,cI,norm", STE_EDGES)
+def test_ste_indexer_kernels_at_tile_edges(dev, B, T, m, topk, nIh, cI, norm):
+    """``kch_csa_ste_scatter`` + ``kch_csa_ste_bwd`` against float64 autograd of the
+    same surrogate: every gradient within 1e-4 of its largest entry (fp32 sums of
+    up to T * nIh <= 2304 terms: at most 2304 * 2^-24 = 1.4e-4 of the terms'
+    absolute sum, and random signs leave its square root)."""
+    import kch
+    rng = np.random.default_rng(B * T + nIh + cI)
+    nb = T // m
+    r = lambda *s: torch.tensor(rng.standard_normal(s))  # noqa: E731
+    K, Z, q, w, Bp = r(B, T, cI), r(B, T, cI), r(B, T, nIh, cI), r(B, T, nIh), 0.3 * r(m, cI)
+    idx = torch.tensor(_selection(rng, B, T, m, topk, hole=T // 2))
+    slot = r(B, T, topk)
+    leaves = [x.clone().requires_grad_(True) for x in (K, Z, q, w, Bp)]
+    Kl, Zl, ql, wl, Bl = leaves
+    kn = (torch.softmax(Zl.view(B, nb, m, cI) + Bl, 2) * Kl.view(B, nb, m, cI)).sum(2)
+    qn = ql
+    if norm:
+        kn, qn = F.normalize(kn, dim=-1), F.normalize(ql, dim=-1)
+    a = torch.einsum('bthd,bnd->bthn', qn, kn) * (1.0 if norm else cI ** -0.5)
+    lg = (torch.relu(a) * wl[..., None]).sum(2)
+    seen = (torch.arange(T)[:, None] + 1) // m > torch.arange(nb)
+    none = ~seen.any(-1, keepdim=True)
+    soft = torch.softmax(lg.masked_fill(~seen, -np.inf).masked_fill(none, 0.0), -1)
+    sel = soft.gather(-1, idx.long().clamp(min=0))
+    ref = torch.autograd.grad((sel * slot * (idx >= 0)).sum(), leaves)
+    f = lambda x: x.to(dev, torch.float32)  # noqa: E731
+    got = kch.ops_csa._ste_indexer_grads(f(K), f(Z), f(q), f(w), f(Bp), idx.to(dev), f(slot),
+                                         m=m, normalize_qk=norm)
+    torch.cuda.synchronize()
+    for name, g, x in zip(("K_idx", "Z_idx", "q_idx", "w_idx", "B_idx"), got, ref):
+        _check(name, g.cpu().numpy(), x.numpy())
