@@ -228,7 +228,9 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
  * nothing); dBap, dBbp [B,T/m,m,c]; sink_part as for HCA; slot_grad
  * [B,T,topk] (zeroed by the caller): the gradient of each selected row dotted
  * with that row, which the STE surrogate (ops_csa.py:1033-1099) turns into
- * the indexer's gradient; gsum [B,T,c] or NULL: the sum over the selected
+ * the indexer's gradient, or NULL; dsel [B,T,T/m] or NULL (normalize = 1,
+ * nh <= 16): the same values at their blocks, 0 at the others (the dsel of
+ * kch_csa_ste_bwd), added to what it holds with dsel_add; gsum [B,T,c] or NULL: the sum over the selected
  * slots of the selected rows' gradients (written), which the full-softmax
  * surrogate's dense term (ops_csa.py:1050-1071) consumes. The window rows'
  * gradient is added into dCa.
@@ -239,9 +241,9 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
                      const float* Cb, const float* Za, const float* Zb, const float* Ba,
                      const float* Bb, const float* sink, void* dq, float* dCa, float* dCb,
                      float* dZa, float* dZb, float* dBap, float* dBbp, float* sink_part,
-                     float* slot_grad, float* gsum, int B, int T, int nh, int c, int m, int topk,
-                     int win, float scale, int normalize, int qdt, void* ws, size_t ws_bytes,
-                     void* stream);
+                     float* slot_grad, float* dsel, int dsel_add, float* gsum, int B, int T, int nh,
+                     int c, int m, int topk, int win, float scale, int normalize, int qdt, void* ws,
+                     size_t ws_bytes, void* stream);
 
 /*
  * The STE surrogate's backward for the CSA indexer (ops_csa.py:1033-1099,

@@ -459,9 +459,9 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
                      const float* Cb, const float* Za, const float* Zb, const float* Ba,
                      const float* Bb, const float* sink, void* dq, float* dCa, float* dCb,
                      float* dZa, float* dZb, float* dBap, float* dBbp, float* sink_part,
-                     float* slot_grad, float* gsum, int B, int T, int nh, int c, int m, int topk,
-                     int win, float scale, int normalize, int qdt, void* ws, size_t ws_bytes,
-                     void* stream) {
+                     float* slot_grad, float* dsel, int dsel_add, float* gsum, int B, int T, int nh,
+                     int c, int m, int topk, int win, float scale, int normalize, int qdt, void* ws,
+                     size_t ws_bytes, void* stream) {
   const char* fn = "kch_csa_attn_bwd";
   if (qdt < 0 || qdt > 2) return fail(KCH_ERR_INVALID, "%s: dtype %d (0 fp32, 1 bf16, 2 fp16)", fn, qdt);
   if (qdt != 0 && (nh > 16 || !normalize))
@@ -477,6 +477,8 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
     return fail(KCH_ERR_UNSUPPORTED, "%s: T=%d rows of a batch row exceed 2 GiB (32-bit row offsets)", fn, T);
   if (nh * (c / 8) > 256)
     return fail(KCH_ERR_UNSUPPORTED, "%s: nh=%d heads of %d exceed one workgroup", fn, nh, c);
+  if (dsel && (nh > 16 || !normalize))
+    return fail(KCH_ERR_UNSUPPORTED, "%s: dsel needs normalize=1 and at most 16 heads a call (nh=%d)", fn, nh);
   if (std::isnan(scale)) return fail(KCH_ERR_INVALID, "%s: scale is NaN", fn);
   if ((long long)B * T * nh * c >= (1LL << 40) || (long long)B * T * topk >= (1LL << 40))
     return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
@@ -503,6 +505,8 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   p.topk = topk;
   p.sparse = 1;
   p.slot_grad = topk > 0 ? slot_grad : nullptr;
+  p.dsel = topk > 0 ? dsel : nullptr;
+  p.dsel_add = dsel && dsel_add ? 1 : 0;
   p.gsum = gsum;
   p.normalize = normalize ? 1 : 0;
   p.qdt = qdt;

@@ -6,29 +6,48 @@
 //   s = scale qn.k,  p = exp(s - lse),  dp = dout.k,  D = sum p dp,
 //   ds = p (dp - D),  dqn = scale sum ds k,  dk += scale ds qn + p dout.
 //
-// Every product is a two-part bf16 split x = hi + lo (2^-16 relative) with
-// three MFMAs, hi*hi + hi*lo + lo*hi, accumulated in fp32; the split rows
-// (queries, dout, keys) are written once by split_rows_kernel.
+// Every operand that is not bf16 already is a two-part bf16 split x = hi + lo
+// (2^-16 relative); a product takes the MFMAs hi*hi + hi*lo + lo*hi of the
+// parts that exist, accumulated in fp32. Queries and dout enter as they are
+// given, with 1/|q| applied to the scores in fp32 (and to ds for dk): bf16
+// ones are exact in one part, so a product with a split key takes two MFMAs
+// and no split copy of them is ever written; fp16 / fp32 ones are split while
+// they are staged. The compressed and window rows are split once by
+// split_rows_kernel.
 //
-// attn_bwd_q_kernel  one wave per query (4 per workgroup), all 16 heads as the
-//   MFMA columns (MQA: every key row is shared by the heads). The query's keys
-//   (selected or causal blocks, then window rows) are gathered 32 rows a step
-//   into the wave's LDS stage (hi and lo tiles, swizzled as the forward's):
-//   S^T = K Qn^T and dP^T = K dout^T per 16 rows. Pass 1: lse and D with a
-//   running maximum; pass 2: ds, and dqn^T += K^T ds^T (K^T fragments from the
-//   transposing LDS read, ds^T from the accumulators, as the forward's
-//   O^T = V^T P^T). Writes dq (after the L2-norm backward), lse, D, and for
-//   CSA each selected slot's gradient dotted with its row and their sum gsum.
-// attn_bwd_k_kernel  one workgroup per 64 key rows (16 per wave) and chunk of
-//   queries, key fragments held in registers; queries are taken in pairs: the
-//   pair's qn and dout rows (32 rows of (query, head)) are staged in LDS once
-//   for the four waves (double-buffered), S = Qn K^T and dP = dout K^T per
-//   query, then dk += ds^T Qn + p^T dout with (query, head) as the
+// attn_bwd_qt_kernel  a workgroup of 4 waves and 8 (bf16) or 4 consecutive
+//   queries, all 16 heads as the MFMA columns (MQA: every key row is shared by
+//   the heads). The queries' key rows (every visible block, masked by the
+//   selection bitmap for CSA, then the window rows) are staged in LDS 32 rows
+//   a step, once for the workgroup, double-buffered, and each K fragment read
+//   serves the wave's two queries: S^T = K Q^T and dP^T = K dout^T per 16
+//   rows. Pass 1: lse and D with a running maximum per lane; pass 2: ds, and
+//   dqn^T += K^T ds^T (K^T fragments from the transposing LDS read, ds^T from
+//   the accumulators, as the forward's O^T = V^T P^T). Writes dq (after the
+//   L2-norm backward), 1/|q|, lse, D, and for CSA each selected block's
+//   gradient dotted with its row (dense, dsel) and their sum gsum.
+// attn_bwd_q_kernel   CSA over long contexts: one wave per query gathers only
+//   the selected rows, 32 a step, into its own LDS stage. Its bound is the L2
+//   gather of 512 bytes a row and pass (8.5 TB/s measured), the tile kernel's
+//   the matrix cores; see attn_bwd_dense_rows for where the line lies.
+// attn_bwd_k_kernel   one workgroup per 64 KG key rows (16 KG per wave, KG 1 or
+//   2, key fragments in registers) and chunk of queries; queries are taken in
+//   pairs: the pair's q and dout rows (32 rows of (query, head)) are staged in
+//   LDS once for the four waves (double-buffered), S = Q K^T and dP = dout K^T
+//   per query, then dk += ds^T Q + p^T dout with (query, head) as the
 //   contraction (the accumulators of the two queries' S are the A operand in
-//   the packed order of the transposing read of Qn / dout). Writes per-chunk
-//   partials of the compressed rows and the window rows' gradient.
+//   the packed order of the transposing read of Q / dout). Every fragment read
+//   serves KG groups of 16 keys. Writes per-chunk partials of the compressed
+//   rows and of the window rows; the chunk length follows the grid size.
 // The L2-norm and compression backwards are hca_backward.hip's block and
 // window kernels on these partials (mfma_parts).
+//
+// Measured, 16 heads of 128, window 128, bf16, against one wave per query with
+// its own copy of every row and 16 keys per wave on three-MFMA products: HCA
+// B2 T8192 (64 blocks) query pass 254 -> 211 us, window keys 233 -> 150,
+// compressed keys 625 (32 workgroups) -> 61, splits of q and dout 68 -> 0; CSA
+// B2 T4096 top-512 (1024 blocks) query pass 565 -> 349, compressed keys 677 ->
+// 247, window keys 197 -> 114.
 
 #include "attn_common.h"
 #include "kch_csa.h"
@@ -38,8 +57,7 @@ namespace kch {
 
 namespace {
 
-constexpr int KQC = 512;  // queries per chunk of the key pass (compressed rows)
-constexpr int KTR = 64;   // key rows per key-pass workgroup
+constexpr float kLn2F = 0.6931471805599453f;
 
 __device__ __forceinline__ bf16_t lo_of(float x) { return (bf16_t)(x - (float)(bf16_t)x); }
 
@@ -145,21 +163,395 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
+// Eight stored values of a query or dout row as bf16 parts: one (exact) for
+// bf16, hi + lo for fp16 and fp32.
+template <typename QT>
+struct Parts {
+  static constexpr bool one = std::is_same<QT, bf16_t>::value;
+};
+template <typename QT>
+__device__ __forceinline__ void load_parts(const QT* p, bool ok, bf16x8& h, bf16x8& l, float& ss) {
+  float v[8];
+  if (ok) {
+    Load8<QT>::run(p, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    ss += v[i] * v[i];
+    h[i] = (bf16_t)v[i];
+    if constexpr (!Parts<QT>::one) l[i] = lo_of(v[i]);
+  }
+}
+// acc + k * x, k split (kh, kl), x in one part (exact) or two
+template <bool ONE>
+__device__ __forceinline__ f32x4 mma_kx(const bf16x8& kh, const bf16x8& kl, const bf16x8& xh, const bf16x8& xl,
+                                        f32x4 acc) {
+  if constexpr (ONE) return mfma2a(kh, kl, xh, acc);
+  else return mfma3(kh, kl, xh, xl, acc);
+}
+// acc + x * k
+template <bool ONE>
+__device__ __forceinline__ f32x4 mma_xk(const bf16x8& xh, const bf16x8& xl, const bf16x8& kh, const bf16x8& kl,
+                                        f32x4 acc) {
+  if constexpr (ONE) return mfma2b(xh, kh, kl, acc);
+  else return mfma3(xh, xl, kh, kl, acc);
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 template <int HD>
 struct QWave {
   static constexpr int NS = HD / 32, NT = HD / 16;
   static constexpr int TPR = HD / 8, RPI = 64 / TPR, NLI = 32 / RPI;
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   struct Rows {
     u32x4 h[NLI], l[NLI];
   };
 };
 
-// ---------------------------------------------------------------- query pass
-// DL0: dout is exactly bf16 (bf16 input; its split's low part is zero), so
-// the products with it take two MFMAs instead of three.
-template <int HD, bool SPARSE, bool DL0>
+// The end of a query's pass: the L2-norm backward of qn and the stores of dq,
+// lse, D, 1/|q| and the sink term (lane: head n, dims 16 tt + 4 q + e).
+template <int HD>
+__device__ __forceinline__ void finish_query(const HcaBwdParams& p, size_t bt, int n, int q, f32x4 (&dq)[HD / 16],
+                                             float rq, float lse2, float D, float sk2) {
+  constexpr int NT = HD / 16;
+  float qv[NT][4];
+  float yd = 0.f;
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (n < p.nh) x = load4(p.q, (bt * p.nh + n) * HD + 16 * tt + 4 * q, p.qdt);
+    qv[tt][0] = x.x * rq; qv[tt][1] = x.y * rq; qv[tt][2] = x.z * rq; qv[tt][3] = x.w * rq;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) yd += qv[tt][e] * dq[tt][e];
+  }
+  yd = colq_sum(yd);
+  if (n < p.nh) {
+    // rq = 1 / max(|q|, eps): for |q| <= eps the norm is the constant eps
+    const bool big = rq < 1e12f;
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (big ? dq[tt][e] - qv[tt][e] * yd : dq[tt][e]) * rq;
+      store4(p.dq, (bt * p.nh + n) * HD + 16 * tt + 4 * q, make_float4(o[0], o[1], o[2], o[3]), p.qdt);
+    }
+  }
+  if (q == 0) {
+    p.lse[bt * 16 + n] = lse2;
+    p.dval[bt * 16 + n] = D;
+    p.rq[bt * 16 + n] = n < p.nh ? rq : 0.f;
+    if (p.sink_part && n < p.nh) p.sink_part[bt * p.nh + n] = p.sink ? fast_exp2(sk2 - lse2) * D : 0.f;
+  }
+}
+
+// gsum = sum over the heads of dssel qn + psel dout (dims 32 s + 8 q + i). The
+// rows are read again: kept as fp32 across the passes they spill.
+template <int HD, typename QT>
+__device__ __forceinline__ void store_gsum(const HcaBwdParams& p, size_t bt, int n, int q, float psel, float dssel,
+                                           float rq) {
+  psel = colq_sum(psel);
+  dssel = colq_sum(dssel) * rq;
+  const bool ok = n < p.nh;
+  const size_t ro = ok ? (bt * p.nh + n) * HD + 8 * q : 0;
+#pragma unroll
+  for (int s = 0; s < HD / 32; ++s) {
+    float qv[8], dv[8], gv[8];
+    Load8<QT>::run(static_cast<const QT*>(p.q) + ro + 32 * s, qv);
+    Load8<QT>::run(static_cast<const QT*>(p.dout) + ro + 32 * s, dv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) gv[i] = row16_sum(ok ? dssel * qv[i] + psel * dv[i] : 0.f);
+    if (n == 0) {
+      float* dst = p.gsum + bt * HD + 32 * s + 8 * q;
+      *reinterpret_cast<float4*>(dst) = make_float4(gv[0], gv[1], gv[2], gv[3]);
+      *reinterpret_cast<float4*>(dst + 4) = make_float4(gv[4], gv[5], gv[6], gv[7]);
+    }
+  }
+}
+
+// lse (log2 units) and D of a head from its four lanes' running m, l, ad and the sink
+struct Soft {
+  float lse2, D, sk2;
+};
+__device__ __forceinline__ Soft close_softmax(const HcaBwdParams& p, int n, float m, float l, float ad) {
+  const float mx = colq_max(m);
+  const float f = m > -INFINITY ? fast_exp2(m - mx) : 0.f;
+  l = colq_sum(l * f);
+  ad = colq_sum(ad * f);
+  m = mx;
+  Soft r;
+  r.sk2 = -INFINITY;
+  if (p.sink && n < p.nh) r.sk2 = p.sink[n] * kLog2eF;
+  if (r.sk2 > -INFINITY) {
+    const float mn = fmaxf(m, r.sk2);
+    const float a = fast_exp2(m - mn);
+    l = l * a + fast_exp2(r.sk2 - mn);
+    ad *= a;
+    m = mn;
+  }
+  const bool live = n < p.nh && l > 0.f;
+  r.lse2 = live ? m + __log2f(l) : INFINITY;
+  r.D = live ? ad / l : 0.f;
+  return r;
+}
+// one step of eight scores (log2 units, -inf: masked) and dp into m, l, ad
+__device__ __forceinline__ void soft_step(const float (&s8)[8], const float (&d8)[8], float& m, float& l, float& ad) {
+  float mx = s8[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s8[e]);
+  if (mx > m) {
+    const float a = fast_exp2(m - mx);  // m = -inf: a = 0
+    l *= a;
+    ad *= a;
+    m = mx;
+  }
+  if (m > -INFINITY) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float pe = fast_exp2(s8[e] - m);  // masked: 0
+      l += pe;
+      ad += pe * d8[e];
+    }
+  }
+}
+
+// --------------------------------------------------- query pass, rows in tiles
+template <int HD, typename QT, bool SEL>
+__global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int ntile) {
+  constexpr bool ONE = Parts<QT>::one;
+  constexpr int QW = ONE ? 2 : 1;             // queries per wave
+  constexpr int NS = HD / 32, NT = HD / 16;
+  constexpr int TILE = 32 * HD, CPR = HD / 8;
+  constexpr int LPT = 2 * TILE / 8 / 256;     // 16-byte pieces per thread per step
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2][2 * TILE];  // hi, lo
+  const int tid = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, q = lane >> 4, n = lane & 15;
+  // the latest queries see the most blocks: they start first
+  const int b = blockIdx.x % p.B;
+  const int t0 = (ntile - 1 - (int)(blockIdx.x / p.B)) * 4 * QW;
+  const int tlast = min(t0 + 4 * QW, p.T) - 1;
+  const int t1 = t0 + wv * QW;                // this wave's queries t1 .. t1 + QW - 1
+  const TileOffsets<HD> to;
+
+  // B operands: q and dout of head n, dims 32s + 8q .. (16 heads, padded rows zero)
+  bf16x8 qh[QW][NS], ql[QW][ONE ? 1 : NS], dh[QW][NS], dl[QW][ONE ? 1 : NS];
+  float rq[QW], scq[QW];
+  int nv[QW];
+#pragma unroll
+  for (int i = 0; i < QW; ++i) {
+    const bool ok = t1 + i < p.T && n < p.nh;
+    const size_t ro = ok ? (((size_t)b * p.T + t1 + i) * p.nh + n) * HD + 8 * q : 0;
+    float ss = 0.f, unused = 0.f;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      load_parts<QT>(static_cast<const QT*>(p.q) + ro + 32 * s, ok, qh[i][s], ql[i][ONE ? 0 : s], ss);
+      load_parts<QT>(static_cast<const QT*>(p.dout) + ro + 32 * s, ok, dh[i][s], dl[i][ONE ? 0 : s], unused);
+    }
+    rq[i] = l2_inv(colq_sum(ss));
+    scq[i] = rq[i] * p.scale * kLog2eF;  // raw score -> log2 units
+    nv[i] = min((t1 + i + 1) / p.m2, p.nb);
+  }
+  const int nvm = SEL && p.topk == 0 ? 0 : min((tlast + 1) / p.m2, p.nb);
+  const int nsc = (nvm + 31) / 32;
+  // window steps start at whole 32-row groups: the rows summed together, and so
+  // the bits, do not depend on how many queries share the workgroup
+  const int w0 = max(0, t0 - p.win + 1) & ~31;
+  const int nwin = p.win > 0 ? tlast - w0 + 1 : 0;
+  const int nsteps = nsc + (nwin + 31) / 32;
+  const int nw = (p.nb + 31) / 32;
+
+  // the 32 rows of step m (hi and lo planes; rows past the end read as zeros)
+  auto fetch = [&](int m, u32x4 (&v)[LPT]) {
+    const bool comp = m < nsc;
+    const int r0 = comp ? 32 * m : 32 * (m - nsc);
+    const int lim = comp ? nvm : nwin;
+    const size_t base = comp ? (size_t)b * p.nb : (size_t)b * p.T + w0;
+    const bf16_t* hi = comp ? p.kc_hi : p.kl_hi;
+    const bf16_t* lo = comp ? p.kc_lo : p.kl_lo;
+#pragma unroll
+    for (int k = 0; k < LPT; ++k) {
+      const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
+      const bf16_t* src = pc < 32 * CPR ? hi : lo;
+      v[k] = u32x4{0, 0, 0, 0};
+      if (r0 + row < lim) v[k] = *reinterpret_cast<const u32x4*>(src + (base + r0 + row) * HD + 8 * c);
+    }
+  };
+  auto put = [&](bf16_t* buf, const u32x4 (&v)[LPT]) {
+#pragma unroll
+    for (int k = 0; k < LPT; ++k) {
+      const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
+      *reinterpret_cast<u32x4*>(buf + (pc / (32 * CPR)) * TILE + row * HD + 8 * (c ^ tile_swz<HD>(row & 15))) = v[k];
+    }
+  };
+  // the selection's word of step m (uniform per query)
+  auto load_word = [&](int m, uint32_t (&w)[QW]) {
+#pragma unroll
+    for (int i = 0; i < QW; ++i)
+      w[i] = m < nsc && t1 + i < p.T ? p.sel[((size_t)b * p.T + t1 + i) * nw + m] : 0u;
+  };
+  // S^T (log2 units, masked) and dP^T of the staged rows: keys 4q+e, 16+4q+e of head n
+  auto scores = [&](int m, const bf16_t* kt, const uint32_t (&sw)[QW], float (&s8)[QW][8], float (&d8)[QW][8]) {
+    const bool comp = m < nsc;
+    const int r0 = comp ? 32 * m : 32 * (m - nsc);
+    const int lim = comp ? nvm : nwin;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      f32x4 sa[QW], da[QW];
+#pragma unroll
+      for (int i = 0; i < QW; ++i) sa[i] = da[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // (rows past the last query's, or before the first query's window)
+      if (r0 + 16 * half < lim && (comp || w0 + r0 + 16 * half + 15 > t0 - p.win)) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const bf16x8 kh = *reinterpret_cast<const bf16x8*>(kt + 16 * HD * half + to.key(s));
+          const bf16x8 kl = *reinterpret_cast<const bf16x8*>(kt + TILE + 16 * HD * half + to.key(s));
+#pragma unroll
+          for (int i = 0; i < QW; ++i) {
+            sa[i] = mma_kx<ONE>(kh, kl, qh[i][s], ql[i][ONE ? 0 : s], sa[i]);
+            da[i] = mma_kx<ONE>(kh, kl, dh[i][s], dl[i][ONE ? 0 : s], da[i]);
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < QW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = r0 + 16 * half + 4 * q + e;
+          bool ok;
+          if (comp) ok = SEL ? (sw[i] >> (16 * half + 4 * q + e)) & 1u : j < nv[i];
+          else ok = (w0 + j <= t1 + i) & (w0 + j > t1 + i - p.win);
+          s8[i][4 * half + e] = ok ? sa[i][e] * scq[i] : -INFINITY;
+          d8[i][4 * half + e] = da[i][e];
+        }
+    }
+  };
+
+  u32x4 pv[LPT];
+  uint32_t sw[QW] = {}, swn[QW] = {};
+  float m_[QW], l_[QW], ad_[QW];
+#pragma unroll
+  for (int i = 0; i < QW; ++i) {
+    m_[i] = -INFINITY;
+    l_[i] = ad_[i] = 0.f;
+  }
+  // ---- pass 1: lse and D ----
+  if (nsteps > 0) {
+    fetch(0, pv);
+    if constexpr (SEL) load_word(0, swn);
+  }
+  for (int m = 0; m < nsteps; ++m) {
+    bf16_t* kt = lds[m & 1];
+    put(kt, pv);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < QW; ++i) sw[i] = swn[i];
+    if (m + 1 < nsteps) {
+      fetch(m + 1, pv);
+      if constexpr (SEL) load_word(m + 1, swn);
+    }
+    float s8[QW][8], d8[QW][8];
+    scores(m, kt, sw, s8, d8);
+#pragma unroll
+    for (int i = 0; i < QW; ++i) soft_step(s8[i], d8[i], m_[i], l_[i], ad_[i]);
+  }
+  Soft sf[QW];
+#pragma unroll
+  for (int i = 0; i < QW; ++i) sf[i] = close_softmax(p, n, m_[i], l_[i], ad_[i]);
+
+  // ---- pass 2: ds, dqn^T += K^T ds^T, the selected rows' terms ----
+  f32x4 dq[QW][NT];
+#pragma unroll
+  for (int i = 0; i < QW; ++i)
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) dq[i][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float psel[QW] = {}, dssel[QW] = {};  // sums over the selected rows (gsum)
+  if (nsteps > 0) {
+    fetch(0, pv);
+    if constexpr (SEL) load_word(0, swn);
+    __syncthreads();  // pass 1's last reads are done
+  }
+  for (int m = 0; m < nsteps; ++m) {
+    bf16_t* kt = lds[m & 1];
+    put(kt, pv);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < QW; ++i) sw[i] = swn[i];
+    if (m + 1 < nsteps) {
+      fetch(m + 1, pv);
+      if constexpr (SEL) load_word(m + 1, swn);
+    }
+    float s8[QW][8], d8[QW][8];
+    scores(m, kt, sw, s8, d8);
+    bf16x8 bh[QW], bl[QW];
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      float pe[8], dse[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        pe[e] = fast_exp2(s8[i][e] - sf[i].lse2);  // masked or dead head: 0
+        dse[e] = pe[e] * (d8[i][e] - sf[i].D) * p.scale;
+        bh[i][e] = (bf16_t)dse[e];
+        bl[i][e] = lo_of(dse[e]);
+      }
+      if constexpr (SEL) {
+        if (m < nsc && (p.dsel || p.gsum)) {
+          // sum over the heads of p ((dp - D) s + dp): the row's gradient dotted with the row
+          float g[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float sraw = s8[i][e] > -INFINITY ? s8[i][e] * kLn2F : 0.f;  // scale qn.k
+            g[e] = row16_sum(pe[e] * ((d8[i][e] - sf[i].D) * sraw + d8[i][e]));
+            psel[i] += pe[e];
+            dssel[i] += dse[e];
+          }
+          if (p.dsel && n == 0 && t1 + i < p.T) {
+            float* dst = p.dsel + ((size_t)b * p.T + t1 + i) * p.nb;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+              const int j = 32 * m + 16 * half + 4 * q;
+              // (added: calls for further groups of heads add theirs)
+              if ((p.nb & 3) == 0 && !p.dsel_add) {
+                if (j < p.nb) *reinterpret_cast<float4*>(dst + j) =
+                    make_float4(g[4 * half], g[4 * half + 1], g[4 * half + 2], g[4 * half + 3]);
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if (j + e < p.nb) dst[j + e] = g[4 * half + e] + (p.dsel_add ? dst[j + e] : 0.f);
+              }
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+      const bf16x8 vh = MqaWave<HD>::vt_frag(kt, to, tt);
+      const bf16x8 vl = MqaWave<HD>::vt_frag(kt + TILE, to, tt);
+#pragma unroll
+      for (int i = 0; i < QW; ++i) dq[i][tt] = mfma3(vh, vl, bh[i], bl[i], dq[i][tt]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < QW; ++i) {
+    if (t1 + i >= p.T) break;  // whole waves
+    const size_t bt = (size_t)b * p.T + t1 + i;
+    finish_query<HD>(p, bt, n, q, dq[i], rq[i], sf[i].lse2, sf[i].D, sf[i].sk2);
+    if constexpr (SEL) {
+      if (p.gsum) store_gsum<HD, QT>(p, bt, n, q, psel[i], dssel[i], rq[i]);
+      // the blocks that no query of the workgroup sees
+      if (p.dsel && !p.dsel_add)
+        for (int j = 32 * nsc + lane; j < p.nb; j += 64) p.dsel[bt * p.nb + j] = 0.f;
+    }
+  }
+}
+
+// -------------------------------------------- query pass, selected rows gathered
+template <int HD, typename QT>
 __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
+  constexpr bool ONE = Parts<QT>::one;
   using W = QWave<HD>;
   constexpr int NS = W::NS, NT = W::NT, TPR = W::TPR, RPI = W::RPI, NLI = W::NLI;
   constexpr int TILE = 32 * HD;  // bf16 per 32-row tile
@@ -175,19 +567,21 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
   const size_t bt = (size_t)b * p.T + t;
   const TileOffsets<HD> to;
 
-  // B operands: qn and dout of head n, dims 32s + 8q .. (16 heads, padded rows zero)
+  // B operands: q and dout of head n, dims 32s + 8q .. (16 heads, padded rows zero)
   bf16x8 qh[NS], ql[NS], dh[NS], dl[NS];
+  float ss = 0.f;
   {
-    const size_t ro = (bt * 16 + n) * HD + 8 * q;
+    const bool ok = n < p.nh;
+    const size_t ro = ok ? (bt * p.nh + n) * HD + 8 * q : 0;
+    float unused = 0.f;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      qh[s] = *reinterpret_cast<const bf16x8*>(p.qs_hi + ro + 32 * s);
-      ql[s] = *reinterpret_cast<const bf16x8*>(p.qs_lo + ro + 32 * s);
-      dh[s] = *reinterpret_cast<const bf16x8*>(p.ds_hi + ro + 32 * s);
-      dl[s] = DL0 ? bf16x8{} : *reinterpret_cast<const bf16x8*>(p.ds_lo + ro + 32 * s);
+      load_parts<QT>(static_cast<const QT*>(p.q) + ro + 32 * s, ok, qh[s], ql[s], ss);
+      load_parts<QT>(static_cast<const QT*>(p.dout) + ro + 32 * s, ok, dh[s], dl[s], unused);
     }
   }
-  const int nsel = SPARSE ? p.topk : min((t + 1) / p.m2, p.nb);
+  const float rq = l2_inv(colq_sum(ss));
+  const int nsel = p.topk;
   const int i0 = p.win > 0 ? max(0, p.win - 1 - t) : 0;
   const int nwin = p.win > 0 ? p.win - i0 : 0;
   const int wpos0 = t - p.win + 1 + i0;
@@ -213,11 +607,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
   const __amdgpu_buffer_rsrc_t rs_cl = rsrc(p.kc_lo + (size_t)b * p.nb * HD, cbytes);
   const __amdgpu_buffer_rsrc_t rs_wh = rsrc(nwin > 0 ? p.kl_hi + (size_t)b * p.T * HD : p.kc_hi, wbytes);
   const __amdgpu_buffer_rsrc_t rs_wl = rsrc(nwin > 0 ? p.kl_lo + (size_t)b * p.T * HD : p.kc_lo, wbytes);
-  const bool has_idx = SPARSE && nsel > 0;
+  const bool has_idx = nsel > 0;
   const __amdgpu_buffer_rsrc_t rs_idx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int*>(has_idx ? p.idx + bt * p.topk : nullptr), 0, has_idx ? nsel * 4 : 0, 0x00020000);
   const bool idx16 = (nsel & 3) == 0;  // 16-byte index loads never straddle the end
-  const float sc = p.scale * kLog2eF;  // raw score -> log2 units
+  const float sc = rq * p.scale * kLog2eF;  // raw score -> log2 units
 
   // the row indices of step m: selected or causal block, or window position
   struct Sel {
@@ -226,24 +620,19 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
   auto load_sel = [&](int m, Sel& sl) {
     const int j0 = 32 * m;
     if (__builtin_amdgcn_readfirstlane(j0 < nsel_pad ? 1 : 0)) {
-      if (SPARSE) {
-        if (idx16) {
-          typedef int i32x4 __attribute__((ext_vector_type(4)));
-          const i32x4 x = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_idx, (j0 + 4 * q) * 4, 0, 0));
-          const i32x4 y = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_idx, (j0 + 16 + 4 * q) * 4, 0, 0));
+      if (idx16) {
+        typedef int i32x4 __attribute__((ext_vector_type(4)));
+        const i32x4 x = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_idx, (j0 + 4 * q) * 4, 0, 0));
+        const i32x4 y = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_idx, (j0 + 16 + 4 * q) * 4, 0, 0));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sl.v[e] = x[e];
-            sl.v[4 + e] = y[e];
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < 8; ++k)
-            sl.v[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_idx, (j0 + MW::row_sl(k, q)) * 4, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+          sl.v[e] = x[e];
+          sl.v[4 + e] = y[e];
         }
       } else {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) sl.v[k] = j0 + MW::row_sl(k, q);
+        for (int k = 0; k < 8; ++k)
+          sl.v[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs_idx, (j0 + MW::row_sl(k, q)) * 4, 0, 0);
       }
     } else {
 #pragma unroll
@@ -278,8 +667,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
     for (int i = 0; i < NLI; ++i) {
       const int r = MW::row_sl(MW::slot_sl(i), q), c = lane % TPR;
       const int off = r * HD + 8 * (c ^ tile_swz<HD>(r & 15));
-      *reinterpret_cast<typename W::u32x4*>(sth + off) = rr.h[i];
-      *reinterpret_cast<typename W::u32x4*>(stl + off) = rr.l[i];
+      *reinterpret_cast<u32x4*>(sth + off) = rr.h[i];
+      *reinterpret_cast<u32x4*>(stl + off) = rr.l[i];
     }
     wave_lds_sync();
   };
@@ -292,8 +681,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
       for (int s = 0; s < NS; ++s) {
         const bf16x8 kh = *reinterpret_cast<const bf16x8*>(sth + 16 * HD * half + to.key(s));
         const bf16x8 kl = *reinterpret_cast<const bf16x8*>(stl + 16 * HD * half + to.key(s));
-        sa = mfma3(kh, kl, qh[s], ql[s], sa);
-        da = DL0 ? mfma2a(kh, kl, dh[s], da) : mfma3(kh, kl, dh[s], dl[s], da);
+        sa = mma_kx<ONE>(kh, kl, qh[s], ql[s], sa);
+        da = mma_kx<ONE>(kh, kl, dh[s], dl[s], da);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -325,40 +714,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
       }
       float s8[8], d8[8];
       scores(ok, s8, d8);
-      float mx = s8[0];
-#pragma unroll
-      for (int e = 1; e < 8; ++e) mx = fmaxf(mx, s8[e]);
-      const float mn = fmaxf(m, colq_max(mx));
-      if (mn > m) {
-        const float a = fast_exp2(m - mn);  // m = -inf: a = 0
-        l *= a;
-        ad *= a;
-        m = mn;
-      }
-      if (m > -INFINITY) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float pe = fast_exp2(s8[e] - m);  // masked: 0
-          l += pe;
-          ad += pe * d8[e];
-        }
-      }
+      soft_step(s8, d8, m, l, ad);
     }
   }
-  l = colq_sum(l);
-  ad = colq_sum(ad);
-  float sk2 = -INFINITY;
-  if (p.sink && n < p.nh) sk2 = p.sink[n] * kLog2eF;
-  if (sk2 > -INFINITY) {
-    const float mn = fmaxf(m, sk2);
-    const float a = fast_exp2(m - mn);
-    l = l * a + fast_exp2(sk2 - mn);
-    ad *= a;
-    m = mn;
-  }
-  const bool live = n < p.nh && l > 0.f;
-  const float lse2 = live ? m + __log2f(l) : INFINITY;
-  const float D = live ? ad / l : 0.f;
+  const Soft sf = close_softmax(p, n, m, l, ad);
+  const float lse2 = sf.lse2, D = sf.D;
 
   // ---- pass 2: ds, dqn^T += K^T ds^T, the slot terms ----
   f32x4 dq[NT];
@@ -400,238 +760,275 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
         const bf16x8 vl = MqaWave<HD>::vt_frag(stl, to, tt);
         dq[tt] = mfma3(vh, vl, bh, bl, dq[tt]);
       }
-      if constexpr (SPARSE) {
-        // the selected rows: sum over the heads of p ((dp - D) s + dp) (the row's
-        // gradient dotted with the row) per slot, and this head's p and ds sums
+      // the selected rows: sum over the heads of p ((dp - D) s + dp) (the row's
+      // gradient dotted with the row) per slot, and this head's p and ds sums
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int j = 32 * st + 16 * (e >> 2) + 4 * q + (e & 3);
-          const bool selk = j < nsel;
-          const float sraw = s8[e] > -INFINITY ? s8[e] / kLog2eF : 0.f;  // scale qn.k
-          float g = selk ? pe[e] * ((d8[e] - D) * sraw + d8[e]) : 0.f;
-          g = row16_sum(g);
-          if (selk) {
-            psel += pe[e];
-            dssel += dse[e];
-          }
-          // (added: calls for further groups of heads add theirs; one wave owns the slot)
-          if (n == 0 && selk && p.slot_grad) p.slot_grad[bt * p.topk + j] += g;
+      for (int e = 0; e < 8; ++e) {
+        const int j = 32 * st + 16 * (e >> 2) + 4 * q + (e & 3);
+        const bool selk = j < nsel;
+        const float sraw = s8[e] > -INFINITY ? s8[e] * kLn2F : 0.f;  // scale qn.k
+        float g = selk ? pe[e] * ((d8[e] - D) * sraw + d8[e]) : 0.f;
+        g = row16_sum(g);
+        if (selk) {
+          psel += pe[e];
+          dssel += dse[e];
         }
+        if (n == 0 && selk && p.slot_ws) p.slot_ws[bt * p.topk + j] = g;
       }
     }
   }
-
-  // ---- dq: the L2-norm backward of qn (lane: head n, dims 16 tt + 4q + e) ----
-  {
-    const float rq = p.rq[bt * 16 + n];
-    float qv[NT][4];
-    float yd = 0.f;
-#pragma unroll
-    for (int tt = 0; tt < NT; ++tt) {
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (n < p.nh) x = load4(p.q, (bt * p.nh + n) * HD + 16 * tt + 4 * q, p.qdt);
-      qv[tt][0] = x.x * rq; qv[tt][1] = x.y * rq; qv[tt][2] = x.z * rq; qv[tt][3] = x.w * rq;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) yd += qv[tt][e] * dq[tt][e];
-    }
-    yd = colq_sum(yd);
-    if (n < p.nh) {
-      // rq = 1 / max(|q|, eps): for |q| <= eps the norm is the constant eps
-      const bool big = rq < 1e12f;
-#pragma unroll
-      for (int tt = 0; tt < NT; ++tt) {
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (big ? dq[tt][e] - qv[tt][e] * yd : dq[tt][e]) * rq;
-        store4(p.dq, (bt * p.nh + n) * HD + 16 * tt + 4 * q, make_float4(o[0], o[1], o[2], o[3]), p.qdt);
-      }
-    }
-    if (q == 0) {
-      p.lse[bt * 16 + n] = lse2;
-      p.dval[bt * 16 + n] = D;
-      if (p.sink_part && n < p.nh) p.sink_part[bt * p.nh + n] = p.sink ? fast_exp2(sk2 - lse2) * D : 0.f;
-    }
-  }
-  if constexpr (SPARSE) {
-    if (p.gsum) {
-      // gsum = sum over the heads of dssel qn + psel dout (dims 32s + 8q + i)
-      psel = colq_sum(psel);
-      dssel = colq_sum(dssel);
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        float gv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float qv = (float)qh[s][i] + (float)ql[s][i];
-          const float dv = (float)dh[s][i] + (float)dl[s][i];
-          gv[i] = row16_sum(dssel * qv + psel * dv);
-        }
-        if (n == 0) {
-          float* dst = p.gsum + bt * HD + 32 * s + 8 * q;
-          *reinterpret_cast<float4*>(dst) = make_float4(gv[0], gv[1], gv[2], gv[3]);
-          *reinterpret_cast<float4*>(dst + 4) = make_float4(gv[4], gv[5], gv[6], gv[7]);
-        }
-      }
-    }
-  }
+  finish_query<HD>(p, bt, n, q, dq, rq, lse2, D, sf.sk2);
+  if (p.gsum) store_gsum<HD, QT>(p, bt, n, q, psel, dssel, rq);
 }
 
 // ------------------------------------------------------------------ key pass
 // MODE 0: compressed rows (HCA: visible when n < (t+1) / m2; CSA: selected),
-// chunk ci of KQC queries; MODE 1: window rows (row u seen by t in [u, u + win)).
-template <int HD, int MODE, bool DL0>
+// chunk ci of part_qc queries; MODE 1: window rows (row u seen by t in
+// [u, u + win)), chunk ci of win_qc of the queries that see the tile.
+template <int HD, int MODE, typename QT, int KG>
 __global__ __launch_bounds__(256, 2) void attn_bwd_k_kernel(HcaBwdParams p, int nchunk) {
+  constexpr bool ONE = Parts<QT>::one;
   constexpr int NS = HD / 32, NT = HD / 16;
   constexpr int TILE = 32 * HD;
-  constexpr int CPR = HD / 8;                 // 16-byte chunks per row
-  constexpr int LPT = 4 * TILE / 8 / 256;     // 16-byte pieces per thread per pair
-  __shared__ __attribute__((aligned(16))) bf16_t lds[2][4 * TILE];  // q hi, q lo, d hi, d lo
+  constexpr int PL = ONE ? 1 : 2;             // planes of q and of dout
+  constexpr int CPR = HD / 8;                 // 8-element chunks per row
+  constexpr int LPT = 2 * TILE / 8 / 256;     // chunks per thread per pair (q and dout)
+  constexpr int KTR = 64 * KG;                // key rows per workgroup
+  __shared__ __attribute__((aligned(16))) bf16_t lds[2][2 * PL * TILE];  // q (hi, lo), dout (hi, lo)
+  __shared__ __attribute__((aligned(16))) float sl[2][32], sd[2][32], sr[2][32];  // lse, D, 1/|q| per row
   const int tid = threadIdx.x;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, q = lane >> 4, n = lane & 15;
   const int b = blockIdx.y;
   const int nrows = MODE == 0 ? p.nb : p.T;
-  const int tile = MODE == 0 ? blockIdx.x / nchunk : blockIdx.x;
-  const int ci = MODE == 0 ? blockIdx.x - tile * nchunk : 0;
+  const int tile = blockIdx.x / nchunk, ci = blockIdx.x - tile * nchunk;
   const int r0 = tile * KTR;
   int tlo, thi;
   if constexpr (MODE == 0) {
-    tlo = max(ci * KQC, (r0 + 1) * p.m2 - 1);
-    thi = min(p.T, (ci + 1) * KQC);
+    tlo = max(ci * p.part_qc, (r0 + 1) * p.m2 - 1);
+    thi = min(p.T, (ci + 1) * p.part_qc);
+    if (tlo >= thi) return;  // no row of the tile is seen by this chunk (nothing is read back)
   } else {
-    tlo = r0;
-    thi = min(p.T, r0 + KTR + p.win - 1);
+    tlo = r0 + ci * p.win_qc;
+    thi = min(min(p.T, r0 + KTR + p.win - 1), tlo + p.win_qc);
   }
-  if (tlo >= thi) return;  // no row of the tile is seen by this chunk (nothing to write)
-  const int rk = r0 + 16 * wv + n;  // this lane's key row (B operand column)
-  const bool rk_ok = rk < nrows;
+  // the queries that see any row of this wave: the others are only staged
+  const int rw = r0 + 16 * KG * wv;
+  const int wlo = MODE == 0 ? (rw + 1) * p.m2 - 1 : rw;
+  const int whi = MODE == 0 ? p.T : rw + 16 * KG - 1 + p.win;
   const TileOffsets<HD> to;
 
-  // key fragments (B operand of S = Qn K^T): row rk, dims 32s + 8q ..
-  bf16x8 kh[NS], kl[NS];
-  {
+  // key fragments (B operand of S = Q K^T): rows rw + 16 g + n, dims 32s + 8q ..
+  bf16x8 kh[KG][NS], kl[KG][NS];
+  f32x4 dk[KG][NT];
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    const int rk = rw + 16 * g + n;
+    const bool ok = rk < nrows;
     const bf16_t* bh = MODE == 0 ? p.kc_hi + (size_t)b * p.nb * HD : p.kl_hi + (size_t)b * p.T * HD;
     const bf16_t* bl = MODE == 0 ? p.kc_lo + (size_t)b * p.nb * HD : p.kl_lo + (size_t)b * p.T * HD;
-    const size_t ro = (size_t)(rk_ok ? rk : 0) * HD + 8 * q;
+    const size_t ro = (size_t)(ok ? rk : 0) * HD + 8 * q;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      kh[s] = *reinterpret_cast<const bf16x8*>(bh + ro + 32 * s);
-      kl[s] = *reinterpret_cast<const bf16x8*>(bl + ro + 32 * s);
-      if (!rk_ok) kh[s] = kl[s] = bf16x8{};
+      kh[g][s] = *reinterpret_cast<const bf16x8*>(bh + ro + 32 * s);
+      kl[g][s] = *reinterpret_cast<const bf16x8*>(bl + ro + 32 * s);
+      if (!ok) kh[g][s] = kl[g][s] = bf16x8{};
     }
-  }
-  f32x4 dk[NT];
 #pragma unroll
-  for (int tt = 0; tt < NT; ++tt) dk[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < NT; ++tt) dk[g][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
-  // staging of a query pair (t, t + 1): 4 tiles of 32 rows (query, head), row
-  // 16 i + h = head h of query t + i; piece k of the thread: tile k / (LPT / 4)
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  auto fetch = [&](int tp, u32x4 (&v)[LPT]) {
+  // staging of a query pair (t, t + 1): rows 16 i + h = head h of query t + i of
+  // q (the thread's first chunks) and dout
+  struct alignas(16) Raw {
+    QT v[8];
+  };
+  struct Pair {
+    Raw x[LPT];
+    float l, d, r;
+  };
+  auto fetch = [&](int tp, Pair& v) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k) {
-      const int pc = tid + 256 * k;              // piece index within the 4 tiles
-      const int tl = pc / (TILE / 8);            // tile 0..3
-      const int w = pc - tl * (TILE / 8);
-      const int row = w / CPR, c = w % CPR;      // row 0..31
-      const int tq = min(tp + (row >> 4), p.T - 1);
-      const bf16_t* src = tl == 0 ? p.qs_hi : tl == 1 ? p.qs_lo : tl == 2 ? p.ds_hi : p.ds_lo;
-      v[k] = *reinterpret_cast<const u32x4*>(src + (((size_t)b * p.T + tq) * 16 + (row & 15)) * HD + 8 * c);
+      const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
+      const int tq = tp + (row >> 4), h = row & 15;
+      const QT* src = static_cast<const QT*>(pc < 32 * CPR ? p.q : p.dout);
+      const bool ok = tq < p.T && h < p.nh;
+      const QT* at = src + (ok ? (((size_t)b * p.T + tq) * p.nh + h) * HD + 8 * c : 0);
+      if (ok) {
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(Raw) / 16; ++i)
+          reinterpret_cast<u32x4*>(v.x[k].v)[i] = reinterpret_cast<const u32x4*>(at)[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < (int)sizeof(Raw) / 16; ++i) reinterpret_cast<u32x4*>(v.x[k].v)[i] = u32x4{0, 0, 0, 0};
+      }
+    }
+    v.l = INFINITY;
+    v.d = v.r = 0.f;
+    if (tid < 32 && tp + (tid >> 4) < p.T) {
+      const size_t li = ((size_t)b * p.T + tp + (tid >> 4)) * 16 + (tid & 15);
+      v.l = p.lse[li];
+      v.d = p.dval[li];
+      v.r = p.rq[li];
     }
   };
-  auto put = [&](bf16_t* buf, const u32x4 (&v)[LPT]) {
+  auto put = [&](int k2, const Pair& v) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k) {
-      const int pc = tid + 256 * k;
-      const int tl = pc / (TILE / 8);
-      const int w = pc - tl * (TILE / 8);
-      const int row = w / CPR, c = w % CPR;
-      *reinterpret_cast<u32x4*>(buf + tl * TILE + row * HD + 8 * (c ^ tile_swz<HD>(row & 15))) = v[k];
+      const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
+      bf16_t* dst = lds[k2] + (pc / (32 * CPR)) * PL * TILE + row * HD + 8 * (c ^ tile_swz<HD>(row & 15));
+      if constexpr (ONE) {
+        *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(v.x[k].v);
+      } else {
+        bf16x8 h, l;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float f = (float)v.x[k].v[i];
+          h[i] = (bf16_t)f;
+          l[i] = lo_of(f);
+        }
+        *reinterpret_cast<bf16x8*>(dst) = h;
+        *reinterpret_cast<bf16x8*>(dst + TILE) = l;
+      }
+    }
+    if (tid < 32) {
+      sl[k2][tid] = v.l;
+      sd[k2][tid] = v.d;
+      sr[k2][tid] = v.r;
     }
   };
   const int nw = (p.nb + 31) / 32;
-  auto visible = [&](int tq) -> bool {
-    if (tq >= thi || !rk_ok) return false;  // (the pair's second query may lie past the chunk)
+  auto visible = [&](int tq, int rk) -> bool {
+    if (tq >= thi || rk >= nrows) return false;  // (the pair's second query may lie past the chunk)
     if constexpr (MODE == 1) return tq >= rk && tq < rk + p.win;
     if (p.sel) return (p.sel[((size_t)b * p.T + tq) * nw + (rk >> 5)] >> (rk & 31)) & 1u;
     return rk < (tq + 1) / p.m2;
   };
 
-  u32x4 pv[LPT];
-  fetch(tlo, pv);
-  put(lds[0], pv);
+  Pair pv;
+  if (tlo < thi) {
+    fetch(tlo, pv);
+    put(0, pv);
+  }
   __syncthreads();
   int buf = 0;
   for (int tp = tlo; tp < thi; tp += 2) {
     const bool more = tp + 2 < thi;
     if (more) fetch(tp + 2, pv);
-    const bf16_t* qs_h = lds[buf];
-    const bf16_t* qs_l = lds[buf] + TILE;
-    const bf16_t* ds_h = lds[buf] + 2 * TILE;
-    const bf16_t* ds_l = lds[buf] + 3 * TILE;
-    bf16x8 ash, asl, aph, apl;  // ds^T and p^T: key n, slots (query i, heads 4q .. 4q+3)
+    if (tp + 1 >= wlo && tp < whi) {
+      const bf16_t* xq = lds[buf];
+      const bf16_t* xd = lds[buf] + PL * TILE;
+      bf16x8 ash[KG], asl[KG], aph[KG], apl[KG];  // ds^T / |q| and p^T: key n, slots (query i, heads 4q .. 4q+3)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int tq = tp + i;
-      f32x4 sa = {0.f, 0.f, 0.f, 0.f}, da = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 2; ++i) {
+        const int tq = tp + i;
+        f32x4 sa[KG], da[KG];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int ko = 16 * HD * i + to.key(s);
-        const bf16x8 xh = *reinterpret_cast<const bf16x8*>(qs_h + ko);
-        const bf16x8 xl = *reinterpret_cast<const bf16x8*>(qs_l + ko);
-        const bf16x8 yh = *reinterpret_cast<const bf16x8*>(ds_h + ko);
-        sa = mfma3(xh, xl, kh[s], kl[s], sa);
-        if constexpr (DL0) {
-          da = mfma2b(yh, kh[s], kl[s], da);
-        } else {
-          const bf16x8 yl = *reinterpret_cast<const bf16x8*>(ds_l + ko);
-          da = mfma3(yh, yl, kh[s], kl[s], da);
+        for (int g = 0; g < KG; ++g) sa[g] = da[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const int ko = 16 * HD * i + to.key(s);
+          const bf16x8 xh = *reinterpret_cast<const bf16x8*>(xq + ko);
+          const bf16x8 yh = *reinterpret_cast<const bf16x8*>(xd + ko);
+          bf16x8 xl = xh, yl = yh;
+          if constexpr (!ONE) {
+            xl = *reinterpret_cast<const bf16x8*>(xq + TILE + ko);
+            yl = *reinterpret_cast<const bf16x8*>(xd + TILE + ko);
+          }
+#pragma unroll
+          for (int g = 0; g < KG; ++g) {
+            sa[g] = mma_xk<ONE>(xh, xl, kh[g][s], kl[g][s], sa[g]);
+            da[g] = mma_xk<ONE>(yh, yl, kh[g][s], kl[g][s], da[g]);
+          }
+        }
+        // lane: heads 4q .. 4q+3 of query tq, keys rw + 16 g + n
+        const float4 L4 = *reinterpret_cast<const float4*>(&sl[buf][16 * i + 4 * q]);
+        const float4 D4 = *reinterpret_cast<const float4*>(&sd[buf][16 * i + 4 * q]);
+        const float4 R4 = *reinterpret_cast<const float4*>(&sr[buf][16 * i + 4 * q]);
+        const float Ls[4] = {L4.x, L4.y, L4.z, L4.w}, Ds[4] = {D4.x, D4.y, D4.z, D4.w};
+        const float Rs[4] = {R4.x, R4.y, R4.z, R4.w};
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+          const bool vis = visible(tq, rw + 16 * g + n);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float pe = vis ? fast_exp2(sa[g][e] * (Rs[e] * p.scale * kLog2eF) - Ls[e]) : 0.f;
+            const float dse = pe * (da[g][e] - Ds[e]) * p.scale * Rs[e];
+            ash[g][4 * i + e] = (bf16_t)dse;
+            asl[g][4 * i + e] = lo_of(dse);
+            aph[g][4 * i + e] = (bf16_t)pe;
+            apl[g][4 * i + e] = lo_of(pe);
+          }
         }
       }
-      // lane: heads 4q .. 4q+3 of query tq, key rk
-      const bool vis = visible(tq);
-      const size_t li = ((size_t)b * p.T + min(tq, p.T - 1)) * 16 + 4 * q;
-      const float4 L4 = *reinterpret_cast<const float4*>(p.lse + li);
-      const float4 D4 = *reinterpret_cast<const float4*>(p.dval + li);
-      const float Ls[4] = {L4.x, L4.y, L4.z, L4.w}, Ds[4] = {D4.x, D4.y, D4.z, D4.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float pe = vis ? fast_exp2(sa[e] * p.scale * kLog2eF - Ls[e]) : 0.f;
-        const float dse = pe * (da[e] - Ds[e]) * p.scale;
-        ash[4 * i + e] = (bf16_t)dse;
-        asl[4 * i + e] = lo_of(dse);
-        aph[4 * i + e] = (bf16_t)pe;
-        apl[4 * i + e] = lo_of(pe);
+      for (int tt = 0; tt < NT; ++tt) {
+        const bf16x8 bq = MqaWave<HD>::vt_frag(xq, to, tt);
+        const bf16x8 bd = MqaWave<HD>::vt_frag(xd, to, tt);
+        bf16x8 bql = bq, bdl = bd;
+        if constexpr (!ONE) {
+          bql = MqaWave<HD>::vt_frag(xq + TILE, to, tt);
+          bdl = MqaWave<HD>::vt_frag(xd + TILE, to, tt);
+        }
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+          dk[g][tt] = mma_kx<ONE>(ash[g], asl[g], bq, bql, dk[g][tt]);
+          dk[g][tt] = mma_kx<ONE>(aph[g], apl[g], bd, bdl, dk[g][tt]);
+        }
       }
     }
-#pragma unroll
-    for (int tt = 0; tt < NT; ++tt) {
-      const bf16x8 bqh = MqaWave<HD>::vt_frag(qs_h, to, tt);
-      const bf16x8 bql = MqaWave<HD>::vt_frag(qs_l, to, tt);
-      const bf16x8 bdh = MqaWave<HD>::vt_frag(ds_h, to, tt);
-      dk[tt] = mfma3(ash, asl, bqh, bql, dk[tt]);
-      if constexpr (DL0) {
-        dk[tt] = mfma2a(aph, apl, bdh, dk[tt]);
-      } else {
-        const bf16x8 bdl = MqaWave<HD>::vt_frag(ds_l, to, tt);
-        dk[tt] = mfma3(aph, apl, bdh, bdl, dk[tt]);
-      }
-    }
-    if (more) put(lds[buf ^ 1], pv);
+    if (more) put(buf ^ 1, pv);
     __syncthreads();
     buf ^= 1;
   }
-  // dk tile tt: rows (keys) 16 wv + 4q + e of the tile, column (dim) 16 tt + n
+  // dk tile tt: rows (keys) rw + 16 g + 4q + e, column (dim) 16 tt + n
   float* out = MODE == 0 ? p.part_b + (((size_t)b * nchunk + ci) * p.nb) * HD
-                         : p.part_w + (size_t)b * p.T * HD;
+                         : p.part_w + ((size_t)ci * p.B + b) * p.T * HD;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int r = r0 + 16 * wv + 4 * q + e;
-    if (r < nrows) {
+  for (int g = 0; g < KG; ++g)
 #pragma unroll
-      for (int tt = 0; tt < NT; ++tt) out[(size_t)r * HD + 16 * tt + n] = dk[tt][e];
+    for (int e = 0; e < 4; ++e) {
+      const int r = rw + 16 * g + 4 * q + e;
+      if (r < nrows) {
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) out[(size_t)r * HD + 16 * tt + n] = dk[g][tt][e];
+      }
     }
-  }
+}
+
+// slot[row, j] += dsel[row, idx[row, j]] (idx < 0: unused slot)
+__global__ __launch_bounds__(256) void slot_gather_kernel(const int* idx, const float* dsel, float* slot,
+                                                          long long n, int topk, int nb) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int k = idx[i];
+  if (k >= 0 && k < nb) slot[i] += dsel[i / topk * nb + k];
+}
+
+// The key passes' grids: groups of 16 keys per wave, queries per chunk.
+struct KeyPlan {
+  int kg, qc, nchunk;    // compressed rows
+  int wqc, wnc;          // window rows
+};
+KeyPlan key_plan(int B, int T, int nb, int win) {
+  KeyPlan k;
+  // two groups of 16 keys per wave halve the LDS reads per product; one group
+  // where two would leave waves without keys
+  k.kg = nb > 64 ? 2 : 1;
+  const long long ntile = (nb + 64 * k.kg - 1) / (64 * k.kg);
+  // chunks of 512 queries, halved (to 64) while the grid, half of which the
+  // causal rule leaves empty, would give the 256 compute units less than two
+  // workgroups each
+  k.qc = 512;
+  while (k.qc > 64 && ntile * ((T + k.qc - 1) / k.qc) * B < 1024) k.qc /= 2;
+  k.nchunk = (T + k.qc - 1) / k.qc;
+  // window: a tile of 128 rows is seen by 127 + win queries, in up to 4 chunks
+  const long long wt = (long long)B * ((T + 127) / 128);
+  k.wnc = 1;
+  while (k.wnc < 4 && wt * k.wnc < 512 && (127 + win) / k.wnc > 64) k.wnc *= 2;
+  k.wqc = ((127 + win + k.wnc - 1) / k.wnc + 1) & ~1;
+  return k;
 }
 
 }  // namespace
@@ -640,28 +1037,74 @@ bool attn_bwd_mfma_supported(const HcaBwdParams& p) {
   return p.normalize && (p.c == 64 || p.c == 128) && p.nh >= 1 && p.nh <= 16;
 }
 
+// CSA: whether the query pass takes every visible block in tiles (true) or
+// gathers the selected rows. The tiles' cost grows with the visible blocks
+// (nb / 2 on average), the gather's with topk; whole backward, 8192 queries,
+// 16 heads of 128, window 128, tiles against gather: topk 512, nb 512 0.655 /
+// 0.852 ms, 1024 0.875 / 1.006, 2048 1.328 / 1.277, 4096 4.51 / 3.61; topk 128,
+// nb 512 0.657 / 0.635; topk 64, nb 512 0.704 / 0.631.
+static bool attn_bwd_dense_rows(int nb, int topk) { return nb <= 3 * topk; }
+
 static size_t al256m(size_t x) { return (x + 255) & ~size_t(255); }
 
 size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
   const size_t BT = (size_t)B * T;
   const int nb = T / m2;
-  const int nchunk = (T + KQC - 1) / KQC;
+  const KeyPlan k = key_plan(B, T, nb, win);
   size_t z = 3 * al256m(BT * 16 * 4);                  // lse, D, 1/|q| (16 heads)
-  z += 4 * al256m(BT * 16 * c * 2);                     // qn, dout hi / lo
   z += 2 * al256m((size_t)B * nb * c * 2);              // compressed rows hi / lo
   if (win > 0) z += 2 * al256m(BT * c * 2);             // window rows hi / lo
-  z += al256m((size_t)B * nchunk * nb * c * 4);         // compressed-row partials
-  if (win > 0) z += al256m(BT * c * 4);                 // window-row gradients
+  z += al256m((size_t)B * k.nchunk * nb * c * 4);       // compressed-row partials
+  if (win > 0) z += al256m(BT * k.wnc * c * 4);         // window-row partials
   if (topk > 0) z += al256m(BT * ((nb + 31) / 32) * 4);  // selection bitmap
+  if (topk > 0) {
+    z += al256m(BT * nb * 4);                            // dense slot gradients
+    if (!attn_bwd_dense_rows(nb, topk)) z += al256m(BT * topk * 4);  // per slot
+  }
   return z;
 }
 
 hipError_t sel_bitmap_launch(const int* idx, uint32_t* sel, long long nq, int topk, int nw, hipStream_t s);
 
+template <int HD, typename QT>
+static void launch_passes(const HcaBwdParams& p, const KeyPlan& k, hipStream_t s) {
+  const int tq = Parts<QT>::one ? 8 : 4;  // queries per workgroup of the tiled query pass
+  const int nt = (p.T + tq - 1) / tq;
+  const dim3 qg((unsigned)((long long)p.B * nt));
+  if (!p.sparse)
+    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, false>), qg, dim3(256), 0, s, p, nt);
+  else if (attn_bwd_dense_rows(p.nb, p.topk))
+    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, true>), qg, dim3(256), 0, s, p, nt);
+  else
+    hipLaunchKernelGGL((attn_bwd_q_kernel<HD, QT>), dim3((unsigned)(p.B * ((p.T + 3) / 4))), dim3(256), 0, s, p);
+  if (p.nb > 0 && !(p.sparse && p.topk == 0)) {
+    const dim3 g((p.nb + 64 * k.kg - 1) / (64 * k.kg) * k.nchunk, p.B);
+    if (k.kg == 2)
+      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 2>), g, dim3(256), 0, s, p, k.nchunk);
+    else
+      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 1>), g, dim3(256), 0, s, p, k.nchunk);
+  }
+  if (p.win > 0)
+    hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 1, QT, 2>), dim3((p.T + 127) / 128 * k.wnc, p.B), dim3(256), 0, s, p,
+                       k.wnc);
+}
+
+template <int HD>
+static void launch_splits(const HcaBwdParams& p, hipStream_t s) {
+  constexpr int rpb = 256 / (HD / 8);  // rows per workgroup
+  const long long BT = (long long)p.B * p.T, bn = (long long)p.B * p.nb;
+  if (p.nb > 0)
+    hipLaunchKernelGGL((split_rows_kernel<HD, float>), dim3((unsigned)((bn + rpb - 1) / rpb)), dim3(256), 0, s, p.kc,
+                       bn, 1, 1, p.kc_hi, p.kc_lo, (float*)nullptr, 0);
+  if (p.win > 0)
+    hipLaunchKernelGGL((split_rows_kernel<HD, float>), dim3((unsigned)((BT + rpb - 1) / rpb)), dim3(256), 0, s, p.kl,
+                       BT, 1, 1, p.kl_hi, p.kl_lo, (float*)nullptr, 0);
+}
+
 hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
   const int HD = p.c;
   const size_t BT = (size_t)p.B * p.T;
-  const int nchunk = (p.T + KQC - 1) / KQC;
+  const KeyPlan k = key_plan(p.B, p.T, p.nb, p.win);
   char* w = static_cast<char*>(ws);
   auto take = [&](size_t bytes) {
     char* r = w;
@@ -671,10 +1114,6 @@ hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
   p.lse = reinterpret_cast<float*>(take(BT * 16 * 4));
   p.dval = reinterpret_cast<float*>(take(BT * 16 * 4));
   p.rq = reinterpret_cast<float*>(take(BT * 16 * 4));
-  p.qs_hi = reinterpret_cast<bf16_t*>(take(BT * 16 * HD * 2));
-  p.qs_lo = reinterpret_cast<bf16_t*>(take(BT * 16 * HD * 2));
-  p.ds_hi = reinterpret_cast<bf16_t*>(take(BT * 16 * HD * 2));
-  p.ds_lo = reinterpret_cast<bf16_t*>(take(BT * 16 * HD * 2));
   p.kc_hi = reinterpret_cast<bf16_t*>(take((size_t)p.B * p.nb * HD * 2));
   p.kc_lo = reinterpret_cast<bf16_t*>(take((size_t)p.B * p.nb * HD * 2));
   p.kl_hi = p.kl_lo = nullptr;
@@ -682,91 +1121,62 @@ hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
     p.kl_hi = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
     p.kl_lo = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
   }
-  p.part_b = reinterpret_cast<float*>(take((size_t)p.B * nchunk * p.nb * HD * 4));
-  p.part_w = p.win > 0 ? reinterpret_cast<float*>(take(BT * HD * 4)) : nullptr;
+  p.part_b = reinterpret_cast<float*>(take((size_t)p.B * k.nchunk * p.nb * HD * 4));
+  p.part_w = p.win > 0 ? reinterpret_cast<float*>(take(BT * k.wnc * HD * 4)) : nullptr;
   p.sel = nullptr;
+  p.mfma_parts = 1;
+  p.part_qc = k.qc;
+  p.win_qc = k.wqc;
+  p.win_nc = k.wnc;
   if (p.idx && p.topk > 0) {
     const int nw = (p.nb + 31) / 32;
     uint32_t* sel = reinterpret_cast<uint32_t*>(take(BT * nw * 4));
-    hipError_t e = fill_u32(sel, (long long)BT * nw, 0u, s);
-    if (e != hipSuccess) return e;
-    e = sel_bitmap_launch(p.idx, sel, (long long)BT, p.topk, nw, s);
+    const hipError_t e = sel_bitmap_launch(p.idx, sel, (long long)BT, p.topk, nw, s);
     if (e != hipSuccess) return e;
     p.sel = sel;
+    float* own = reinterpret_cast<float*>(take(BT * p.nb * 4));
+    if (!p.dsel && p.slot_grad) {
+      p.dsel = own;
+      p.dsel_add = 0;
+    }
+    if (p.dsel && !attn_bwd_dense_rows(p.nb, p.topk)) p.slot_ws = reinterpret_cast<float*>(take(BT * p.topk * 4));
   }
-  p.mfma_parts = 1;
-  p.part_qc = KQC;
-  // split_rows_kernel: 256 / (HD / 8) rows per workgroup
-  auto grid_rows = [](long long rows, int hd) {
-    const long long rpb = 256 / (hd / 8);
-    return dim3((unsigned)((rows + rpb - 1) / rpb));
-  };
-#define KCH_SPLIT_Q(HDV, QT)                                                                       \
-  do {                                                                                             \
-    hipLaunchKernelGGL((split_rows_kernel<HDV, QT>), grid_rows((long long)BT * 16, HDV), dim3(256), 0, \
-                       s, static_cast<const QT*>(p.q), (long long)BT, p.nh, 16, p.qs_hi, p.qs_lo, p.rq, 1); \
-    hipLaunchKernelGGL((split_rows_kernel<HDV, QT>), grid_rows((long long)BT * 16, HDV), dim3(256), 0, \
-                       s, static_cast<const QT*>(p.dout), (long long)BT, p.nh, 16, p.ds_hi, p.ds_lo,  \
-                       (float*)nullptr, 0);                                                        \
+#define KCH_BWD(HDV)                             \
+  do {                                           \
+    launch_splits<HDV>(p, s);                    \
+    if (p.qdt == DT_BF16)                        \
+      launch_passes<HDV, bf16_t>(p, k, s);       \
+    else if (p.qdt == DT_F16)                    \
+      launch_passes<HDV, _Float16>(p, k, s);     \
+    else                                         \
+      launch_passes<HDV, float>(p, k, s);        \
   } while (0)
-#define KCH_SPLIT(HDV)                                                                              \
-  do {                                                                                              \
-    if (p.qdt == DT_BF16)                                                                           \
-      KCH_SPLIT_Q(HDV, bf16_t);                                                                     \
-    else if (p.qdt == DT_F16)                                                                       \
-      KCH_SPLIT_Q(HDV, _Float16);                                                                   \
-    else                                                                                            \
-      KCH_SPLIT_Q(HDV, float);                                                                      \
-    if (p.nb > 0)                                                                                   \
-      hipLaunchKernelGGL((split_rows_kernel<HDV, float>), grid_rows((long long)p.B * p.nb, HDV),    \
-                         dim3(256), 0, s, p.kc, (long long)p.B * p.nb, 1, 1, p.kc_hi, p.kc_lo,      \
-                         (float*)nullptr, 0);                                                       \
-    if (p.win > 0)                                                                                  \
-      hipLaunchKernelGGL((split_rows_kernel<HDV, float>), grid_rows((long long)BT, HDV), dim3(256), \
-                         0, s, p.kl, (long long)BT, 1, 1, p.kl_hi, p.kl_lo, (float*)nullptr, 0);    \
-  } while (0)
-#define KCH_PASSES_D(HDV, DL)                                                                      \
-  do {                                                                                             \
-    const unsigned qg = (unsigned)(p.B * ((p.T + 3) / 4));                                         \
-    if (p.sparse)                                                                                  \
-      hipLaunchKernelGGL((attn_bwd_q_kernel<HDV, true, DL>), dim3(qg), dim3(256), 0, s, p);        \
-    else                                                                                           \
-      hipLaunchKernelGGL((attn_bwd_q_kernel<HDV, false, DL>), dim3(qg), dim3(256), 0, s, p);       \
-    if (p.nb > 0 && !(p.sparse && p.topk == 0)) {                                                  \
-      const int ntile = (p.nb + KTR - 1) / KTR;                                                    \
-      hipLaunchKernelGGL((attn_bwd_k_kernel<HDV, 0, DL>), dim3(ntile * nchunk, p.B), dim3(256), 0, s, \
-                         p, nchunk);                                                               \
-    }                                                                                              \
-    if (p.win > 0)                                                                                 \
-      hipLaunchKernelGGL((attn_bwd_k_kernel<HDV, 1, DL>), dim3((p.T + KTR - 1) / KTR, p.B), dim3(256), \
-                         0, s, p, nchunk);                                                         \
-  } while (0)
-#define KCH_PASSES(HDV)                                                                            \
-  do {                                                                                             \
-    if (p.qdt == DT_BF16)                                                                          \
-      KCH_PASSES_D(HDV, true);                                                                     \
-    else                                                                                           \
-      KCH_PASSES_D(HDV, false);                                                                    \
-  } while (0)
-  if (HD == 64) {
-    KCH_SPLIT(64);
-    KCH_PASSES(64);
-  } else {
-    KCH_SPLIT(128);
-    KCH_PASSES(128);
+  if (HD == 64)
+    KCH_BWD(64);
+  else
+    KCH_BWD(128);
+#undef KCH_BWD
+  if (p.slot_ws) {
+    if (!p.dsel_add) {
+      hipError_t e = fill_u32(p.dsel, (long long)BT * p.nb, 0u, s);
+      if (e != hipSuccess) return e;
+    }
+    hipError_t e = ste_scatter_launch(p.idx, p.slot_ws, p.dsel, (long long)BT, p.topk, p.nb, s);
+    if (e != hipSuccess) return e;
   }
-#undef KCH_SPLIT
-#undef KCH_SPLIT_Q
-#undef KCH_PASSES
-#undef KCH_PASSES_D
+  if (p.slot_grad && p.idx) {
+    const long long ns = (long long)BT * p.topk;
+    hipLaunchKernelGGL(slot_gather_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, s, p.idx, p.dsel,
+                       p.slot_grad, ns, p.topk, p.nb);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (p.nb > 0 && p.sparse && p.topk == 0) {
     // no selection: the compressed rows receive nothing
-    e = fill_u32(p.part_b, (long long)p.B * nchunk * p.nb * HD, 0u, s);
+    e = fill_u32(p.part_b, (long long)p.B * k.nchunk * p.nb * HD, 0u, s);
     if (e != hipSuccess) return e;
   }
-  return hca_bwd_finish_launch(p, nchunk, s);
+  return hca_bwd_finish_launch(p, k.nchunk, s);
 }
 
 }  // namespace kch

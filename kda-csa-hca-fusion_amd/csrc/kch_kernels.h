@@ -99,6 +99,11 @@ struct HcaBwdParams {
   float* dZb = nullptr;
   float* dBbp = nullptr;
   float* slot_grad = nullptr;
+  // the same values dense over the blocks, [B,T,nb] (0 at the others); dsel_add:
+  // added to what it holds (calls for further groups of heads)
+  float* dsel = nullptr;
+  int dsel_add = 0;
+  float* slot_ws = nullptr;  // workspace: the gathering query pass's values per slot
   // CSA, full-softmax STE: the sum over the selected slots of each selected
   // row's gradient, gsum [B,T,c] (written, the heads of this call summed)
   float* gsum = nullptr;
@@ -107,21 +112,18 @@ struct HcaBwdParams {
   float* rq = nullptr;
   float* part_b = nullptr;
   float* part_w = nullptr;
-  // MFMA path (attn_bwd_mfma.hip): the two-part bf16 splits of qn and dout
-  // ([B,T,16,c], heads padded to 16) and of the compressed and window rows;
-  // mfma_parts: part_b holds [B, nchunk, nb, c] per-chunk partials of the
-  // compressed rows (chunk ci = queries [ci part_qc, (ci+1) part_qc), written
-  // for the chunks a row's queries reach), part_w the window rows' [B, T, c]
-  bf16_t* qs_hi = nullptr;
-  bf16_t* qs_lo = nullptr;
-  bf16_t* ds_hi = nullptr;
-  bf16_t* ds_lo = nullptr;
+  // MFMA path (attn_bwd_mfma.hip): the two-part bf16 splits of the compressed
+  // and window rows; mfma_parts: part_b holds [B, nchunk, nb, c] per-chunk
+  // partials of the compressed rows (chunk ci = queries [ci part_qc, (ci+1)
+  // part_qc), written for the chunks a row's queries reach), part_w the window
+  // rows' [win_nc, B, T, c]
   bf16_t* kc_hi = nullptr;
   bf16_t* kc_lo = nullptr;
   bf16_t* kl_hi = nullptr;
   bf16_t* kl_lo = nullptr;
   int mfma_parts = 0;
   int part_qc = 0;
+  int win_qc = 0, win_nc = 1;
   int B, T, nh, c, m2, nb, win;
   float scale;
 };

@@ -514,7 +514,7 @@ def _csa_core(Ca, Cb, Za, Zb, K_idx, Z_idx, q, q_idx, w_idx, Ba, Bb, B_idx, *, m
 
 
 def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
-                  sink_logits=None, normalize_qk=True, scale=None, want_gsum=False):
+                  sink_logits=None, normalize_qk=True, scale=None, want_gsum=False, _dense=False):
     """Gradients of the CSA attention (``ops_csa.py:869-1155``) with the selection
     ``idx`` ``[B,T,topk]`` (int32, -1 = unused) held fixed, on
     ``kch_csa_attn_bwd`` (fp32 arithmetic). Returns a dict with ``Ca, Cb, Za, Zb, q, Ba,
@@ -522,7 +522,9 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     (fp32): each selected row's gradient dotted with the row; with
     ``want_gsum`` also ``gsum`` ``[B,T,c]`` (fp32): the sum of the selected
     rows' gradients over the slots. Channels are zero-padded to the kernel's
-    size; more than 16 heads run as groups."""
+    size; more than 16 heads run as groups. ``_dense`` (internal,
+    ``normalize_qk`` only): the slots' values as ``dsel`` ``[B,T,T/m]`` at their
+    blocks (0 at the others) in place of ``slot``."""
     fn = "csa_attn_grad"
     B_, T, c = Ca.shape
     nh = q.shape[2]
@@ -561,7 +563,8 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     dCb, dZa, dZb = torch.zeros_like(dCa), torch.zeros_like(dCa), torch.zeros_like(dCa)
     dBa = torch.zeros(m, cp, device=dev, dtype=f32)
     dBb = torch.zeros_like(dBa)
-    slot = torch.zeros(B_, T, topk, device=dev, dtype=f32)
+    slot = None if _dense else torch.zeros(B_, T, topk, device=dev, dtype=f32)
+    dsel = torch.empty(B_, T, nb, device=dev, dtype=f32) if _dense else None
     gsum = torch.zeros(B_, T, cp, device=dev, dtype=f32) if want_gsum else None
     dsink = None if sink is None else torch.zeros(nh, device=dev, dtype=f32)
     # 16 heads a call on the MFMA kernels (normalised rows), else as many as
@@ -586,8 +589,8 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
                   _lib.ptr(Zaf), _lib.ptr(Zbf), _lib.ptr(Baf), _lib.ptr(Bbf),
                   _lib.ptr(None if sink is None else sink[h0:h1].contiguous()), _lib.ptr(dqg),
                   _lib.ptr(oa), _lib.ptr(ob), _lib.ptr(za), _lib.ptr(zb), _lib.ptr(bap),
-                  _lib.ptr(bbp), _lib.ptr(sp), _lib.ptr(slot if topk else None), _lib.ptr(gs),
-                  B_, T, g, cp, m, topk, win, float(scale), int(bool(normalize_qk)),
+                  _lib.ptr(bbp), _lib.ptr(sp), _lib.ptr(slot if topk else None), _lib.ptr(dsel),
+                  int(h0 > 0), _lib.ptr(gs), B_, T, g, cp, m, topk, win, float(scale), int(bool(normalize_qk)),
                   _lib.dtype_code(fn, qdt), _lib.ptr(ws), nbytes, _lib.stream_of(qg))
         if dqg is not dq:
             dq[:, :, h0:h1] = dqg
@@ -604,7 +607,11 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     out = {"Ca": dCa[..., :c].to(Ca.dtype), "Cb": dCb[..., :c].to(Cb.dtype),
            "Za": dZa[..., :c].to(Za.dtype), "Zb": dZb[..., :c].to(Zb.dtype),
            "q": dq[..., :c].to(q.dtype), "Ba": dBa[:, :c].to(Ba.dtype),
-           "Bb": dBb[:, :c].to(Bb.dtype), "slot": slot}
+           "Bb": dBb[:, :c].to(Bb.dtype)}
+    if _dense:
+        out["dsel"] = dsel
+    else:
+        out["slot"] = slot
     if gsum is not None:
         out["gsum"] = gsum[..., :c]
     if sink_logits is not None:
@@ -612,8 +619,15 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     return out
 
 
+def _ste_kernel_sizes(cI, nIh):
+    """(padded cI, padded nIh) of ``kch_csa_ste_bwd``, or None beyond its sizes."""
+    cIp = 64 if cI <= 64 else 128
+    nIp = next((n for n in (1, 2, 4, 8) if n >= nIh), None)
+    return None if cI > 128 or nIp is None or nIp * cIp > 512 else (cIp, nIp)
+
+
 def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, normalize_qk,
-                       dsel_extra=None):
+                       dsel_extra=None, dsel=None):
     """The straight-through surrogate's gradients for the indexer inputs
     (``ops_csa.py:1033-1099``): the selected columns of the soft weights
     (``softmax`` over every causal block of the indexer logits,
@@ -621,15 +635,16 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
     ``dsel_extra`` ``[B,T,nb]`` every column receives that too (the dense term
     of ``full_softmax``), carried through the logits (``ops_csa.py:503-536``)
     and the key compression (``ops_csa.py:198-234``). On ``kch_csa_ste_bwd``
-    when the padded ``nIh * c_I <= 512`` (a wave per query); beyond that,
-    ``_ste_indexer_grads_dense``."""
+    when the padded ``nIh * c_I <= 512``; beyond that,
+    ``_ste_indexer_grads_dense``. ``dsel`` ``[B,T,nb]`` (those sizes only):
+    the slots' values already at their blocks, in place of ``slot``."""
     B_, T, cI = K_idx.shape
     nIh = q_idx.shape[2]
-    cIp = 64 if cI <= 64 else 128
-    nIp = next((n for n in (1, 2, 4, 8) if n >= nIh), None)
-    if cI > 128 or nIp is None or nIp * cIp > 512:
+    sizes = _ste_kernel_sizes(cI, nIh)
+    if sizes is None:
         return _ste_indexer_grads_dense(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, m=m,
                                         normalize_qk=normalize_qk, dsel_extra=dsel_extra)
+    cIp, nIp = sizes
     fn = "csa_ste_grad"
     dev = K_idx.device
     f32 = torch.float32
@@ -647,12 +662,15 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
     raw = _compress(fn, Kf, Zf, Bf, m, out_raw=True, key=kc, normalize=bool(normalize_qk))
     if not normalize_qk:
         kc = raw
-    dsel = (torch.zeros(B_, T, nb, device=dev, dtype=f32) if dsel_extra is None
-            else dsel_extra.to(f32).clone(memory_format=torch.contiguous_format))
-    idx32 = idx.to(dtype=torch.int32).contiguous()
-    slot = slot.to(f32).contiguous()
-    _lib.call("kch_csa_ste_scatter", _lib.ptr(idx32), _lib.ptr(slot), _lib.ptr(dsel), B_, T,
-              idx.shape[-1], nb, _lib.stream_of(qf))
+    if dsel is not None:
+        dsel = dsel if dsel_extra is None else dsel + dsel_extra
+    else:
+        dsel = (torch.zeros(B_, T, nb, device=dev, dtype=f32) if dsel_extra is None
+                else dsel_extra.to(f32).clone(memory_format=torch.contiguous_format))
+        idx32 = idx.to(dtype=torch.int32).contiguous()
+        slot = slot.to(f32).contiguous()
+        _lib.call("kch_csa_ste_scatter", _lib.ptr(idx32), _lib.ptr(slot), _lib.ptr(dsel), B_, T,
+                  idx.shape[-1], nb, _lib.stream_of(qf))
     scale = 1.0 if normalize_qk else cI ** -0.5
     dq = torch.empty_like(qf)
     dw = torch.empty_like(wf)
@@ -794,9 +812,14 @@ class _CsaCoreFunction(torch.autograd.Function):
         Ca, Cb, Za, Zb, K_idx, Z_idx, q, q_idx, w_idx, Ba, Bb, B_idx, sink, idx = ctx.saved_tensors
         cfg = ctx.cfg
         full = cfg["use_ste"] and cfg["ste_mode"] == "full_softmax" and idx.shape[-1] > 0
+        ste = cfg["use_ste"] and idx.shape[-1] > 0 and any(
+            x.requires_grad for x in (K_idx, Z_idx, q_idx, w_idx, B_idx))
+        dense = ste and bool(cfg["normalize_qk"]) and _ste_kernel_sizes(
+            K_idx.shape[-1], q_idx.shape[2]) is not None
         g = csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx if idx.shape[-1] else None, d_out,
                           m=cfg["m"], sliding_window=cfg["sliding_window"], sink_logits=sink,
-                          normalize_qk=cfg["normalize_qk"], scale=cfg["scale"], want_gsum=full)
+                          normalize_qk=cfg["normalize_qk"], scale=cfg["scale"], want_gsum=full,
+                          _dense=dense)
         dsel_extra = None
         if full:
             dsel_extra, extra = _full_softmax_grads(
@@ -806,11 +829,10 @@ class _CsaCoreFunction(torch.autograd.Function):
                                   extra):
                 g[name] = (g[name].to(torch.float32) + e).to(x.dtype)
         ig = [None] * 5
-        if cfg["use_ste"] and idx.shape[-1] and any(
-                x.requires_grad for x in (K_idx, Z_idx, q_idx, w_idx, B_idx)):
-            ig = _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, g["slot"],
+        if ste:
+            ig = _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, g.get("slot"),
                                     m=cfg["m"], normalize_qk=cfg["normalize_qk"],
-                                    dsel_extra=dsel_extra)
+                                    dsel_extra=dsel_extra, dsel=g.get("dsel"))
         return (g["Ca"], g["Cb"], g["Za"], g["Zb"], ig[0], ig[1], g["q"], ig[2], ig[3], g["Ba"],
                 g["Bb"], ig[4], g.get("sink_logits"), None)
 

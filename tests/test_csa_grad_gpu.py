@@ -426,3 +426,47 @@ def test_ste_indexer_kernels_at_tile_edges(dev, B, T, m, topk, nIh, cI, norm):
     torch.cuda.synchronize()
     for name, g, x in zip(("K_idx", "Z_idx", "q_idx", "w_idx", "B_idx"), got, ref):
         _check(name, g.cpu().numpy(), x.numpy())
+
+
+TILE_EDGES = [
+    # B, T, nh, c, m, topk, win, dtype: blocks in tiles (nb <= 3 topk) or gathered
+    (2, 9, 16, 128, 1, 3, 5, torch.bfloat16),      # 9 queries: a workgroup of one; in tiles
+    (1, 132, 5, 64, 2, 66, 37, torch.bfloat16),    # 66 blocks: a second group of 64 keys, 3-row step
+    (1, 301, 16, 128, 7, 20, 128, torch.float16),  # 43 blocks, window of whole steps
+    (2, 264, 18, 128, 4, 23, 33, torch.float32),   # 66 blocks in tiles, two head groups
+    (1, 264, 16, 128, 4, 21, 33, torch.bfloat16),  # 66 blocks > 3 topk: gathered
+    (1, 260, 17, 64, 4, 6, 40, torch.float32),     # gathered, two head groups
+]
+
+
+@pytest.mark.parametrize("B,T,nh,c,m,topk,win,dtype", TILE_EDGES)
+def test_attn_grad_at_tile_edges(dev, B, T, nh, c, m, topk, win, dtype):
+    """The tiled and the gathering query pass and both key passes at remainders of
+    their tiles, against the fp64 oracle on the same (dtype-representable) q and
+    d_out: within 1e-4 of each tensor's largest entry (two-part products, 2^-16);
+    dq one rounding of dtype more. ``_dense`` gives the slots' values at their
+    blocks."""
+    import kch
+    rng = np.random.default_rng(T + nh + topk)
+    t = lambda x: torch.tensor(x, dtype=torch.float32, device=dev)  # noqa: E731
+    X = {k: rng.standard_normal((B, T, c)).astype(np.float32) for k in ("Ca", "Cb", "Za", "Zb")}
+    q, W = (t(rng.standard_normal((B, T, nh, c))).to(dtype) for _ in range(2))
+    Ba, Bb = ((rng.standard_normal((m, c)) * 0.3).astype(np.float32) for _ in range(2))
+    sk = rng.standard_normal(nh).astype(np.float32)
+    idx = _selection(rng, B, T, m, topk, hole=T // 2)
+    ref = o_grad(X["Ca"], X["Cb"], X["Za"], X["Zb"], q.float().cpu().numpy(), Ba, Bb, idx,
+                 W.float().cpu().numpy(), m=m, sliding_window=win, sink_logits=sk, normalize_qk=True)
+    args = [t(X[k]) for k in ("Ca", "Cb", "Za", "Zb")] + [q, t(Ba), t(Bb)]
+    kw = dict(m=m, sliding_window=win, sink_logits=t(sk))
+    ix = torch.tensor(idx, device=dev)
+    g = kch.ops_csa.csa_attn_grad(*args, ix, W, **kw)
+    dsel = kch.ops_csa.csa_attn_grad(*args, ix, W, _dense=True, **kw)["dsel"].cpu().numpy()
+    torch.cuda.synchronize()
+    ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for name in ("Ca", "Cb", "Za", "Zb", "q", "Ba", "Bb", "slot", "sink_logits"):
+        _check(name, g[name].float().cpu().numpy(), ref[name], 1e-4 + (ulp if name == "q" else 0.0))
+    want = np.zeros((B, T, T // m))
+    np.put_along_axis(want, np.maximum(idx, 0), 0.0, -1)
+    for b, i, j in zip(*np.nonzero(idx >= 0)):
+        want[b, i, idx[b, i, j]] = ref["slot"][b, i, j]
+    _check("dsel", dsel, want)
