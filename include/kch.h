@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define KCH_ABI_VERSION 20
+#define KCH_ABI_VERSION 21
 
 #define KCH_OK 0
 #define KCH_ERR_INVALID 1     /* bad pointer / shape / argument */
@@ -194,26 +194,26 @@ int kch_gen_attn(const void* q, const void* kv, const long long* idx, const void
  * Gradients of the HCA attention: the backward of hca_core (ops_hca.py:132-194,
  * which the reference differentiates with autograd; the gradient check of the
  * hybrid stack, run_correctness.py:2710-2830, runs through it). q, d_out and
- * dq [B,T,nh,c] are stored in qdt (KCH_DT_F32 / BF16 / F16; bf16 and fp16
- * need nh <= 16, the MFMA kernels' limit: the caller runs more heads as
- * groups), the queries as given (the kernel normalises them); the other
- * tensors are fp32: kc / raw
- * [B,T/m2,c] (the L2-normalised and the raw compressed rows of C, Z, B_pos,
- * from kch_compress), kl / lsrc [B,T,c] (the normalised window rows and the
- * rows they normalise; NULL when win = 0), C, Z [B,T,c], B_pos [m2,c], sink
- * [nh] or NULL. Outputs: dq [B,T,nh,c]; dC, dZ [B,T,c]; dBp [B,T/m2,m2,c]
- * (summed over the first two axes it is dB_pos); dlocal [B,T,c] (the window
- * rows' source gradient) or NULL to add it into dC; sink_part [B,T,nh]
- * (p_sink * D; dsink = -its sum over B and T) or NULL. Coverage: c in {64,
- * 128}, nh <= 16 (c = 128) or 32 (c = 64), T a multiple of m2, T >= 1. ws:
- * 256-byte aligned, kch_hca_attn_bwd_ws_bytes bytes.
+ * dq [B,T,nh,c] are stored in qdt (KCH_DT_F32 / BF16 / F16), the queries as
+ * given (the kernel normalises them). C, Z and the window rows lsrc (C itself,
+ * or other rows; unused when win = 0) are rows of c values in cdt, ld* elements
+ * apart, 16-byte aligned; dC, dZ and dlocal [B,T,c] contiguous in odt (cdt, or
+ * KCH_DT_F32). bf16 / fp16 tensors need nh <= 16 (the MFMA kernels' limit: the
+ * caller runs more heads as groups); beyond that the rows are contiguous fp32.
+ * The other tensors are fp32: kc / raw [B,T/m2,c] (the L2-normalised and the
+ * raw compressed rows of C, Z, B_pos, from kch_compress), B_pos [m2,c], sink
+ * [nh] or NULL. Outputs: dq; dC, dZ; dB_pos [m2,c]; dlocal (the window rows'
+ * source gradient) or NULL to add it into dC; dsink [nh] or NULL. Coverage: c
+ * in {64, 128}, nh <= 16 (c = 128) or 32 (c = 64), T a multiple of m2, T >= 1.
+ * ws: 256-byte aligned, kch_hca_attn_bwd_ws_bytes bytes.
  */
 size_t kch_hca_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win);
 int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
-                     const float* kl, const float* lsrc, const float* C, const float* Z,
-                     const float* B_pos, const float* sink, void* dq, float* dC, float* dZ,
-                     float* dBp, float* dlocal, float* sink_part, int B, int T, int nh, int c,
-                     int m2, int win, float scale, int qdt, void* ws, size_t ws_bytes, void* stream);
+                     const void* lsrc, long long ld_l, const void* C, long long ldC, const void* Z,
+                     long long ldZ, const float* B_pos, const float* sink, void* dq, void* dC, void* dZ,
+                     float* dB_pos, void* dlocal, float* dsink, int B, int T, int nh, int c, int m2,
+                     int win, float scale, int qdt, int cdt, int odt, void* ws, size_t ws_bytes,
+                     void* stream);
 
 /*
  * Gradients of the CSA attention: the backward of the sparse attention of
@@ -221,47 +221,48 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
  * reference; run_correctness.py:1312-1473, 2710-2830) with the selection held
  * fixed. Tensors as for kch_hca_attn_bwd, plus: idx [B,T,topk] int32 (the
  * selection, -1 = unused slot), the overlapped compression's inputs Ca, Cb,
- * Za, Zb [B,T,c], Ba, Bb [m,c] (kc / raw from kch_compress_overlapped; kl,
- * lsrc the window rows of Ca), normalize = 0 for normalize_qk=False (queries
- * and keys used as given; q, d_out, dq then fp32). Outputs: dq; dCa, dCb, dZa, dZb [B,T,c] (dCb, dZb
- * must be zeroed by the caller: the last block's second-branch rows receive
- * nothing); dBap, dBbp [B,T/m,m,c]; sink_part as for HCA; slot_grad
- * [B,T,topk] (zeroed by the caller): the gradient of each selected row dotted
- * with that row, which the STE surrogate (ops_csa.py:1033-1099) turns into
- * the indexer's gradient, or NULL; dsel [B,T,T/m] or NULL (normalize = 1,
- * nh <= 16): the same values at their blocks, 0 at the others (the dsel of
- * kch_csa_ste_bwd), added to what it holds with dsel_add; gsum [B,T,c] or NULL: the sum over the selected
- * slots of the selected rows' gradients (written), which the full-softmax
- * surrogate's dense term (ops_csa.py:1050-1071) consumes. The window rows'
- * gradient is added into dCa.
+ * Za, Zb (rows as C and Z), Ba, Bb [m,c] (kc / raw from
+ * kch_compress_overlapped; the window rows are Ca's), normalize = 0 for
+ * normalize_qk=False (queries and keys used as given; every tensor then fp32
+ * and contiguous). Outputs: dq; dCa, dCb, dZa, dZb [B,T,c] (every row written);
+ * dBa, dBb [m,c]; dsink; slot_grad [B,T,topk] (zeroed by the caller) or NULL:
+ * the gradient of each selected row dotted with that row, which the STE
+ * surrogate (ops_csa.py:1033-1099) turns into the indexer's gradient; dsel
+ * [B,T,T/m] or NULL (normalize = 1, nh <= 16): the same values at their blocks,
+ * 0 at the others (the dsel of kch_csa_ste_bwd), added to what it holds with
+ * dsel_add; gsum [B,T,c] or NULL: the sum over the selected slots of the
+ * selected rows' gradients (written), which the full-softmax surrogate's dense
+ * term (ops_csa.py:1050-1071) consumes. The window rows' gradient is added into
+ * dCa.
  */
 size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk);
 int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
-                     const float* kl, const float* lsrc, const int* idx, const float* Ca,
-                     const float* Cb, const float* Za, const float* Zb, const float* Ba,
-                     const float* Bb, const float* sink, void* dq, float* dCa, float* dCb,
-                     float* dZa, float* dZb, float* dBap, float* dBbp, float* sink_part,
-                     float* slot_grad, float* dsel, int dsel_add, float* gsum, int B, int T, int nh,
-                     int c, int m, int topk, int win, float scale, int normalize, int qdt, void* ws,
-                     size_t ws_bytes, void* stream);
+                     const int* idx, const void* Ca, long long ldCa, const void* Cb, long long ldCb,
+                     const void* Za, long long ldZa, const void* Zb, long long ldZb, const float* Ba,
+                     const float* Bb, const float* sink, void* dq, void* dCa, void* dCb, void* dZa,
+                     void* dZb, float* dBa, float* dBb, float* dsink, float* slot_grad, float* dsel,
+                     int dsel_add, float* gsum, int B, int T, int nh, int c, int m, int topk, int win,
+                     float scale, int normalize, int qdt, int cdt, int odt, void* ws, size_t ws_bytes,
+                     void* stream);
 
 /*
  * The STE surrogate's backward for the CSA indexer (ops_csa.py:1033-1099,
  * ste_mode='topk_columns'; the soft weights of ops_csa.py:545-572 over the
  * logits of ops_csa.py:503-536): given dsel [B,T,nb] (each selected slot's
- * value from kch_csa_attn_bwd's slot_grad, scattered to its block, 0
- * elsewhere), the indexer queries q_idx [B,T,nIh,cI], head weights w_idx
- * [B,T,nIh], the compressed indexer keys kc / raw [B,nb,cI] (kch_compress of
- * K_idx, Z_idx, B_idx; kc normalised when normalize), writes dq_idx, dw_idx,
- * dK_idx, dZ_idx and the per-block dB_idx terms dBp [B,nb,m,cI]. fp32; cI in
- * {64, 128}, nIh in {1, 2, 4, 8}, nIh * cI <= 512.
+ * value from kch_csa_attn_bwd at its block, 0 elsewhere), the indexer queries
+ * q_idx [B,T,nIh,cI] and head weights w_idx [B,T,nIh] (qdt, contiguous), the
+ * compressed indexer keys kc / raw [B,nb,cI] (kch_compress of K_idx, Z_idx,
+ * B_idx; kc normalised when normalize) and their sources K_idx, Z_idx (rows of
+ * cI values in cdt, ld* elements apart, 16-byte aligned), writes dq_idx, dw_idx
+ * (qdt), dK_idx, dZ_idx [B,T,cI] (odt: cdt or KCH_DT_F32) and dB_idx [m,cI].
+ * fp32 arithmetic; cI in {64, 128}, nIh in {1, 2, 4, 8}, nIh * cI <= 512.
  */
 size_t kch_csa_ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m);
-int kch_csa_ste_bwd(const float* q_idx, const float* w_idx, const float* kc, const float* raw,
-                    const float* K_idx, const float* Z_idx, const float* B_idx, const float* dsel,
-                    float* dq_idx, float* dw_idx, float* dK_idx, float* dZ_idx, float* dBp, int B,
-                    int T, int m, int nIh, int cI, float scale, int normalize, void* ws,
-                    size_t ws_bytes, void* stream);
+int kch_csa_ste_bwd(const void* q_idx, const void* w_idx, const float* kc, const float* raw,
+                    const void* K_idx, long long ldK, const void* Z_idx, long long ldZ,
+                    const float* B_idx, const float* dsel, void* dq_idx, void* dw_idx, void* dK_idx,
+                    void* dZ_idx, float* dB_idx, int B, int T, int m, int nIh, int cI, float scale,
+                    int normalize, int qdt, int cdt, int odt, void* ws, size_t ws_bytes, void* stream);
 
 /*
  * The dense dsel of kch_csa_ste_bwd from the selection's slots:

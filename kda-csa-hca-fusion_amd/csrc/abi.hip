@@ -399,53 +399,81 @@ int kch_gen_attn(const void* q, const void* kv, const long long* idx, const void
   return hip_status(fn, kch::gen_attn_launch(p, dtype == KCH_DT_F64, (hipStream_t)stream));
 }
 
-size_t kch_hca_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win) {
-  if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m2 < 1 || T % m2 || win < 0) return 0;
-  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, 0);
+// rows of c values of a backward's compression inputs (cdt, ld elements apart):
+// read and written 16 bytes at a time
+static int check_bwd_rows(const char* fn, const char* name, const void* p, long long ld, int c, int dt) {
+  const long long es = dt == 0 ? 4 : 2;
+  if (!p) return fail(KCH_ERR_INVALID, "%s: null tensor pointer (%s)", fn, name);
+  if (ld < c) return fail(KCH_ERR_INVALID, "%s: %s rows of %d values lie %lld apart", fn, name, c, ld);
+  if (((uintptr_t)p & 15) || (ld * es) % 16)
+    return fail(KCH_ERR_INVALID, "%s: %s rows must be 16-byte aligned", fn, name);
+  return KCH_OK;
 }
-
-int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
-                     const float* kl, const float* lsrc, const float* C, const float* Z,
-                     const float* B_pos, const float* sink, void* dq, float* dC, float* dZ,
-                     float* dBp, float* dlocal, float* sink_part, int B, int T, int nh, int c,
-                     int m2, int win, float scale, int qdt, void* ws, size_t ws_bytes, void* stream) {
-  const char* fn = "kch_hca_attn_bwd";
+// gradients' storage: the inputs' or fp32
+static int check_bwd_types(const char* fn, int qdt, int cdt, int odt) {
   if (qdt < 0 || qdt > 2) return fail(KCH_ERR_INVALID, "%s: dtype %d (0 fp32, 1 bf16, 2 fp16)", fn, qdt);
-  if (qdt != 0 && nh > 16)
-    return fail(KCH_ERR_UNSUPPORTED, "%s: bf16 / fp16 q and d_out take at most 16 heads a call (nh=%d)",
-                fn, nh);
-  if (B < 0 || T < 1 || nh < 1 || m2 < 1 || win < 0)
-    return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d T=%d nh=%d m2=%d win=%d (T >= 1)", fn, B, T, nh,
-                m2, win);
-  if (T % m2) return fail(KCH_ERR_INVALID, "%s: T=%d must be a multiple of m2=%d", fn, T, m2);
+  if (cdt < 0 || cdt > 2 || (odt != 0 && odt != cdt))
+    return fail(KCH_ERR_INVALID, "%s: cdt %d, odt %d (cdt 0 fp32, 1 bf16, 2 fp16; odt 0 or cdt)", fn, cdt, odt);
+  return KCH_OK;
+}
+// what the HCA and the CSA attention backward check alike
+static int check_attn_bwd(const char* fn, int B, int T, int nh, int c, int m, int win, float scale, int normalize,
+                          int qdt, int cdt) {
+  if ((qdt != 0 || cdt != 0) && (nh > 16 || !normalize))
+    return fail(KCH_ERR_UNSUPPORTED, "%s: bf16 / fp16 tensors need normalize=1 and at most 16 heads a call (nh=%d)", fn,
+                nh);
+  if (B < 0 || T < 1 || nh < 1 || m < 1 || win < 0)
+    return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d T=%d nh=%d m=%d win=%d (T >= 1)", fn, B, T, nh, m, win);
+  if (T % m) return fail(KCH_ERR_INVALID, "%s: T=%d must be a multiple of m=%d", fn, T, m);
   if (c != 64 && c != 128) return fail(KCH_ERR_UNSUPPORTED, "%s: c=%d not supported (64 or 128)", fn, c);
   if ((long long)T * c * 4 >= (1LL << 31))
     return fail(KCH_ERR_UNSUPPORTED, "%s: T=%d rows of a batch row exceed 2 GiB (32-bit row offsets)", fn, T);
   if (nh * (c / 8) > 256)
     return fail(KCH_ERR_UNSUPPORTED, "%s: nh=%d heads of %d exceed one workgroup", fn, nh, c);
   if (std::isnan(scale)) return fail(KCH_ERR_INVALID, "%s: scale is NaN", fn);
-  if ((long long)B * T * nh * c >= (1LL << 40))
-    return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
+  if ((long long)B * T * nh * c >= (1LL << 40)) return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
+  return KCH_OK;
+}
+
+size_t kch_hca_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win) {
+  if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m2 < 1 || T % m2 || win < 0) return 0;
+  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, -1);
+}
+
+int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
+                     const void* lsrc, long long ld_l, const void* C, long long ldC, const void* Z,
+                     long long ldZ, const float* B_pos, const float* sink, void* dq, void* dC, void* dZ,
+                     float* dB_pos, void* dlocal, float* dsink, int B, int T, int nh, int c, int m2,
+                     int win, float scale, int qdt, int cdt, int odt, void* ws, size_t ws_bytes,
+                     void* stream) {
+  const char* fn = "kch_hca_attn_bwd";
+  if (int rc = check_bwd_types(fn, qdt, cdt, odt)) return rc;
+  if (int rc = check_attn_bwd(fn, B, T, nh, c, m2, win, scale, 1, qdt, cdt)) return rc;
   if (B == 0) return KCH_OK;
-  if (!q || !d_out || !kc || !raw || !C || !Z || !B_pos || !dq || !dC || !dZ || !dBp)
+  if (!q || !d_out || !kc || !raw || !B_pos || !dq || !dC || !dZ || !dB_pos)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
-  if (win > 0 && (!kl || !lsrc)) return fail(KCH_ERR_INVALID, "%s: window rows required (win > 0)", fn);
+  if (int rc = check_bwd_rows(fn, "C", C, ldC, c, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Z", Z, ldZ, c, cdt)) return rc;
+  if (win > 0)
+    if (int rc = check_bwd_rows(fn, "window", lsrc, ld_l, c, cdt)) return rc;
   const size_t need = kch_hca_attn_bwd_ws_bytes(B, T, nh, c, m2, win);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
                 ws ? ws_bytes : (size_t)0);
   if ((uintptr_t)ws & 255) return fail(KCH_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
-  for (const void* ptr : {(const void*)q, (const void*)d_out, (const void*)kc, (const void*)kl,
-                          (const void*)dq})
-    if ((uintptr_t)ptr & 15) return fail(KCH_ERR_INVALID, "%s: q, d_out, kc, kl, dq must be 16-byte aligned", fn);
+  for (const void* ptr : {(const void*)q, (const void*)d_out, (const void*)kc, (const void*)raw, (const void*)B_pos,
+                          (const void*)dq, (const void*)dC, (const void*)dZ, (const void*)dlocal})
+    if ((uintptr_t)ptr & 15) return fail(KCH_ERR_INVALID, "%s: tensors must be 16-byte aligned", fn);
   kch::HcaBwdParams p;
-  p.q = q; p.dout = d_out; p.kc = kc; p.raw = raw; p.kl = kl; p.lsrc = lsrc;
-  p.C = C; p.Z = Z; p.Bpos = B_pos; p.sink = sink;
-  p.dq = dq; p.dC = dC; p.dZ = dZ; p.dBp = dBp; p.dlocal = dlocal; p.sink_part = sink_part;
+  p.q = q; p.dout = d_out; p.sink = sink; p.dq = dq; p.dB = dB_pos; p.dsink = dsink;
   p.qdt = qdt;
   p.B = B; p.T = T; p.nh = nh; p.c = c; p.m2 = m2; p.nb = T / m2; p.win = win;
   p.scale = scale;
-  return hip_status(fn, kch::hca_bwd_dispatch(p, ws, (hipStream_t)stream));
+  kch::BwdFinish f;
+  f.C = C; f.ldC = ldC; f.Z = Z; f.ldZ = ldZ; f.lsrc = lsrc; f.ldl = ld_l; f.Bpos = B_pos; f.kc = kc; f.raw = raw;
+  f.dC = dC; f.dZ = dZ; f.dlocal = dlocal;
+  f.B = B; f.T = T; f.nb = p.nb; f.m = m2; f.win = win; f.cdt = cdt; f.odt = odt;
+  return hip_status(fn, kch::hca_bwd_dispatch(p, f, ws, (hipStream_t)stream));
 }
 
 size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk) {
@@ -455,52 +483,39 @@ size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, in
 }
 
 int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
-                     const float* kl, const float* lsrc, const int* idx, const float* Ca,
-                     const float* Cb, const float* Za, const float* Zb, const float* Ba,
-                     const float* Bb, const float* sink, void* dq, float* dCa, float* dCb,
-                     float* dZa, float* dZb, float* dBap, float* dBbp, float* sink_part,
-                     float* slot_grad, float* dsel, int dsel_add, float* gsum, int B, int T, int nh,
-                     int c, int m, int topk, int win, float scale, int normalize, int qdt, void* ws,
-                     size_t ws_bytes, void* stream) {
+                     const int* idx, const void* Ca, long long ldCa, const void* Cb, long long ldCb,
+                     const void* Za, long long ldZa, const void* Zb, long long ldZb, const float* Ba,
+                     const float* Bb, const float* sink, void* dq, void* dCa, void* dCb, void* dZa,
+                     void* dZb, float* dBa, float* dBb, float* dsink, float* slot_grad, float* dsel,
+                     int dsel_add, float* gsum, int B, int T, int nh, int c, int m, int topk, int win,
+                     float scale, int normalize, int qdt, int cdt, int odt, void* ws, size_t ws_bytes,
+                     void* stream) {
   const char* fn = "kch_csa_attn_bwd";
-  if (qdt < 0 || qdt > 2) return fail(KCH_ERR_INVALID, "%s: dtype %d (0 fp32, 1 bf16, 2 fp16)", fn, qdt);
-  if (qdt != 0 && (nh > 16 || !normalize))
-    return fail(KCH_ERR_UNSUPPORTED,
-                "%s: bf16 / fp16 q and d_out need normalize=1 and at most 16 heads a call (nh=%d)", fn,
-                nh);
-  if (B < 0 || T < 1 || nh < 1 || m < 1 || win < 0 || topk < 0)
-    return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d T=%d nh=%d m=%d win=%d topk=%d (T >= 1)", fn, B,
-                T, nh, m, win, topk);
-  if (T % m) return fail(KCH_ERR_INVALID, "%s: T=%d must be a multiple of m=%d", fn, T, m);
-  if (c != 64 && c != 128) return fail(KCH_ERR_UNSUPPORTED, "%s: c=%d not supported (64 or 128)", fn, c);
-  if ((long long)T * c * 4 >= (1LL << 31))
-    return fail(KCH_ERR_UNSUPPORTED, "%s: T=%d rows of a batch row exceed 2 GiB (32-bit row offsets)", fn, T);
-  if (nh * (c / 8) > 256)
-    return fail(KCH_ERR_UNSUPPORTED, "%s: nh=%d heads of %d exceed one workgroup", fn, nh, c);
+  if (int rc = check_bwd_types(fn, qdt, cdt, odt)) return rc;
+  if (topk < 0) return fail(KCH_ERR_INVALID, "%s: topk=%d must be >= 0", fn, topk);
+  if (int rc = check_attn_bwd(fn, B, T, nh, c, m, win, scale, normalize, qdt, cdt)) return rc;
   if (dsel && (nh > 16 || !normalize))
     return fail(KCH_ERR_UNSUPPORTED, "%s: dsel needs normalize=1 and at most 16 heads a call (nh=%d)", fn, nh);
-  if (std::isnan(scale)) return fail(KCH_ERR_INVALID, "%s: scale is NaN", fn);
-  if ((long long)B * T * nh * c >= (1LL << 40) || (long long)B * T * topk >= (1LL << 40))
-    return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
+  if ((long long)B * T * topk >= (1LL << 39)) return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
   if (B == 0) return KCH_OK;
-  if (!q || !d_out || !kc || !raw || !Ca || !Cb || !Za || !Zb || !Ba || !Bb || !dq || !dCa || !dCb ||
-      !dZa || !dZb || !dBap || !dBbp || (topk > 0 && !idx))
+  if (!q || !d_out || !kc || !raw || !Ba || !Bb || !dq || !dCa || !dCb || !dZa || !dZb || !dBa || !dBb ||
+      (topk > 0 && !idx))
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
-  if (win > 0 && (!kl || !lsrc)) return fail(KCH_ERR_INVALID, "%s: window rows required (win > 0)", fn);
+  if (int rc = check_bwd_rows(fn, "Ca", Ca, ldCa, c, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Cb", Cb, ldCb, c, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Za", Za, ldZa, c, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Zb", Zb, ldZb, c, cdt)) return rc;
   const size_t need = kch_csa_attn_bwd_ws_bytes(B, T, nh, c, m, win, topk);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
                 ws ? ws_bytes : (size_t)0);
   if ((uintptr_t)ws & 255) return fail(KCH_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
-  for (const void* ptr : {(const void*)q, (const void*)d_out, (const void*)kc, (const void*)kl,
-                          (const void*)dq})
-    if ((uintptr_t)ptr & 15) return fail(KCH_ERR_INVALID, "%s: q, d_out, kc, kl, dq must be 16-byte aligned", fn);
+  for (const void* ptr : {(const void*)q, (const void*)d_out, (const void*)kc, (const void*)raw, (const void*)Ba,
+                          (const void*)Bb, (const void*)dq, (const void*)dCa, (const void*)dCb, (const void*)dZa,
+                          (const void*)dZb, (const void*)dsel, (const void*)gsum})
+    if ((uintptr_t)ptr & 15) return fail(KCH_ERR_INVALID, "%s: tensors must be 16-byte aligned", fn);
   kch::HcaBwdParams p;
-  p.q = q; p.dout = d_out; p.kc = kc; p.raw = raw; p.kl = kl; p.lsrc = lsrc;
-  p.C = Ca; p.Z = Za; p.Bpos = Ba; p.sink = sink;
-  p.Cb = Cb; p.Zb = Zb; p.Bb = Bb;
-  p.dq = dq; p.dC = dCa; p.dZ = dZa; p.dBp = dBap; p.dlocal = nullptr; p.sink_part = sink_part;
-  p.dCb = dCb; p.dZb = dZb; p.dBbp = dBbp;
+  p.q = q; p.dout = d_out; p.sink = sink; p.dq = dq; p.dB = dBa; p.dBb = dBb; p.dsink = dsink;
   p.idx = topk > 0 ? idx : nullptr;
   p.topk = topk;
   p.sparse = 1;
@@ -512,7 +527,12 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   p.qdt = qdt;
   p.B = B; p.T = T; p.nh = nh; p.c = c; p.m2 = m; p.nb = T / m; p.win = win;
   p.scale = scale;
-  return hip_status(fn, kch::hca_bwd_dispatch(p, ws, (hipStream_t)stream));
+  kch::BwdFinish f;
+  f.C = Ca; f.ldC = ldCa; f.Z = Za; f.ldZ = ldZa; f.Cb = Cb; f.ldCb = ldCb; f.Zb = Zb; f.ldZb = ldZb;
+  f.lsrc = Ca; f.ldl = ldCa; f.Bpos = Ba; f.Bb = Bb; f.kc = kc; f.raw = raw;
+  f.dC = dCa; f.dZ = dZa; f.dCb = dCb; f.dZb = dZb;
+  f.B = B; f.T = T; f.nb = p.nb; f.m = m; f.win = win; f.normalize = p.normalize; f.cdt = cdt; f.odt = odt;
+  return hip_status(fn, kch::hca_bwd_dispatch(p, f, ws, (hipStream_t)stream));
 }
 
 size_t kch_csa_ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m) {
@@ -521,12 +541,13 @@ size_t kch_csa_ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m) {
   return kch::ste_bwd_ws_bytes(B, T, nIh, cI, m);
 }
 
-int kch_csa_ste_bwd(const float* q_idx, const float* w_idx, const float* kc, const float* raw,
-                    const float* K_idx, const float* Z_idx, const float* B_idx, const float* dsel,
-                    float* dq_idx, float* dw_idx, float* dK_idx, float* dZ_idx, float* dBp, int B,
-                    int T, int m, int nIh, int cI, float scale, int normalize, void* ws,
-                    size_t ws_bytes, void* stream) {
+int kch_csa_ste_bwd(const void* q_idx, const void* w_idx, const float* kc, const float* raw,
+                    const void* K_idx, long long ldK, const void* Z_idx, long long ldZ,
+                    const float* B_idx, const float* dsel, void* dq_idx, void* dw_idx, void* dK_idx,
+                    void* dZ_idx, float* dB_idx, int B, int T, int m, int nIh, int cI, float scale,
+                    int normalize, int qdt, int cdt, int odt, void* ws, size_t ws_bytes, void* stream) {
   const char* fn = "kch_csa_ste_bwd";
+  if (int rc = check_bwd_types(fn, qdt, cdt, odt)) return rc;
   if (B < 0 || T < 1 || m < 1 || nIh < 1)
     return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d T=%d m=%d nIh=%d (T >= 1)", fn, B, T, m, nIh);
   if (T % m) return fail(KCH_ERR_INVALID, "%s: T=%d must be a multiple of m=%d", fn, T, m);
@@ -536,26 +557,28 @@ int kch_csa_ste_bwd(const float* q_idx, const float* w_idx, const float* kc, con
   if (std::isnan(scale)) return fail(KCH_ERR_INVALID, "%s: scale is NaN", fn);
   if ((long long)B * T * (T / m) >= (1LL << 40)) return fail(KCH_ERR_UNSUPPORTED, "%s: too large", fn);
   if (B == 0) return KCH_OK;
-  if (!q_idx || !w_idx || !kc || !raw || !K_idx || !Z_idx || !B_idx || !dsel || !dq_idx || !dw_idx ||
-      !dK_idx || !dZ_idx || !dBp)
+  if (!q_idx || !w_idx || !kc || !raw || !B_idx || !dsel || !dq_idx || !dw_idx || !dK_idx || !dZ_idx || !dB_idx)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
+  if (int rc = check_bwd_rows(fn, "K_idx", K_idx, ldK, cI, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Z_idx", Z_idx, ldZ, cI, cdt)) return rc;
   const size_t need = kch_csa_ste_bwd_ws_bytes(B, T, nIh, cI, m);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
                 ws ? ws_bytes : (size_t)0);
   if ((uintptr_t)ws & 255) return fail(KCH_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
+  for (const void* ptr : {(const void*)q_idx, (const void*)kc, (const void*)raw, (const void*)B_idx, (const void*)dsel,
+                          (const void*)dq_idx, (const void*)dK_idx, (const void*)dZ_idx})
+    if ((uintptr_t)ptr & 15) return fail(KCH_ERR_INVALID, "%s: tensors must be 16-byte aligned", fn);
   kch::SteBwdParams p;
-  p.qi = q_idx; p.w = w_idx; p.kc = kc; p.dsel = dsel; p.dqi = dq_idx; p.dw = dw_idx;
+  p.qi = q_idx; p.w = w_idx; p.kc = kc; p.dsel = dsel; p.dqi = dq_idx; p.dw = dw_idx; p.dB = dB_idx;
+  p.qdt = qdt;
   p.B = B; p.T = T; p.nb = T / m; p.m = m; p.nIh = nIh; p.cI = cI; p.normalize = normalize ? 1 : 0;
   p.scale = scale;
-  kch::HcaBwdParams bp;
-  bp.q = nullptr; bp.dout = nullptr; bp.kc = kc; bp.raw = raw; bp.kl = nullptr; bp.lsrc = nullptr;
-  bp.C = K_idx; bp.Z = Z_idx; bp.Bpos = B_idx; bp.sink = nullptr;
-  bp.dq = nullptr; bp.dC = dK_idx; bp.dZ = dZ_idx; bp.dBp = dBp; bp.dlocal = nullptr;
-  bp.sink_part = nullptr;
-  bp.normalize = p.normalize;
-  bp.B = B; bp.T = T; bp.nh = 1; bp.c = cI; bp.m2 = m; bp.nb = T / m; bp.win = 0; bp.scale = scale;
-  return hip_status(fn, kch::ste_bwd_dispatch(p, bp, ws, (hipStream_t)stream));
+  kch::BwdFinish f;
+  f.C = K_idx; f.ldC = ldK; f.Z = Z_idx; f.ldZ = ldZ; f.Bpos = B_idx; f.kc = kc; f.raw = raw;
+  f.dC = dK_idx; f.dZ = dZ_idx;
+  f.B = B; f.T = T; f.nb = p.nb; f.m = m; f.normalize = p.normalize; f.cdt = cdt; f.odt = odt;
+  return hip_status(fn, kch::ste_bwd_dispatch(p, f, ws, (hipStream_t)stream));
 }
 
 int kch_csa_ste_scatter(const int* idx, const float* slot, float* dsel, int B, int T, int topk, int nb,

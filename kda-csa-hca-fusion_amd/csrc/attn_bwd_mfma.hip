@@ -12,8 +12,9 @@
 // given, with 1/|q| applied to the scores in fp32 (and to ds for dk): bf16
 // ones are exact in one part, so a product with a split key takes two MFMAs
 // and no split copy of them is ever written; fp16 / fp32 ones are split while
-// they are staged. The compressed and window rows are split once by
-// split_rows_kernel.
+// they are staged. The window rows enter the same way (1/|x| in fp32): with
+// bf16 queries and rows their products take one MFMA. The compressed rows,
+// fp32 sums, are split once by split_rows_kernel.
 //
 // attn_bwd_qt_kernel  a workgroup of 4 waves and 8 (bf16) or 4 consecutive
 //   queries, all 16 heads as the MFMA columns (MQA: every key row is shared by
@@ -39,15 +40,16 @@
 //   the packed order of the transposing read of Q / dout). Every fragment read
 //   serves KG groups of 16 keys. Writes per-chunk partials of the compressed
 //   rows and of the window rows; the chunk length follows the grid size.
-// The L2-norm and compression backwards are hca_backward.hip's block and
-// window kernels on these partials (mfma_parts).
+// The L2-norm and compression backwards follow on these partials
+// (attn_bwd_finish.hip).
 //
 // Measured, 16 heads of 128, window 128, bf16, against one wave per query with
 // its own copy of every row and 16 keys per wave on three-MFMA products: HCA
-// B2 T8192 (64 blocks) query pass 254 -> 211 us, window keys 233 -> 150,
-// compressed keys 625 (32 workgroups) -> 61, splits of q and dout 68 -> 0; CSA
-// B2 T4096 top-512 (1024 blocks) query pass 565 -> 349, compressed keys 677 ->
-// 247, window keys 197 -> 114.
+// B2 T8192 (64 blocks) query pass 254 -> 168 us, window keys 233 -> 105,
+// compressed keys 625 (32 workgroups) -> 62, splits of q and dout 68 -> 0; CSA
+// B2 T4096 top-512 (1024 blocks) query pass 565 -> 316, compressed keys 677 ->
+// 261, window keys 197 -> 73. (The window rows in two parts: 211, 150 and 349,
+// 114.)
 
 #include "attn_common.h"
 #include "kch_csa.h"
@@ -104,49 +106,58 @@ __device__ __forceinline__ void store4(void* base, long long off, float4 v, int 
   }
 }
 
-// Rows of HD values, grouped nin to a group, into bf16 hi / lo rows grouped nout
-// to a group (rows nin .. nout-1 of a group zero): x * f = hi + lo, f = 1 /
-// max(|row|, 1e-12) with normalize (written to rinv per output row), else 1.
-// Each lane splits 8 consecutive values (16-byte stores of hi and lo), HD / 8
-// lanes per row; input in T (the rows as given: fp32, bf16 or fp16).
-template <int HD, typename T>
-__global__ __launch_bounds__(256) void split_rows_kernel(const T* x, long long ngroups, int nin,
-                                                         int nout, bf16_t* hi, bf16_t* lo, float* rinv,
-                                                         int normalize) {
+// Rows of HD fp32 values as bf16 hi / lo rows (x = hi + lo): the compressed
+// rows, 8 values a lane.
+template <int HD>
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* x, long long rows, bf16_t* hi, bf16_t* lo) {
   constexpr int LPR = HD / 8;  // lanes per row
-  constexpr int RPB = 256 / LPR;
-  const long long orow = (long long)blockIdx.x * RPB + threadIdx.x / LPR;
-  const int lc = threadIdx.x % LPR;
-  const bool act = orow < ngroups * nout;  // no early return: the row sum shuffles
-  const long long g = act ? orow / nout : 0;
-  const int r = act ? (int)(orow - g * nout) : nin;
+  const long long r = (long long)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  if (r >= rows) return;
+  const long long o = r * HD + 8 * (threadIdx.x % LPR);
   float v[8];
-  if (r < nin) {
-    Load8<T>::run(x + (g * nin + r) * HD + 8 * lc, v);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = 0.f;
-  }
-  float f = 1.f;
-  if (normalize) {
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
-#pragma unroll
-    for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
-    f = r < nin ? l2_inv(ss) : 0.f;
-  }
-  if (!act) return;
+  Load8<float>::run(x + o, v);
   bf16x8 h, l;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float y = v[i] * f;
-    h[i] = (bf16_t)y;
-    l[i] = (bf16_t)(y - (float)h[i]);
+    h[i] = (bf16_t)v[i];
+    l[i] = lo_of(v[i]);
   }
-  *reinterpret_cast<bf16x8*>(hi + orow * HD + 8 * lc) = h;
-  *reinterpret_cast<bf16x8*>(lo + orow * HD + 8 * lc) = l;
-  if (rinv && lc == 0) rinv[orow] = f;
+  *reinterpret_cast<bf16x8*>(hi + o) = h;
+  *reinterpret_cast<bf16x8*>(lo + o) = l;
+}
+
+// The window rows' 1 / max(|row|, 1e-12) and, where asked for, the splits of
+// the rows as given (hi, lo) and normalised (nhi, nlo). Rows ld elements apart
+// in, contiguous out.
+template <int HD, typename T>
+__global__ __launch_bounds__(256) void window_rows_kernel(const T* x, long long ld, long long rows, float* rl,
+                                                          bf16_t* hi, bf16_t* lo, bf16_t* nhi, bf16_t* nlo) {
+  constexpr int LPR = HD / 8;
+  const long long r = (long long)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  const int lc = threadIdx.x % LPR;
+  const bool act = r < rows;  // no early return: the row sum shuffles
+  float v[8];
+  Load8<T>::run(x + (act ? r : 0) * ld + 8 * lc, v);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
+#pragma unroll
+  for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
+  if (!act) return;
+  const float f = l2_inv(ss);
+  if (lc == 0) rl[r] = f;
+  auto split = [&](bf16_t* h, bf16_t* l, float g) {
+    bf16x8 a, b;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a[i] = (bf16_t)(v[i] * g);
+      b[i] = lo_of(v[i] * g);
+    }
+    *reinterpret_cast<bf16x8*>(h + r * HD + 8 * lc) = a;
+    *reinterpret_cast<bf16x8*>(l + r * HD + 8 * lc) = b;
+  };
+  if (hi) split(hi, lo, 1.f);
+  if (nhi) split(nhi, nlo, f);
 }
 
 template <int CTRL>
@@ -318,7 +329,8 @@ __device__ __forceinline__ void soft_step(const float (&s8)[8], const float (&d8
 }
 
 // --------------------------------------------------- query pass, rows in tiles
-template <int HD, typename QT, bool SEL>
+// KX: the window rows are exact in one part (bf16 rows and queries).
+template <int HD, typename QT, bool SEL, bool KX>
 __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int ntile) {
   constexpr bool ONE = Parts<QT>::one;
   constexpr int QW = ONE ? 2 : 1;             // queries per wave
@@ -326,6 +338,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
   constexpr int TILE = 32 * HD, CPR = HD / 8;
   constexpr int LPT = 2 * TILE / 8 / 256;     // 16-byte pieces per thread per step
   __shared__ __attribute__((aligned(16))) bf16_t lds[2][2 * TILE];  // hi, lo
+  __shared__ __attribute__((aligned(16))) float srl[2][32];         // the rows' factors: 1, or 1/|x| (window)
   const int tid = threadIdx.x;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, q = lane >> 4, n = lane & 15;
@@ -364,27 +377,38 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
   const int nw = (p.nb + 31) / 32;
 
   // the 32 rows of step m (hi and lo planes; rows past the end read as zeros)
-  auto fetch = [&](int m, u32x4 (&v)[LPT]) {
+  struct Rows {
+    u32x4 v[LPT];
+    float f;
+  };
+  auto fetch = [&](int m, Rows& x) {
     const bool comp = m < nsc;
     const int r0 = comp ? 32 * m : 32 * (m - nsc);
     const int lim = comp ? nvm : nwin;
     const size_t base = comp ? (size_t)b * p.nb : (size_t)b * p.T + w0;
+    const long long ld = comp ? HD : p.ldl;
     const bf16_t* hi = comp ? p.kc_hi : p.kl_hi;
     const bf16_t* lo = comp ? p.kc_lo : p.kl_lo;
 #pragma unroll
     for (int k = 0; k < LPT; ++k) {
       const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
+      if (KX && k >= LPT / 2 && !comp) break;  // the rows' low parts are zero
       const bf16_t* src = pc < 32 * CPR ? hi : lo;
-      v[k] = u32x4{0, 0, 0, 0};
-      if (r0 + row < lim) v[k] = *reinterpret_cast<const u32x4*>(src + (base + r0 + row) * HD + 8 * c);
+      x.v[k] = u32x4{0, 0, 0, 0};
+      if (r0 + row < lim) x.v[k] = *reinterpret_cast<const u32x4*>(src + (base + r0 + row) * ld + 8 * c);
     }
+    x.f = 1.f;
+    if (tid < 32 && !comp) x.f = r0 + tid < lim ? p.rl[base + r0 + tid] : 0.f;
   };
-  auto put = [&](bf16_t* buf, const u32x4 (&v)[LPT]) {
+  auto put = [&](int k2, int m, const Rows& x) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k) {
       const int pc = tid + 256 * k, w = pc % (32 * CPR), row = w / CPR, c = w % CPR;
-      *reinterpret_cast<u32x4*>(buf + (pc / (32 * CPR)) * TILE + row * HD + 8 * (c ^ tile_swz<HD>(row & 15))) = v[k];
+      if (KX && k >= LPT / 2 && m >= nsc) break;
+      *reinterpret_cast<u32x4*>(lds[k2] + (pc / (32 * CPR)) * TILE + row * HD + 8 * (c ^ tile_swz<HD>(row & 15))) =
+          x.v[k];
     }
+    if (tid < 32) srl[k2][tid] = x.f;
   };
   // the selection's word of step m (uniform per query)
   auto load_word = [&](int m, uint32_t (&w)[QW]) {
@@ -392,9 +416,11 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
     for (int i = 0; i < QW; ++i)
       w[i] = m < nsc && t1 + i < p.T ? p.sel[((size_t)b * p.T + t1 + i) * nw + m] : 0u;
   };
-  // S^T (log2 units, masked) and dP^T of the staged rows: keys 4q+e, 16+4q+e of head n
-  auto scores = [&](int m, const bf16_t* kt, const uint32_t (&sw)[QW], float (&s8)[QW][8], float (&d8)[QW][8]) {
-    const bool comp = m < nsc;
+  // S^T (log2 units, masked) and dP^T of the staged rows of step m (comp: block
+  // rows, else window rows): keys 4q+e, 16+4q+e of head n
+  auto scores = [&](auto comp_, int m, const uint32_t (&sw)[QW], float (&s8)[QW][8], float (&d8)[QW][8]) {
+    constexpr bool comp = decltype(comp_)::value;
+    const bf16_t* kt = lds[m & 1];
     const int r0 = comp ? 32 * m : 32 * (m - nsc);
     const int lim = comp ? nvm : nwin;
 #pragma unroll
@@ -404,16 +430,30 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
       for (int i = 0; i < QW; ++i) sa[i] = da[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       // (rows past the last query's, or before the first query's window)
       if (r0 + 16 * half < lim && (comp || w0 + r0 + 16 * half + 15 > t0 - p.win)) {
+        const bf16_t* kr = kt + 16 * HD * half;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-          const bf16x8 kh = *reinterpret_cast<const bf16x8*>(kt + 16 * HD * half + to.key(s));
-          const bf16x8 kl = *reinterpret_cast<const bf16x8*>(kt + TILE + 16 * HD * half + to.key(s));
+          const bf16x8 kh = *reinterpret_cast<const bf16x8*>(kr + to.key(s));
+          if constexpr (KX && !comp) {
 #pragma unroll
-          for (int i = 0; i < QW; ++i) {
-            sa[i] = mma_kx<ONE>(kh, kl, qh[i][s], ql[i][ONE ? 0 : s], sa[i]);
-            da[i] = mma_kx<ONE>(kh, kl, dh[i][s], dl[i][ONE ? 0 : s], da[i]);
+            for (int i = 0; i < QW; ++i) {
+              sa[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh[i][s], sa[i], 0, 0, 0);
+              da[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, dh[i][s], da[i], 0, 0, 0);
+            }
+          } else {
+            const bf16x8 kl = *reinterpret_cast<const bf16x8*>(kr + TILE + to.key(s));
+#pragma unroll
+            for (int i = 0; i < QW; ++i) {
+              sa[i] = mma_kx<ONE>(kh, kl, qh[i][s], ql[i][ONE ? 0 : s], sa[i]);
+              da[i] = mma_kx<ONE>(kh, kl, dh[i][s], dl[i][ONE ? 0 : s], da[i]);
+            }
           }
         }
+      }
+      float f[4] = {1.f, 1.f, 1.f, 1.f};
+      if constexpr (!comp) {
+        const float4 f4 = *reinterpret_cast<const float4*>(&srl[m & 1][16 * half + 4 * q]);
+        f[0] = f4.x; f[1] = f4.y; f[2] = f4.z; f[3] = f4.w;
       }
 #pragma unroll
       for (int i = 0; i < QW; ++i)
@@ -423,14 +463,27 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
           bool ok;
           if (comp) ok = SEL ? (sw[i] >> (16 * half + 4 * q + e)) & 1u : j < nv[i];
           else ok = (w0 + j <= t1 + i) & (w0 + j > t1 + i - p.win);
-          s8[i][4 * half + e] = ok ? sa[i][e] * scq[i] : -INFINITY;
-          d8[i][4 * half + e] = da[i][e];
+          s8[i][4 * half + e] = ok ? sa[i][e] * (scq[i] * f[e]) : -INFINITY;
+          d8[i][4 * half + e] = da[i][e] * f[e];
         }
     }
   };
 
-  u32x4 pv[LPT];
+  Rows pv;
   uint32_t sw[QW] = {}, swn[QW] = {};
+  // the staged rows of step m to LDS, the next step's requested
+  auto begin = [&](int m) {
+    put(m & 1, m, pv);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < QW; ++i) sw[i] = swn[i];
+    if (m + 1 < nsteps) {
+      fetch(m + 1, pv);
+      if constexpr (SEL) load_word(m + 1, swn);
+    }
+  };
+  typedef std::integral_constant<bool, true> Comp;
+  typedef std::integral_constant<bool, false> Win;
   float m_[QW], l_[QW], ad_[QW];
 #pragma unroll
   for (int i = 0; i < QW; ++i) {
@@ -442,21 +495,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
     fetch(0, pv);
     if constexpr (SEL) load_word(0, swn);
   }
-  for (int m = 0; m < nsteps; ++m) {
-    bf16_t* kt = lds[m & 1];
-    put(kt, pv);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < QW; ++i) sw[i] = swn[i];
-    if (m + 1 < nsteps) {
-      fetch(m + 1, pv);
-      if constexpr (SEL) load_word(m + 1, swn);
-    }
+  auto pass1 = [&](auto comp_, int m) {
+    begin(m);
     float s8[QW][8], d8[QW][8];
-    scores(m, kt, sw, s8, d8);
+    scores(comp_, m, sw, s8, d8);
 #pragma unroll
     for (int i = 0; i < QW; ++i) soft_step(s8[i], d8[i], m_[i], l_[i], ad_[i]);
-  }
+  };
+  for (int m = 0; m < nsc; ++m) pass1(Comp{}, m);
+  for (int m = nsc; m < nsteps; ++m) pass1(Win{}, m);
   Soft sf[QW];
 #pragma unroll
   for (int i = 0; i < QW; ++i) sf[i] = close_softmax(p, n, m_[i], l_[i], ad_[i]);
@@ -473,19 +520,20 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
     if constexpr (SEL) load_word(0, swn);
     __syncthreads();  // pass 1's last reads are done
   }
-  for (int m = 0; m < nsteps; ++m) {
-    bf16_t* kt = lds[m & 1];
-    put(kt, pv);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < QW; ++i) sw[i] = swn[i];
-    if (m + 1 < nsteps) {
-      fetch(m + 1, pv);
-      if constexpr (SEL) load_word(m + 1, swn);
-    }
+  auto pass2 = [&](auto comp_, int m) {
+    constexpr bool comp = decltype(comp_)::value;
+    begin(m);
     float s8[QW][8], d8[QW][8];
-    scores(m, kt, sw, s8, d8);
-    bf16x8 bh[QW], bl[QW];
+    scores(comp_, m, sw, s8, d8);
+    const bf16_t* kt = lds[m & 1];
+    bf16x8 bh[QW], bl[QW];  // ds^T, times the rows' factors
+    float f[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+    if constexpr (!comp) {
+      const float4 x = *reinterpret_cast<const float4*>(&srl[m & 1][4 * q]);
+      const float4 y = *reinterpret_cast<const float4*>(&srl[m & 1][16 + 4 * q]);
+      f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w;
+      f[4] = y.x; f[5] = y.y; f[6] = y.z; f[7] = y.w;
+    }
 #pragma unroll
     for (int i = 0; i < QW; ++i) {
       float pe[8], dse[8];
@@ -493,11 +541,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
       for (int e = 0; e < 8; ++e) {
         pe[e] = fast_exp2(s8[i][e] - sf[i].lse2);  // masked or dead head: 0
         dse[e] = pe[e] * (d8[i][e] - sf[i].D) * p.scale;
-        bh[i][e] = (bf16_t)dse[e];
-        bl[i][e] = lo_of(dse[e]);
+        const float x = dse[e] * f[e];
+        bh[i][e] = (bf16_t)x;
+        bl[i][e] = lo_of(x);
       }
-      if constexpr (SEL) {
-        if (m < nsc && (p.dsel || p.gsum)) {
+      if constexpr (SEL && comp) {
+        if (p.dsel || p.gsum) {
           // sum over the heads of p ((dp - D) s + dp): the row's gradient dotted with the row
           float g[8];
 #pragma unroll
@@ -529,11 +578,18 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_qt_kernel(HcaBwdParams p, int
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
       const bf16x8 vh = MqaWave<HD>::vt_frag(kt, to, tt);
-      const bf16x8 vl = MqaWave<HD>::vt_frag(kt + TILE, to, tt);
+      if constexpr (KX && !comp) {
 #pragma unroll
-      for (int i = 0; i < QW; ++i) dq[i][tt] = mfma3(vh, vl, bh[i], bl[i], dq[i][tt]);
+        for (int i = 0; i < QW; ++i) dq[i][tt] = mfma2b(vh, bh[i], bl[i], dq[i][tt]);
+      } else {
+        const bf16x8 vl = MqaWave<HD>::vt_frag(kt + TILE, to, tt);
+#pragma unroll
+        for (int i = 0; i < QW; ++i) dq[i][tt] = mfma3(vh, vl, bh[i], bl[i], dq[i][tt]);
+      }
     }
-  }
+  };
+  for (int m = 0; m < nsc; ++m) pass2(Comp{}, m);
+  for (int m = nsc; m < nsteps; ++m) pass2(Win{}, m);
 #pragma unroll
   for (int i = 0; i < QW; ++i) {
     if (t1 + i >= p.T) break;  // whole waves
@@ -605,8 +661,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
   const long long cbytes = (long long)p.nb * ROWB, wbytes = nwin > 0 ? (long long)p.T * ROWB : 0;
   const __amdgpu_buffer_rsrc_t rs_ch = rsrc(p.kc_hi + (size_t)b * p.nb * HD, cbytes);
   const __amdgpu_buffer_rsrc_t rs_cl = rsrc(p.kc_lo + (size_t)b * p.nb * HD, cbytes);
-  const __amdgpu_buffer_rsrc_t rs_wh = rsrc(nwin > 0 ? p.kl_hi + (size_t)b * p.T * HD : p.kc_hi, wbytes);
-  const __amdgpu_buffer_rsrc_t rs_wl = rsrc(nwin > 0 ? p.kl_lo + (size_t)b * p.T * HD : p.kc_lo, wbytes);
+  const __amdgpu_buffer_rsrc_t rs_wh = rsrc(nwin > 0 ? p.kn_hi + (size_t)b * p.T * HD : p.kc_hi, wbytes);
+  const __amdgpu_buffer_rsrc_t rs_wl = rsrc(nwin > 0 ? p.kn_lo + (size_t)b * p.T * HD : p.kc_lo, wbytes);
   const bool has_idx = nsel > 0;
   const __amdgpu_buffer_rsrc_t rs_idx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int*>(has_idx ? p.idx + bt * p.topk : nullptr), 0, has_idx ? nsel * 4 : 0, 0x00020000);
@@ -785,7 +841,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
 // MODE 0: compressed rows (HCA: visible when n < (t+1) / m2; CSA: selected),
 // chunk ci of part_qc queries; MODE 1: window rows (row u seen by t in
 // [u, u + win)), chunk ci of win_qc of the queries that see the tile.
-template <int HD, int MODE, typename QT, int KG>
+// KX (MODE 1): the window rows are exact in one part (bf16 rows and queries).
+template <int HD, int MODE, typename QT, int KG, bool KX>
 __global__ __launch_bounds__(256, 2) void attn_bwd_k_kernel(HcaBwdParams p, int nchunk) {
   constexpr bool ONE = Parts<QT>::one;
   constexpr int NS = HD / 32, NT = HD / 16;
@@ -819,21 +876,25 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_k_kernel(HcaBwdParams p, int 
   const TileOffsets<HD> to;
 
   // key fragments (B operand of S = Q K^T): rows rw + 16 g + n, dims 32s + 8q ..
-  bf16x8 kh[KG][NS], kl[KG][NS];
+  bf16x8 kh[KG][NS], kl[KG][KX ? 1 : NS];
+  float rk1[KG];  // the row's factor: 1, or 1/|x| (window)
   f32x4 dk[KG][NT];
 #pragma unroll
   for (int g = 0; g < KG; ++g) {
     const int rk = rw + 16 * g + n;
     const bool ok = rk < nrows;
-    const bf16_t* bh = MODE == 0 ? p.kc_hi + (size_t)b * p.nb * HD : p.kl_hi + (size_t)b * p.T * HD;
-    const bf16_t* bl = MODE == 0 ? p.kc_lo + (size_t)b * p.nb * HD : p.kl_lo + (size_t)b * p.T * HD;
-    const size_t ro = (size_t)(ok ? rk : 0) * HD + 8 * q;
+    const size_t row = (size_t)b * nrows + (ok ? rk : 0);
+    const size_t ro = row * (MODE == 0 ? HD : p.ldl) + 8 * q;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      kh[g][s] = *reinterpret_cast<const bf16x8*>(bh + ro + 32 * s);
-      kl[g][s] = *reinterpret_cast<const bf16x8*>(bl + ro + 32 * s);
-      if (!ok) kh[g][s] = kl[g][s] = bf16x8{};
+      kh[g][s] = *reinterpret_cast<const bf16x8*>((MODE == 0 ? p.kc_hi : p.kl_hi) + ro + 32 * s);
+      if (!ok) kh[g][s] = bf16x8{};
+      if constexpr (!KX) {
+        kl[g][s] = *reinterpret_cast<const bf16x8*>((MODE == 0 ? p.kc_lo : p.kl_lo) + ro + 32 * s);
+        if (!ok) kl[g][s] = bf16x8{};
+      }
     }
+    rk1[g] = MODE == 0 ? 1.f : p.rl[row];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) dk[g][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -938,8 +999,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_k_kernel(HcaBwdParams p, int 
           }
 #pragma unroll
           for (int g = 0; g < KG; ++g) {
-            sa[g] = mma_xk<ONE>(xh, xl, kh[g][s], kl[g][s], sa[g]);
-            da[g] = mma_xk<ONE>(yh, yl, kh[g][s], kl[g][s], da[g]);
+            if constexpr (KX) {
+              sa[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, kh[g][s], sa[g], 0, 0, 0);
+              da[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yh, kh[g][s], da[g], 0, 0, 0);
+            } else {
+              sa[g] = mma_xk<ONE>(xh, xl, kh[g][s], kl[g][s], sa[g]);
+              da[g] = mma_xk<ONE>(yh, yl, kh[g][s], kl[g][s], da[g]);
+            }
           }
         }
         // lane: heads 4q .. 4q+3 of query tq, keys rw + 16 g + n
@@ -953,8 +1019,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_k_kernel(HcaBwdParams p, int 
           const bool vis = visible(tq, rw + 16 * g + n);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float pe = vis ? fast_exp2(sa[g][e] * (Rs[e] * p.scale * kLog2eF) - Ls[e]) : 0.f;
-            const float dse = pe * (da[g][e] - Ds[e]) * p.scale * Rs[e];
+            const float pe = vis ? fast_exp2(sa[g][e] * (Rs[e] * (rk1[g] * p.scale * kLog2eF)) - Ls[e]) : 0.f;
+            const float dse = pe * (da[g][e] * rk1[g] - Ds[e]) * p.scale * Rs[e];
             ash[g][4 * i + e] = (bf16_t)dse;
             asl[g][4 * i + e] = lo_of(dse);
             aph[g][4 * i + e] = (bf16_t)pe;
@@ -1053,11 +1119,12 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
   const KeyPlan k = key_plan(B, T, nb, win);
   size_t z = 3 * al256m(BT * 16 * 4);                  // lse, D, 1/|q| (16 heads)
   z += 2 * al256m((size_t)B * nb * c * 2);              // compressed rows hi / lo
-  if (win > 0) z += 2 * al256m(BT * c * 2);             // window rows hi / lo
+  // window rows: factors, the splits of the rows and of the normalised rows
+  if (win > 0) z += al256m(BT * 4) + 4 * al256m(BT * c * 2);
   z += al256m((size_t)B * k.nchunk * nb * c * 4);       // compressed-row partials
   if (win > 0) z += al256m(BT * k.wnc * c * 4);         // window-row partials
-  if (topk > 0) z += al256m(BT * ((nb + 31) / 32) * 4);  // selection bitmap
   if (topk > 0) {
+    z += al256m(BT * ((nb + 31) / 32) * 4);              // selection bitmap
     z += al256m(BT * nb * 4);                            // dense slot gradients
     if (!attn_bwd_dense_rows(nb, topk)) z += al256m(BT * topk * 4);  // per slot
   }
@@ -1066,42 +1133,65 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
 
 hipError_t sel_bitmap_launch(const int* idx, uint32_t* sel, long long nq, int topk, int nw, hipStream_t s);
 
-template <int HD, typename QT>
+template <int HD, typename QT, bool KX>
 static void launch_passes(const HcaBwdParams& p, const KeyPlan& k, hipStream_t s) {
   const int tq = Parts<QT>::one ? 8 : 4;  // queries per workgroup of the tiled query pass
   const int nt = (p.T + tq - 1) / tq;
   const dim3 qg((unsigned)((long long)p.B * nt));
   if (!p.sparse)
-    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, false>), qg, dim3(256), 0, s, p, nt);
+    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, false, KX>), qg, dim3(256), 0, s, p, nt);
   else if (attn_bwd_dense_rows(p.nb, p.topk))
-    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, true>), qg, dim3(256), 0, s, p, nt);
+    hipLaunchKernelGGL((attn_bwd_qt_kernel<HD, QT, true, KX>), qg, dim3(256), 0, s, p, nt);
   else
     hipLaunchKernelGGL((attn_bwd_q_kernel<HD, QT>), dim3((unsigned)(p.B * ((p.T + 3) / 4))), dim3(256), 0, s, p);
   if (p.nb > 0 && !(p.sparse && p.topk == 0)) {
     const dim3 g((p.nb + 64 * k.kg - 1) / (64 * k.kg) * k.nchunk, p.B);
     if (k.kg == 2)
-      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 2>), g, dim3(256), 0, s, p, k.nchunk);
+      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 2, false>), g, dim3(256), 0, s, p, k.nchunk);
     else
-      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 1>), g, dim3(256), 0, s, p, k.nchunk);
+      hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 0, QT, 1, false>), g, dim3(256), 0, s, p, k.nchunk);
   }
   if (p.win > 0)
-    hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 1, QT, 2>), dim3((p.T + 127) / 128 * k.wnc, p.B), dim3(256), 0, s, p,
-                       k.wnc);
+    hipLaunchKernelGGL((attn_bwd_k_kernel<HD, 1, QT, 2, KX>), dim3((p.T + 127) / 128 * k.wnc, p.B), dim3(256), 0, s,
+                       p, k.wnc);
+}
+
+// The window rows' factors and splits: the rows as given unless they are used in
+// place (ldl = f.ldl), the normalised rows for the gathering query pass.
+template <int HD, typename T>
+static void launch_window_rows(const HcaBwdParams& p, const BwdFinish& f, hipStream_t s) {
+  constexpr int rpb = 256 / (HD / 8);
+  const long long BT = (long long)p.B * p.T;
+  hipLaunchKernelGGL((window_rows_kernel<HD, T>), dim3((unsigned)((BT + rpb - 1) / rpb)), dim3(256), 0, s,
+                     static_cast<const T*>(f.lsrc), f.ldl, BT, const_cast<float*>(p.rl),
+                     p.kl_lo ? const_cast<bf16_t*>(p.kl_hi) : nullptr, const_cast<bf16_t*>(p.kl_lo),
+                     const_cast<bf16_t*>(p.kn_hi), const_cast<bf16_t*>(p.kn_lo));
 }
 
 template <int HD>
-static void launch_splits(const HcaBwdParams& p, hipStream_t s) {
+static hipError_t run_passes(const HcaBwdParams& p, const BwdFinish& f, const KeyPlan& k, hipStream_t s) {
   constexpr int rpb = 256 / (HD / 8);  // rows per workgroup
-  const long long BT = (long long)p.B * p.T, bn = (long long)p.B * p.nb;
-  if (p.nb > 0)
-    hipLaunchKernelGGL((split_rows_kernel<HD, float>), dim3((unsigned)((bn + rpb - 1) / rpb)), dim3(256), 0, s, p.kc,
-                       bn, 1, 1, p.kc_hi, p.kc_lo, (float*)nullptr, 0);
-  if (p.win > 0)
-    hipLaunchKernelGGL((split_rows_kernel<HD, float>), dim3((unsigned)((BT + rpb - 1) / rpb)), dim3(256), 0, s, p.kl,
-                       BT, 1, 1, p.kl_hi, p.kl_lo, (float*)nullptr, 0);
+  const long long bn = (long long)p.B * p.nb;
+  if (bn > 0)
+    hipLaunchKernelGGL((split_rows_kernel<HD>), dim3((unsigned)((bn + rpb - 1) / rpb)), dim3(256), 0, s, f.kc, bn,
+                       const_cast<bf16_t*>(p.kc_hi), const_cast<bf16_t*>(p.kc_lo));
+  if (p.win > 0) {
+    if (f.cdt == DT_BF16) launch_window_rows<HD, bf16_t>(p, f, s);
+    else if (f.cdt == DT_F16) launch_window_rows<HD, _Float16>(p, f, s);
+    else launch_window_rows<HD, float>(p, f, s);
+  }
+  if (p.qdt == DT_BF16) {
+    if (p.win > 0 && !p.kl_lo) launch_passes<HD, bf16_t, true>(p, k, s);
+    else launch_passes<HD, bf16_t, false>(p, k, s);
+  } else if (p.qdt == DT_F16) {
+    launch_passes<HD, _Float16, false>(p, k, s);
+  } else {
+    launch_passes<HD, float, false>(p, k, s);
+  }
+  return hipGetLastError();
 }
 
-hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
+hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t s) {
   const int HD = p.c;
   const size_t BT = (size_t)p.B * p.T;
   const KeyPlan k = key_plan(p.B, p.T, p.nb, p.win);
@@ -1116,18 +1206,26 @@ hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
   p.rq = reinterpret_cast<float*>(take(BT * 16 * 4));
   p.kc_hi = reinterpret_cast<bf16_t*>(take((size_t)p.B * p.nb * HD * 2));
   p.kc_lo = reinterpret_cast<bf16_t*>(take((size_t)p.B * p.nb * HD * 2));
-  p.kl_hi = p.kl_lo = nullptr;
+  const bool tiled = !p.sparse || attn_bwd_dense_rows(p.nb, p.topk);
   if (p.win > 0) {
-    p.kl_hi = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
-    p.kl_lo = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
+    p.rl = reinterpret_cast<float*>(take(BT * 4));
+    if (f.cdt == DT_BF16 && p.qdt == DT_BF16) {
+      p.kl_hi = static_cast<const bf16_t*>(f.lsrc);
+      p.ldl = f.ldl;
+    } else {
+      p.kl_hi = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
+      p.kl_lo = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
+      p.ldl = HD;
+    }
+    if (!tiled) {
+      p.kn_hi = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
+      p.kn_lo = reinterpret_cast<bf16_t*>(take(BT * HD * 2));
+    }
   }
   p.part_b = reinterpret_cast<float*>(take((size_t)p.B * k.nchunk * p.nb * HD * 4));
   p.part_w = p.win > 0 ? reinterpret_cast<float*>(take(BT * k.wnc * HD * 4)) : nullptr;
-  p.sel = nullptr;
-  p.mfma_parts = 1;
   p.part_qc = k.qc;
   p.win_qc = k.wqc;
-  p.win_nc = k.wnc;
   if (p.idx && p.topk > 0) {
     const int nw = (p.nb + 31) / 32;
     uint32_t* sel = reinterpret_cast<uint32_t*>(take(BT * nw * 4));
@@ -1139,44 +1237,37 @@ hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s) {
       p.dsel = own;
       p.dsel_add = 0;
     }
-    if (p.dsel && !attn_bwd_dense_rows(p.nb, p.topk)) p.slot_ws = reinterpret_cast<float*>(take(BT * p.topk * 4));
+    if (p.dsel && !tiled) p.slot_ws = reinterpret_cast<float*>(take(BT * p.topk * 4));
   }
-#define KCH_BWD(HDV)                             \
-  do {                                           \
-    launch_splits<HDV>(p, s);                    \
-    if (p.qdt == DT_BF16)                        \
-      launch_passes<HDV, bf16_t>(p, k, s);       \
-    else if (p.qdt == DT_F16)                    \
-      launch_passes<HDV, _Float16>(p, k, s);     \
-    else                                         \
-      launch_passes<HDV, float>(p, k, s);        \
-  } while (0)
-  if (HD == 64)
-    KCH_BWD(64);
-  else
-    KCH_BWD(128);
-#undef KCH_BWD
+  hipError_t e = HD == 64 ? run_passes<64>(p, f, k, s) : run_passes<128>(p, f, k, s);
+  if (e != hipSuccess) return e;
   if (p.slot_ws) {
     if (!p.dsel_add) {
-      hipError_t e = fill_u32(p.dsel, (long long)BT * p.nb, 0u, s);
+      e = fill_u32(p.dsel, (long long)BT * p.nb, 0u, s);
       if (e != hipSuccess) return e;
     }
-    hipError_t e = ste_scatter_launch(p.idx, p.slot_ws, p.dsel, (long long)BT, p.topk, p.nb, s);
+    e = ste_scatter_launch(p.idx, p.slot_ws, p.dsel, (long long)BT, p.topk, p.nb, s);
     if (e != hipSuccess) return e;
   }
   if (p.slot_grad && p.idx) {
     const long long ns = (long long)BT * p.topk;
     hipLaunchKernelGGL(slot_gather_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, s, p.idx, p.dsel,
                        p.slot_grad, ns, p.topk, p.nb);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   if (p.nb > 0 && p.sparse && p.topk == 0) {
     // no selection: the compressed rows receive nothing
     e = fill_u32(p.part_b, (long long)p.B * k.nchunk * p.nb * HD, 0u, s);
     if (e != hipSuccess) return e;
   }
-  return hca_bwd_finish_launch(p, k.nchunk, s);
+  f.part_b = p.part_b;
+  f.part_w = p.part_w;
+  f.rl = p.rl;
+  f.nchunk = k.nchunk;
+  f.part_qc = k.qc;
+  f.win_nc = k.wnc;
+  return bwd_finish_launch(f, HD, s);
 }
 
 }  // namespace kch

@@ -344,14 +344,8 @@ __global__ __launch_bounds__(HD) void hca_bwd_block_kernel(HcaBwdParams p, int n
   const int n = blockIdx.x, b = blockIdx.y, c = threadIdx.x;
   const int tile = n / NBT, i = n % NBT;
   float dk = 0.f;
-  if (p.mfma_parts) {
-    // the chunks from the first one that holds a query seeing block n
-    for (int ci = ((n + 1) * p.m2 - 1) / p.part_qc; ci < nchunk; ++ci)
-      dk += p.part_b[(((size_t)b * nchunk + ci) * p.nb + n) * HD + c];
-  } else {
-    for (int ci = 0; ci < nchunk; ++ci)
-      dk += p.part_b[((((size_t)b * ntile + tile) * nchunk + ci) * NBT + i) * HD + c];
-  }
+  for (int ci = 0; ci < nchunk; ++ci)
+    dk += p.part_b[((((size_t)b * ntile + tile) * nchunk + ci) * NBT + i) * HD + c];
   const size_t ri = ((size_t)b * p.nb + n) * HD + c;
   const float y = p.kc[ri], r = p.raw[ri];
   const float yd = block_sum<HD>(y * dk, sh);
@@ -391,6 +385,10 @@ __global__ __launch_bounds__(HD) void hca_bwd_block_kernel(HcaBwdParams p, int n
         p.dZb[ti] = dz;
       }
       p.dBbp[(((size_t)b * p.nb + n) * m2 + j) * HD + c] = dz;
+      if (n == p.nb - 1) {  // the last block's second branch feeds no block
+        const size_t ti = ((size_t)b * p.T + (size_t)n * m2 + j) * HD + c;
+        p.dCb[ti] = p.dZb[ti] = 0.f;
+      }
     }
     return;
   }
@@ -421,12 +419,8 @@ __global__ __launch_bounds__(HD) void hca_bwd_window_kernel(HcaBwdParams p, int 
   const int u = blockIdx.x, b = blockIdx.y, c = threadIdx.x;
   const int tile = u / NBT, i = u % NBT;
   float dk = 0.f;
-  if (p.mfma_parts) {
-    for (int ci = 0; ci < p.win_nc; ++ci) dk += p.part_w[(((size_t)ci * p.B + b) * p.T + u) * HD + c];
-  } else {
-    for (int ci = 0; ci < nchunk; ++ci)
-      dk += p.part_w[((((size_t)b * ntile + tile) * nchunk + ci) * NBT + i) * HD + c];
-  }
+  for (int ci = 0; ci < nchunk; ++ci)
+    dk += p.part_w[((((size_t)b * ntile + tile) * nchunk + ci) * NBT + i) * HD + c];
   const size_t ri = ((size_t)b * p.T + u) * HD + c;
   const float y = p.kl[ri], x = p.lsrc[ri];
   const float yd = block_sum<HD>(y * dk, sh);
@@ -518,50 +512,92 @@ hipError_t sel_bitmap_launch(const int* idx, uint32_t* sel, long long nq, int to
   return hipGetLastError();
 }
 
-// The L2-norm and compression backward of the compressed rows and the window
-// rows' L2-norm backward, from MFMA-path partials (p.mfma_parts).
-hipError_t hca_bwd_finish_launch(const HcaBwdParams& p, int nchunk, hipStream_t s) {
-  if (p.nb > 0) {
-    if (p.c == 64)
-      hipLaunchKernelGGL((hca_bwd_block_kernel<64>), dim3(p.nb, p.B), dim3(64), 0, s, p, nchunk, 0);
-    else
-      hipLaunchKernelGGL((hca_bwd_block_kernel<128>), dim3(p.nb, p.B), dim3(128), 0, s, p, nchunk, 0);
-  }
-  if (p.win > 0) {
-    if (p.c == 64)
-      hipLaunchKernelGGL((hca_bwd_window_kernel<64>), dim3(p.T, p.B), dim3(64), 0, s, p, 0, 0);
-    else
-      hipLaunchKernelGGL((hca_bwd_window_kernel<128>), dim3(p.T, p.B), dim3(128), 0, s, p, 0, 0);
-  }
-  return hipGetLastError();
+// The regions behind either path's own: the per-block dB terms, the sink's
+// per-query terms and the scratch of their sums.
+struct Tail {
+  size_t terms, sink, scratch;  // bytes
+};
+static Tail tail(int B, int T, int nh, int c, int m2) {
+  Tail t;
+  t.terms = al256((size_t)B * T * c * 4);
+  t.sink = al256((size_t)B * T * nh * 4);
+  const size_t a = sum_rows_ws_bytes((long long)B * (T / m2), m2 * c), b = sum_rows_ws_bytes((long long)B * T, nh);
+  t.scratch = a > b ? a : b;
+  return t;
 }
 
-size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk) {
+static size_t path_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk) {
   const Plan z = plan(B, T, T / m2, win, c);
   const size_t sel = topk > 0 ? al256((size_t)B * T * ((T / m2 + 31) / 32) * 4) : 0;
-  const size_t simt = 3 * al256((size_t)B * T * nh * 4) + al256(z.part_b * 4) + al256(z.part_w * 4) + sel;
+  const size_t simt = 3 * al256((size_t)B * T * nh * 4) + al256(z.part_b * 4) + al256(z.part_w * 4) + sel +
+                      al256((size_t)B * T * c * 4);
   // the MFMA path (normalised rows) needs its own regions; the larger of the two
   const size_t mfma = nh <= 16 ? attn_bwd_mfma_ws_bytes(B, T, c, m2, win, topk) : 0;
   return simt > mfma ? simt : mfma;
 }
 
-hipError_t hca_bwd_dispatch(HcaBwdParams p, void* ws, hipStream_t stream) {
-  if (attn_bwd_mfma_supported(p)) return attn_bwd_mfma_dispatch(p, ws, stream);
-  if (p.qdt != DT_F32) return hipErrorInvalidValue;  // the SIMT kernels read fp32 rows
+size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk) {
+  const Tail t = tail(B, T, nh, c, m2);
+  return path_ws_bytes(B, T, nh, c, m2, win, topk < 0 ? 0 : topk) + (topk >= 0 ? 2 : 1) * t.terms + t.sink + t.scratch;
+}
+
+static hipError_t simt_dispatch(HcaBwdParams p, const BwdFinish& f, void* ws, hipStream_t stream) {
+  // the SIMT kernels read and write contiguous fp32 rows
+  if (p.qdt != DT_F32 || f.cdt != DT_F32 || f.odt != DT_F32 || f.ldC != p.c || f.ldZ != p.c ||
+      (f.Cb && (f.ldCb != p.c || f.ldZb != p.c)) || p.dsel)
+    return hipErrorInvalidValue;
+  p.C = static_cast<const float*>(f.C); p.Z = static_cast<const float*>(f.Z);
+  p.Cb = static_cast<const float*>(f.Cb); p.Zb = static_cast<const float*>(f.Zb);
+  p.lsrc = static_cast<const float*>(f.lsrc);
+  p.Bpos = f.Bpos; p.Bb = f.Bb; p.kc = f.kc; p.raw = f.raw;
+  p.dC = static_cast<float*>(f.dC); p.dZ = static_cast<float*>(f.dZ);
+  p.dCb = static_cast<float*>(f.dCb); p.dZb = static_cast<float*>(f.dZb);
+  p.dlocal = static_cast<float*>(f.dlocal);
+  p.dBp = f.dBp; p.dBbp = f.dBbp;
   const Plan z = plan(p.B, p.T, p.nb, p.win, p.c);
   char* w = static_cast<char*>(ws);
   const size_t per = al256((size_t)p.B * p.T * p.nh * 4);
   p.lse = reinterpret_cast<float*>(w);
   p.dval = reinterpret_cast<float*>(w + per);
   p.rq = reinterpret_cast<float*>(w + 2 * per);
-  p.part_b = reinterpret_cast<float*>(w + 3 * per);
-  p.part_w = reinterpret_cast<float*>(w + 3 * per + al256(z.part_b * 4));
-  p.sel = nullptr;
-  if (p.idx && p.topk > 0) {
-    uint32_t* sel = reinterpret_cast<uint32_t*>(w + 3 * per + al256(z.part_b * 4) + al256(z.part_w * 4));
-    p.sel = sel;
+  w += 3 * per;
+  p.part_b = reinterpret_cast<float*>(w);
+  w += al256(z.part_b * 4);
+  p.part_w = reinterpret_cast<float*>(w);
+  w += al256(z.part_w * 4);
+  if (p.win > 0) {
+    // window rows as fp32 keys
+    float* kl = reinterpret_cast<float*>(w);
+    const hipError_t e = l2norm_rows_dispatch(f.lsrc, f.ldl, kl, 1, p.B * p.T, p.c, p.normalize, DT_F32, stream);
+    if (e != hipSuccess) return e;
+    p.kl = kl;
   }
+  w += al256((size_t)p.B * p.T * p.c * 4);
+  p.sel = nullptr;
+  if (p.idx && p.topk > 0) p.sel = reinterpret_cast<uint32_t*>(w);
   return p.c == 64 ? launch_hca_bwd<64>(p, z, stream) : launch_hca_bwd<128>(p, z, stream);
+}
+
+hipError_t hca_bwd_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t stream) {
+  const bool two = f.Cb != nullptr;
+  const Tail t = tail(p.B, p.T, p.nh, p.c, p.m2);
+  char* w = static_cast<char*>(ws) + path_ws_bytes(p.B, p.T, p.nh, p.c, p.m2, p.win, p.topk);
+  f.dBp = reinterpret_cast<float*>(w);
+  w += t.terms;
+  if (two) {
+    f.dBbp = reinterpret_cast<float*>(w);
+    w += t.terms;
+  }
+  p.sink_part = p.dsink ? reinterpret_cast<float*>(w) : nullptr;
+  void* scratch = w + t.sink;
+  hipError_t e = attn_bwd_mfma_supported(p) ? attn_bwd_mfma_dispatch(p, f, ws, stream) : simt_dispatch(p, f, ws, stream);
+  if (e != hipSuccess) return e;
+  const long long blocks = (long long)p.B * p.nb;
+  e = sum_rows_launch(f.dBp, p.dB, blocks, p.m2 * p.c, 1.f, scratch, stream);
+  if (e == hipSuccess && two) e = sum_rows_launch(f.dBbp, p.dBb, blocks, p.m2 * p.c, 1.f, scratch, stream);
+  if (e == hipSuccess && p.dsink)
+    e = sum_rows_launch(p.sink_part, p.dsink, (long long)p.B * p.T, p.nh, -1.f, scratch, stream);
+  return e;
 }
 
 }  // namespace kch

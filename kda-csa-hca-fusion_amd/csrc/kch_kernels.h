@@ -63,85 +63,132 @@ bool kda_chunk_bwd_supported(int K, int V, int dtype);
 size_t kda_chunk_bwd_ws_bytes(int B, int T, int H, int HV, int K, int V);
 hipError_t kda_chunk_bwd_dispatch(KdaBwdParams p, int dtype, void* ws, hipStream_t stream);
 
-// Gradients of the HCA attention (hca_backward.hip), fp32 tensors, c in
-// {64, 128}, nh <= 256 / (c / 8), T a multiple of m2.
+// The last stage of the attention and indexer backwards (attn_bwd_finish.hip):
+// the compression's inputs and their gradients, rows of c channels, ld* elements
+// apart where given (gradients contiguous), in cdt / odt.
+struct BwdFinish {
+  const void* C = nullptr;     // [B,T,c]
+  const void* Z = nullptr;
+  const void* Cb = nullptr;    // the overlapped compression's second branch, or null
+  const void* Zb = nullptr;
+  const void* lsrc = nullptr;  // [B,T,c] rows the window keys normalise (win > 0)
+  long long ldC = 0, ldZ = 0, ldCb = 0, ldZb = 0, ldl = 0;
+  const float* Bpos = nullptr;  // [m,c]
+  const float* Bb = nullptr;
+  const float* kc = nullptr;   // [B,nb,c] compressed rows, L2-normalised when normalize
+  const float* raw = nullptr;  // [B,nb,c] compressed rows
+  void* dC = nullptr;          // [B,T,c]
+  void* dZ = nullptr;
+  void* dCb = nullptr;
+  void* dZb = nullptr;
+  void* dlocal = nullptr;      // gradient of the window rows' source, or null: added to dC
+  int B = 0, T = 0, nb = 0, m = 0, win = 0, normalize = 1;
+  int cdt = 0, odt = 0;        // DType; odt = cdt or DT_F32
+  // set by the dispatch: the per-block terms of dB_pos, dBb [B,nb,m,c]; part_b
+  // [B,nchunk,nb,c], the key pass's partials (chunk ci = queries [ci part_qc,
+  // (ci+1) part_qc), read for the chunks a row's queries reach); part_w
+  // [win_nc,B,T,c], the window rows'; rl [B,T] 1 / max(|window row|, eps)
+  float* dBp = nullptr;
+  float* dBbp = nullptr;
+  const float* part_b = nullptr;
+  const float* part_w = nullptr;
+  const float* rl = nullptr;
+  int nchunk = 0, part_qc = 1, win_nc = 1;
+};
+hipError_t bwd_finish_launch(const BwdFinish& p, int c, hipStream_t s);
+// out[c] = sign * sum over the rows of x [rows, cols]
+size_t sum_rows_ws_bytes(long long rows, int cols);
+hipError_t sum_rows_launch(const float* x, float* out, long long rows, int cols, float sign, void* ws, hipStream_t s);
+
+// Gradients of the HCA / CSA attention (hca_backward.hip, attn_bwd_mfma.hip), c
+// in {64, 128}, nh <= 256 / (c / 8), T a multiple of m2.
 struct HcaBwdParams {
   const void* q;        // [B,T,nh,c] queries as given (not normalised), in qdt
   const void* dout;     // [B,T,nh,c], in qdt
-  const float* kc;      // [B,nb,c] L2-normalised compressed rows
-  const float* raw;     // [B,nb,c] compressed rows
-  const float* kl;      // [B,T,c] L2-normalised window rows (win > 0)
-  const float* lsrc;    // [B,T,c] rows the window keys normalise (win > 0)
-  const float* C;       // [B,T,c] compression inputs
-  const float* Z;
-  const float* Bpos;    // [m2,c]
   const float* sink;    // [nh] or null
   void* dq;             // [B,T,nh,c], in qdt
-  float* dC;            // [B,T,c]
-  float* dZ;            // [B,T,c]
-  float* dBp;           // [B,nb,m2,c] per-block terms of dB_pos
-  float* dlocal;        // [B,T,c] gradient of the window rows' source, or null: added to dC
-  float* sink_part;     // [B,T,nh] p_sink * D per query and head, or null
+  float* dB;            // [m2,c]
+  float* dBb = nullptr; // [m2,c]
+  float* dsink;         // [nh] or null
   int normalize = 1;    // 0: queries and keys are used as given (no L2 norms)
   int qdt = 0;          // storage of q, dout, dq: 0 fp32, 1 bf16, 2 fp16 (the SIMT path: fp32)
   // CSA: the selected blocks (idx [B,T,topk], -1 = unused) instead of every
-  // causal block, its bitmap sel [B,T,ceil(nb/32)], the overlapped
-  // compression's second branch, and the per-slot gradient of the selected
-  // rows against themselves (slot_grad [B,T,topk], for the STE surrogate)
+  // causal block, its bitmap sel [B,T,ceil(nb/32)], and the per-slot gradient
+  // of the selected rows against themselves (slot_grad [B,T,topk], for the STE
+  // surrogate)
   const int* idx = nullptr;
   const uint32_t* sel = nullptr;
   int topk = 0;
   int sparse = 0;  // CSA: only the selected blocks (none when topk = 0)
-  const float* Cb = nullptr;
-  const float* Zb = nullptr;
-  const float* Bb = nullptr;
-  float* dCb = nullptr;
-  float* dZb = nullptr;
-  float* dBbp = nullptr;
   float* slot_grad = nullptr;
   // the same values dense over the blocks, [B,T,nb] (0 at the others); dsel_add:
   // added to what it holds (calls for further groups of heads)
   float* dsel = nullptr;
   int dsel_add = 0;
-  float* slot_ws = nullptr;  // workspace: the gathering query pass's values per slot
   // CSA, full-softmax STE: the sum over the selected slots of each selected
   // row's gradient, gsum [B,T,c] (written, the heads of this call summed)
   float* gsum = nullptr;
-  float* lse = nullptr;  // workspace regions, set by hca_bwd_dispatch
+  int B, T, nh, c, m2, nb, win;
+  float scale;
+  // set by the dispatch
+  float* sink_part = nullptr;  // [B,T,nh] p_sink * D per query and head
+  float* slot_ws = nullptr;    // the gathering query pass's values per slot
+  float* lse = nullptr;
   float* dval = nullptr;
   float* rq = nullptr;
   float* part_b = nullptr;
   float* part_w = nullptr;
-  // MFMA path (attn_bwd_mfma.hip): the two-part bf16 splits of the compressed
-  // and window rows; mfma_parts: part_b holds [B, nchunk, nb, c] per-chunk
-  // partials of the compressed rows (chunk ci = queries [ci part_qc, (ci+1)
-  // part_qc), written for the chunks a row's queries reach), part_w the window
-  // rows' [win_nc, B, T, c]
-  bf16_t* kc_hi = nullptr;
-  bf16_t* kc_lo = nullptr;
-  bf16_t* kl_hi = nullptr;
-  bf16_t* kl_lo = nullptr;
-  int mfma_parts = 0;
-  int part_qc = 0;
-  int win_qc = 0, win_nc = 1;
-  int B, T, nh, c, m2, nb, win;
-  float scale;
+  // SIMT path (fp32, contiguous)
+  const float* kc = nullptr;
+  const float* raw = nullptr;
+  const float* kl = nullptr;
+  const float* lsrc = nullptr;
+  const float* C = nullptr;
+  const float* Z = nullptr;
+  const float* Cb = nullptr;
+  const float* Zb = nullptr;
+  const float* Bpos = nullptr;
+  const float* Bb = nullptr;
+  float* dC = nullptr;
+  float* dZ = nullptr;
+  float* dCb = nullptr;
+  float* dZb = nullptr;
+  float* dBp = nullptr;
+  float* dBbp = nullptr;
+  float* dlocal = nullptr;
+  // MFMA path: the compressed rows' two-part bf16 split; the window rows as
+  // given, ldl elements apart: exact in kl_hi (kl_lo null) or their split; rl
+  // [B,T] = 1 / max(|row|, eps); kn: the split of the normalised window rows
+  // (for the gathering query pass)
+  const bf16_t* kc_hi = nullptr;
+  const bf16_t* kc_lo = nullptr;
+  const bf16_t* kl_hi = nullptr;
+  const bf16_t* kl_lo = nullptr;
+  const bf16_t* kn_hi = nullptr;
+  const bf16_t* kn_lo = nullptr;
+  const float* rl = nullptr;
+  long long ldl = 0;
+  int part_qc = 0, win_qc = 0;
 };
 // MFMA attention backward (normalised queries and keys, c in {64, 128}, nh <= 16)
 bool attn_bwd_mfma_supported(const HcaBwdParams& p);
 size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk);
-hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, void* ws, hipStream_t s);
+hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t s);
+// topk < 0: HCA (single-branch compression)
 size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk);
+hipError_t hca_bwd_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t stream);
 
-// The STE surrogate's backward for the indexer (ste_backward.hip): fp32,
-// cI in {64, 128}, nIh in {1, 2, 4, 8}, nIh * cI <= 512.
+// The STE surrogate's backward for the indexer (ste_backward.hip), fp32
+// arithmetic: cI in {64, 128}, nIh in {1, 2, 4, 8}, nIh * cI <= 512.
 struct SteBwdParams {
-  const float* qi;    // [B,T,nIh,cI] indexer queries as given
-  const float* w;     // [B,T,nIh] head weights
+  const void* qi;     // [B,T,nIh,cI] indexer queries as given, in qdt
+  const void* w;      // [B,T,nIh] head weights, in qdt
   const float* kc;    // [B,nb,cI] compressed indexer keys (L2-normalised when normalize)
   const float* dsel;  // [B,T,nb] the slot gradients at the selected blocks, 0 elsewhere
-  float* dqi;         // [B,T,nIh,cI]
-  float* dw;          // [B,T,nIh]
+  void* dqi;          // [B,T,nIh,cI], in qdt
+  void* dw;           // [B,T,nIh], in qdt
+  float* dB;          // [m,cI]
+  int qdt = 0;        // DType
   float* part = nullptr;  // workspace regions, set by ste_bwd_dispatch
   float* lse = nullptr;
   float* dval = nullptr;
@@ -150,14 +197,11 @@ struct SteBwdParams {
   float scale;
 };
 size_t ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m);
-// bp: the key compression's inputs and outputs for the block kernel
-hipError_t ste_bwd_dispatch(SteBwdParams p, HcaBwdParams bp, void* ws, hipStream_t stream);
+// f: the key compression's inputs and gradients
+hipError_t ste_bwd_dispatch(SteBwdParams p, BwdFinish f, void* ws, hipStream_t stream);
 // dsel[row, idx[row, j]] += slot[row, j] over rows of topk slots, nb columns
 hipError_t ste_scatter_launch(const int* idx, const float* slot, float* dsel, long long rows, int topk, int nb,
                               hipStream_t s);
-// the block and window kernels on the partials (hca_backward.hip)
-hipError_t hca_bwd_finish_launch(const HcaBwdParams& p, int nchunk, hipStream_t s);
-hipError_t hca_bwd_dispatch(HcaBwdParams p, void* ws, hipStream_t stream);
 
 hipError_t kda_chunk_dispatch(const KdaParams& p, int dtype, hipStream_t stream);
 // fp64 inputs, state and arithmetic (kda_recurrent.hip)

@@ -1,5 +1,6 @@
 // The STE surrogate's backward for the CSA indexer (ops_csa.py:1033-1099) for
-// gfx950, fp32 throughout.
+// gfx950, in fp32; queries, head weights and their gradients in their own
+// storage type.
 //
 // soft = softmax over the visible blocks n of the indexer logits
 //   lg_n = sum_h w_h relu(a_hn),  a_hn = scale qn_h . k_n
@@ -9,7 +10,7 @@
 //   dw_h = sum_n dl_n relu(a_hn),  dqn_h = sum_n dl_n w_h [a_hn > 0] scale k_n,
 //   dk_n = sum_t sum_h dl_tn w_th [a > 0] scale qn_th,
 // then the L2-norm and compression backwards of the indexer keys
-// (hca_backward.hip's block kernel on the partials written here).
+// (attn_bwd_finish.hip on the partials written here).
 //
 // Every sum over channels, blocks or queries is a contraction, and runs on the
 // fp32 matrix instruction 16x16x4 (the same precision as the vector units):
@@ -76,15 +77,27 @@ __device__ __forceinline__ f32x4 mma4(float4 a, const float* b, f32x4 acc) {
 // same side. (Raw rows keep the matrix sum.)
 constexpr float kNearZero = 2e-6f;
 
-template <int CPL, int N>
-__device__ __forceinline__ float tree_dot(const float* q, float rq, const float* k) {
+// four consecutive stored values as fp32
+template <typename T>
+__device__ __forceinline__ float4 load4(const T* p) {
+  if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const float4*>(p);
+  } else {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    const t4 v = *reinterpret_cast<const t4*>(p);
+    return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+  }
+}
+
+template <int CPL, int N, typename T>
+__device__ __forceinline__ float tree_dot(const T* q, float rq, const float* k) {
   if constexpr (N == 1) {
     float d = 0.f;
 #pragma unroll
-    for (int e = 0; e < CPL; ++e) d = __builtin_fmaf(q[e] * rq, k[e], d);
+    for (int e = 0; e < CPL; ++e) d = __builtin_fmaf((float)q[e] * rq, k[e], d);
     return d;
   } else {
-    return tree_dot<CPL, N / 2>(q, rq, k) + tree_dot<CPL, N / 2>(q + N / 2 * CPL, rq, k + N / 2 * CPL);
+    return tree_dot<CPL, N / 2, T>(q, rq, k) + tree_dot<CPL, N / 2, T>(q + N / 2 * CPL, rq, k + N / 2 * CPL);
   }
 }
 // sum of squares of v[0 .. N CPL) in the same order
@@ -100,7 +113,7 @@ __device__ __forceinline__ float tree_sq(const float* v) {
   }
 }
 // a[e] summed again where it is near zero; row(e): the query and key row of a[e]
-template <int NIH, int CI, typename Rows>
+template <int NIH, int CI, typename T, typename Rows>
 __device__ __forceinline__ void settle_zero(f32x4& a, int normalize, Rows rows) {
   unsigned near = 0;
 #pragma unroll
@@ -109,17 +122,17 @@ __device__ __forceinline__ void settle_zero(f32x4& a, int normalize, Rows rows) 
   while (near) {
     const int e = __builtin_ctz(near);
     near &= near - 1;
-    const float* q;
+    const T* q;
     const float* k;
     float rq;
     if (!rows(e, q, rq, k)) continue;
-    const float d = tree_dot<CI * NIH / 64, 64 / NIH>(q, rq, k);
+    const float d = tree_dot<CI * NIH / 64, 64 / NIH, T>(q, rq, k);
 #pragma unroll
     for (int i = 0; i < 4; ++i) a[i] = e == i ? d : a[i];
   }
 }
 
-template <int NIH, int CI>
+template <int NIH, int CI, typename T>
 __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int ntile) {
   constexpr int QPW = 16 / NIH, QPB = 4 * QPW;  // queries per wave, per workgroup
   constexpr int LD = CI + 4;                    // padded row: 16 rows' float4 reads free of conflicts
@@ -141,12 +154,12 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
   const bool vec = (p.nb & 3) == 0;
 
   // B operand: qn of this lane's (query, head), channels q CI/4 + j
-  const float* qrow = p.qi + (bt * NIH + h) * CI;
+  const T* qrow = static_cast<const T*>(p.qi) + (bt * NIH + h) * CI;
   float qv[CI / 4];
 #pragma unroll
   for (int j = 0; j < CI / 16; ++j) {
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) x = *reinterpret_cast<const float4*>(qrow + q * (CI / 4) + 4 * j);
+    if (live) x = load4<T>(qrow + q * (CI / 4) + 4 * j);
     qv[4 * j] = x.x; qv[4 * j + 1] = x.y; qv[4 * j + 2] = x.z; qv[4 * j + 3] = x.w;
   }
   const float ss = tree_sq<CI * NIH / 64, 16 / NIH>(qv);
@@ -154,7 +167,7 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
   const float rq = p.normalize ? 1.f / fmaxf(nrm, kEps) : 1.f;
 #pragma unroll
   for (int j = 0; j < CI / 4; ++j) qv[j] *= rq;
-  const float wh = live ? p.w[bt * NIH + h] : 0.f;
+  const float wh = live ? (float)static_cast<const T*>(p.w)[bt * NIH + h] : 0.f;
   const float* dsel = p.dsel + bt * p.nb;
   const float* kc = p.kc + (size_t)b * p.nb * CI;
 
@@ -182,7 +195,10 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
       if (vec) {
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (n0 < nvis) x = *reinterpret_cast<const float4*>(dsel + n0);
-        d[4 * u] = x.x; d[4 * u + 1] = x.y; d[4 * u + 2] = x.z; d[4 * u + 3] = x.w;
+        d[4 * u] = x.x;
+        d[4 * u + 1] = n0 + 1 < nvis ? x.y : 0.f;
+        d[4 * u + 2] = n0 + 2 < nvis ? x.z : 0.f;
+        d[4 * u + 3] = n0 + 3 < nvis ? x.w : 0.f;
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) d[4 * u + e] = n0 + e < nvis ? dsel[n0 + e] : 0.f;
@@ -195,7 +211,7 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
 #pragma unroll
     for (int j = 0; j < CI / 16; ++j)
       a = mma4(*reinterpret_cast<const float4*>(buf + (16 * u + n) * LD + q * (CI / 4) + 4 * j), qv + 4 * j, a);
-    settle_zero<NIH, CI>(a, p.normalize, [&](int e, const float*& qr, float& f, const float*& kr) {
+    settle_zero<NIH, CI, T>(a, p.normalize, [&](int e, const T*& qr, float& f, const float*& kr) {
       qr = qrow;
       f = rq;
       kr = buf + (16 * u + 4 * q + e) * LD;
@@ -309,7 +325,7 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt) {
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) x = *reinterpret_cast<const float4*>(qrow + 16 * tt + 4 * q);
+    if (live) x = load4<T>(qrow + 16 * tt + 4 * q);
     y[tt] = f32x4{x.x * rq, x.y * rq, x.z * rq, x.w * rq};
 #pragma unroll
     for (int e = 0; e < 4; ++e) yd += y[tt][e] * dq[tt][e];
@@ -317,16 +333,16 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
   yd = colq_sum(yd);
   if (!live) return;
   const bool big = p.normalize && nrm > kEps;
-  float* dst = p.dqi + (bt * NIH + h) * CI;
+  T* dst = static_cast<T*>(p.dqi) + (bt * NIH + h) * CI;
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt) {
     float o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (big ? dq[tt][e] - y[tt][e] * yd : dq[tt][e]) * rq;
-    *reinterpret_cast<float4*>(dst + 16 * tt + 4 * q) = make_float4(o[0], o[1], o[2], o[3]);
+    Store4<T>::run(dst + 16 * tt + 4 * q, f32x4{o[0], o[1], o[2], o[3]}, 1.f);
   }
   if (q == 0) {
-    p.dw[bt * NIH + h] = dwh;
+    static_cast<T*>(p.dw)[bt * NIH + h] = (T)dwh;
     p.rq[bt * NIH + h] = rq;
     if (h == 0) {
       p.lse[bt] = lse;
@@ -335,7 +351,7 @@ __global__ __launch_bounds__(256) void ste_bwd_query_kernel(SteBwdParams p, int 
   }
 }
 
-template <int NIH, int CI>
+template <int NIH, int CI, typename T>
 __global__ __launch_bounds__(256) void ste_bwd_key_kernel(SteBwdParams p, int qc, int nchunk) {
   constexpr int LD = CI + 4;
   constexpr int NP = KS * CI / 4 / 256;
@@ -385,13 +401,13 @@ __global__ __launch_bounds__(256) void ste_bwd_key_kernel(SteBwdParams p, int qc
       x.v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (row < live) {
         const float f = p.rq[row0 + row];
-        const float4 y = *reinterpret_cast<const float4*>(p.qi + (row0 + row) * CI + 4 * c);
+        const float4 y = load4<T>(static_cast<const T*>(p.qi) + (row0 + row) * CI + 4 * c);
         x.v[i] = make_float4(y.x * f, y.y * f, y.z * f, y.w * f);
       }
     }
     x.w = x.l = x.d = 0.f;
     if (tid < KS && tid < live) {
-      x.w = p.w[row0 + tid];
+      x.w = (float)static_cast<const T*>(p.w)[row0 + tid];
       x.l = p.lse[(size_t)b * p.T + ts + tid / NIH];
       x.d = p.dval[(size_t)b * p.T + ts + tid / NIH];
     }
@@ -438,10 +454,10 @@ __global__ __launch_bounds__(256) void ste_bwd_key_kernel(SteBwdParams p, int qc
         for (int j = 0; j < CI / 16; ++j)
           a = mma4(*reinterpret_cast<const float4*>(buf + (16 * g + n) * LD + q * (CI / 4) + 4 * j), kv + 4 * j, a);
         const int r = 16 * g + 4 * q;
-        settle_zero<NIH, CI>(a, p.normalize, [&](int e, const float*& qr, float& f, const float*& kr) {
+        settle_zero<NIH, CI, T>(a, p.normalize, [&](int e, const T*& qr, float& f, const float*& kr) {
           const size_t row = ((size_t)b * p.T + ts) * NIH + r + e;
           const bool ok = rk_ok && ts + (r + e) / NIH < thi;
-          qr = p.qi + (ok ? row * CI : 0);
+          qr = static_cast<const T*>(p.qi) + (ok ? row * CI : 0);
           f = ok ? p.rq[row] : 0.f;
           kr = p.kc + ((size_t)b * p.nb + (rk_ok ? rk : 0)) * CI;
           return ok;
@@ -515,19 +531,15 @@ int ste_chunk(int B, int T, int nb) {
   return qc;
 }
 
-template <int NIH, int CI>
-hipError_t launch_ste(const SteBwdParams& p, const HcaBwdParams& bp, hipStream_t s) {
+template <int NIH, int CI, typename T>
+hipError_t launch_ste(const SteBwdParams& p, const BwdFinish& f, hipStream_t s) {
   const int qpb = 64 / NIH, nt = (p.T + qpb - 1) / qpb;
-  hipLaunchKernelGGL((ste_bwd_query_kernel<NIH, CI>), dim3((unsigned)((long long)nt * p.B)), dim3(256), 0, s, p, nt);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.nb == 0) return e;
-  const int nchunk = (p.T + bp.part_qc - 1) / bp.part_qc;
-  hipLaunchKernelGGL((ste_bwd_key_kernel<NIH, CI>), dim3((p.nb + KT - 1) / KT * nchunk, p.B), dim3(256), 0, s,
-                     p, bp.part_qc, nchunk);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  // compression and L2-norm backward of the indexer keys
-  return hca_bwd_finish_launch(bp, nchunk, s);
+  hipLaunchKernelGGL((ste_bwd_query_kernel<NIH, CI, T>), dim3((unsigned)((long long)nt * p.B)), dim3(256), 0, s, p,
+                     nt);
+  if (p.nb > 0)
+    hipLaunchKernelGGL((ste_bwd_key_kernel<NIH, CI, T>), dim3((p.nb + KT - 1) / KT * f.nchunk, p.B), dim3(256), 0, s,
+                       p, f.part_qc, f.nchunk);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -535,25 +547,37 @@ hipError_t launch_ste(const SteBwdParams& p, const HcaBwdParams& bp, hipStream_t
 size_t ste_bwd_ws_bytes(int B, int T, int nIh, int cI, int m) {
   const int nb = T / m, qc = ste_chunk(B, T, nb);
   return 2 * al256((size_t)B * T * 4) + al256((size_t)B * T * nIh * 4) +
-         al256((size_t)B * ((T + qc - 1) / qc) * nb * cI * 4);
+         al256((size_t)B * ((T + qc - 1) / qc) * nb * cI * 4) + al256((size_t)B * T * cI * 4) +
+         sum_rows_ws_bytes((long long)B * nb, m * cI);
 }
 
-hipError_t ste_bwd_dispatch(SteBwdParams p, HcaBwdParams bp, void* ws, hipStream_t stream) {
+hipError_t ste_bwd_dispatch(SteBwdParams p, BwdFinish f, void* ws, hipStream_t stream) {
   char* w = static_cast<char*>(ws);
   const size_t per = al256((size_t)p.B * p.T * 4);
+  f.part_qc = ste_chunk(p.B, p.T, p.nb);
+  f.nchunk = (p.T + f.part_qc - 1) / f.part_qc;
   p.lse = reinterpret_cast<float*>(w);
   p.dval = reinterpret_cast<float*>(w + per);
   p.rq = reinterpret_cast<float*>(w + 2 * per);
-  p.part = reinterpret_cast<float*>(w + 2 * per + al256((size_t)p.B * p.T * p.nIh * 4));
-  bp.part_b = p.part;
-  bp.mfma_parts = 1;
-  bp.part_qc = ste_chunk(p.B, p.T, p.nb);
-#define KCH_STE(NIH, CI) \
-  if (p.nIh == NIH && p.cI == CI) return launch_ste<NIH, CI>(p, bp, stream);
+  w += 2 * per + al256((size_t)p.B * p.T * p.nIh * 4);
+  p.part = reinterpret_cast<float*>(w);
+  f.part_b = p.part;
+  w += al256((size_t)p.B * f.nchunk * p.nb * p.cI * 4);
+  f.dBp = reinterpret_cast<float*>(w);
+  w += al256((size_t)p.B * p.T * p.cI * 4);
+  hipError_t e = hipErrorInvalidValue;
+#define KCH_STE(NIH, CI)                                                    \
+  if (p.nIh == NIH && p.cI == CI)                                           \
+    e = p.qdt == DT_BF16  ? launch_ste<NIH, CI, bf16_t>(p, f, stream)       \
+        : p.qdt == DT_F16 ? launch_ste<NIH, CI, _Float16>(p, f, stream)     \
+                          : launch_ste<NIH, CI, float>(p, f, stream);
   KCH_STE(1, 64) KCH_STE(1, 128) KCH_STE(2, 64) KCH_STE(2, 128) KCH_STE(4, 64) KCH_STE(4, 128)
   KCH_STE(8, 64)
 #undef KCH_STE
-  return hipErrorInvalidValue;
+  // compression and L2-norm backward of the indexer keys
+  if (e == hipSuccess) e = bwd_finish_launch(f, p.cI, stream);
+  if (e == hipSuccess) e = sum_rows_launch(f.dBp, p.dB, (long long)p.B * p.nb, p.m * p.cI, 1.f, w, stream);
+  return e;
 }
 
 hipError_t ste_scatter_launch(const int* idx, const float* slot, float* dsel, long long rows, int topk, int nb,

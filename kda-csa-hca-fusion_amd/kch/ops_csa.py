@@ -198,6 +198,33 @@ def _attn_bwd_qdtype(q, d_out, normalize=True):
     return torch.float32
 
 
+def _bwd_rows(dt, n, *xs):
+    """The rows of a backward's compression inputs ``[B, T, <= n]`` in ``dt``,
+    zero-padded to ``n`` channels, as alternating (tensor, row stride): views are
+    used in place when their rows lie 16-byte aligned at one stride."""
+    out = []
+    for x in xs:
+        if x is None:
+            out += [None, n]
+            continue
+        x = _pad_last(x.detach().to(dt), n)
+        ld = x.stride(1)
+        if not (x.stride(2) == 1 and ld >= n and ld * x.element_size() % 16 == 0
+                and (x.shape[0] == 1 or x.stride(0) == x.shape[1] * ld)
+                and x.data_ptr() % 16 == 0):
+            x, ld = _aligned(x), n
+        out += [x, ld]
+    return out
+
+
+def _bwd_dtype(xs, direct):
+    """Storage dtype of a backward's compression inputs: theirs when they share
+    one that the kernels read (and ``direct``), else float32."""
+    dts = {x.dtype for x in xs if x is not None}
+    dt = dts.pop()
+    return dt if direct and not dts and dt in _lib.DTYPE_CODE else torch.float32
+
+
 def _compress(fn, C, Z, B_pos, m, *, out_raw=True, key=None, normalize=False, local=None,
               key_split=0):
     """``key_split``: 0 keys as ``key``'s dtype (bf16 / fp32); 1 bf16 three-part
@@ -541,69 +568,63 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
         x = x.to(device=dev, dtype=dt)
         return (_pad_last(x, cp) if cp != c else x).contiguous()
 
-    # q, d_out and dq move in their storage dtype where the MFMA kernels run
+    # q, d_out and dq, the compression's inputs and their gradients move in their
+    # storage dtype where the MFMA kernels run
     qdt = _attn_bwd_qdtype(q, d_out, normalize_qk)
-    Caf, Cbf, Zaf, Zbf, Baf, Bbf = (prep(x) for x in (Ca, Cb, Za, Zb, Ba, Bb))
+    cdt = _bwd_dtype((Ca, Cb, Za, Zb), bool(normalize_qk))
+    # 16 heads a call on the MFMA kernels (normalised rows), else as many as
+    # one SIMT workgroup holds
+    hmax = _MAX_HEADS if normalize_qk else 256 // (cp // 8)
+    one = nh <= hmax
+    odt = cdt if one else f32
+    rows = _bwd_rows(cdt, cp, Ca, Cb, Za, Zb)
+    Car, Cbr, Zar, Zbr = rows[::2]
+    if not normalize_qk:
+        Car, Cbr, Zar, Zbr = (x.contiguous() for x in (Car, Cbr, Zar, Zbr))
+        rows = [Car, cp, Cbr, cp, Zar, cp, Zbr, cp]
+    rowargs = [_lib.ptr(x) if isinstance(x, torch.Tensor) else x for x in rows]
+    Baf, Bbf = (_aligned(prep(x)) for x in (Ba, Bb))
     qf, dof = _aligned(prep(q, qdt)), _aligned(prep(d_out, qdt))
     nb = T // m
     kc = torch.empty(B_, nb, cp, device=dev, dtype=f32)
-    raw = _compress_overlapped(fn, Caf, Cbf, Zaf, Zbf, Baf, Bbf, m, out_raw=True, key=kc,
+    raw = _compress_overlapped(fn, Car, Cbr, Zar, Zbr, Baf, Bbf, m, out_raw=True, key=kc,
                                normalize=bool(normalize_qk))
     if not normalize_qk:
         kc = raw
     win = int(sliding_window)
-    kl = lsrc = None
-    if win > 0:
-        lsrc = Caf
-        kl = l2_normalize_rows(Caf, out_dtype=f32) if normalize_qk else Caf
     idx32 = None if topk == 0 else idx.to(device=dev, dtype=torch.int32).contiguous()
     sink = None if sink_logits is None else sink_logits.detach().to(device=dev, dtype=f32).contiguous()
     dq = torch.empty_like(qf)
-    dCa = torch.zeros(B_, T, cp, device=dev, dtype=f32)
-    dCb, dZa, dZb = torch.zeros_like(dCa), torch.zeros_like(dCa), torch.zeros_like(dCa)
-    dBa = torch.zeros(m, cp, device=dev, dtype=f32)
-    dBb = torch.zeros_like(dBa)
+    # (zeros: the SIMT kernels add into it)
     slot = None if _dense else torch.zeros(B_, T, topk, device=dev, dtype=f32)
     dsel = torch.empty(B_, T, nb, device=dev, dtype=f32) if _dense else None
-    gsum = torch.zeros(B_, T, cp, device=dev, dtype=f32) if want_gsum else None
-    dsink = None if sink is None else torch.zeros(nh, device=dev, dtype=f32)
-    # 16 heads a call on the MFMA kernels (normalised rows), else as many as
-    # one SIMT workgroup holds
-    hmax = _MAX_HEADS if normalize_qk else 256 // (cp // 8)
+    gsum = None
+    dsink = None if sink is None else torch.empty(nh, device=dev, dtype=f32)
+    nbytes = _lib.load().kch_csa_attn_bwd_ws_bytes(B_, T, min(nh, hmax), cp, m, win, topk)
+    ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+    total = None
     for h0 in range(0, nh, hmax):
         h1 = min(nh, h0 + hmax)
         g = h1 - h0
-        qg = qf if g == nh else qf[:, :, h0:h1].contiguous()
-        dog = dof if g == nh else dof[:, :, h0:h1].contiguous()
-        dqg = dq if g == nh else torch.empty_like(qg)
-        oa, ob = torch.empty_like(dCa), torch.zeros_like(dCa)
-        za, zb = torch.empty_like(dCa), torch.zeros_like(dCa)
-        bap = torch.empty(B_, nb, m, cp, device=dev, dtype=f32)
-        bbp = torch.empty_like(bap)
-        sp = None if sink is None else torch.empty(B_, T, g, device=dev, dtype=f32)
-        gs = None if gsum is None else (gsum if g == nh else torch.empty_like(gsum))
-        nbytes = _lib.load().kch_csa_attn_bwd_ws_bytes(B_, T, g, cp, m, win, topk)
-        ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+        qg = qf if one else qf[:, :, h0:h1].contiguous()
+        dog = dof if one else dof[:, :, h0:h1].contiguous()
+        dqg = dq if one else torch.empty_like(qg)
+        part = [torch.empty(B_, T, cp, device=dev, dtype=odt) for _ in range(4)]
+        part += [torch.empty(m, cp, device=dev, dtype=f32) for _ in range(2)]
+        gs = torch.empty(B_, T, cp, device=dev, dtype=f32) if want_gsum else None
         _lib.call("kch_csa_attn_bwd", _lib.ptr(qg), _lib.ptr(dog), _lib.ptr(kc), _lib.ptr(raw),
-                  _lib.ptr(kl), _lib.ptr(lsrc), _lib.ptr(idx32), _lib.ptr(Caf), _lib.ptr(Cbf),
-                  _lib.ptr(Zaf), _lib.ptr(Zbf), _lib.ptr(Baf), _lib.ptr(Bbf),
-                  _lib.ptr(None if sink is None else sink[h0:h1].contiguous()), _lib.ptr(dqg),
-                  _lib.ptr(oa), _lib.ptr(ob), _lib.ptr(za), _lib.ptr(zb), _lib.ptr(bap),
-                  _lib.ptr(bbp), _lib.ptr(sp), _lib.ptr(slot if topk else None), _lib.ptr(dsel),
-                  int(h0 > 0), _lib.ptr(gs), B_, T, g, cp, m, topk, win, float(scale), int(bool(normalize_qk)),
-                  _lib.dtype_code(fn, qdt), _lib.ptr(ws), nbytes, _lib.stream_of(qg))
-        if dqg is not dq:
+                  _lib.ptr(idx32), *rowargs, _lib.ptr(Baf), _lib.ptr(Bbf),
+                  _lib.ptr(None if sink is None else sink[h0:h1]), _lib.ptr(dqg),
+                  *(_lib.ptr(x) for x in part), _lib.ptr(None if sink is None else dsink[h0:h1]),
+                  _lib.ptr(slot if topk else None), _lib.ptr(dsel), int(h0 > 0), _lib.ptr(gs), B_, T,
+                  g, cp, m, topk, win, float(scale), int(bool(normalize_qk)),
+                  _lib.dtype_code(fn, qdt), _lib.dtype_code(fn, cdt), _lib.dtype_code(fn, odt),
+                  _lib.ptr(ws), ws.numel(), _lib.stream_of(qg))
+        if not one:
             dq[:, :, h0:h1] = dqg
-        if gs is not None and gs is not gsum:
-            gsum += gs
-        dCa += oa
-        dCb += ob
-        dZa += za
-        dZb += zb
-        dBa += bap.sum(dim=(0, 1))
-        dBb += bbp.sum(dim=(0, 1))
-        if sp is not None:
-            dsink[h0:h1] = -sp.sum(dim=(0, 1))
+        total = part if total is None else [a + b for a, b in zip(total, part)]
+        gsum = gs if gsum is None or gs is None else gsum + gs
+    dCa, dCb, dZa, dZb, dBa, dBb = total
     out = {"Ca": dCa[..., :c].to(Ca.dtype), "Cb": dCb[..., :c].to(Cb.dtype),
            "Za": dZa[..., :c].to(Za.dtype), "Zb": dZb[..., :c].to(Zb.dtype),
            "q": dq[..., :c].to(q.dtype), "Ba": dBa[:, :c].to(Ba.dtype),
@@ -650,16 +671,17 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
     f32 = torch.float32
     nb = T // m
 
-    def prep(x, n):
-        x = x.detach().to(device=dev, dtype=f32)
-        return (_pad_last(x, n) if x.shape[-1] != n else x).contiguous()
-
-    Kf, Zf = prep(K_idx, cIp), prep(Z_idx, cIp)
-    Bf = prep(B_idx, cIp)
-    qf = F.pad(q_idx.detach().to(f32), (0, cIp - cI, 0, nIp - nIh)).contiguous()
-    wf = prep(w_idx, nIp)
+    qdt = _bwd_dtype((q_idx, w_idx), True)
+    cdt = _bwd_dtype((K_idx, Z_idx), True)
+    rows = _bwd_rows(cdt, cIp, K_idx, Z_idx)
+    Bf = _aligned(_pad_last(B_idx.detach().to(device=dev, dtype=f32), cIp))
+    qf = q_idx.detach().to(qdt)
+    if (cIp, nIp) != (cI, nIh):
+        qf = F.pad(qf, (0, cIp - cI, 0, nIp - nIh))
+    qf = _aligned(qf)
+    wf = _pad_last(w_idx.detach().to(qdt), nIp).contiguous()
     kc = torch.empty(B_, nb, cIp, device=dev, dtype=f32)
-    raw = _compress(fn, Kf, Zf, Bf, m, out_raw=True, key=kc, normalize=bool(normalize_qk))
+    raw = _compress(fn, rows[0], rows[2], Bf, m, out_raw=True, key=kc, normalize=bool(normalize_qk))
     if not normalize_qk:
         kc = raw
     if dsel is not None:
@@ -674,18 +696,19 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
     scale = 1.0 if normalize_qk else cI ** -0.5
     dq = torch.empty_like(qf)
     dw = torch.empty_like(wf)
-    dK = torch.zeros(B_, T, cIp, device=dev, dtype=f32)
-    dZ = torch.zeros_like(dK)
-    dBp = torch.empty(B_, nb, m, cIp, device=dev, dtype=f32)
+    dK, dZ = (torch.empty(B_, T, cIp, device=dev, dtype=cdt) for _ in range(2))
+    dB = torch.empty(m, cIp, device=dev, dtype=f32)
     nbytes = _lib.load().kch_csa_ste_bwd_ws_bytes(B_, T, nIp, cIp, m)
     ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+    qcode, ccode = _lib.dtype_code(fn, qdt), _lib.dtype_code(fn, cdt)
     _lib.call("kch_csa_ste_bwd", _lib.ptr(qf), _lib.ptr(wf), _lib.ptr(kc), _lib.ptr(raw),
-              _lib.ptr(Kf), _lib.ptr(Zf), _lib.ptr(Bf), _lib.ptr(dsel), _lib.ptr(dq), _lib.ptr(dw),
-              _lib.ptr(dK), _lib.ptr(dZ), _lib.ptr(dBp), B_, T, m, nIp, cIp, float(scale),
-              int(bool(normalize_qk)), _lib.ptr(ws), nbytes, _lib.stream_of(qf))
+              _lib.ptr(rows[0]), rows[1], _lib.ptr(rows[2]), rows[3], _lib.ptr(Bf), _lib.ptr(dsel),
+              _lib.ptr(dq), _lib.ptr(dw), _lib.ptr(dK), _lib.ptr(dZ), _lib.ptr(dB), B_, T, m, nIp,
+              cIp, float(scale), int(bool(normalize_qk)), qcode, ccode, ccode, _lib.ptr(ws),
+              nbytes, _lib.stream_of(qf))
     return [dK[..., :cI].to(K_idx.dtype), dZ[..., :cI].to(Z_idx.dtype),
             dq[:, :, :nIh, :cI].to(q_idx.dtype), dw[..., :nIh].to(w_idx.dtype),
-            dBp.sum(dim=(0, 1))[:, :cI].to(B_idx.dtype)]
+            dB[:, :cI].to(B_idx.dtype)]
 
 
 def _ste_indexer_grads_dense(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, normalize_qk,

@@ -17,8 +17,8 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib, generic
-from .ops_csa import (_HEAD_DIMS, _MAX_HEADS, _aligned, _attn_bwd_qdtype, _cat_cached,
-                      _check_gpu_dtype, _compress, _f32_cached, _head_groups, _kernel_size,
+from .ops_csa import (_HEAD_DIMS, _MAX_HEADS, _aligned, _attn_bwd_qdtype, _bwd_dtype, _bwd_rows,
+                      _cat_cached, _check_gpu_dtype, _compress, _f32_cached, _head_groups, _kernel_size,
                       _linear_up, _pad_last, l2_normalize_rows)
 
 
@@ -62,60 +62,55 @@ def hca_core_grad(C, Z, q, B_pos, d_out, *, m2, sliding_window=0, sink_logits=No
         x = x.to(dt)
         return (_pad_last(x, cp) if cp != c else x).contiguous()
 
-    # q, d_out and dq move in their storage dtype (the MFMA kernels, 16 heads a call)
+    # q, d_out and dq, the compression's inputs and their gradients move in their
+    # storage dtype (the MFMA kernels, 16 heads a call)
     qdt = _attn_bwd_qdtype(q, d_out)
-    Cf, Zf, Bp = (prep(x) for x in (C, Z, B_pos))
-    qf, dof = _aligned(prep(q, qdt)), _aligned(prep(d_out, qdt))
-    Clr = None if C_local_raw is None else prep(C_local_raw)
-    nb = T // m2
     win = int(sliding_window)
+    cdt = _bwd_dtype((C, Z, C_local_raw if win > 0 else None), True)
+    one = nh <= _MAX_HEADS
+    odt = cdt if one else f32
+    Cr, ldC, Zr, ldZ, lr, ldl = _bwd_rows(cdt, cp, C, Z, C_local_raw if win > 0 else None)
+    if lr is None:
+        lr, ldl = Cr, ldC
+    Bp = _aligned(prep(B_pos))
+    qf, dof = _aligned(prep(q, qdt)), _aligned(prep(d_out, qdt))
+    nb = T // m2
     kc = torch.empty(B_, nb, cp, device=dev, dtype=f32)
-    raw = _compress(fn, Cf, Zf, Bp, m2, out_raw=True, key=kc, normalize=True)
-    lsrc = kl = None
-    if win > 0:
-        lsrc = Cf if Clr is None else Clr
-        kl = l2_normalize_rows(lsrc, out_dtype=f32)
+    raw = _compress(fn, Cr, Zr, Bp, m2, out_raw=True, key=kc, normalize=True)
     sink = None if sink_logits is None else sink_logits.detach().to(device=dev, dtype=f32).contiguous()
     dq = torch.empty_like(qf)
-    dC = torch.zeros(B_, T, cp, device=dev, dtype=f32)
-    dZ = torch.zeros_like(dC)
-    dB = torch.zeros(cp, device=dev, dtype=f32).new_zeros(m2, cp)
-    dloc = None if Clr is None else torch.zeros_like(dC)
-    dsink = None if sink is None else torch.zeros(nh, device=dev, dtype=f32)
-    hmax = _MAX_HEADS
-    for h0 in range(0, nh, hmax):
-        h1 = min(nh, h0 + hmax)
+    dsink = None if sink is None else torch.empty(nh, device=dev, dtype=f32)
+    nbytes = _lib.load().kch_hca_attn_bwd_ws_bytes(B_, T, min(nh, _MAX_HEADS), cp, m2, win)
+    ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+    total = None
+    for h0 in range(0, nh, _MAX_HEADS):
+        h1 = min(nh, h0 + _MAX_HEADS)
         g = h1 - h0
-        qg = qf if g == nh else qf[:, :, h0:h1].contiguous()
-        dog = dof if g == nh else dof[:, :, h0:h1].contiguous()
-        dqg = dq if g == nh else torch.empty_like(qg)
-        dCg, dZg = torch.empty_like(dC), torch.empty_like(dZ)
-        dBp = torch.empty(B_, nb, m2, cp, device=dev, dtype=f32)
-        dlg = None if dloc is None else torch.empty_like(dloc)
-        sp = None if sink is None else torch.empty(B_, T, g, device=dev, dtype=f32)
-        nbytes = _lib.load().kch_hca_attn_bwd_ws_bytes(B_, T, g, cp, m2, win)
-        ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+        qg = qf if one else qf[:, :, h0:h1].contiguous()
+        dog = dof if one else dof[:, :, h0:h1].contiguous()
+        dqg = dq if one else torch.empty_like(qg)
+        part = [torch.empty(B_, T, cp, device=dev, dtype=odt) for _ in range(2)]
+        part.append(torch.empty(m2, cp, device=dev, dtype=f32))
+        if C_local_raw is not None:
+            part.append(torch.empty_like(part[0]) if win > 0 else torch.zeros_like(part[0]))
         _lib.call("kch_hca_attn_bwd", _lib.ptr(qg), _lib.ptr(dog), _lib.ptr(kc), _lib.ptr(raw),
-                  _lib.ptr(kl), _lib.ptr(lsrc), _lib.ptr(Cf), _lib.ptr(Zf), _lib.ptr(Bp),
-                  _lib.ptr(None if sink is None else sink[h0:h1].contiguous()), _lib.ptr(dqg),
-                  _lib.ptr(dCg), _lib.ptr(dZg), _lib.ptr(dBp), _lib.ptr(dlg), _lib.ptr(sp),
-                  B_, T, g, cp, m2, win, float(scale), _lib.dtype_code(fn, qdt), _lib.ptr(ws),
-                  nbytes, _lib.stream_of(qg))
-        if dqg is not dq:
+                  _lib.ptr(lr), ldl, _lib.ptr(Cr), ldC, _lib.ptr(Zr), ldZ, _lib.ptr(Bp),
+                  _lib.ptr(None if sink is None else sink[h0:h1]), _lib.ptr(dqg),
+                  _lib.ptr(part[0]), _lib.ptr(part[1]), _lib.ptr(part[2]),
+                  _lib.ptr(part[3] if len(part) > 3 else None),
+                  _lib.ptr(None if sink is None else dsink[h0:h1]), B_, T, g, cp, m2, win,
+                  float(scale), _lib.dtype_code(fn, qdt), _lib.dtype_code(fn, cdt),
+                  _lib.dtype_code(fn, odt), _lib.ptr(ws), ws.numel(), _lib.stream_of(qg))
+        if not one:
             dq[:, :, h0:h1] = dqg
-        dC += dCg
-        dZ += dZg
-        dB += dBp.sum(dim=(0, 1))
-        if dlg is not None:
-            dloc += dlg
-        if sp is not None:
-            dsink[h0:h1] = -sp.sum(dim=(0, 1))
+        total = part if total is None else [a + b for a, b in zip(total, part)]
+    dC, dZ, dB = total[:3]
     out = {"C": dC[..., :c].to(C.dtype), "Z": dZ[..., :c].to(Z.dtype),
            "q": dq[..., :c].to(q.dtype), "B_pos": dB[:, :c].to(B_pos.dtype)}
     if sink_logits is not None:
         out["sink_logits"] = dsink.to(sink_logits.dtype)
     if C_local_raw is not None:
-        out["C_local_raw"] = dloc[..., :c].to(C_local_raw.dtype)
+        out["C_local_raw"] = total[3][..., :c].to(C_local_raw.dtype)
     return out
 
 

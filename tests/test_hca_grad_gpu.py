@@ -198,3 +198,42 @@ def test_core_grad_edges(dev, T, m2, win):
     torch.cuda.synchronize()
     for name, x in (("C", Ct), ("Z", Zt), ("q", qt), ("B_pos", Bt), ("sink_logits", st)):
         _check(name, x.grad.cpu().numpy(), ref[name], 1e-4)
+
+
+STORAGE = [
+    # B, T, nh, c, m2, win, local, dtype, views: block form, storage, strided rows
+    (2, 36, 3, 64, 4, 6, False, torch.bfloat16, True),      # lane groups per block
+    (1, 256, 16, 128, 128, 40, False, torch.bfloat16, True),  # long blocks, split over workgroups
+    (1, 99, 2, 128, 33, 5, True, torch.float16, True),       # 33 tokens a block, window rows of their own
+    (1, 160, 18, 64, 32, 33, False, torch.bfloat16, False),  # two head groups: fp32 gradients added
+    (1, 132, 4, 48, 66, 0, True, torch.bfloat16, True),      # padded channels, no window
+]
+
+
+@pytest.mark.parametrize("B,T,nh,c,m2,win,local,dtype,views", STORAGE)
+def test_core_grad_in_storage_type(dev, B, T, nh, c, m2, win, local, dtype, views):
+    """C, Z and the window rows are read, and their gradients written, in their own
+    storage type and row stride: against the fp64 oracle on the same values, one
+    rounding of the type (half an ulp of the largest entry, 2^-8 / 2^-11 of it at
+    most) and 1e-4 of the largest entry."""
+    from kch.ops_hca import hca_core_grad
+    C, Z, q, Bp, sk, Cl, W = _make(T + nh + c + m2, B, T, nh, c, m2)
+    t = lambda x: torch.tensor(x, dtype=torch.float32, device=dev).to(dtype)  # noqa: E731
+    Ct, Zt, Clt, qt, Wt = (t(x) for x in (C, Z, Cl, q, W))
+    if views:  # column ranges of one projection, as the layers pass them
+        Ct, Zt, Clt = torch.cat([Ct, Zt, Clt], -1).split(c, -1)
+    f = lambda x: x.double().cpu().numpy()  # noqa: E731
+    kw = dict(m2=m2, sliding_window=win, scale=0.9)
+    ref = o_grad(f(Ct), f(Zt), f(qt), Bp, f(Wt), sink_logits=sk, C_local_raw=f(Clt) if local else None,
+                 **kw)
+    got = hca_core_grad(Ct, Zt, qt, torch.tensor(Bp, dtype=torch.float32, device=dev), Wt,
+                        sink_logits=torch.tensor(sk, dtype=torch.float32, device=dev),
+                        C_local_raw=Clt if local else None, **kw)
+    torch.cuda.synchronize()
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for name in ("C", "Z", "q", "B_pos", "sink_logits") + (("C_local_raw",) if local else ()):
+        half = name in ("C", "Z", "q", "C_local_raw")
+        assert got[name].dtype == (dtype if half else torch.float32)
+        r = ref.get(name)
+        r = np.zeros((B, T, c)) if r is None else r
+        _check(name, got[name].double().cpu().numpy(), r, 1e-4 + (ulp if half else 0.0))
