@@ -28,19 +28,25 @@
 // Kernels (one launch each):
 //   cb_prep_kernel  per (b, hv, chunk): M, Aqk, X, W, U, Qg, Kd, el -> workspace
 //                   (8 waves, two per SIMD, sharing one LDS allocation)
-//   cb_fwd_kernel   per (b, hv, 64 columns of V), chunks in order: S_n, v_n
-//   cb_bwd_kernel   per (b, hv, 64 columns of V), chunks in reverse: dS', dv_n, dS_0
+//   cb_fwd_kernel   per (b, hv, slice of V), chunks in order: S_n, v_n
+//   cb_bwd_kernel   per (b, hv, slice of V), chunks in reverse: dS', dv_n, dS_0
 //   cb_grad_kernel  per (b, hv, chunk): dq, dk, dv, dg, dbeta (or per-value-head
 //                   partials that kda_bwd_reduce_launch sums when HV > H)
-// The state kernels keep the state in MFMA accumulators; the operands shared
-// by the waves sit in LDS, the rest is read straight from L2 in fragment form.
+// Every operand that passes from one kernel to the next is split once, where
+// it is made, and lies in the workspace in the order the matrix instruction
+// reads it (Rec): a consumer's fragment is two 16-byte loads a lane, whole
+// 1 KB tiles, with no conversion, transpose or LDS staging. Between the two
+// products of a state kernel's chunk the state and v_n (dv_n) pass through
+// LDS as split planes; the transposed fragments that cb_grad_kernel reads are
+// taken from the same planes by transposing reads.
 // The decay-weighted products (M, Aqk and their gradients) factor as
 // e^(G_i - G_a) e^(G_a - G_j) around token a = 31 and run on MFMA when every
-// gate of the chunk (or channel block) is <= 0 and every |G - G_a| <= 60 nats:
+// gate of the chunk (channel tile) is <= 0 and every |G - G_a| <= 60 nats:
 // the factors then stay in fp32 range with normal low parts, and no exponent
 // reaches the clamp. Otherwise they are formed exactly, one exponential per
 // (i, j, channel), with the clamp and its zero gradient.
 
+#include <atomic>
 #include <type_traits>
 
 #include "kch_device.h"
@@ -77,6 +83,123 @@ __device__ __forceinline__ f32x4 mm3(const Sp& a, const Sp& b, f32x4 acc) {
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, b.hi, acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.lo, acc, 0, 0, 0);
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, acc, 0, 0, 0);
+}
+
+// Buffer addressing: a scalar base, one 32-bit byte offset per lane and a
+// constant, so no 64-bit address lives in vector registers; an offset at or
+// past `bytes` reads zero and stores nothing, which is how rows past the end
+// of a sequence drop out.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(const void* base, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(unsigned)bytes, 0x00020000);
+}
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// N consecutive values of InT as dwords
+template <typename InT, int N>
+__device__ __forceinline__ auto buf_load(__amdgpu_buffer_rsrc_t r, unsigned off) {
+  if constexpr (N * sizeof(InT) == 32) {
+    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  } else if constexpr (N * sizeof(InT) == 16) {
+    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return a;
+  } else {
+    static_assert(N * sizeof(InT) == 8, "dwords");
+    const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+    return a;
+  }
+}
+
+// a b with b of NP exact parts (1: b.lo is zero)
+template <int NP>
+__device__ __forceinline__ f32x4 mmp(const Sp& a, const Sp& b, f32x4 acc) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, b.hi, acc, 0, 0, 0);
+  if constexpr (NP == 2) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.lo, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, acc, 0, 0, 0);
+}
+
+// parts of an input value: bf16 is one part exactly
+template <typename T> constexpr int kParts = std::is_same<T, bf16_t>::value ? 1 : 2;
+
+struct Sp4 {
+  bf16x4 hi, lo;
+};
+
+__device__ __forceinline__ Sp4 sp4(f32x4 f) {
+  Sp4 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bf16_t h = (bf16_t)f[i];
+    s.hi[i] = h;
+    s.lo[i] = (bf16_t)(f[i] - (float)h);
+  }
+  return s;
+}
+
+// Fragment tiles: a matrix of R rows and D contraction columns as tiles of
+// 16 x 32, tile (r / 16) * (D / 32) + d / 32; in a tile lane r % 16 + 16 (d %
+// 32 / 8) holds columns d .. d + 7 of its row, the high parts of all lanes
+// before the low parts (1024 bf16 a tile).
+constexpr int kTile = 1024;
+
+__device__ __forceinline__ Sp ft_load(const bf16_t* m, int tile) {
+  const bf16_t* p = m + (size_t)tile * kTile + 8 * (threadIdx.x & 63);
+  return {*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + 512)};
+}
+
+__device__ __forceinline__ Sp ft_load(__amdgpu_buffer_rsrc_t m, int off, int tile) {
+  const int v = 16 * (threadIdx.x & 63), so = 2 * (off + tile * kTile);
+  return {__builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(m, v, so, 0)),
+          __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(m, v + 1024, so, 0))};
+}
+
+__device__ __forceinline__ void ft_store(bf16_t* m, int tile, int lane, const Sp& s) {
+  bf16_t* p = m + (size_t)tile * kTile + 8 * lane;
+  *reinterpret_cast<bf16x8*>(p) = s.hi;
+  *reinterpret_cast<bf16x8*>(p + 512) = s.lo;
+}
+
+// Accumulator rows 16 tc + 4 kq + e, column r16 into a matrix whose rows are
+// the accumulator's columns (row tile tr) and whose contraction columns (nk
+// tiles of 32) are the accumulator's rows.
+__device__ __forceinline__ void ft_store_acc(bf16_t* m, int tr, int nk, int tc, const Sp4& s) {
+  const int l = threadIdx.x & 63, r16 = l & 15, kq = l >> 4;
+  bf16_t* p = m + (size_t)(tr * nk + (tc >> 1)) * kTile + 8 * (r16 + 16 * (2 * (tc & 1) + (kq >> 1))) +
+              4 * (kq & 1);
+  *reinterpret_cast<bf16x4*>(p) = s.hi;
+  *reinterpret_cast<bf16x4*>(p + 512) = s.lo;
+}
+
+// 4 rows (this lane: r0 .. r0 + 3, r0 by lane / 16) of column col0 + lane % 16
+// of an LDS plane of row stride ld
+__device__ __forceinline__ bf16x4 tr4(const bf16_t* plane, int ld, int r0, int col0) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  const int n = threadIdx.x & 15;
+  return __builtin_bit_cast(
+      bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(
+                  plane + (r0 + (n >> 2)) * ld + col0 + 4 * (n & 3))));
+}
+
+__device__ __forceinline__ bf16x8 cat4(bf16x4 a, bf16x4 b) {
+  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// rows r0 + 8 kq .. + 7 of column col0 + lane % 16
+__device__ __forceinline__ bf16x8 tr8(const bf16_t* plane, int ld, int r0, int col0) {
+  const int r = r0 + 8 * ((threadIdx.x & 63) >> 4);
+  return cat4(tr4(plane, ld, r, col0), tr4(plane, ld, r + 4, col0));
+}
+
+__device__ __forceinline__ Sp plane8(const bf16_t* hi, const bf16_t* lo, int off) {
+  return {*reinterpret_cast<const bf16x8*>(hi + off), *reinterpret_cast<const bf16x8*>(lo + off)};
+}
+
+// the wave's index, known to be uniform
+__device__ __forceinline__ int wave_id() {
+  return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
 // 8 consecutive fp32 values (16-byte aligned)
@@ -135,20 +258,33 @@ __device__ __forceinline__ float quad_sum(float v) {
   return v + dppf<0x4E>(v);
 }
 
-// Workspace record of one (b, hv, chunk), fp32, row-major:
-//   W [C][K] | Kd [C][K] | Qg [C][K] | U [C][V] | Aqk^T [C][C] | X^T [C][C] | el [K]
+// Workspace record of one (b, hv, chunk), offsets in bf16 elements: fragment
+// tiles (rows x contraction), U as accumulator tiles (16 tokens x 16 columns, a
+// float4 of 4 tokens a lane) and el as floats. cb_fwd_kernel is the only reader
+// of the first three, so cb_bwd_kernel puts dS' over W1 and KD2 (2 K V <= 4 C K)
+// and dv_n over U.
 template <int K, int V>
 struct Rec {
-  static constexpr int W = 0, KD = C * K, QG = 2 * C * K, U = 3 * C * K, AQK = U + C * V,
-                       XT = AQK + C * C, EL = XT + C * C, RS = (EL + K + 63) / 64 * 64;
+  static constexpr int W1 = 0;                 // W        C x K
+  static constexpr int KD2 = 2 * C * K;        // Kd^T     K x C
+  static constexpr int U = 4 * C * K;          // U        fp32
+  static constexpr int KD1 = U + 2 * C * V;    // Kd       C x K
+  static constexpr int QG2 = KD1 + 2 * C * K;  // Qg^T     K x C
+  static constexpr int W2 = QG2 + 2 * C * K;   // -W^T     K x C
+  static constexpr int AQ = W2 + 2 * C * K;    // Aqk^T    C x C
+  static constexpr int XT = AQ + 2 * C * C;    // X^T      C x C
+  static constexpr int EL = XT + 2 * C * C;    // el       fp32 [K]
+  static constexpr int FL = EL + 2 * K;        // per 64 channels: decay products factored (int)
+  static constexpr int RS = FL + 128;
+  static constexpr int DSN = 0;                // dL/dS after the chunk, K x V
+  static constexpr int DVN = U;                // dL/dv_n transposed, V x C
+  static_assert(V <= 2 * C && RS % 128 == 0, "record layout");
 };
 
 struct CbWs {
-  float* rec;   // [B*HV*NT][RS]
-  float* sn;    // [B*HV*NT][K][V]   state at the start of each chunk
-  float* dsn;   // [B*HV*NT][K][V]   dL/dS after each chunk
-  float* vn;    // [B*HV*NT][C][V]   v_n
-  float* dvn;   // [B*HV*NT][C][V]   dL/dv_n
+  bf16_t* rec;  // [B*HV*NT][RS]
+  bf16_t* sn;   // [B*HV*NT] state at the start of each chunk, tiles K x V
+  bf16_t* vn;   // [B*HV*NT] v_n, tiles C x V
   float* part;  // [B,T,HV,3K+1] per-value-head partials (HV > H), else null
   int nt;
 };
@@ -188,7 +324,10 @@ __device__ __forceinline__ void col_scan(float* m, int ld, float* tot, const flo
 }
 
 // ---------------------------------------------------------------------------
-// cb_prep_kernel: one workgroup (8 waves) per (b, hv, chunk)
+// cb_prep_kernel: one workgroup (8 waves) per (b, hv, chunk). It writes W and Kd
+// in both orders, which the two state kernels need (64 KB a chunk more than
+// one order each; 467 us at 4096 chunks against 420, for the 601 us that the
+// state kernels no longer spend on transposing).
 // ---------------------------------------------------------------------------
 template <int K, int V, typename InT>
 __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
@@ -196,10 +335,10 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   constexpr int LK = K + 4, LC = C + 4, LV = V + 4;
   constexpr int SQ = C * LK > C * LV ? C * LK : C * LV;
   __shared__ float sk[C * LK], sG[C * LK], sq[SQ], sM[C * LC], sX[C * LC], sb[C], stot[NTH];
-  __shared__ int sflag;
+  __shared__ int sflag[K / 64];
   float* const sv = sq;  // v [C][LV] once q^ is consumed
 
-  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, r16 = l & 15, kq = l >> 4;
+  const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   const int nt = w.nt;
   const int n = blockIdx.x % nt, bh = blockIdx.x / nt;
   const int hv = bh % p.HV, b = bh / p.HV, h = hv / (p.HV / p.H);
@@ -207,11 +346,10 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   const float scale = (float)p.scale;
   const bool clampg = p.g_clamp_min > -INFINITY;
   const float gmin = (float)p.g_clamp_min;
-  float* rec = w.rec + (size_t)blockIdx.x * R::RS;
+  bf16_t* rec = w.rec + (size_t)blockIdx.x * R::RS;
 
-  if (tid == 0) sflag = 1;
+  if (tid < K / 64) sflag[tid] = 1;
   __syncthreads();
-  bool pos = false;
   for (int it = tid; it < C * (K / 8); it += NTH) {
     const int c = it / (K / 8), c8 = (it % (K / 8)) * 8, t = t0 + c;
     float fq[8], fk[8], fg[8];
@@ -223,6 +361,7 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
     } else {
       zero8(fq); zero8(fk); zero8(fg);
     }
+    bool pos = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float gc = clampg ? fmaxf(fg[i], gmin) : fg[i];
@@ -231,8 +370,8 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
       sk[c * LK + c8 + i] = fk[i];
       sG[c * LK + c8 + i] = gc;
     }
+    if (pos) sflag[c8 / 64] = 0;
   }
-  if (pos) sflag = 0;
   if (tid < C) {
     const int t = t0 + tid;
     sb[tid] = t < T ? to_f32(static_cast<const InT*>(p.beta)[(size_t)(b * T + t) * p.HV + hv]) : 0.f;
@@ -241,10 +380,13 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   col_scan<K, false>(sG, LK, stot, nullptr);
   if (tid < K) {
     const float ga = sG[kAnc * LK + tid];
-    if (sG[tid] - ga > kAncRange || ga - sG[(C - 1) * LK + tid] > kAncRange) sflag = 0;
+    if (sG[tid] - ga > kAncRange || ga - sG[(C - 1) * LK + tid] > kAncRange) sflag[tid / 64] = 0;
   }
   __syncthreads();
-  const bool anchored = sflag != 0;
+  bool anchored = true;
+#pragma unroll
+  for (int i = 0; i < K / 64; ++i) anchored &= sflag[i] != 0;
+  if (tid < K / 64) reinterpret_cast<int*>(rec + R::FL)[tid] = sflag[tid];
 
   // M and Aqk: wave wv owns column tile wv & 3 (j) of row tiles rt0, rt0 + 1 (i)
   {
@@ -300,22 +442,45 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
       }
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
+      f32x4 a;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 16 * (rt0 + u) + 4 * kq + e;
         sM[i * LC + jc] = jc < i ? sb[i] * am[u][e] : 0.f;
-        rec[R::AQK + jc * C + i] = jc <= i ? aa[u][e] : 0.f;  // stored transposed
+        a[e] = jc <= i ? aa[u][e] : 0.f;
       }
+      ft_store_acc(rec + R::AQ, wv & 3, 2, rt0 + u, sp4(a));
+    }
   }
-  // Qg, Kd, el
-  for (int it = tid; it < C * K; it += NTH) {
-    const int c = it / K, ch = it % K;
-    const float G = sG[c * LK + ch];
-    rec[R::QG + it] = sq[c * LK + ch] * ex(G);
-    rec[R::KD + it] = sk[c * LK + ch] * ex(sG[(C - 1) * LK + ch] - G);
+  // Qg^T and Kd^T (8 tokens of a channel), Kd (8 channels of a token), el
+  for (int it = tid; it < K * (C / 8); it += NTH) {
+    const int ch = it % K, c8 = it / K;
+    const float Gl = sG[(C - 1) * LK + ch];
+    float fq[8], fk[8], gc[8];
+    ld8s(&sq[8 * c8 * LK + ch], LK, fq);
+    ld8s(&sk[8 * c8 * LK + ch], LK, fk);
+    ld8s(&sG[8 * c8 * LK + ch], LK, gc);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      fq[i] *= ex(gc[i]);
+      fk[i] *= ex(Gl - gc[i]);
+    }
+    const int tile = (ch >> 4) * 2 + (c8 >> 2), lane = (ch & 15) + 16 * (c8 & 3);
+    ft_store(rec + R::QG2, tile, lane, sp8(fq));
+    ft_store(rec + R::KD2, tile, lane, sp8(fk));
   }
-  if (tid < K) rec[R::EL + tid] = ex(sG[(C - 1) * LK + tid]);
+  for (int it = tid; it < C * (K / 8); it += NTH) {
+    const int c = it % C, k8 = it / C;
+    float fk[8], gc[8], gl[8];
+    ld8c(&sk[c * LK + 8 * k8], fk);
+    ld8c(&sG[c * LK + 8 * k8], gc);
+    ld8c(&sG[(C - 1) * LK + 8 * k8], gl);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) fk[i] *= ex(gl[i] - gc[i]);
+    ft_store(rec + R::KD1, (c >> 4) * (K / 32) + (k8 >> 2), (c & 15) + 16 * (k8 & 3), sp8(fk));
+  }
+  if (tid < K) reinterpret_cast<float*>(rec + R::EL)[tid] = ex(sG[(C - 1) * LK + tid]);
   __syncthreads();
 
   // v -> LDS (over q^); X = (I + M)^-1, column cc by the eight lanes of a half row
@@ -352,24 +517,38 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
     for (int jj = 0; jj < 8; ++jj) {
       const int j = 8 * jj + part;
       sX[j * LC + cc] = xr[jj];
-      rec[R::XT + cc * C + j] = xr[jj];
     }
   }
   __syncthreads();
 
-  // W^T = Bk^T X^T and U^T = Bv^T X^T, one row tile (of K, then of V) at a
-  // time over the four column tiles of the chunk; stored row-major as W [C][K]
-  // and U [C][V]
+  {
+    const int c = tid & 63, j8 = tid >> 6;
+    float f[8];
+    ld8s(&sX[8 * j8 * LC + c], LC, f);
+    ft_store(rec + R::XT, (c >> 4) * 2 + (j8 >> 2), (c & 15) + 16 * (j8 & 3), sp8(f));
+  }
+  // W = X Bk in both orientations (the same fragments with the operands
+  // exchanged) and U = X Bv, one tile of K (then of V) at a time over the
+  // chunk's four row tiles; X's rows are split once per wave, its upper
+  // triangle left out
+  Sp xs[4][2];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      if (2 * ks > ct) continue;
+      float fb[8];
+      ld8c(&sX[(16 * ct + r16) * LC + 32 * ks + 8 * kq], fb);
+      xs[ct][ks] = sp8(fb);
+    }
 #pragma unroll 1
   for (int rtg = wv; rtg < K / 16 + V / 16; rtg += NTH / 64) {
     const bool isw = rtg < K / 16;
     const int r = 16 * (isw ? rtg : rtg - K / 16) + r16;
-    f32x4 acc[4];
+    Sp as[2];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < C; ks += 32) {
-      const int j0 = ks + 8 * kq;
+    for (int ks = 0; ks < 2; ++ks) {
+      const int j0 = 32 * ks + 8 * kq;
       float fa[8];
       if (isw) {
         float gj[8];
@@ -382,434 +561,353 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) fa[i] *= sb[j0 + i];
       }
-      const Sp as = sp8(fa);
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        float fb[8];
-        ld8c(&sX[(16 * ct + r16) * LC + j0], fb);
-        acc[ct] = mm3(as, sp8(fb), acc[ct]);
-      }
+      as[ks] = sp8(fa);
     }
-    const int r4 = r - r16 + 4 * kq;
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) {
-      float* dst = isw ? &rec[R::W + (16 * ct + r16) * K + r4] : &rec[R::U + (16 * ct + r16) * V + r4];
-      *reinterpret_cast<float4*>(dst) = make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
+      f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        if (2 * ks <= ct) x = mm3(xs[ct][ks], as[ks], x);
+      if (isw) {
+        f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          if (2 * ks <= ct) y = mm3(as[ks], xs[ct][ks], y);
+        ft_store_acc(rec + R::W1, ct, K / 32, rtg, sp4(y));
+        ft_store_acc(rec + R::W2, rtg, 2, ct, sp4(-x));
+      } else {
+        reinterpret_cast<f32x4*>(rec + R::U)[(ct * (V / 16) + rtg - K / 16) * 64 + l] = x;
+      }
     }
   }
 }
 
 // (slice of V, head) of a state-kernel workgroup. Workgroups are dealt to the
-// 8 XCDs round-robin; with two slices per head, blocks g and g + 8 of every
-// 16 take the two slices of one head, so they share an XCD and its L2 and the
-// head's per-chunk operands are read from HBM once.
+// 8 XCDs round-robin; the NVS slices of a head are blocks 8 apart, so they
+// share an XCD and its L2 and the head's per-chunk operands are read from HBM
+// once.
 template <int NVS>
 __device__ __forceinline__ void slice_of(int& vs, int& bh) {
   const int g = blockIdx.x;
-  if (NVS == 2 && (gridDim.x % 16) == 0) {
-    vs = (g >> 3) & 1;
-    bh = (g >> 4) * 8 + (g & 7);
+  if (NVS > 1 && (gridDim.x % (8 * NVS)) == 0) {
+    vs = (g >> 3) % NVS;
+    bh = g / (8 * NVS) * 8 + (g & 7);
   } else {
     vs = g % NVS;
     bh = g / NVS;
   }
 }
 
+// State rows in accumulators: wave wv owns rows [K/4 wv, K/4 (wv+1)) (KT tiles),
+// lane: rows 4 kq + e of a tile, column r16 of the slice's column tile vt. Its
+// split planes in LDS are [v][k].
+template <int K, int VS>
+struct StateTile {
+  static constexpr int KT = K / 64, VT = VS / 16, LK = K + 8;
+
+  // from fp32 [K][V] (null: zero) at column v0
+  static __device__ __forceinline__ void load(f32x4 (&S)[KT][VT], const float* src, int V, int v0) {
+    const int l = threadIdx.x & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          S[kt][vt][e] =
+              src ? src[(size_t)(16 * (wv * KT + kt) + 4 * kq + e) * V + v0 + 16 * vt + r16] : 0.f;
+  }
+
+  static __device__ __forceinline__ void to_planes(const f32x4 (&S)[KT][VT], bf16_t* hi, bf16_t* lo) {
+    const int l = threadIdx.x & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        const Sp4 x = sp4(S[kt][vt]);
+        const int o = (16 * vt + r16) * LK + 16 * (wv * KT + kt) + 4 * kq;
+        *reinterpret_cast<bf16x4*>(hi + o) = x.hi;
+        *reinterpret_cast<bf16x4*>(lo + o) = x.lo;
+      }
+  }
+
+  // the wave's own rows of the planes as fragment tiles K x V of the slice
+  static __device__ __forceinline__ void store_tiles(bf16_t* dst, const bf16_t* hi, const bf16_t* lo,
+                                                     int V, int v0) {
+    const int wv = wave_id();
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int vk = 0; vk < VS / 32; ++vk) {
+        const int k0 = 16 * (wv * KT + kt);
+        const Sp x = {tr8(hi, LK, 32 * vk, k0), tr8(lo, LK, 32 * vk, k0)};
+        ft_store(dst, (wv * KT + kt) * (V / 32) + v0 / 32 + vk, threadIdx.x & 63, x);
+      }
+  }
+};
+
 // ---------------------------------------------------------------------------
-// cb_fwd_kernel: one workgroup per (b, hv, 64 columns of V); S^T in
-// accumulators (rows v, columns K), wave wv owning columns [K/4 wv, K/4 (wv+1)).
-// The operands of chunk n+1 read from L2 in fragment form (W rows, U, el) are
-// loaded into registers while chunk n runs; Kd, transposed into LDS, is
-// loaded at the start of its own chunk and stored after the v_n product.
+// cb_fwd_kernel: one workgroup per (b, hv, VS columns of V), chunks in order.
+// Bound by HBM (at K = V = 128: 96 KB read and 96 KB written a chunk) and by
+// the chain of a chunk: two products with an LDS pass of split planes and a
+// barrier after each. A wave's share of W, Kd^T, U and el of chunk n + 1 is in
+// flight, in registers, through the whole of chunk n. At 64 heads of
+// 64 chunks 224 us (3.5 TB/s), where splitting fp32 operands in every consumer
+// and staging Kd through LDS took 456.
 // ---------------------------------------------------------------------------
-template <int K, int V>
-__global__ __launch_bounds__(256) void cb_fwd_kernel(KdaBwdParams p, CbWs w) {
+template <int K, int V, int VS>
+__global__ __launch_bounds__(256, 1) void cb_fwd_kernel(KdaBwdParams p, CbWs w) {
   using R = Rec<K, V>;
-  constexpr int VS = 64, NVS = V / VS, LK = K + 4, LC = C + 4, KT = K / 64, KS = K / 32;
-  constexpr int NKD = C * K / 4 / 256;
-  __shared__ float sST[VS * LK], sVT[VS * LC], sKT[K * LC];
-  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, r16 = l & 15, kq = l >> 4;
+  using ST = StateTile<K, VS>;
+  constexpr int KT = ST::KT, VT = ST::VT, LK = ST::LK, LC = C + 8, KS = K / 32;
+  __shared__ __attribute__((aligned(16))) bf16_t sS[2][VS * LK], sV[2][VS * LC];
+  const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   int vs, bh;
-  slice_of<NVS>(vs, bh);
-  const int v0 = vs * VS;
-  const int nt = w.nt;
-  const int cw = 16 * wv + r16;  // this lane's token row of the v_n^T column tile
+  slice_of<V / VS>(vs, bh);
+  const int v0 = vs * VS, nt = w.nt;
+
+  f32x4 S[KT][VT];
   const float* s0 = static_cast<const float*>(p.s0);
+  ST::load(S, s0 ? s0 + (size_t)bh * K * V : nullptr, V, v0);
+  ST::to_planes(S, sS[0], sS[1]);
 
-  f32x4 S[4][KT];
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int a = 0; a < KT; ++a) {
-      const int kch = 16 * (wv * KT + a) + r16, vr = 16 * rt + 4 * kq;
-      if (s0) {
-        const float4 x = *reinterpret_cast<const float4*>(&s0[((size_t)bh * K + kch) * V + v0 + vr]);
-        S[rt][a] = f32x4{x.x, x.y, x.z, x.w};
-      } else {
-        S[rt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sST[(vr + e) * LK + kch] = S[rt][a][e];
-    }
-
-  float wb[KS][8];
-  float4 ub[4];
-  float elb[KT];
-  auto prefetch = [&](int n) {
-    const float* rec = w.rec + ((size_t)bh * nt + n) * R::RS;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) ld8c(&rec[R::W + cw * K + 32 * ks + 8 * kq], wb[ks]);
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-      ub[rt] = *reinterpret_cast<const float4*>(&rec[R::U + cw * V + v0 + 16 * rt + 4 * kq]);
-#pragma unroll
-    for (int a = 0; a < KT; ++a) elb[a] = rec[R::EL + 16 * (wv * KT + a) + r16];
+  struct Ops {
+    Sp w[KS], kd[KT][2];
+    f32x4 u[VT], el[KT];
   };
-  prefetch(0);
-  __syncthreads();
-
-#pragma unroll 1
-  for (int n = 0; n < nt; ++n) {
+  auto fetch = [&](int n, Ops& o) {
+    const bf16_t* rec = w.rec + ((size_t)bh * nt + n) * R::RS;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) o.w[ks] = ft_load(rec + R::W1, wv * KS + ks);
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt)
+      o.u[vt] = reinterpret_cast<const f32x4*>(rec + R::U)[(wv * (V / 16) + v0 / 16 + vt) * 64 + l];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) o.kd[kt][ks] = ft_load(rec + R::KD2, (wv * KT + kt) * 2 + ks);
+      o.el[kt] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(rec + R::EL) +
+                                                 16 * (wv * KT + kt) + 4 * kq);
+    }
+  };
+  auto chunk = [&](int n, Ops& cur, Ops& nxt) {
     const size_t ci = (size_t)bh * nt + n;
-    const float* rec = w.rec + ci * R::RS;
-    // Kd of this chunk: lane-consecutive rows c, so the transposed LDS
-    // stores below hit distinct banks
-    float4 kd[NKD];
+    if (n + 1 < nt) fetch(n + 1, nxt);
+    // v_n = U - W S: the wave's 16 tokens
+    f32x4 vn[VT];
 #pragma unroll
-    for (int i = 0; i < NKD; ++i) {
-      const int it = tid + 256 * i, c = it % C, k4 = (it / C) * 4;
-      kd[i] = *reinterpret_cast<const float4*>(&rec[R::KD + c * K + k4]);
+    for (int vt = 0; vt < VT; ++vt) vn[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+        vn[vt] = mm3(cur.w[ks], plane8(sS[0], sS[1], (16 * vt + r16) * LK + 32 * ks + 8 * kq), vn[vt]);
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) {
+      const Sp4 x = sp4(cur.u[vt] - vn[vt]);
+      const int o = (16 * vt + r16) * LC + 16 * wv + 4 * kq;
+      *reinterpret_cast<bf16x4*>(&sV[0][o]) = x.hi;
+      *reinterpret_cast<bf16x4*>(&sV[1][o]) = x.lo;
     }
-    float* sn = w.sn + ci * K * V;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
-        *reinterpret_cast<float4*>(&sn[(size_t)kch * V + v0 + 16 * rt + 4 * kq]) =
-            make_float4(S[rt][a][0], S[rt][a][1], S[rt][a][2], S[rt][a][3]);
-      }
-    // v_n^T = U^T - S^T W^T: wave wv owns column tile wv (tokens)
-    f32x4 vn[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) vn[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const Sp bs = sp8(wb[ks]);
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        float fa[8];
-        ld8c(&sST[(16 * rt + r16) * LK + 32 * ks + 8 * kq], fa);
-        vn[rt] = mm3(sp8(fa), bs, vn[rt]);
-      }
-    }
-    float* vng = w.vn + ci * C * V;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      const int vr = 16 * rt + 4 * kq;
-      const float4 x = make_float4(ub[rt].x - vn[rt][0], ub[rt].y - vn[rt][1], ub[rt].z - vn[rt][2],
-                                   ub[rt].w - vn[rt][3]);
-      *reinterpret_cast<float4*>(&vng[cw * V + v0 + vr]) = x;
-      sVT[(vr + 0) * LC + cw] = x.x;
-      sVT[(vr + 1) * LC + cw] = x.y;
-      sVT[(vr + 2) * LC + cw] = x.z;
-      sVT[(vr + 3) * LC + cw] = x.w;
-    }
-    float el[KT];
-#pragma unroll
-    for (int a = 0; a < KT; ++a) el[a] = elb[a];
-    if (n + 1 < nt) prefetch(n + 1);
-#pragma unroll
-    for (int i = 0; i < NKD; ++i) {
-      const int it = tid + 256 * i, c = it % C, k4 = (it / C) * 4;
-      sKT[(k4 + 0) * LC + c] = kd[i].x;
-      sKT[(k4 + 1) * LC + c] = kd[i].y;
-      sKT[(k4 + 2) * LC + c] = kd[i].z;
-      sKT[(k4 + 3) * LC + c] = kd[i].w;
-    }
+    ST::store_tiles(w.sn + ci * 2 * K * V, sS[0], sS[1], V, v0);
     __syncthreads();
-    // S_n+1^T = el S^T + v_n^T Kd
 #pragma unroll
-    for (int a = 0; a < KT; ++a)
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) S[rt][a] *= el[a];
-#pragma unroll
-    for (int ks = 0; ks < C; ks += 32) {
-      const int c0 = ks + 8 * kq;
-      Sp bs[KT];
-#pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        float fb[8];
-        ld8c(&sKT[(16 * (wv * KT + a) + r16) * LC + c0], fb);
-        bs[a] = sp8(fb);
-      }
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        float fa[8];
-        ld8c(&sVT[(16 * rt + r16) * LC + c0], fa);
-        const Sp as = sp8(fa);
-#pragma unroll
-        for (int a = 0; a < KT; ++a) S[rt][a] = mm3(as, bs[a], S[rt][a]);
-      }
+    for (int vk = 0; vk < VS / 32; ++vk) {
+      const Sp x = {tr8(sV[0], LC, 32 * vk, 16 * wv), tr8(sV[1], LC, 32 * vk, 16 * wv)};
+      ft_store(w.vn + ci * 2 * C * V, wv * (V / 32) + v0 / 32 + vk, l, x);
     }
+    // S = el S + Kd^T v_n
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
+      for (int vt = 0; vt < VT; ++vt) S[kt][vt] *= cur.el[kt];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sST[(16 * rt + 4 * kq + e) * LK + kch] = S[rt][a][e];
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt) {
+        const Sp b = plane8(sV[0], sV[1], (16 * vt + r16) * LC + 32 * ks + 8 * kq);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) S[kt][vt] = mm3(cur.kd[kt][ks], b, S[kt][vt]);
       }
+    ST::to_planes(S, sS[0], sS[1]);
     __syncthreads();
+  };
+  Ops oa, ob;
+  fetch(0, oa);
+  __syncthreads();
+#pragma unroll 1
+  for (int n = 0; n < nt; n += 2) {
+    chunk(n, oa, ob);
+    if (n + 1 < nt) chunk(n + 1, ob, oa);
   }
 }
 
 // ---------------------------------------------------------------------------
-// cb_bwd_kernel: one workgroup per (b, hv, 64 columns of V), chunks in
-// reverse; dS^T in accumulators, wave wv owning columns [K/4 wv, K/4 (wv+1)).
-// Aqk^T and Kd rows (fragments), el and the dO slice of chunk n-1 are loaded
-// while chunk n runs (dO^T into the other of two LDS buffers); Qg and W,
-// transposed into LDS, are loaded at the start of their own chunk and stored
-// after the dv_n product.
+// cb_bwd_kernel: one workgroup per (b, hv, VS columns of V), chunks in
+// reverse; the shape of cb_fwd_kernel with dS' as the state, the operands of
+// chunk n - 1 (and its dO rows, for the other of two LDS buffers) in flight
+// through chunk n. Bound by HBM (at K = V = 128, bf16: 128 KB read and 96 KB
+// written a chunk). 64 heads of 64 chunks: 314 us (2.9 TB/s; 683 with fp32
+// operands, split by each wave and transposed through LDS).
 // ---------------------------------------------------------------------------
-template <int K, int V, typename InT>
-__global__ __launch_bounds__(256) void cb_bwd_kernel(KdaBwdParams p, CbWs w) {
+template <int K, int V, int VS, typename InT>
+__global__ __launch_bounds__(256, 1) void cb_bwd_kernel(KdaBwdParams p, CbWs w) {
   using R = Rec<K, V>;
-  constexpr int VS = 64, NVS = V / VS, LK = K + 4, LC = C + 4, KT = K / 64, KS = K / 32;
-  constexpr int NKD = C * K / 4 / 256;
-  constexpr int NDO = C * VS / 8 / 256;
-  __shared__ float sdST[VS * LK], sDOT[2][VS * LC], sdVT[VS * LC], sQT[K * LC], sWT[K * LC];
-  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, r16 = l & 15, kq = l >> 4;
+  using ST = StateTile<K, VS>;
+  constexpr int KT = ST::KT, VT = ST::VT, LK = ST::LK, LC = C + 8, KS = K / 32, LV = VS + 8;
+  constexpr int NP = kParts<InT>, NDO = C * VS / 8 / 256;
+  __shared__ __attribute__((aligned(16))) bf16_t sD[2][VS * LK], sdV[2][VS * LC], sdO[2][NP][C * LV];
+  const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   int vs, bh;
-  slice_of<NVS>(vs, bh);
-  const int v0 = vs * VS;
+  slice_of<V / VS>(vs, bh);
+  const int v0 = vs * VS, nt = w.nt, T = p.T;
   const int hv = bh % p.HV, b = bh / p.HV;
-  const int nt = w.nt, T = p.T;
-  const int cw = 16 * wv + r16;
+  const InT* dO = static_cast<const InT*>(p.d_o) + ((size_t)b * T * p.HV + hv) * V + v0;
+  const size_t ldo = (size_t)p.HV * V;
+
+  f32x4 D[KT][VT];
   const float* dsf = static_cast<const float*>(p.ds_final);
-  const InT* dO = static_cast<const InT*>(p.d_o);
+  ST::load(D, dsf ? dsf + (size_t)bh * K * V : nullptr, V, v0);
+  ST::to_planes(D, sD[0], sD[1]);
 
-  f32x4 D[4][KT];
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int a = 0; a < KT; ++a) {
-      const int kch = 16 * (wv * KT + a) + r16, vr = 16 * rt + 4 * kq;
-      if (dsf) {
-        const float4 x = *reinterpret_cast<const float4*>(&dsf[((size_t)bh * K + kch) * V + v0 + vr]);
-        D[rt][a] = f32x4{x.x, x.y, x.z, x.w};
-      } else {
-        D[rt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sdST[(vr + e) * LK + kch] = D[rt][a][e];
-    }
-
-  float ab[2][8], kb[KS][8], elb[KT], dob[NDO][8];
-  auto prefetch = [&](int n) {
-    const float* rec = w.rec + ((size_t)bh * nt + n) * R::RS;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) ld8c(&rec[R::AQK + cw * C + 32 * ks + 8 * kq], ab[ks]);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) ld8c(&rec[R::KD + cw * K + 32 * ks + 8 * kq], kb[ks]);
-#pragma unroll
-    for (int a = 0; a < KT; ++a) elb[a] = rec[R::EL + 16 * (wv * KT + a) + r16];
+  struct Ops {
+    Sp aq[2], kd[KS], qg[KT][2], wt[KT][2];
+    f32x4 el[KT];
+    float d_o[NDO][8];
+  };
+  auto fetch = [&](int n, Ops& o) {
+    const bf16_t* rec = w.rec + ((size_t)bh * nt + n) * R::RS;
 #pragma unroll
     for (int i = 0; i < NDO; ++i) {
-      const int it = tid + 256 * i, c = it % C, v8 = (it / C) * 8, t = n * C + c;
+      const int it = tid + 256 * i, c = it / (VS / 8), v8 = it % (VS / 8), t = n * C + c;
       if (t < T)
-        ld8g(dO + ((size_t)(b * T + t) * p.HV + hv) * V + v0 + v8, dob[i]);
+        ld8g(dO + t * ldo + 8 * v8, o.d_o[i]);
       else
-        zero8(dob[i]);
+        zero8(o.d_o[i]);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) o.aq[ks] = ft_load(rec + R::AQ, wv * 2 + ks);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) o.kd[ks] = ft_load(rec + R::KD1, wv * KS + ks);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        o.qg[kt][ks] = ft_load(rec + R::QG2, (wv * KT + kt) * 2 + ks);
+        o.wt[kt][ks] = ft_load(rec + R::W2, (wv * KT + kt) * 2 + ks);
+      }
+      o.el[kt] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(rec + R::EL) +
+                                                 16 * (wv * KT + kt) + 4 * kq);
     }
   };
-  auto store_dot = [&](float* dst) {
+  auto put_do = [&](int buf, const Ops& o) {
 #pragma unroll
     for (int i = 0; i < NDO; ++i) {
-      const int it = tid + 256 * i, c = it % C, v8 = (it / C) * 8;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dst[(v8 + j) * LC + c] = dob[i][j];
+      const int it = tid + 256 * i, c = it / (VS / 8), v8 = it % (VS / 8);
+      const Sp x = sp8(o.d_o[i]);
+      *reinterpret_cast<bf16x8*>(&sdO[buf][0][c * LV + 8 * v8]) = x.hi;
+      if constexpr (NP == 2) *reinterpret_cast<bf16x8*>(&sdO[buf][1][c * LV + 8 * v8]) = x.lo;
     }
   };
-  prefetch(nt - 1);
-  store_dot(sDOT[(nt - 1) & 1]);
-  __syncthreads();
-
-#pragma unroll 1
-  for (int n = nt - 1; n >= 0; --n) {
+  auto chunk = [&](int n, Ops& cur, Ops& nxt) {
     const size_t ci = (size_t)bh * nt + n;
-    const float* rec = w.rec + ci * R::RS;
-    const float* sdo = sDOT[n & 1];
-    float4 qr[NKD], wr[NKD];
+    bf16_t* rec = w.rec + ci * R::RS;
+    if (n > 0) fetch(n - 1, nxt);
+    // dv_n = Aqk^T dO + Kd dS': the wave's 16 tokens
+    Sp dof[2][VT];
 #pragma unroll
-    for (int i = 0; i < NKD; ++i) {
-      const int it = tid + 256 * i, c = it % C, k4 = (it / C) * 4;
-      qr[i] = *reinterpret_cast<const float4*>(&rec[R::QG + c * K + k4]);
-      wr[i] = *reinterpret_cast<const float4*>(&rec[R::W + c * K + k4]);
-    }
-    float* dsn = w.dsn + ci * K * V;
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
-        *reinterpret_cast<float4*>(&dsn[(size_t)kch * V + v0 + 16 * rt + 4 * kq]) =
-            make_float4(D[rt][a][0], D[rt][a][1], D[rt][a][2], D[rt][a][3]);
+      for (int vt = 0; vt < VT; ++vt) {
+        dof[ks][vt].hi = tr8(sdO[n & 1][0], LV, 32 * ks, 16 * vt);
+        if constexpr (NP == 2) dof[ks][vt].lo = tr8(sdO[n & 1][NP - 1], LV, 32 * ks, 16 * vt);
       }
-    // dv_n^T = dO^T Aqk + dS^T Kd^T (B operands: rows c of Aqk^T and of Kd);
-    // wave wv owns column tile wv (tokens)
-    f32x4 dv[4];
+    f32x4 dv[VT];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) dv[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int vt = 0; vt < VT; ++vt) dv[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const Sp bs = sp8(ab[ks]);
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        float fa[8];
-        ld8c(&sdo[(16 * rt + r16) * LC + 32 * ks + 8 * kq], fa);
-        dv[rt] = mm3(sp8(fa), bs, dv[rt]);
-      }
+      for (int vt = 0; vt < VT; ++vt) dv[vt] = mmp<NP>(cur.aq[ks], dof[ks][vt], dv[vt]);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+        dv[vt] = mm3(cur.kd[ks], plane8(sD[0], sD[1], (16 * vt + r16) * LK + 32 * ks + 8 * kq), dv[vt]);
+#pragma unroll
+    for (int vt = 0; vt < VT; ++vt) {
+      const Sp4 x = sp4(dv[vt]);
+      const int o = (16 * vt + r16) * LC + 16 * wv + 4 * kq;
+      *reinterpret_cast<bf16x4*>(&sdV[0][o]) = x.hi;
+      *reinterpret_cast<bf16x4*>(&sdV[1][o]) = x.lo;
+      ft_store_acc(rec + R::DVN, v0 / 16 + vt, 2, wv, x);
     }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const Sp bs = sp8(kb[ks]);
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        float fa[8];
-        ld8c(&sdST[(16 * rt + r16) * LK + 32 * ks + 8 * kq], fa);
-        dv[rt] = mm3(sp8(fa), bs, dv[rt]);
-      }
-    }
-    float* dvg = w.dvn + ci * C * V;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      const int vr = 16 * rt + 4 * kq;
-      *reinterpret_cast<float4*>(&dvg[cw * V + v0 + vr]) =
-          make_float4(dv[rt][0], dv[rt][1], dv[rt][2], dv[rt][3]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sdVT[(vr + e) * LC + cw] = dv[rt][e];
-    }
-    float el[KT];
-#pragma unroll
-    for (int a = 0; a < KT; ++a) el[a] = elb[a];
-    if (n > 0) prefetch(n - 1);
-#pragma unroll
-    for (int i = 0; i < NKD; ++i) {
-      const int it = tid + 256 * i, c = it % C, k4 = (it / C) * 4;
-      sQT[(k4 + 0) * LC + c] = qr[i].x; sQT[(k4 + 1) * LC + c] = qr[i].y;
-      sQT[(k4 + 2) * LC + c] = qr[i].z; sQT[(k4 + 3) * LC + c] = qr[i].w;
-      sWT[(k4 + 0) * LC + c] = wr[i].x; sWT[(k4 + 1) * LC + c] = wr[i].y;
-      sWT[(k4 + 2) * LC + c] = wr[i].z; sWT[(k4 + 3) * LC + c] = wr[i].w;
-    }
+    ST::store_tiles(rec + R::DSN, sD[0], sD[1], V, v0);
     __syncthreads();
-    // dS_n^T = el dS^T + dO^T Qg - dv_n^T W
+    // dS = el dS' + Qg^T dO - W^T dv_n
 #pragma unroll
-    for (int a = 0; a < KT; ++a)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) D[rt][a] *= el[a];
+      for (int vt = 0; vt < VT; ++vt) D[kt][vt] *= cur.el[kt];
 #pragma unroll
-    for (int ks = 0; ks < C; ks += 32) {
-      const int c0 = ks + 8 * kq;
-      Sp bq[KT], bw[KT];
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
-        float fb[8];
-        ld8c(&sQT[kch * LC + c0], fb);
-        bq[a] = sp8(fb);
-        ld8c(&sWT[kch * LC + c0], fb);
-        bw[a] = sp8(fb);
-      }
+      for (int vt = 0; vt < VT; ++vt) {
+        const Sp x = plane8(sdV[0], sdV[1], (16 * vt + r16) * LC + 32 * ks + 8 * kq);
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        float fa[8], fd[8];
-        ld8c(&sdo[(16 * rt + r16) * LC + c0], fa);
-        ld8c(&sdVT[(16 * rt + r16) * LC + c0], fd);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) fd[i] = -fd[i];
-        const Sp as = sp8(fa), ds = sp8(fd);
-#pragma unroll
-        for (int a = 0; a < KT; ++a) {
-          D[rt][a] = mm3(as, bq[a], D[rt][a]);
-          D[rt][a] = mm3(ds, bw[a], D[rt][a]);
+        for (int kt = 0; kt < KT; ++kt) {
+          D[kt][vt] = mmp<NP>(cur.qg[kt][ks], dof[ks][vt], D[kt][vt]);
+          D[kt][vt] = mm3(cur.wt[kt][ks], x, D[kt][vt]);
         }
       }
-    }
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sdST[(16 * rt + 4 * kq + e) * LK + kch] = D[rt][a][e];
-      }
-    if (n > 0) store_dot(sDOT[(n - 1) & 1]);
+    ST::to_planes(D, sD[0], sD[1]);
+    if (n > 0) put_do((n - 1) & 1, nxt);
     __syncthreads();
+  };
+  Ops oa, ob;
+  fetch(nt - 1, oa);
+  put_do((nt - 1) & 1, oa);
+  __syncthreads();
+#pragma unroll 1
+  for (int n = nt - 1; n >= 0; n -= 2) {
+    chunk(n, oa, ob);
+    if (n > 0) chunk(n - 1, ob, oa);
   }
   if (p.ds0) {
-    float* ds0 = static_cast<float*>(p.ds0);
+    float* ds0 = static_cast<float*>(p.ds0) + (size_t)bh * K * V;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        const int kch = 16 * (wv * KT + a) + r16;
-        *reinterpret_cast<float4*>(&ds0[((size_t)bh * K + kch) * V + v0 + 16 * rt + 4 * kq]) =
-            make_float4(D[rt][a][0], D[rt][a][1], D[rt][a][2], D[rt][a][3]);
-      }
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          ds0[(size_t)(16 * (wv * KT + kt) + 4 * kq + e) * V + v0 + 16 * vt + r16] = D[kt][vt][e];
   }
-}
-
-// Exact decay-weighted gradient terms of row i, channel chl of a block of 64
-// held in LDS with row stride 68: one exponential per (i, j), with the clamp
-// at 50 and its zero gradient in dG. Returns the additions to (dk, dq^, dG,
-// dbeta).
-__device__ __forceinline__ float4 exact_decay_terms(const float* sG, const float* sk, const float* sq,
-                                                 const float* sdM, const float* sdA, const float* sb,
-                                                 int chl, int i) {
-  constexpr int LC = C + 4, LH = 64 + 4;
-  const float Gi = sG[i * LH + chl], ki = sk[i * LH + chl], qi = sq[i * LH + chl], bi = sb[i];
-  float r1 = 0.f, r2 = 0.f, r1g = 0.f, r2g = 0.f;
-  for (int j = 0; j <= i; ++j) {
-    const float d = Gi - sG[j * LH + chl];
-    const float x = ex(fminf(d, kCap)) * sk[j * LH + chl];
-    const float gm = d > kCap ? 0.f : 1.f;
-    const float m = sdM[i * LC + j] * x, a = sdA[i * LC + j] * x;
-    r1 += m;
-    r2 += a;
-    r1g += gm * m;
-    r2g += gm * a;
-  }
-  float c1 = 0.f, c1g = 0.f;
-  for (int r = i; r < C; ++r) {
-    const float d = sG[r * LH + chl] - Gi;
-    const float x = ex(fminf(d, kCap));
-    const float gm = d > kCap ? 0.f : 1.f;
-    const float m = (sb[r] * sdM[r * LC + i] * sk[r * LH + chl] + sdA[r * LC + i] * sq[r * LH + chl]) * x;
-    c1 += m;
-    c1g += gm * m;
-  }
-  return make_float4(bi * r1 + c1, r2, bi * ki * r1g + qi * r2g - ki * c1g, ki * r1);
 }
 
 // ---------------------------------------------------------------------------
-// cb_grad_kernel: one workgroup (8 waves) per (b, hv, chunk)
+// cb_grad_kernel: one workgroup (4 waves) per (b, hv, chunk), two per CU.
+// Bound by HBM (at K = V = 128, bf16: 288 KB read and 64 KB written a chunk).
+// A wave owns whole columns of the chunk (16-channel tiles, all 64 tokens), so
+// the gate sums, their reversed sums and the sums over tokens stay in its
+// registers (in-lane steps and two shuffles), the key and query factors of the
+// decay products are made once, by the lanes that need them, and S and dS'
+// fragments are read by one wave only. The decay products contract over the
+// tokens in accumulator order (lane kq: tokens 16 rt + 4 kq + e), which makes
+// those registers the operand as they stand. The row offsets
+// go through buffer addressing: as 64-bit lane addresses they spilled (805 us).
+// 4096 chunks: 494 us (2.9 TB/s), where fp32 operands split by every reader, two
+// waves a SIMD of one workgroup and a load round trip per step took 1190.
 // ---------------------------------------------------------------------------
 template <int K, int V, typename InT>
-__global__ __launch_bounds__(NTH) void cb_grad_kernel(KdaBwdParams p, CbWs w) {
+__global__ __launch_bounds__(256, 2) void cb_grad_kernel(KdaBwdParams p, CbWs w) {
   using R = Rec<K, V>;
-  constexpr int LC = C + 4, LV = V + 4, KH = 64, LH = KH + 4;
-  constexpr int RG = 3 * C * LH > C * LV ? 3 * C * LH : C * LV;
-  constexpr int NCT1 = V / 16, RT1 = 4 * NCT1 / (NTH / 64);
-  __shared__ float sdBv[C * LV], sdA[C * LC], sdM[C * LC], sR[RG], sb[C], sbeta[C], sext[KH],
-      stot[NTH];
-  __shared__ int sflag;
-  float* const sV = sR;  // dv_n [C][LV] (phase 1)
-  float* const sk = sR;  // channel block: k, q^, G [C][LH]; q^ then dG
-  float* const sq = sR + C * LH;
-  float* const sG = sR + 2 * C * LH;
+  constexpr int LV = V + 8, LC = C + 8, KT = K / 64, VT = V / 64, VS = V / 32, NP = kParts<InT>;
+  __shared__ __attribute__((aligned(16))) bf16_t sdB[2][C * LV], sdA[2][C * LC], sdM[2][C * LC];
+  __shared__ __attribute__((aligned(16))) float sb[C], sbeta[2][4][C];
 
-  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, r16 = l & 15, kq = l >> 4;
+  const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   const int nt = w.nt;
   const int n = blockIdx.x % nt, bh = blockIdx.x / nt;
   const int hv = bh % p.HV, b = bh / p.HV, h = hv / (p.HV / p.H);
@@ -819,346 +917,571 @@ __global__ __launch_bounds__(NTH) void cb_grad_kernel(KdaBwdParams p, CbWs w) {
   const float gmin = (float)p.g_clamp_min;
   const bool direct = w.part == nullptr;
   const size_t ci = blockIdx.x;
-  const float* rec = w.rec + ci * R::RS;
-  const float* Sn = w.sn + ci * K * V;
-  const float* dSn = w.dsn + ci * K * V;
-  const float* vng = w.vn + ci * C * V;
-  const float* dvg = w.dvn + ci * C * V;
-  const InT* dO = static_cast<const InT*>(p.d_o) + ((size_t)b * T * HV + hv) * V;  // row t at t*HV*V
-  const InT* vin = static_cast<const InT*>(p.v) + ((size_t)b * T * HV + hv) * V;
-  const size_t rs = (size_t)HV * V;
-  // phases 2 and 3: wave wv owns column tile ct of row tiles rt0, rt0 + 1
-  const int ct = wv & 3, rt0 = 2 * (wv >> 2);
+  const __amdgpu_buffer_rsrc_t rec = buf(w.rec + ci * R::RS, 2 * (size_t)R::RS);
+  const __amdgpu_buffer_rsrc_t sn = buf(w.sn + ci * 2 * K * V, 4 * (size_t)K * V);
+  const __amdgpu_buffer_rsrc_t vng = buf(w.vn + ci * 2 * C * V, 4 * (size_t)C * V);
+  // the chunk's rows of an input or gradient (row stride ld elements, first
+  // element base0), up to the sequence's end
+  const int last = min(T - 1 - t0, C - 1);
+  constexpr unsigned SZ = sizeof(InT);
+  auto rows = [&](const void* x, int heads, int head, int D) {
+    return buf(static_cast<const char*>(x) + (((size_t)b * T + t0) * heads + head) * D * SZ,
+               (size_t)(last + 1) * heads * D * SZ);
+  };
+  const unsigned rs = HV * V * SZ, rq = p.H * K * SZ, rg = HV * K * SZ;  // row strides, bytes
+  const __amdgpu_buffer_rsrc_t dO = rows(p.d_o, HV, hv, V), vin = rows(p.v, HV, hv, V),
+                               dvout = rows(p.dv, HV, hv, V);
 
-  // phase 1: dBv = X^T dv_n; dv = beta dBv; dbeta += v . dBv
-  for (int it = tid; it < C * V / 4; it += NTH) {
-    const int c = it / (V / 4), v4 = (it % (V / 4)) * 4;
-    *reinterpret_cast<float4*>(&sV[c * LV + v4]) = *reinterpret_cast<const float4*>(&dvg[c * V + v4]);
-  }
+  // dO rows 16 rt + r16, columns 32 ks + 8 kq .. + 7
+  auto do_load = [&](unsigned od, int rt, int ks) {
+    return buf_load<InT, 8>(dO, od + 16 * rt * rs + 32 * ks * SZ);
+  };
+  const unsigned od0 = r16 * rs + 8 * kq * SZ;
+  auto do_split = [](auto raw) {
+    Sp x;
+    if constexpr (NP == 1) {
+      x.hi = __builtin_bit_cast(bf16x8, raw);
+      x.lo = bf16x8{};
+    } else {
+      typedef InT in8 __attribute__((ext_vector_type(8)));
+      const in8 t = __builtin_bit_cast(in8, raw);
+      float f[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] = to_f32((InT)t[i]);
+      x = sp8(f);
+    }
+    return x;
+  };
+  auto raw_f32 = [](uint32_t r) {
+    if constexpr (SZ == 4)
+      return __uint_as_float(r);
+    else
+      return to_f32(__builtin_bit_cast(InT, (uint16_t)r));
+  };
+  auto load1 = [](__amdgpu_buffer_rsrc_t r, unsigned off) -> uint32_t {
+    if constexpr (SZ == 4)
+      return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+    else
+      return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
+  };
+  auto store1 = [](float x, __amdgpu_buffer_rsrc_t r, unsigned off) {
+    const InT y = from_f32<InT>(x);
+    if constexpr (SZ == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), r, off, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, y), r, off, 0, 0);
+  };
+  auto dB_frag = [&](int rt, int ks) {
+    return plane8(sdB[0], sdB[1], (16 * rt + r16) * LV + 32 * ks + 8 * kq);
+  };
+  // dO as the left operand
+  auto mma_do = [](const Sp& a, const Sp& x, f32x4 acc) {
+    if constexpr (SZ == 4) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, x.lo, acc, 0, 0, 0);
+    if constexpr (NP == 2) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, x.hi, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, x.lo, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, x.hi, acc, 0, 0, 0);
+  };
+
+  // fp32 gradients also take the product of the low parts: what S and dS' lose
+  // in their two parts (del needs both) is then no more than the parts' products
+  // lost before
+  auto mmg = [](const Sp& a, const Sp& x, f32x4 acc) {
+    if constexpr (SZ == 4) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, x.lo, acc, 0, 0, 0);
+    return mm3(a, x, acc);
+  };
   if (tid < C) {
     const int t = t0 + tid;
     sb[tid] = t < T ? to_f32(static_cast<const InT*>(p.beta)[(size_t)(b * T + t) * HV + hv]) : 0.f;
-    sbeta[tid] = 0.f;
-  }
-  __syncthreads();
-  {
-    const int ct1 = wv % NCT1, r1 = (wv / NCT1) * RT1, vv = 16 * ct1 + r16;
-    f32x4 acc[RT1];
-#pragma unroll
-    for (int u = 0; u < RT1; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < C; ks += 32) {
-      const int j0 = ks + 8 * kq;
-      float fb[8];
-      ld8s(&sV[j0 * LV + vv], LV, fb);
-      const Sp bs = sp8(fb);
-#pragma unroll
-      for (int u = 0; u < RT1; ++u) {
-        float fa[8];
-        ld8c(&rec[R::XT + (16 * (r1 + u) + r16) * C + j0], fa);
-        acc[u] = mm3(sp8(fa), bs, acc[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < RT1; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = 16 * (r1 + u) + 4 * kq + e, t = t0 + c;
-        const float x = acc[u][e];
-        sdBv[c * LV + vv] = x;
-        float s = 0.f;
-        if (t < T) {
-          const size_t o = (size_t)t * rs + vv;
-          static_cast<InT*>(p.dv)[((size_t)b * T * HV + hv) * V + o] = from_f32<InT>(sb[c] * x);
-          s = to_f32(vin[o]) * x;
-        }
-        s = row16_sum(s);
-        if (r16 == 0) atomicAdd(&sbeta[c], s);
-      }
   }
   __syncthreads();
 
-  // phase 2: dAqk = dO v_n^T (j <= i), dM = -dBv v_n^T (j < i)
-  {
-    f32x4 a1[2], a2[2];
+  bool factored = true;  // every block of 64 channels
 #pragma unroll
-    for (int u = 0; u < 2; ++u) a1[u] = a2[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int ks = 0; ks < V; ks += 32) {
-      const int v0 = ks + 8 * kq;
-      float fb[8];
-      ld8c(&vng[(16 * ct + r16) * V + v0], fb);
-      const Sp bs = sp8(fb);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int c = 16 * (rt0 + u) + r16;
-        float fa[8], fd[8];
-        if (t0 + c < T)
-          ld8g(dO + (size_t)(t0 + c) * rs + v0, fa);
-        else
-          zero8(fa);
-        ld8c(&sdBv[c * LV + v0], fd);
-        a1[u] = mm3(sp8(fa), bs, a1[u]);
-        a2[u] = mm3(sp8(fd), bs, a2[u]);
-      }
-    }
-    const int j = 16 * ct + r16;
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 16 * (rt0 + u) + 4 * kq + e;
-        sdA[i * LC + j] = j <= i ? a1[u][e] : 0.f;
-        sdM[i * LC + j] = j < i ? -a2[u][e] : 0.f;
-      }
-  }
-  __syncthreads();
+  for (int i = 0; i < K / 64; ++i)
+    factored &= __builtin_amdgcn_raw_buffer_load_b32(rec, 0, 2 * R::FL + 4 * i, 0) != 0;
 
-  // phase 3: channel blocks of 64 (lane: channel 16 ct + r16 of the block,
-  // rows 16 (rt0 + u) + 4 kq + e)
-  float dbeta[2][4];
+  // phase 1: dBv^T = dv_n^T X (rows of V, lanes tokens); dv = beta dBv;
+  // dbeta += v . dBv
+  {
+    f32x4 acc[VT][4];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < VT; ++u)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) dbeta[u][e] = 0.f;
-  const int chl = 16 * ct + r16;
-#pragma unroll 1
-  for (int ch0 = 0; ch0 < K; ch0 += KH) {
-    const int chg = ch0 + chl;
-    if (tid == 0) sflag = 1;
-    __syncthreads();
-    bool pos = false;
-    for (int it = tid; it < C * (KH / 8); it += NTH) {
-      const int c = it / (KH / 8), c8 = (it % (KH / 8)) * 8, t = t0 + c;
-      float fq[8], fk[8], fg[8];
-      if (t < T) {
-        const size_t qk = ((size_t)(b * T + t) * p.H + h) * K + ch0 + c8;
-        ld8g(static_cast<const InT*>(p.q) + qk, fq);
-        ld8g(static_cast<const InT*>(p.k) + qk, fk);
-        ld8g(static_cast<const InT*>(p.g) + ((size_t)(b * T + t) * HV + hv) * K + ch0 + c8, fg);
-      } else {
-        zero8(fq); zero8(fk); zero8(fg);
+      for (int ct = 0; ct < 4; ++ct) acc[u][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Sp a[VT][2];
+    typedef InT in4 __attribute__((ext_vector_type(4)));
+    decltype(buf_load<InT, 4>(vin, 0)) vr[VT][4];
+#pragma unroll
+    for (int u = 0; u < VT; ++u) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) a[u][ks] = ft_load(rec, R::DVN, (wv * VT + u) * 2 + ks);
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+        vr[u][ct] = buf_load<InT, 4>(vin, (16 * ct + r16) * rs + (16 * (wv * VT + u) + 4 * kq) * SZ);
+    }
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        if (2 * ks + 1 < ct) continue;  // X^T is upper triangular
+        const Sp x = ft_load(rec, R::XT, ct * 2 + ks);
+#pragma unroll
+        for (int u = 0; u < VT; ++u) acc[u][ct] = mmg(a[u][ks], x, acc[u][ct]);
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float gc = clampg ? fmaxf(fg[i], gmin) : fg[i];
-        pos |= gc > 0.f;
-        sq[c * LH + c8 + i] = scale * fq[i];
-        sk[c * LH + c8 + i] = fk[i];
-        sG[c * LH + c8 + i] = gc;
-      }
-    }
-    if (pos) sflag = 0;
-    __syncthreads();
-    col_scan<KH, false>(sG, LH, stot, nullptr);
-    if (tid < KH) {
-      const float ga = sG[kAnc * LH + tid];
-      if (sG[tid] - ga > kAncRange || ga - sG[(C - 1) * LH + tid] > kAncRange) sflag = 0;
-    }
-    {
-      // el * del for the block's channels: eight lanes per channel
-      const int cl = tid >> 3, part = tid & 7;
-      const float* s1 = Sn + (size_t)(ch0 + cl) * V + part * (V / 8);
-      const float* s2 = dSn + (size_t)(ch0 + cl) * V + part * (V / 8);
+    for (int ct = 0; ct < 4; ++ct) {
+      const int c = 16 * ct + r16;
+      const float bb = sb[c];
       float s = 0.f;
 #pragma unroll
-      for (int i = 0; i < V / 8; i += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(s1 + i);
-        const float4 y = *reinterpret_cast<const float4*>(s2 + i);
-        s += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
-      }
-      s = oct_sum(s);
-      if (part == 0) sext[cl] = ex(sG[(C - 1) * LH + cl]) * s;
-    }
-    __syncthreads();
-    const bool anchored = sflag != 0;
-
-    float dq[2][4], dk[2][4], dg[2][4];
-    {
-      // dQg = dO S^T, dBk = -dBv S^T, dKd = v_n dS'^T
-      f32x4 x1[2], x2[2], x3[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) x1[u] = x2[u] = x3[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int ks = 0; ks < V; ks += 32) {
-        const int v0 = ks + 8 * kq;
-        float fb[8];
-        ld8c(&Sn[(size_t)chg * V + v0], fb);
-        const Sp b1 = sp8(fb);
-        ld8c(&dSn[(size_t)chg * V + v0], fb);
-        const Sp b3 = sp8(fb);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int c = 16 * (rt0 + u) + r16;
-          float fa[8];
-          if (t0 + c < T)
-            ld8g(dO + (size_t)(t0 + c) * rs + v0, fa);
-          else
-            zero8(fa);
-          x1[u] = mm3(sp8(fa), b1, x1[u]);
-          ld8c(&sdBv[c * LV + v0], fa);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) fa[i] = -fa[i];
-          x2[u] = mm3(sp8(fa), b1, x2[u]);
-          ld8c(&vng[c * V + v0], fa);
-          x3[u] = mm3(sp8(fa), b3, x3[u]);
-        }
-      }
-      const float Gl = sG[(C - 1) * LH + chl];
-      float colsum = 0.f;
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < VT; ++u) {
+        const int vv = 16 * (wv * VT + u) + 4 * kq;
+        const f32x4 x = acc[u][ct];
+        const Sp4 y = sp4(x);
+        *reinterpret_cast<bf16x4*>(&sdB[0][c * LV + vv]) = y.hi;
+        *reinterpret_cast<bf16x4*>(&sdB[1][c * LV + vv]) = y.lo;
+        const in4 vin4 = __builtin_bit_cast(in4, vr[u][ct]);
+        in4 dr;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int c = 16 * (rt0 + u) + 4 * kq + e;
-          const float G = sG[c * LH + chl], kk = sk[c * LH + chl], qq = sq[c * LH + chl], bb = sb[c];
-          const float eG = ex(G), ed = ex(Gl - G);
-          const float y1 = x1[u][e], y2 = x2[u][e], y3 = x3[u][e];
-          dq[u][e] = eG * y1;
-          dk[u][e] = ed * y3 + bb * eG * y2;
-          dg[u][e] = qq * eG * y1 - kk * ed * y3 + bb * kk * eG * y2;
-          colsum += kk * ed * y3;
-          dbeta[u][e] += kk * eG * y2;
+          s += to_f32((InT)vin4[e]) * x[e];
+          dr[e] = from_f32<InT>(bb * x[e]);
         }
-      atomicAdd(&sext[chl], colsum);
+        const unsigned o = c * rs + vv * SZ;
+        if constexpr (SZ == 4)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, dr), dvout, o, 0, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, dr), dvout, o, 0, 0);
+      }
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (kq == 0) sbeta[0][wv][c] = s;
     }
+  }
+  __syncthreads();
 
-    if (anchored) {
-      // R1' = dM KN, R2 = dAqk KN, C1 = (beta dM)^T KP, C2 = dAqk^T QP with
-      // KN = k e^(G_a - G), KP = k e^(G - G_a), QP = q^ e^(G - G_a)
-      f32x4 r1[2], r2[2], c1[2], c2[2];
+  // phase 2: dAqk = dO v_n^T (j <= i), dM = -dBv v_n^T (j < i), transposed: the
+  // wave's rows are tokens j of its tile, lanes tokens i
+  {
+    f32x4 a1[4], a2[4];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) r1[u] = r2[u] = c1[u] = c2[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const float Ga = sG[kAnc * LH + chl];
+    for (int rt = 0; rt < 4; ++rt) a1[rt] = a2[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < C; ks += 32) {
-        const int j0 = ks + 8 * kq;
-        float kj[8], gj[8], qj[8], fN[8], fP[8], fQ[8];
-        ld8s(&sk[j0 * LH + chl], LH, kj);
-        ld8s(&sG[j0 * LH + chl], LH, gj);
-        ld8s(&sq[j0 * LH + chl], LH, qj);
+    for (int ks = 0; ks < VS; ++ks) {
+      const Sp a = ft_load(vng, 0, wv * VS + ks);
+      decltype(do_load(0, 0, 0)) d[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float P = ex(gj[i] - Ga), N = ex(Ga - gj[i]);
-          fN[i] = kj[i] * N;
-          fP[i] = kj[i] * P;
-          fQ[i] = qj[i] * P;
-        }
-        const Sp bN = sp8(fN), bP = sp8(fP), bQ = sp8(fQ);
+      for (int rt = 0; rt < 4; ++rt) d[rt] = do_load(od0, rt, ks);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int i0 = 16 * (rt0 + u) + r16;
-          float fa[8];
-          ld8c(&sdM[i0 * LC + j0], fa);
-          r1[u] = mm3(sp8(fa), bN, r1[u]);
-          ld8c(&sdA[i0 * LC + j0], fa);
-          r2[u] = mm3(sp8(fa), bN, r2[u]);
-          ld8s(&sdM[j0 * LC + i0], LC, fa);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) fa[i] *= sb[j0 + i];
-          c1[u] = mm3(sp8(fa), bP, c1[u]);
-          ld8s(&sdA[j0 * LC + i0], LC, fa);
-          c2[u] = mm3(sp8(fa), bQ, c2[u]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int c = 16 * (rt0 + u) + 4 * kq + e;
-          const float G = sG[c * LH + chl], kk = sk[c * LH + chl], qq = sq[c * LH + chl], bb = sb[c];
-          const float P = ex(G - Ga), N = ex(Ga - G);
-          const float y1 = P * r1[u][e], y2 = P * r2[u][e], yc = N * (c1[u][e] + c2[u][e]);
-          dk[u][e] += bb * y1 + yc;
-          dq[u][e] += y2;
-          dg[u][e] += bb * kk * y1 + qq * y2 - kk * yc;
-          dbeta[u][e] += kk * y1;
-        }
-    } else {
-      // one row at a time (a rolled loop keeps the slow path's registers
-      // few); the sums land in the row's registers through an unrolled select
-#pragma unroll 1
-      for (int ue = 0; ue < 8; ++ue) {
-        const float4 x = exact_decay_terms(sG, sk, sq, sdM, sdA, sb, chl,
-                                           16 * (rt0 + (ue >> 2)) + 4 * kq + (ue & 3));
-#pragma unroll
-        for (int z = 0; z < 8; ++z)
-          if (z == ue) {
-            dk[z >> 2][z & 3] += x.x;
-            dq[z >> 2][z & 3] += x.y;
-            dg[z >> 2][z & 3] += x.z;
-            dbeta[z >> 2][z & 3] += x.w;
-          }
+      for (int rt = 0; rt < 4; ++rt) {
+        a1[rt] = mmp<NP>(a, do_split(d[rt]), a1[rt]);
+        a2[rt] = mmg(a, dB_frag(rt, ks), a2[rt]);
       }
     }
-    __syncthreads();  // every read of q^ (sq) done, sext complete
-    // dG -> LDS (over q^); suffix sums over the chunk plus the G_l gradient
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sq[(16 * (rt0 + u) + 4 * kq + e) * LH + chl] = dg[u][e];
-    __syncthreads();
-    col_scan<KH, true>(sq, LH, stot, sext);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int rt = 0; rt < 4; ++rt) {
+      const int i = 16 * rt + r16, j = 16 * wv + 4 * kq;
+      f32x4 x, y;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int c = 16 * (rt0 + u) + 4 * kq + e, t = t0 + c;
-        if (t >= T) continue;
-        const float dgv = sq[c * LH + chl];
-        if (direct) {
-          const size_t qi = ((size_t)(b * T + t) * p.H + h) * K + chg;
-          const size_t gi = ((size_t)(b * T + t) * HV + hv) * K + chg;
-          static_cast<InT*>(p.dq)[qi] = from_f32<InT>(scale * dq[u][e]);
-          static_cast<InT*>(p.dk)[qi] = from_f32<InT>(dk[u][e]);
-          const bool pass = !clampg || to_f32(static_cast<const InT*>(p.g)[gi]) >= gmin;
-          static_cast<InT*>(p.dg)[gi] = from_f32<InT>(pass ? dgv : 0.f);
-        } else {
-          float* pr = w.part + ((size_t)(b * T + t) * HV + hv) * (3 * K + 1);
-          pr[chg] = dq[u][e];
-          pr[K + chg] = dk[u][e];
-          pr[2 * K + chg] = dgv;
+        x[e] = j + e <= i ? a1[rt][e] : 0.f;
+        y[e] = j + e < i ? -a2[rt][e] : 0.f;
+      }
+      if (!factored) {
+        // for the exact decay terms, in fp32 and both orders, over Aqk^T and X^T
+        float* xa = reinterpret_cast<float*>(w.rec + ci * R::RS + R::AQ);
+#pragma unroll 1
+        for (int z = 0; z < 8; ++z) {
+          const int jj = j + (z & 3);
+          float val = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if ((z & 3) == e) val = z < 4 ? x[e] : y[e];
+          if (jj <= i) xa[(z < 4 ? 0 : C * C) + jj * C + i] = xa[(z < 4 ? 0 : C * C) + i * C + jj] = val;
         }
       }
-    __syncthreads();  // before the next block overwrites sR and sext
+      const Sp4 xs = sp4(x), ys = sp4(y);
+      *reinterpret_cast<bf16x4*>(&sdA[0][i * LC + j]) = xs.hi;
+      *reinterpret_cast<bf16x4*>(&sdA[1][i * LC + j]) = xs.lo;
+      *reinterpret_cast<bf16x4*>(&sdM[0][i * LC + j]) = ys.hi;
+      *reinterpret_cast<bf16x4*>(&sdM[1][i * LC + j]) = ys.lo;
+    }
+  }
+  __syncthreads();
+
+  // phase 3: the wave's channel tiles; lane: channel ch, tokens 16 rt + 4 kq + e
+  float dbeta[4][4];
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dbeta[rt][e] = 0.f;
+#pragma unroll 1
+  for (int kt = 0; kt < KT; ++kt) {
+    const int ctg = wv * KT + kt, ch = 16 * ctg + r16;
+    // dQg = dO S^T, dBk = -dBv S^T, dKd = v_n dS'^T; del
+    f32x4 x1[4], x2[4], x3[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) x1[rt] = x2[rt] = x3[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float del = 0.f;
+    // the next step's state tiles (read here only) are in flight through each
+    // step, the gates, keys and queries through the last
+    const __amdgpu_buffer_rsrc_t qb = rows(p.q, p.H, h, K), kb = rows(p.k, p.H, h, K),
+                                 gb = rows(p.g, HV, hv, K);
+    unsigned oq = 4 * kq * rq + ch * SZ, og = 4 * kq * rg + ch * SZ;
+    unsigned od = od0;
+    // (opaque, or the loop keeps every row's offset in a register of its own)
+    asm volatile("" : "+v"(oq), "+v"(og), "+v"(od));
+    uint32_t xg[4][4], xq[4][4], xk[4][4];
+    Sp b1 = ft_load(sn, 0, ctg * VS), b3 = ft_load(rec, R::DSN, ctg * VS);
+#pragma unroll
+    for (int ks = 0; ks < VS; ++ks) {
+      decltype(do_load(0, 0, 0)) d[4];
+      Sp v[4], n1, n3;
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        d[rt] = do_load(od, rt, ks);
+        v[rt] = ft_load(vng, 0, rt * VS + ks);
+      }
+      if (ks + 1 < VS) {
+        n1 = ft_load(sn, 0, ctg * VS + ks + 1);
+        n3 = ft_load(rec, R::DSN, ctg * VS + ks + 1);
+      } else {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            xg[rt][e] = load1(gb, og + (16 * rt + e) * rg);
+            xq[rt][e] = load1(qb, oq + (16 * rt + e) * rq);
+            xk[rt][e] = load1(kb, oq + (16 * rt + e) * rq);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        del += ((float)b1.hi[i] + (float)b1.lo[i]) * ((float)b3.hi[i] + (float)b3.lo[i]);
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        x1[rt] = mma_do(do_split(d[rt]), b1, x1[rt]);
+        x2[rt] = mmg(dB_frag(rt, ks), b1, x2[rt]);
+        x3[rt] = mmg(v[rt], b3, x3[rt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      b1 = n1;
+      b3 = n3;
+    }
+    del += __shfl_xor(del, 16);
+    del += __shfl_xor(del, 32);
+
+    float G[4][4], kk[4][4], qq[4][4];
+    unsigned pass = 0;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float g = raw_f32(xg[rt][e]);
+        if (!clampg || g >= gmin) pass |= 1u << (4 * rt + e);
+        G[rt][e] = clampg ? fmaxf(g, gmin) : g;
+        qq[rt][e] = scale * raw_f32(xq[rt][e]);
+        kk[rt][e] = raw_f32(xk[rt][e]);
+      }
+    // prefix sums over the chunk's tokens: in runs of 8 (lanes kq, kq + 1), then
+    // over the runs
+    float run = 0.f;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      const float half = ((G[rt][0] + G[rt][1]) + G[rt][2]) + G[rt][3];
+      const float before = __shfl_xor(half, 16);
+      if (kq & 1) G[rt][0] += before;
+#pragma unroll
+      for (int e = 1; e < 4; ++e) G[rt][e] += G[rt][e - 1];
+      const float t0r = __shfl(G[rt][3], 16 + r16), t1r = __shfl(G[rt][3], 48 + r16);
+      const float off = kq < 2 ? run : run + t0r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) G[rt][e] += off;
+      run = (run + t0r) + t1r;
+    }
+    const float Ga = __shfl(G[1][3], 48 + r16), Gl = __shfl(G[3][3], 48 + r16);
+    const bool anchored =
+        factored || __builtin_amdgcn_raw_buffer_load_b32(rec, 0, 2 * R::FL + 4 * (ctg / 4), 0) != 0;
+
+    float dq[4][4], dk[4][4], dg[4][4], ext = 0.f;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      const float4 b4 = *reinterpret_cast<const float4*>(&sb[16 * rt + 4 * kq]);
+      const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float eG = ex(G[rt][e]), ed = ex(Gl - G[rt][e]);
+        const float y1 = eG * x1[rt][e], y2 = -eG * x2[rt][e], y3 = ed * x3[rt][e];
+        dq[rt][e] = y1;
+        dk[rt][e] = y3 + bb[e] * y2;
+        dg[rt][e] = qq[rt][e] * y1 - kk[rt][e] * y3 + bb[e] * kk[rt][e] * y2;
+        ext += kk[rt][e] * y3;
+        dbeta[rt][e] += kk[rt][e] * y2;
+      }
+    }
+    ext += __shfl_xor(ext, 16);
+    ext += __shfl_xor(ext, 32);
+    ext += ex(Gl) * del;
+
+    if (anchored) {
+      // R1' = dM KN, R2 = dAqk KN, then C = dM^T (beta KP) + dAqk^T QP with
+      // KN = k e^(G_a - G), KP = k e^(G - G_a), QP = q^ e^(G - G_a); one after
+      // the other, as all accumulators at once do not fit the registers
+      {
+        f32x4 r1[4], r2[4];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) r1[rt] = r2[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          float f[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            f[i] = kk[2 * ks + (i >> 2)][i & 3] * ex(Ga - G[2 * ks + (i >> 2)][i & 3]);
+          const Sp bN = sp8(f);
+          // tokens j <= i: rows of dM and dAqk
+          auto rows = [&](const bf16_t* hi, const bf16_t* lo, int rt) {
+            const int o = (16 * rt + r16) * LC + 32 * ks + 4 * kq;
+            return Sp{cat4(*reinterpret_cast<const bf16x4*>(hi + o),
+                           *reinterpret_cast<const bf16x4*>(hi + o + 16)),
+                      cat4(*reinterpret_cast<const bf16x4*>(lo + o),
+                           *reinterpret_cast<const bf16x4*>(lo + o + 16))};
+          };
+#pragma unroll
+          for (int rt = 2 * ks; rt < 4; ++rt) {
+            r1[rt] = mmg(rows(sdM[0], sdM[1], rt), bN, r1[rt]);
+            r2[rt] = mmg(rows(sdA[0], sdA[1], rt), bN, r2[rt]);
+          }
+        }
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+          const f32x4 bb = *reinterpret_cast<const f32x4*>(&sb[16 * rt + 4 * kq]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float P = ex(G[rt][e] - Ga);
+            const float y1 = kk[rt][e] * (P * r1[rt][e]), y2 = P * r2[rt][e];
+            dk[rt][e] += bb[e] * (P * r1[rt][e]);
+            dq[rt][e] += y2;
+            dg[rt][e] += bb[e] * y1 + qq[rt][e] * y2;
+            dbeta[rt][e] += y1;
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4 cc[4];
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) cc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        float fP[8], fQ[8];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+          const f32x4 bb = *reinterpret_cast<const f32x4*>(&sb[16 * (2 * ks + z) + 4 * kq]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float P = ex(G[2 * ks + z][e] - Ga);
+            fP[4 * z + e] = bb[e] * kk[2 * ks + z][e] * P;
+            fQ[4 * z + e] = qq[2 * ks + z][e] * P;
+          }
+        }
+        const Sp bP = sp8(fP), bQ = sp8(fQ);
+        // tokens i >= j: columns of dM and dAqk
+        auto cols = [&](const bf16_t* hi, const bf16_t* lo, int rt) {
+          const int r0 = 32 * ks + 4 * kq;
+          return Sp{cat4(tr4(hi, LC, r0, 16 * rt), tr4(hi, LC, r0 + 16, 16 * rt)),
+                    cat4(tr4(lo, LC, r0, 16 * rt), tr4(lo, LC, r0 + 16, 16 * rt))};
+        };
+#pragma unroll
+        for (int rt = 0; rt < 2 * ks + 2; ++rt) {
+          cc[rt] = mmg(cols(sdM[0], sdM[1], rt), bP, cc[rt]);
+          cc[rt] = mmg(cols(sdA[0], sdA[1], rt), bQ, cc[rt]);
+        }
+      }
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float yc = ex(Ga - G[rt][e]) * cc[rt][e];
+          dk[rt][e] += yc;
+          dg[rt][e] -= kk[rt][e] * yc;
+        }
+    } else {
+      // The exact products, one exponential per token pair and channel, with the
+      // clamp at 50 and its zero gradient in dG: over tokens j in turn, each lane
+      // adds the pair's term to its 16 tokens i (j < i: row i of dM and dAqk, j >
+      // i: column i). G, k, q^ of the tile pass through the chunk's record (its
+      // Kd, Qg^T and W^T are not read any more); token j + 1's values are in
+      // flight through token j's 16 terms.
+      auto at = [&](unsigned v, int off) {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rec, v, off, 0));
+      };
+      auto at4 = [&](unsigned v, int off) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rec, v, off, 0));
+      };
+      auto put = [&](float x, unsigned v, int off) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rec, v, off, 0);
+      };
+      constexpr int oG = 2 * R::KD1, ok = oG + 4 * C * K, oq2 = ok + 4 * C * K;
+      constexpr int oA = 2 * R::AQ, oM = oA + 4 * C * C;
+      unsigned vo = 4 * ch, vd = 4 * (4 * kq * (C + 1)), vr = 16 * kq;
+      asm volatile("" : "+v"(vo), "+v"(vd), "+v"(vr));
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned v = vo + 16 * kq * K;
+          const int o = 4 * (16 * rt + e) * K;
+          put(G[rt][e], v, oG + o);
+          put(kk[rt][e], v, ok + o);
+          put(qq[rt][e], v, oq2 + o);
+          const float a = at(vd, oA + 4 * (16 * rt + e) * (C + 1));  // dAqk[i][i]
+          dq[rt][e] += a * kk[rt][e];
+          dk[rt][e] += a * qq[rt][e];
+        }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+      float nG = at(vo, oG), nk = at(vo, ok), nq = at(vo, oq2);
+#pragma unroll 1
+      for (int j = 0; j < C; ++j) {
+        const float Gj = nG, kj = nk, qj = nq, bk = sb[j] * nk;
+        int i0 = 4 * kq;
+        asm volatile("" : "+v"(i0));  // (as above)
+        const int jn = 4 * K * min(j + 1, C - 1);
+        nG = at(vo, oG + jn);
+        nk = at(vo, ok + jn);
+        nq = at(vo, oq2 + jn);
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+          const f32x4 A = at4(vr, oA + 4 * (j * C + 16 * rt)), M = at4(vr, oM + 4 * (j * C + 16 * rt));
+          const f32x4 bb = *reinterpret_cast<const f32x4*>(&sb[16 * rt + i0]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 16 * rt + e + i0;
+            const float d0 = G[rt][e] - Gj, d = j < i ? d0 : -d0;
+            const float E = ex(fminf(d, kCap)), x = E * kj;
+            const float m = j < i ? M[e] * x : 0.f, a = j < i ? A[e] * x : 0.f;
+            const float c = j > i ? (M[e] * bk + A[e] * qj) * E : 0.f;
+            const float km = kk[rt][e] * m;
+            dk[rt][e] += bb[e] * m + c;
+            dq[rt][e] += a;
+            dbeta[rt][e] += km;
+            const float t = bb[e] * km + qq[rt][e] * a - kk[rt][e] * c;
+            dg[rt][e] += d > kCap ? 0.f : t;
+          }
+        }
+      }
+    }
+    // suffix sums of dG over the chunk's tokens, plus the G_l gradient
+    run = ext;
+#pragma unroll
+    for (int rt = 3; rt >= 0; --rt) {
+      const float half = ((dg[rt][3] + dg[rt][2]) + dg[rt][1]) + dg[rt][0];
+      const float after = __shfl_xor(half, 16);
+      if (!(kq & 1)) dg[rt][3] += after;
+#pragma unroll
+      for (int e = 2; e >= 0; --e) dg[rt][e] += dg[rt][e + 1];
+      const float t1r = __shfl(dg[rt][0], 32 + r16), t0r = __shfl(dg[rt][0], r16);
+      const float off = kq >= 2 ? run : run + t1r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dg[rt][e] += off;
+      run = (run + t1r) + t0r;
+    }
+    if (direct) {
+      const __amdgpu_buffer_rsrc_t dqb = rows(p.dq, p.H, h, K), dkb = rows(p.dk, p.H, h, K),
+                                   dgb = rows(p.dg, HV, hv, K);
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          store1(scale * dq[rt][e], dqb, oq + (16 * rt + e) * rq);
+          store1(dk[rt][e], dkb, oq + (16 * rt + e) * rq);
+          store1((pass >> (4 * rt + e)) & 1 ? dg[rt][e] : 0.f, dgb, og + (16 * rt + e) * rg);
+        }
+    } else {
+      const unsigned ld = HV * (3 * K + 1) * 4;
+      const __amdgpu_buffer_rsrc_t prb =
+          buf(w.part + ((size_t)(b * T + t0) * HV + hv) * (3 * K + 1), (size_t)(last + 1) * ld);
+      unsigned op = 4 * kq * ld + 4 * ch;
+      asm volatile("" : "+v"(op));
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned o = op + (16 * rt + e) * ld;
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dq[rt][e]), prb, o, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dk[rt][e]), prb, o + 4 * K, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dg[rt][e]), prb, o + 8 * K, 0, 0);
+        }
+    }
   }
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float s = row16_sum(dbeta[u][e]);
-      if (r16 == 0) atomicAdd(&sbeta[16 * (rt0 + u) + 4 * kq + e], s);
+      const float s = row16_sum(dbeta[rt][e]);
+      if (r16 == 0) sbeta[1][wv][16 * rt + 4 * kq + e] = s;
     }
   __syncthreads();
   if (tid < C && t0 + tid < T) {
     const int t = t0 + tid;
+    float s = 0.f;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) s += sbeta[0][z][tid] + sbeta[1][z][tid];
     if (direct)
-      static_cast<InT*>(p.dbeta)[(size_t)(b * T + t) * HV + hv] = from_f32<InT>(sbeta[tid]);
+      static_cast<InT*>(p.dbeta)[(size_t)(b * T + t) * HV + hv] = from_f32<InT>(s);
     else
-      w.part[((size_t)(b * T + t) * HV + hv) * (3 * K + 1) + 3 * K] = sbeta[tid];
+      w.part[((size_t)(b * T + t) * HV + hv) * (3 * K + 1) + 3 * K] = s;
   }
 }
 
 size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
 
-size_t rec_floats(int K, int V) {
-  const int el = 3 * C * K + C * V + 2 * C * C;
-  return (size_t)((el + K + 63) / 64 * 64);
+int cu_count() {
+  // multiprocessor count of each device, queried once
+  static std::atomic<int> counts[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int c = counts[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
+    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
+    counts[dev].store(c, std::memory_order_relaxed);
+  }
+  return c;
+}
+
+size_t rec_bytes(int K, int V) {
+  return 2 * ((size_t)10 * C * K + 2 * C * V + 4 * C * C + 2 * K + 128);
+}
+
+// Slices of V per state workgroup: 32 columns when 64-column slices would
+// leave half of the CUs without one (a workgroup's share of a chunk is then
+// half as long; the rows of W, Kd and Qg that both halves read come from their
+// XCD's L2). Forward and backward of
+// 16 heads of 128 at T 2048: B 4 (128 workgroups of 64 columns) 966 us against
+// 870 with 32, B 5 (160) 1113 against 1169; heads of 64 at B 8 (128) 831 against
+// 777, B 12 (192) 1112 against 1129.
+template <int K, int V, int VS, typename InT>
+hipError_t state_launch(const KdaBwdParams& p, const CbWs& w, hipStream_t s) {
+  const unsigned grid = (unsigned)((size_t)p.B * p.HV * (V / VS));
+  hipLaunchKernelGGL((cb_fwd_kernel<K, V, VS>), dim3(grid), dim3(256), 0, s, p, w);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((cb_bwd_kernel<K, V, VS, InT>), dim3(grid), dim3(256), 0, s, p, w);
+  return hipGetLastError();
 }
 
 template <int K, int V, typename InT>
 hipError_t cb_launch(const KdaBwdParams& p, const CbWs& w, hipStream_t s) {
   constexpr int dt = sizeof(InT) == 4 ? DT_F32 : (std::is_same<InT, bf16_t>::value ? DT_BF16 : DT_F16);
   const unsigned chunks = (unsigned)((size_t)p.B * p.HV * w.nt);
-  const unsigned heads = (unsigned)((size_t)p.B * p.HV * (V / 64));
   hipLaunchKernelGGL((cb_prep_kernel<K, V, InT>), dim3(chunks), dim3(NTH), 0, s, p, w);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((cb_fwd_kernel<K, V>), dim3(heads), dim3(256), 0, s, p, w);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL((cb_bwd_kernel<K, V, InT>), dim3(heads), dim3(256), 0, s, p, w);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL((cb_grad_kernel<K, V, InT>), dim3(chunks), dim3(NTH), 0, s, p, w);
+  if (2LL * p.B * p.HV * (V / 64) <= cu_count())
+    e = state_launch<K, V, 32, InT>(p, w, s);
+  else
+    e = state_launch<K, V, 64, InT>(p, w, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((cb_grad_kernel<K, V, InT>), dim3(chunks), dim3(256), 0, s, p, w);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (w.part) {
     KdaBwdParams q = p;
@@ -1178,8 +1501,6 @@ hipError_t cb_by_shape(const KdaBwdParams& p, const CbWs& w, hipStream_t s) {
 
 }  // namespace
 
-static_assert(Rec<128, 128>::RS % 64 == 0 && Rec<64, 64>::RS % 64 == 0, "record alignment");
-
 bool kda_chunk_bwd_supported(int K, int V, int dtype) {
   return dtype != DT_F64 && (K == 64 || K == 128) && (V == 64 || V == 128);
 }
@@ -1187,9 +1508,9 @@ bool kda_chunk_bwd_supported(int K, int V, int dtype) {
 size_t kda_chunk_bwd_ws_bytes(int B, int T, int H, int HV, int K, int V) {
   const size_t nt = (size_t)(T + C - 1) / C;
   const size_t chunks = (size_t)B * HV * nt;
-  size_t total = al256(chunks * rec_floats(K, V) * 4);
-  total += 2 * al256(chunks * K * V * 4);
-  total += 2 * al256(chunks * C * V * 4);
+  size_t total = al256(chunks * rec_bytes(K, V));
+  total += al256(chunks * K * V * 4);
+  total += al256(chunks * C * V * 4);
   if (HV != H) total += al256((size_t)B * T * HV * (3 * K + 1) * 4);
   return total;
 }
@@ -1200,15 +1521,11 @@ hipError_t kda_chunk_bwd_dispatch(KdaBwdParams p, int dtype, void* ws, hipStream
   char* base = static_cast<char*>(ws);
   CbWs w;
   w.nt = nt;
-  w.rec = reinterpret_cast<float*>(base);
-  base += al256(chunks * rec_floats(p.K, p.V) * 4);
-  w.sn = reinterpret_cast<float*>(base);
+  w.rec = reinterpret_cast<bf16_t*>(base);
+  base += al256(chunks * rec_bytes(p.K, p.V));
+  w.sn = reinterpret_cast<bf16_t*>(base);
   base += al256(chunks * p.K * p.V * 4);
-  w.dsn = reinterpret_cast<float*>(base);
-  base += al256(chunks * p.K * p.V * 4);
-  w.vn = reinterpret_cast<float*>(base);
-  base += al256(chunks * C * p.V * 4);
-  w.dvn = reinterpret_cast<float*>(base);
+  w.vn = reinterpret_cast<bf16_t*>(base);
   base += al256(chunks * C * p.V * 4);
   w.part = p.HV != p.H ? reinterpret_cast<float*>(base) : nullptr;
   if (dtype == DT_F32) return cb_by_shape<float>(p, w, stream);

@@ -323,3 +323,30 @@ def test_chunk_bwd_clamp_matches_chunk_form_autograd(dev):
     assert np.abs(rec[0] - ref[0]).max() > 0.5 * np.abs(ref[0]).max()
     assert np.abs(rec[3] - ref[3]).max() > 1e-2 * np.abs(ref[3]).max()
     _check(got, ref, 1e-4, label="clamp")
+
+
+@pytest.mark.parametrize("B,T,H,HV,K,V,exact", [
+    (1, 63, 2, 2, 128, 128, None),     # one short chunk, 32-column slices of the state
+    (1, 129, 1, 2, 128, 64, "upper"),  # one row past two chunks, per-value-head partials
+    (2, 64, 1, 1, 64, 128, "all"),     # a whole chunk, the exact products throughout
+    (9, 65, 16, 16, 64, 64, None),     # 64-column slices
+    (3, 70, 32, 32, 128, 128, "lower"),
+])
+def test_chunk_bwd_tile_edges(dev, B, T, H, HV, K, V, exact):
+    """``kch_kda_chunk_bwd`` at the edges of its chunks of 64 tokens, on both
+    widths of the state kernels' slices, with the decay products of a half of
+    the channels formed exactly (gates of both signs) beside factored ones;
+    fp32 at 1e-4 of each tensor's largest gradient (two-part bf16 products,
+    2^-16 each, over at most 128 + 64 terms of random sign)."""
+    import kch
+    host, s0, w_o, w_s = _make(T + K + V, B, T, H, HV, K, V)
+    sel = {None: slice(0, 0), "all": slice(0, K), "lower": slice(0, K // 2),
+           "upper": slice(K // 2, K)}[exact]
+    g = host[3].copy()
+    g[..., sel] = 0.3 * np.random.default_rng(T).standard_normal(g[..., sel].shape)
+    host[3] = g
+    host = [np.asarray(x, np.float32).astype(np.float64) for x in host]
+    s0 = s0.astype(np.float32).astype(np.float64)
+    ts, s0t = _leaves(host, s0, dev, torch.float32, torch.float32)
+    got = _hip_grads(kch.naive_chunk_kda, ts, s0t, w_o, w_s)
+    _check(got, _ref(host, s0, w_o, w_s), 1e-4, label=f"{B} {T} {exact}")
