@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define KCH_ABI_VERSION 21
+#define KCH_ABI_VERSION 22
 
 #define KCH_OK 0
 #define KCH_ERR_INVALID 1     /* bad pointer / shape / argument */
@@ -625,6 +625,21 @@ int kch_csa_cache_append(const void* proj, long long ld_proj, void* acc, void* p
 int kch_hca_cache_append(const void* proj, long long ld_proj, void* acc, const float* B_pos,
                          void* ring, void* c_rows, void* c_keys, const int* n_seen, int B, int c,
                          int m2, int win, int cap, int normalize, int dtype, void* stream);
+
+/*
+ * kch_csa_cache_append / kch_hca_cache_append with the count of tokens cached
+ * before this one given by value (n_seen >= 0). What only a token that completes
+ * a block uses (prev, the biases, c_rows, c_keys, k_rows, k_inv, cap) may be
+ * null (0) for the others.
+ */
+int kch_csa_cache_append_at(const void* proj, long long ld_proj, void* acc, void* prev,
+                            const float* Ba, const float* Bb, const float* B_idx, void* ring,
+                            void* c_rows, void* c_keys, void* k_rows, float* k_inv, int n_seen,
+                            int B, int c, int cI, int m, int win, int cap, int normalize,
+                            int dtype, void* stream);
+int kch_hca_cache_append_at(const void* proj, long long ld_proj, void* acc, const float* B_pos,
+                            void* ring, void* c_rows, void* c_keys, int n_seen, int B, int c,
+                            int m2, int win, int cap, int normalize, int dtype, void* stream);
 
 /*
  * The front of a KDA sub-layer and its input projection for one token, in one

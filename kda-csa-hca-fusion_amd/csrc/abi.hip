@@ -1112,6 +1112,58 @@ int kch_hca_cache_append(const void* proj, long long ld_proj, void* acc, const f
   return hip_status(fn, kch::cache_step_dispatch(p, dtype, (hipStream_t)stream));
 }
 
+// the same by a host count: block operands are needed only where the token
+// completes block n_seen / m
+static int check_cache_append_at(const char* fn, const void* proj, long long ld_proj,
+                                 long long width, const void* acc, const void* block_ptrs_ok,
+                                 int n_seen, int B, int c, int m, int win, const void* ring,
+                                 int cap, int dtype) {
+  if (n_seen < 0) return fail(KCH_ERR_INVALID, "%s: n_seen=%d", fn, n_seen);
+  const bool ends = m >= 1 && n_seen % m == m - 1;
+  const int rc = check_cache_append(fn, proj, ld_proj, width, acc, acc, acc, &n_seen, B, c, m, win,
+                                    ring, ends ? cap : 1, dtype);
+  if (rc) return rc;
+  if (ends && !block_ptrs_ok) return fail(KCH_ERR_INVALID, "%s: null pointer", fn);
+  if (ends && n_seen / m >= cap)
+    return fail(KCH_ERR_INVALID, "%s: block %d of a store of %d", fn, n_seen / m, cap);
+  return KCH_OK;
+}
+
+int kch_csa_cache_append_at(const void* proj, long long ld_proj, void* acc, void* prev,
+                            const float* Ba, const float* Bb, const float* B_idx, void* ring,
+                            void* c_rows, void* c_keys, void* k_rows, float* k_inv, int n_seen,
+                            int B, int c, int cI, int m, int win, int cap, int normalize,
+                            int dtype, void* stream) {
+  const char* fn = "kch_csa_cache_append_at";
+  if (c < 1 || cI < 1 || c > 256 || c + cI > 256)
+    return fail(KCH_ERR_UNSUPPORTED, "%s: c=%d, cI=%d (c + cI at most 256)", fn, c, cI);
+  const void* ok = prev && Ba && Bb && B_idx && c_rows && c_keys && k_rows && k_inv ? prev : nullptr;
+  const int rc = check_cache_append_at(fn, proj, ld_proj, 4LL * c + 2LL * cI, acc, ok, n_seen, B, c,
+                                       m, win, ring, cap, dtype);
+  if (rc) return rc;
+  if (B == 0) return KCH_OK;
+  kch::CacheStepParams p{proj, ld_proj, acc, prev, Ba, Bb, B_idx, win > 0 ? ring : nullptr,
+                         c_rows, c_keys, k_rows, k_inv, nullptr, B, c, cI, m, win, cap,
+                         normalize != 0, 1, n_seen};
+  return hip_status(fn, kch::cache_step_dispatch(p, dtype, (hipStream_t)stream));
+}
+
+int kch_hca_cache_append_at(const void* proj, long long ld_proj, void* acc, const float* B_pos,
+                            void* ring, void* c_rows, void* c_keys, int n_seen, int B, int c,
+                            int m2, int win, int cap, int normalize, int dtype, void* stream) {
+  const char* fn = "kch_hca_cache_append_at";
+  if (c < 1 || c > 256) return fail(KCH_ERR_UNSUPPORTED, "%s: c=%d > 256", fn, c);
+  const void* ok = B_pos && c_rows && c_keys ? c_rows : nullptr;
+  const int rc = check_cache_append_at(fn, proj, ld_proj, 2LL * c, acc, ok, n_seen, B, c, m2, win,
+                                       ring, cap, dtype);
+  if (rc) return rc;
+  if (B == 0) return KCH_OK;
+  kch::CacheStepParams p{proj, ld_proj, acc, nullptr, B_pos, nullptr, nullptr,
+                         win > 0 ? ring : nullptr, c_rows, c_keys, nullptr, nullptr, nullptr, B, c,
+                         0, m2, win, cap, normalize != 0, 0, n_seen};
+  return hip_status(fn, kch::cache_step_dispatch(p, dtype, (hipStream_t)stream));
+}
+
 // A row projection y = x W^T launched beside a cache append: bf16 / fp16, M
 // rows (M <= 16), K a multiple of 32, 16-byte aligned x and w rows.
 static int rows_beside(const char* fn, const void* x, long long ldx, const void* w, long long ldw,

@@ -285,7 +285,7 @@ template <typename T>
 __device__ __forceinline__ void cache_step_block(const CacheStepParams& p, int b) {
   __shared__ float red[8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int t = p.n_seen[0];
+  const int t = p.n_seen ? p.n_seen[0] : p.n_host;
   const int m = p.m, c = p.c, cI = p.cI;
   const int W = p.csa ? 4 * c + 2 * cI : 2 * c;
   const int j_cur = t % m, blk = t / m;

@@ -414,8 +414,9 @@ struct CacheStepParams {
   void* c_keys;      // [B, cap, c] bf16
   void* k_rows;      // [B, cap, cI] (CSA)
   float* k_inv;      // [B, cap] (CSA)
-  const int* n_seen;
+  const int* n_seen;  // device count of the tokens cached before this one, or null: n_host
   int B, c, cI, m, win, cap, normalize, csa;
+  int n_host = 0;
 };
 hipError_t cache_step_dispatch(const CacheStepParams& p, int dtype, hipStream_t s);
 // The append and a row projection (no norm, residual or counter; bf16 / fp16)

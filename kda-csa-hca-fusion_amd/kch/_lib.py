@@ -78,6 +78,8 @@ _SIGNATURES = {
                                                                                _P],
     "kch_csa_cache_append": [_P, _L] + [_P] * 11 + [_I] * 8 + [_P],
     "kch_hca_cache_append": [_P, _L] + [_P] * 6 + [_I] * 7 + [_P],
+    "kch_csa_cache_append_at": [_P, _L] + [_P] * 10 + [_I] * 9 + [_P],
+    "kch_hca_cache_append_at": [_P, _L] + [_P] * 5 + [_I] * 8 + [_P],
     "kch_csa_cache_append_rows": [_P, _L] + [_P] * 11 + [_I] * 7 + [_P, _L, _P, _L, _P, _L, _I, _I,
                                                                     _I, _P],
     "kch_hca_cache_append_rows": [_P, _L] + [_P] * 6 + [_I] * 6 + [_P, _L, _P, _L, _P, _L, _I, _I,

@@ -238,6 +238,45 @@ def _column_group(ts):
     return t0.as_strided((*lead, w), st)
 
 
+# widths of the one-launch append: those of the bulk compression (the append
+# kernel itself takes c + c_I <= 256), so that a cache refuses the same sizes
+# however its tokens arrive
+_ONE_TOKEN_MAX = 128
+
+
+def _one_token_rows(cache, new, widths):
+    """The ``[B, W]`` rows of one token's projections for the one-launch append,
+    or None where the general path has to take the call: projections and buffers
+    of one dtype on one device, in the shapes the cache holds, and ring and key
+    rows normalised alike."""
+    B, dt, sw = cache.B, cache.dtype, cache._sw
+    dev = new[0].get_device()
+    if cache.device.index != dev:
+        return None
+    for t, w in zip(new, widths):
+        if t.dtype != dt or t.get_device() != dev or t.shape != (B, 1, w):
+            return None
+    if not cache._device_ready(dt) or cache._C.key_norm not in (None, cache._normalize_qk):
+        return None
+    if sw is not None and (sw._written != cache._n_tokens_seen or sw._buf.get_device() != dev
+                           or sw._buf.dtype != dt):
+        return None
+    if cache._acc is not None and cache._acc_buf.get_device() != dev:
+        return None
+    rows = _column_group(new)
+    if rows is None or rows.stride(0) < rows.shape[-1]:
+        rows = torch.cat(new, -1)
+    return rows
+
+
+def _bias_rows(biases, m, widths, dev):
+    """fp32 position biases ``[m, w]`` on ``dev``, or None if one has another form."""
+    if any(t.shape != (m, w) or t.device != dev or t.dtype == torch.float64
+           for t, w in zip(biases, widths)):
+        return None
+    return [_f32(t, dev) for t in biases]
+
+
 def _ring_rows(x, dtype, normalize):
     """Sliding-window rows of ``x``: L2-normalised in fp32 and rounded to the
     cache dtype (the kernel writes bf16 itself, rounding the same fp32 value)."""
@@ -348,6 +387,10 @@ class CSADecodingCache:
         _lib.require_gpu("CSADecodingCache.append_step", Ca_new)
         new = [Ca_new, Cb_new, Za_new, Zb_new, K_idx_new, Z_idx_new]
         with torch.no_grad():
+            if T_new == 1 and max(c, self.c_I) <= _ONE_TOKEN_MAX:
+                out_idx = self._append_one(new, (Ba, Bb, B_idx))
+                if out_idx is not None:
+                    return out_idx
             if self._sw is not None:
                 self._sw.append(_ring_rows(Ca_new, self.dtype, self._normalize_qk))
             if self._acc is None:
@@ -392,6 +435,49 @@ class CSADecodingCache:
             self._acc_len = rem
             self._n_tokens_seen += T_new
         return out_idx
+
+    def _append_one(self, new, biases):
+        """``append_step`` of one token in one launch (``kch_csa_cache_append_at``),
+        or None where the general path has to take it (before any change)."""
+        B, m, c, cI = self.B, self.m, self.c, self.c_I
+        rows = _one_token_rows(self, new, (c, c, c, c, cI, cI))
+        if rows is None:
+            return None
+        n, dev, dt = self._n_tokens_seen, rows.device, self.dtype
+        nb = self._n_blocks
+        ends = self._acc_len == m - 1
+        if n != nb * m + self._acc_len or n >= 2 ** 31 - 1:
+            return None
+        C, K, cap = self._C, self._K, 0
+        prev = Ba = Bb = Bi = None
+        if ends:
+            fp = _bias_rows(biases, m, (c, c, cI), dev)
+            if fp is None or (C.rows is not None and C.rows.device != dev):
+                return None
+            Ba, Bb, Bi = fp
+            if self._prev_buf is None:
+                self._set_prev_buf(torch.empty(B, m, 2 * c, device=dev, dtype=dt))
+            prev = self._prev_buf
+            C.ensure(nb, nb + 1)
+            K.ensure(nb, nb + 1)
+            cap = max(C.rows.shape[1], K.rows.shape[1])
+            # (the kernel addresses both stores with one block stride)
+            C.ensure(nb, cap)
+            K.ensure(nb, cap)
+            if C.key_norm is None:
+                C.key_norm = self._normalize_qk
+        if self._acc is None:
+            self._acc_buf, self._acc = _alloc_acc(new, B, m)
+        ptr = _lib.ptr
+        _lib.call("kch_csa_cache_append_at", ptr(rows), rows.stride(0), ptr(self._acc_buf),
+                  ptr(prev), ptr(Ba), ptr(Bb), ptr(Bi),
+                  None if self._sw is None else ptr(self._sw._buf),
+                  ptr(C.rows) if ends else None, ptr(C.keys) if ends else None,
+                  ptr(K.rows) if ends else None, ptr(K.inv) if ends else None, n, B, c, cI, m,
+                  self.win, cap, int(self._normalize_qk),
+                  _lib.dtype_code("CSADecodingCache.append_step", dt), _lib.stream_of(rows))
+        self._device_advance()
+        return [nb] if ends else []
 
     def _set_prev_buf(self, buf):
         self._prev_buf = buf
@@ -614,6 +700,10 @@ class HCADecodingCache:
         _lib.require_gpu("HCADecodingCache.append_step", C_new)
         new = [C_new, Z_new]
         with torch.no_grad():
+            if T_new == 1 and c <= _ONE_TOKEN_MAX:
+                out_idx = self._append_one(new, B_pos)
+                if out_idx is not None:
+                    return out_idx
             if self._sw is not None:
                 self._sw.append(_ring_rows(C_new, self.dtype, self._normalize_qk))
             if self._acc is None:
@@ -643,6 +733,38 @@ class HCADecodingCache:
             self._acc_len = rem
             self._n_tokens_seen += T_new
         return out_idx
+
+    def _append_one(self, new, B_pos):
+        """``append_step`` of one token in one launch (``kch_hca_cache_append_at``),
+        or None where the general path has to take it (before any change)."""
+        B, m2, c = self.B, self.m2, self.c
+        rows = _one_token_rows(self, new, (c, c))
+        if rows is None:
+            return None
+        n, dev, dt, nb, C = self._n_tokens_seen, rows.device, self.dtype, self._n_blocks, self._C
+        ends = self._acc_len == m2 - 1
+        if n != nb * m2 + self._acc_len or n >= 2 ** 31 - 1:
+            return None
+        Bp, cap = None, 0
+        if ends:
+            fp = _bias_rows([B_pos], m2, (c,), dev)
+            if fp is None or (C.rows is not None and C.rows.device != dev):
+                return None
+            Bp = fp[0]
+            C.ensure(nb, nb + 1)
+            cap = C.rows.shape[1]
+            if C.key_norm is None:
+                C.key_norm = self._normalize_qk
+        if self._acc is None:
+            self._acc_buf, self._acc = _alloc_acc(new, B, m2)
+        ptr = _lib.ptr
+        _lib.call("kch_hca_cache_append_at", ptr(rows), rows.stride(0), ptr(self._acc_buf), ptr(Bp),
+                  None if self._sw is None else ptr(self._sw._buf),
+                  ptr(C.rows) if ends else None, ptr(C.keys) if ends else None, n, B, c, m2,
+                  self.win, cap, int(self._normalize_qk),
+                  _lib.dtype_code("HCADecodingCache.append_step", dt), _lib.stream_of(rows))
+        self._device_advance()
+        return [nb] if ends else []
 
     # ---- device-driven steps (kch_hca_cache_append, kch_hca_decode_dyn) ----
     def _device_ready(self, dtype) -> bool:

@@ -361,3 +361,58 @@ def test_kda_front_rows_matches_separate_calls(dev, d):
         assert exact > 0.99, f"step {step}: only {exact:.4f} of the lookback bit-identical"
         look[1].copy_(look[0])  # keep the two paths on the same history
         state[1].copy_(state[0])
+
+
+@pytest.mark.parametrize("kind,c,cI,dt,win", [
+    ("csa", 128, 64, torch.bfloat16, 8), ("csa", 128, 128, torch.float32, 0),
+    ("csa", 72, 40, torch.float16, 3), ("csa", 1, 1, torch.bfloat16, 5),
+    ("hca", 128, 0, torch.bfloat16, 8), ("hca", 96, 0, torch.float16, 1),
+    ("hca", 56, 0, torch.float32, 0)])
+def test_append_one_matches_chunk_append(dev, kind, c, cI, dt, win):
+    """``append_step`` token by token (``kch_*_cache_append_at``) from the first token on, against one ``append_step`` of all tokens and
+    against a token, then the rest: the same ring, counters and accumulator, the
+    block rows of the bulk compression to one rounding of the cache dtype (both
+    sum at most 2 m fp32 terms, then round); token rows as slices of one projection and as separate
+    tensors, of a sequence-expanded batch too."""
+    import kch
+    torch.manual_seed(c + win)
+    B, T = 2, 19
+    m = 4 if kind == "csa" else 6
+    widths = [c] * 4 + [cI] * 2 if kind == "csa" else [c] * 2
+    P = torch.randn(B, T, sum(widths), device=dev).to(dt)
+    P[1] = P[0]
+    pos = [0.1 * torch.randn(m, w, device=dev) for w in ((c, c, cI) if kind == "csa" else (c,))]
+
+    def cache():
+        return (kch.CSADecodingCache(B, c, cI, m, win, dev, dt) if kind == "csa"
+                else kch.HCADecodingCache(B, c, m, win, dev, dt))
+
+    whole, one, split = cache(), cache(), cache()
+    idx = whole.append_step(*P.split(widths, -1), *pos)
+    got = []
+    for t in range(T):
+        x = P[:, t:t + 1]
+        if t % 3 == 1:
+            x = x[:1].expand(B, 1, -1)
+        parts = x.split(widths, -1)
+        if t % 3 == 2:
+            parts = [p.clone() for p in parts]
+        got += one.append_step(*parts, *pos)
+    split.append_step(*P[:, :1].split(widths, -1), *pos)
+    split.append_step(*P[:, 1:].split(widths, -1), *pos)
+    assert got == idx == list(range(T // m))
+    a = whole.accumulator_len
+    for k in (one, split):
+        assert k.n_tokens_seen == T and k.n_blocks == T // m and k.accumulator_len == a
+        for x, y in zip(k._acc, whole._acc):
+            assert torch.equal(x[:, :a], y[:, :a])
+        if win:
+            _ulps_close("ring", k._sw.get(), whole._sw.get(), dt)
+        _ulps_close("rows", k.C_comp, whole.C_comp, torch.float16 if dt == torch.float32 else dt)
+        if kind == "csa":
+            _ulps_close("index rows", k.K_IComp, whole.K_IComp,
+                        torch.float16 if dt == torch.float32 else dt)
+            torch.testing.assert_close(k._K.inv[:, :T // m], whole._K.inv[:, :T // m], rtol=1e-3,
+                                       atol=0)
+            assert torch.equal(k._prev[0], whole._prev[0]) and torch.equal(k._prev[1], whole._prev[1])
+    torch.cuda.synchronize()
