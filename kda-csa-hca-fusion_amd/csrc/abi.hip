@@ -1257,6 +1257,11 @@ DecodePlan decode_plan(int B, int nb, int nh, int hd, int topk, int ring_len, bo
     pl.nr = (nb + 255) / 256;
     pl.ko = (nb + 3) & ~3;
   }
+  if (sel && pl.nr > 1 && !pl.split && kch::decode_pick_keys(B, nb, topk, pl.nr, &pl.rb)) {
+    pl.split = true;
+    pl.nr = (nb + pl.rb - 1) / pl.rb;
+    pl.ko = (nb + 3) & ~3;
+  }
   pl.na = sparse ? (sel ? topk : 0) : nb;
   // the attention takes the attended blocks in whole 32-row steps (padded)
   const long long rows = (long long)((pl.na + 31) & ~31) + ring_len;
@@ -1381,6 +1386,10 @@ int kch_csa_decode(const void* q, const void* q_idx, const void* w_idx, const vo
     ip.idx_out = idx;
     ip.B = B; ip.nb = nb; ip.nIh = nIh; ip.cI = cI; ip.topk = topk; ip.rb = pl.rb; ip.nr = pl.nr;
     ip.normalize_q = normalize_qidx; ip.scale = idx_scale;
+    if (pl.split) {
+      ip.keys_out = (uint32_t*)(w + pl.off_keys);
+      ip.ko_bstride = pl.ko;
+    }
     rc = hip_status(fn, kch::decode_idx_dispatch(ip, qdtype, kdtype, s));
     if (rc) return rc;
   } else if (idx_out && topk > 0) {

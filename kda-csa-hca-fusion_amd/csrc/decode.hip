@@ -21,14 +21,16 @@
 //   values when the estimate misses. One range per sequence: sorted and final; otherwise the range's
 //   top-k are candidates.
 //   With keys_out the range only writes its logit keys there (score pass of
-//   a score / select split).
+//   a score / select split, or of a merge from all keys).
 // idx_select_kernel  the top-k of all logit keys of a sequence (at most
 //   RB_MAX, held in LDS): radix select over the ordered 64-bit values, gather,
 //   rank sort; output sorted, -1 padded.
 // idx_merge_kernel   the top-k of the candidates of all ranges of a sequence
 //   (a global top-k lies in the union of the per-range top-ks), by the same
 //   estimate-gather-select over the candidates streamed from global memory;
-//   output sorted by value (logit desc, index asc).
+//   output sorted by value (logit desc, index asc). Up to KEYS_MAX blocks (and
+//   where the candidates would be as many bytes) it streams all logit keys of a
+//   score pass instead, and the ranges select nothing.
 // attn_kernel   joint-softmax MQA over a group of the attended rows of a
 //   sequence (selected or all compressed blocks, then the ring window): per
 //   wave and head M, L and the unnormalised o (MqaWave), merged across the
@@ -50,6 +52,15 @@ constexpr int RB_MAX = 8192;     // blocks per indexer range (keys held in LDS)
 constexpr int WG_TARGET = 1024;  // indexer workgroups worth splitting a small batch for
 constexpr int SV_CAP = 2048;     // key positions a range gathers at or above its estimate
 constexpr int MV_CAP = 4096;     // candidates the merge gathers at or above its estimate
+// Blocks up to which the merge selects from all logit keys of a sequence
+// instead of from the ranges' top-k candidates (decode_pick_keys): a range's
+// own selection costs more than scoring it, while one workgroup streams a
+// sequence's keys at about 3 us per 8192. Step time of the two in us (candidates
+// / keys): B 16, 9000 blocks, top-512 55 / 46; 32769 blocks, top-64 60 / 56, top-512 83 /
+// 66; past this line only where the candidates are at least as many bytes:
+// B 4, 131073 blocks, top-512 126 / 107, but B 4, 65536, top-256 59 / 68 and B 1,
+// 131073, top-64 49 / 89.
+constexpr int KEYS_MAX = 40960;
 
 __device__ __forceinline__ uint32_t okey(float f) {
   uint32_t u = __float_as_uint(f);
@@ -929,6 +940,9 @@ __host__ __device__ inline int merge_cap(int topk) { return topk <= MV_CAP / 2 ?
 
 // LDS of the merge kernel: sv [merge_cap u64] | sel [pow2(topk + 1) u64] |
 // hist [512] | scratch [48] | counter [4]
+// KEYS: the candidates are all logit keys of the sequence, as the score pass
+// left them (candidate f = block f).
+template <bool KEYS>
 __global__ __launch_bounds__(256) void idx_merge_kernel(DecodeIdxParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int topk = p.topk, nr = p.nr;
@@ -939,17 +953,19 @@ __global__ __launch_bounds__(256) void idx_merge_kernel(DecodeIdxParams p) {
   int* scratch = reinterpret_cast<int*>(hist + 512);         // [48]
   int* counter = scratch + 48;                               // [4]
   const int tid = threadIdx.x, b = blockIdx.x;
-  const u64* src = p.cand + (size_t)b * nr * topk;
+  const u64* src = KEYS ? nullptr : p.cand + (size_t)b * nr * topk;
+  const uint32_t* ksrc = KEYS ? p.keys_out + (size_t)b * p.ko_bstride : nullptr;
   // ranges holding blocks (all nr unless the step is device-driven)
   const int nb = p.n_seen ? min((p.n_seen[0] + 1) / p.m, p.cap) : p.nb;
   const int na = (nb + p.rb - 1) / p.rb;
   // candidate f of the sequence: ranges before the last hold c0 each
   const int c0 = min(p.rb, topk);
   const int cl = na > 0 ? min(nb - (na - 1) * p.rb, topk) : 0;
-  const int N = na > 0 ? (na - 1) * c0 + cl : 0;
+  const int N = KEYS ? nb : (na > 0 ? (na - 1) * c0 + cl : 0);
   // (when every range holds topk candidates they are contiguous)
   const bool contig = c0 == topk;
   auto gval = [&](int f) {
+    if constexpr (KEYS) return kv64(ksrc[f], f);
     if (contig) return src[f];
     const int r = min(f / c0, na - 1);
     return src[(size_t)r * topk + (f - r * c0)];
@@ -965,21 +981,76 @@ __global__ __launch_bounds__(256) void idx_merge_kernel(DecodeIdxParams p) {
       // stream the candidates once: those at or above the estimate into sv
       if (tid == 0) counter[0] = 0;
       __syncthreads();
-      constexpr int U = 32;  // loads in flight per thread
       const int lane = tid & 63;
-      for (int base = wave_id() * 64 * U; base < N; base += 256 * U) {
-        u64 v[U];
+      if constexpr (KEYS) {
+        // 16-byte loads (a row is padded to whole ones), the next 8 of a thread
+        // in flight while its 32 keys are compared as 32-bit words; one LDS
+        // atomic per wave and 2048 keys
+        constexpr int U = 8;
+        const uint32_t ek = (uint32_t)(est >> 32);
+        const int end4 = (N - 1) & ~3;
+        auto fetch = [&](int base, uint4 (&q)[U]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = gval(min(base + 64 * u + lane, N - 1));
+          for (int u = 0; u < U; ++u)
+            q[u] = *reinterpret_cast<const uint4*>(ksrc + min(base + 256 * u + 4 * lane, end4));
+        };
+        uint4 cur[U], nxt[U];
+        int base = wave_id() * 256 * U;
+        fetch(base, cur);
+        for (; base < N; base += 1024 * U) {
+          fetch(base + 1024 * U, nxt);
+          uint32_t hit = 0u;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const bool t = base + 64 * u + lane < N && v[u] >= est;
-          const u64 m = __ballot(t);
-          if (m) {
-            int at = 0;
-            if (lane == 0) at = atomicAdd(counter, __popcll(m));
-            at = __builtin_amdgcn_readlane(at, 0) + mbcnt64(m);
-            if (t && at < mcap) sv[at] = v[u];
+          for (int u = 0; u < U; ++u) {
+            const uint32_t k4[4] = {cur[u].x, cur[u].y, cur[u].z, cur[u].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int f = base + 256 * u + 4 * lane + e;
+              const bool t = f < N && (k4[e] > ek || (k4[e] == ek && kv64(k4[e], f) >= est));
+              hit |= (uint32_t)t << (4 * u + e);
+            }
+          }
+          const int c = __popc(hit);
+          int x = c;
+#pragma unroll
+          for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(x, d);
+            if (lane >= d) x += y;
+          }
+          int slot = 0;
+          if (lane == 63 && x) slot = atomicAdd(counter, x);
+          slot = __builtin_amdgcn_readlane(slot, 63) + x - c;
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const uint32_t k4[4] = {cur[u].x, cur[u].y, cur[u].z, cur[u].w};
+            if ((hit >> (4 * u)) & 15u) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if ((hit >> (4 * u + e)) & 1u) {
+                  if (slot < mcap) sv[slot] = kv64(k4[e], base + 256 * u + 4 * lane + e);
+                  ++slot;
+                }
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+        }
+      } else {
+        constexpr int U = 32;  // loads in flight per thread
+        for (int base = wave_id() * 64 * U; base < N; base += 256 * U) {
+          u64 v[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] = gval(min(base + 64 * u + lane, N - 1));
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const bool t = base + 64 * u + lane < N && v[u] >= est;
+            const u64 m = __ballot(t);
+            if (m) {
+              int at = 0;
+              if (lane == 0) at = atomicAdd(counter, __popcll(m));
+              at = __builtin_amdgcn_readlane(at, 0) + mbcnt64(m);
+              if (t && at < mcap) sv[at] = v[u];
+            }
           }
         }
       }
@@ -1390,6 +1461,19 @@ size_t decode_merge_lds(int topk) {
   return (size_t)merge_cap(topk) * 8 + (size_t)pow2_at_least(topk + 1) * 8 + 512 * 4 + 52 * 4;
 }
 
+bool decode_pick_keys(int B, int nb, int topk, int nr, int* rb) {
+  if (nb <= RB_MAX || topk > MV_CAP / 2) return false;
+  if (nb > KEYS_MAX && 2LL * nr * topk < nb) return false;
+  // the merge's sampled estimate has to hold (sample_estimate's own terms)
+  const float ex = (float)topk * 256.f / (float)nb;
+  const int r = (int)ceilf(ex + 3.f * sqrtf(ex) + 2.f);
+  if (2 * r > 256 || (float)r * (float)nb / 256.f * 1.25f > (float)MV_CAP) return false;
+  // score ranges of about WG_TARGET workgroups over the batch
+  const long long want = min((long long)RB_MAX, max(256LL, ((long long)B * nb + WG_TARGET - 1) / WG_TARGET));
+  *rb = (int)((want + 15) & ~15LL);
+  return true;
+}
+
 bool decode_merge_fits(int topk) { return decode_merge_lds(topk) <= 160 * 1024; }
 
 bool decode_idx_fits(int rb, int topk, int nr) { return decode_idx_lds(rb, topk, nr) <= 160 * 1024; }
@@ -1421,12 +1505,16 @@ hipError_t decode_idx_dispatch(const DecodeIdxParams& p, int qdtype, int kdtype,
 #undef KCH_DIDX
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (p.keys_out && p.nb > RB_MAX) {
+    hipLaunchKernelGGL((idx_merge_kernel<true>), dim3((unsigned)p.B), dim3(256), decode_merge_lds(p.topk), s, p);
+    return hipGetLastError();
+  }
   if (p.keys_out) {
     hipLaunchKernelGGL(idx_select_kernel, dim3((unsigned)p.B), dim3(256), decode_select_lds(p.topk), s, p);
     return hipGetLastError();
   }
   if (p.nr == 1) return e;
-  hipLaunchKernelGGL(idx_merge_kernel, dim3((unsigned)p.B), dim3(256), decode_merge_lds(p.topk), s, p);
+  hipLaunchKernelGGL((idx_merge_kernel<false>), dim3((unsigned)p.B), dim3(256), decode_merge_lds(p.topk), s, p);
   return hipGetLastError();
 }
 

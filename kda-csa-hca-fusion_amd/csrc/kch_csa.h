@@ -82,12 +82,16 @@ struct DecodeIdxParams {
   // device-driven step: nb = (*n_seen + 1) / m, at most cap (nr ranges cover cap)
   const int* n_seen = nullptr;
   int m = 1, cap = 0;
-  // score / select split (nb <= decode_range_max()): the ranges only write
-  // their logit keys to keys_out [B, ko_bstride], then one workgroup per
-  // sequence selects from all of them
+  // score / select split: the ranges only write their logit keys to keys_out
+  // [B, ko_bstride], then one workgroup per sequence selects from all of them
+  // (held in LDS up to decode_range_max() blocks, streamed past that)
   uint32_t* keys_out = nullptr;
   long long ko_bstride = 0;
 };
+// Whether the selection of a plan of nr > 1 ranges takes all logit keys of the
+// sequence from a score pass (in ranges of *rb blocks) instead of the ranges'
+// candidates.
+bool decode_pick_keys(int B, int nb, int topk, int nr, int* rb);
 void decode_idx_plan(int B, int nb, int topk, int* rb, int* nr);
 int decode_range_max();  // most blocks one indexer range holds
 size_t decode_select_lds(int topk);

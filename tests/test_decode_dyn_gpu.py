@@ -106,6 +106,35 @@ def test_csa_decode_dyn_matches_planned(dev, nb, topk, cap, m):
             assert 7 in idx_d[b] and 40 not in idx_d[b]
 
 
+@pytest.mark.parametrize("nb,topk,form", [
+    (8193, 8, "random"),        # one block past the in-LDS selection
+    (9000, 512, "equal"),       # every logit the same: the lowest indices win
+    (8200, 2048, "random"),     # the largest selection merged from keys
+    (40960, 64, "random"),      # the last size merged from keys whatever the selection
+    (40961, 64, "random"),      # ranges and their candidates
+    (40961, 1024, "random"),    # keys again: as many bytes as the candidates
+    (12000, 512, "sampled"),    # large logits where the estimate samples: it misses
+])
+def test_csa_decode_selects_from_keys(dev, nb, topk, form):
+    """The planned step's selection past 8192 blocks against the oracle's order
+    (within the logits' fp32 rounding), where it is merged from all logit keys
+    and where from the ranges' candidates."""
+    rng = np.random.default_rng(nb + topk)
+    c, cI, nh, nIh = 64, 32, 16, 2
+    kraw, crow, ring, q, qi, wi, sink = make_csa(rng, 1, nb, c, cI, nh, nIh, 4)
+    if form == "equal":
+        kraw[:] = kraw[:, :1]
+    elif form == "sampled":
+        at = (np.arange(256) * nb) // 256
+        kraw[0, at] = qi[0, 0] + 0.01 * rng.standard_normal((256, cI))
+    out, idx, kr = run_csa(dev, kraw, q, qi, wi, crow, ring, sink, topk, nIh, cI)
+    lg = indexer_logits(qi[:, None], kr, wi[:, None], None, None, True, compute=np.float64)[:, 0]
+    if form == "equal":
+        assert np.array_equal(idx[0], np.arange(topk))
+    check_selection(f"keys nb={nb}", idx, topk_desc_lowest_index(lg, topk), lg,
+                    logit_eps(wi, nIh), sorted_=True)
+
+
 def test_csa_decode_dyn_no_blocks(dev):
     """n_seen = 1 < m - 1: no block yet; the window alone (its first 2 rows)."""
     rng = np.random.default_rng(3)
