@@ -27,7 +27,6 @@
 //
 // Kernels (one launch each):
 //   cb_prep_kernel  per (b, hv, chunk): M, Aqk, X, W, U, Qg, Kd, el -> workspace
-//                   (8 waves, two per SIMD, sharing one LDS allocation)
 //   cb_fwd_kernel   per (b, hv, slice of V), chunks in order: S_n, v_n
 //   cb_bwd_kernel   per (b, hv, slice of V), chunks in reverse: dS', dv_n, dS_0
 //   cb_grad_kernel  per (b, hv, chunk): dq, dk, dv, dg, dbeta (or per-value-head
@@ -324,19 +323,26 @@ __device__ __forceinline__ void col_scan(float* m, int ld, float* tot, const flo
 }
 
 // ---------------------------------------------------------------------------
-// cb_prep_kernel: one workgroup (8 waves) per (b, hv, chunk). It writes W and Kd
-// in both orders, which the two state kernels need (64 KB a chunk more than
-// one order each; 467 us at 4096 chunks against 420, for the 601 us that the
-// state kernels no longer spend on transposing).
+// cb_prep_kernel: one workgroup (8 waves) per (b, hv, chunk), two per CU (16-bit
+// inputs). Bound by HBM writes (K = V = 128: 224 KB a chunk; W and Kd in both
+// orders, which the two state kernels need) and by the chain of phases between
+// barriers, which the second workgroup fills: k is held as stored, q and v are
+// read where they are used (L2), X takes M's place as split planes, 72 KB of
+// LDS in all. 4096 chunks: 329 us (467 with fp32 copies of k, q, v and X, 138 KB
+// and one workgroup a CU; 420 before the second orders were written).
 // ---------------------------------------------------------------------------
 template <int K, int V, typename InT>
-__global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
+__global__ __launch_bounds__(NTH, sizeof(InT) == 4 ? 2 : 4) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   using R = Rec<K, V>;
-  constexpr int LK = K + 4, LC = C + 4, LV = V + 4;
-  constexpr int SQ = C * LK > C * LV ? C * LK : C * LV;
-  __shared__ float sk[C * LK], sG[C * LK], sq[SQ], sM[C * LC], sX[C * LC], sb[C], stot[NTH];
+  constexpr unsigned SZ = sizeof(InT);
+  constexpr int LK = K + 4, LC = C + 4, LX = C + 8, LI = K + 16 / (int)SZ;
+  __shared__ __attribute__((aligned(16))) InT sk[C * LI];
+  __shared__ __attribute__((aligned(16))) float sG[C * LK], stot[NTH], sb[C];
+  // M (fp32), then the split planes of X
+  __shared__ __attribute__((aligned(16))) bf16_t sX[2][C * LX];
   __shared__ int sflag[K / 64];
-  float* const sv = sq;  // v [C][LV] once q^ is consumed
+  float* const sM = reinterpret_cast<float*>(sX);
+  static_assert(C * LC * 4 <= 4 * C * LX, "M fits where X goes");
 
   const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   const int nt = w.nt;
@@ -347,27 +353,46 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   const bool clampg = p.g_clamp_min > -INFINITY;
   const float gmin = (float)p.g_clamp_min;
   bf16_t* rec = w.rec + (size_t)blockIdx.x * R::RS;
+  // the chunk's rows of an input, zero past the sequence's end
+  const int last = min(T - 1 - t0, C - 1);
+  auto rows = [&](const void* x, int heads, int head, int D) {
+    return buf(static_cast<const char*>(x) + (((size_t)b * T + t0) * heads + head) * D * SZ,
+               (size_t)(last + 1) * heads * D * SZ);
+  };
+  const __amdgpu_buffer_rsrc_t qb = rows(p.q, p.H, h, K), kb = rows(p.k, p.H, h, K),
+                               gb = rows(p.g, p.HV, hv, K), vb = rows(p.v, p.HV, hv, V);
+  const unsigned rq = p.H * K * SZ, rg = p.HV * K * SZ, rv = p.HV * V * SZ;
+  typedef InT in8 __attribute__((ext_vector_type(8)));
+  auto cvt8 = [](auto raw, float* f) {
+    const in8 t = __builtin_bit_cast(in8, raw);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = to_f32((InT)t[i]);
+  };
+  // 8 tokens of one channel, rows r0 .. r0 + 7 of row stride ld
+  auto col8 = [&](__amdgpu_buffer_rsrc_t r, unsigned ld, int r0, int ch, float* f) {
+    const unsigned o = r0 * ld + ch * SZ;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (SZ == 4)
+        f[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, o + i * ld, 0, 0));
+      else
+        f[i] = to_f32(__builtin_bit_cast(InT, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, o + i * ld, 0, 0)));
+    }
+  };
 
   if (tid < K / 64) sflag[tid] = 1;
   __syncthreads();
   for (int it = tid; it < C * (K / 8); it += NTH) {
-    const int c = it / (K / 8), c8 = (it % (K / 8)) * 8, t = t0 + c;
-    float fq[8], fk[8], fg[8];
-    if (t < T) {
-      const size_t qk = ((size_t)(b * T + t) * p.H + h) * K + c8;
-      ld8g(static_cast<const InT*>(p.q) + qk, fq);
-      ld8g(static_cast<const InT*>(p.k) + qk, fk);
-      ld8g(static_cast<const InT*>(p.g) + ((size_t)(b * T + t) * p.HV + hv) * K + c8, fg);
-    } else {
-      zero8(fq); zero8(fk); zero8(fg);
-    }
+    const int c = it / (K / 8), c8 = (it % (K / 8)) * 8;
+    const auto kr = buf_load<InT, 8>(kb, c * rq + c8 * SZ);
+    float fg[8];
+    cvt8(buf_load<InT, 8>(gb, c * rg + c8 * SZ), fg);
+    *reinterpret_cast<in8*>(&sk[c * LI + c8]) = __builtin_bit_cast(in8, kr);
     bool pos = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float gc = clampg ? fmaxf(fg[i], gmin) : fg[i];
       pos |= gc > 0.f;
-      sq[c * LK + c8 + i] = scale * fq[i];
-      sk[c * LK + c8 + i] = fk[i];
       sG[c * LK + c8 + i] = gc;
     }
     if (pos) sflag[c8 / 64] = 0;
@@ -395,11 +420,19 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) am[u] = aa[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (anchored) {
+      decltype(buf_load<InT, 8>(qb, 0)) qc[2], qn[2];
+      auto qload = [&](int ks, auto& o) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          o[u] = buf_load<InT, 8>(qb, (16 * (rt0 + u) + r16) * rq + (ks + 8 * kq) * SZ);
+      };
+      qload(0, qc);
 #pragma unroll 1
       for (int ks = 0; ks < K; ks += 32) {
         const int ch = ks + 8 * kq;
+        if (ks + 32 < K) qload(ks + 32, qn);
         float fb[8], gj[8], ga[8];
-        ld8c(&sk[jc * LK + ch], fb);
+        ld8g(&sk[jc * LI + ch], fb);
         ld8c(&sG[jc * LK + ch], gj);
         ld8c(&sG[kAnc * LK + ch], ga);
 #pragma unroll
@@ -409,18 +442,21 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
         for (int u = 0; u < 2; ++u) {
           const int i0 = 16 * (rt0 + u) + r16;
           float fk[8], fq[8], gi[8];
-          ld8c(&sk[i0 * LK + ch], fk);
-          ld8c(&sq[i0 * LK + ch], fq);
+          ld8g(&sk[i0 * LI + ch], fk);
+          cvt8(qc[u], fq);
           ld8c(&sG[i0 * LK + ch], gi);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const float P = ex(gi[i] - ga[i]);
             fk[i] *= P;
+            fq[i] *= scale;
             fq[i] *= P;
           }
           am[u] = mm3(sp8(fk), bs, am[u]);
           aa[u] = mm3(sp8(fq), bs, aa[u]);
         }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) qc[u] = qn[u];
       }
     } else {
 #pragma unroll
@@ -430,10 +466,18 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
           const int i = 16 * (rt0 + u) + 4 * kq + e;
           float m = 0.f, a = 0.f;
           if (jc <= i) {
-            for (int ch = 0; ch < K; ++ch) {
-              const float x = ex(fminf(sG[i * LK + ch] - sG[jc * LK + ch], kCap)) * sk[jc * LK + ch];
-              m += sk[i * LK + ch] * x;
-              a += sq[i * LK + ch] * x;
+#pragma unroll 1
+            for (int c8 = 0; c8 < K; c8 += 8) {
+              float fq[8];
+              cvt8(buf_load<InT, 8>(qb, i * rq + c8 * SZ), fq);
+#pragma unroll
+              for (int z = 0; z < 8; ++z) {
+                const int ch = c8 + z;
+                const float x =
+                    ex(fminf(sG[i * LK + ch] - sG[jc * LK + ch], kCap)) * to_f32(sk[jc * LI + ch]);
+                m += to_f32(sk[i * LI + ch]) * x;
+                a += scale * fq[z] * x;
+              }
             }
           }
           am[u][e] = m;
@@ -454,26 +498,28 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
     }
   }
   // Qg^T and Kd^T (8 tokens of a channel), Kd (8 channels of a token), el
+#pragma unroll 1
   for (int it = tid; it < K * (C / 8); it += NTH) {
     const int ch = it % K, c8 = it / K;
     const float Gl = sG[(C - 1) * LK + ch];
-    float fq[8], fk[8], gc[8];
-    ld8s(&sq[8 * c8 * LK + ch], LK, fq);
-    ld8s(&sk[8 * c8 * LK + ch], LK, fk);
-    ld8s(&sG[8 * c8 * LK + ch], LK, gc);
+    float fq[8], fk[8];
+    col8(qb, rq, 8 * c8, ch, fq);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      fq[i] *= ex(gc[i]);
-      fk[i] *= ex(Gl - gc[i]);
+      const float G = sG[(8 * c8 + i) * LK + ch];
+      fq[i] *= scale;
+      fq[i] *= ex(G);
+      fk[i] = to_f32(sk[(8 * c8 + i) * LI + ch]) * ex(Gl - G);
     }
     const int tile = (ch >> 4) * 2 + (c8 >> 2), lane = (ch & 15) + 16 * (c8 & 3);
     ft_store(rec + R::QG2, tile, lane, sp8(fq));
     ft_store(rec + R::KD2, tile, lane, sp8(fk));
   }
+#pragma unroll 1
   for (int it = tid; it < C * (K / 8); it += NTH) {
     const int c = it % C, k8 = it / C;
     float fk[8], gc[8], gl[8];
-    ld8c(&sk[c * LK + 8 * k8], fk);
+    ld8g(&sk[c * LI + 8 * k8], fk);
     ld8c(&sG[c * LK + 8 * k8], gc);
     ld8c(&sG[(C - 1) * LK + 8 * k8], gl);
 #pragma unroll
@@ -483,17 +529,7 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
   if (tid < K) reinterpret_cast<float*>(rec + R::EL)[tid] = ex(sG[(C - 1) * LK + tid]);
   __syncthreads();
 
-  // v -> LDS (over q^); X = (I + M)^-1, column cc by the eight lanes of a half row
-  for (int it = tid; it < C * (V / 8); it += NTH) {
-    const int c = it / (V / 8), c8 = (it % (V / 8)) * 8, t = t0 + c;
-    float fv[8];
-    if (t < T)
-      ld8g(static_cast<const InT*>(p.v) + ((size_t)(b * T + t) * p.HV + hv) * V + c8, fv);
-    else
-      zero8(fv);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sv[c * LV + c8 + i] = fv[i];
-  }
+  // X = (I + M)^-1, column cc by the eight lanes of a half row
   {
     const int cc = tid >> 3, part = tid & 7;
     float xr[8];
@@ -513,34 +549,22 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
       const float xi = (i == cc ? 1.f : 0.f) - s;
       if (part == (i & 7)) xr[i >> 3] = xi;
     }
+    __syncthreads();  // every read of M done
 #pragma unroll
     for (int jj = 0; jj < 8; ++jj) {
-      const int j = 8 * jj + part;
-      sX[j * LC + cc] = xr[jj];
+      const int o = (8 * jj + part) * LX + cc;
+      const bf16_t hi = (bf16_t)xr[jj];
+      sX[0][o] = hi;
+      sX[1][o] = (bf16_t)(xr[jj] - (float)hi);
     }
   }
   __syncthreads();
 
-  {
-    const int c = tid & 63, j8 = tid >> 6;
-    float f[8];
-    ld8s(&sX[8 * j8 * LC + c], LC, f);
-    ft_store(rec + R::XT, (c >> 4) * 2 + (j8 >> 2), (c & 15) + 16 * (j8 & 3), sp8(f));
-  }
+  ft_store(rec + R::XT, wv, l,
+           Sp{tr8(sX[0], LX, 32 * (wv & 1), 16 * (wv >> 1)), tr8(sX[1], LX, 32 * (wv & 1), 16 * (wv >> 1))});
   // W = X Bk in both orientations (the same fragments with the operands
   // exchanged) and U = X Bv, one tile of K (then of V) at a time over the
-  // chunk's four row tiles; X's rows are split once per wave, its upper
-  // triangle left out
-  Sp xs[4][2];
-#pragma unroll
-  for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      if (2 * ks > ct) continue;
-      float fb[8];
-      ld8c(&sX[(16 * ct + r16) * LC + 32 * ks + 8 * kq], fb);
-      xs[ct][ks] = sp8(fb);
-    }
+  // chunk's four row tiles, X's upper triangle left out
 #pragma unroll 1
   for (int rtg = wv; rtg < K / 16 + V / 16; rtg += NTH / 64) {
     const bool isw = rtg < K / 16;
@@ -551,13 +575,11 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
       const int j0 = 32 * ks + 8 * kq;
       float fa[8];
       if (isw) {
-        float gj[8];
-        ld8s(&sk[j0 * LK + r], LK, fa);
-        ld8s(&sG[j0 * LK + r], LK, gj);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) fa[i] *= sb[j0 + i] * ex(gj[i]);
+        for (int i = 0; i < 8; ++i)
+          fa[i] = to_f32(sk[(j0 + i) * LI + r]) * (sb[j0 + i] * ex(sG[(j0 + i) * LK + r]));
       } else {
-        ld8s(&sv[j0 * LV + r], LV, fa);
+        col8(vb, rv, j0, r, fa);
 #pragma unroll
         for (int i = 0; i < 8; ++i) fa[i] *= sb[j0 + i];
       }
@@ -565,15 +587,15 @@ __global__ __launch_bounds__(NTH) void cb_prep_kernel(KdaBwdParams p, CbWs w) {
     }
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) {
-      f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f}, y = x;
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        if (2 * ks <= ct) x = mm3(xs[ct][ks], as[ks], x);
+      for (int ks = 0; ks < 2; ++ks) {
+        if (2 * ks > ct) continue;
+        const Sp xs = plane8(sX[0], sX[1], (16 * ct + r16) * LX + 32 * ks + 8 * kq);
+        x = mm3(xs, as[ks], x);
+        if (isw) y = mm3(as[ks], xs, y);
+      }
       if (isw) {
-        f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          if (2 * ks <= ct) y = mm3(as[ks], xs[ct][ks], y);
         ft_store_acc(rec + R::W1, ct, K / 32, rtg, sp4(y));
         ft_store_acc(rec + R::W2, rtg, 2, ct, sp4(-x));
       } else {
