@@ -1244,7 +1244,7 @@ struct DecodePlan {
 size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 DecodePlan decode_plan(int B, int nb, int nh, int hd, int topk, int ring_len, bool sparse,
-                       bool one_range = false) {
+                       bool one_range = false, bool keys = true) {
   DecodePlan pl;
   const bool sel = sparse && nb > 0 && topk > 0;
   if (sel) kch::decode_idx_plan(B, nb, topk, &pl.rb, &pl.nr);
@@ -1257,7 +1257,8 @@ DecodePlan decode_plan(int B, int nb, int nh, int hd, int topk, int ring_len, bo
     pl.nr = (nb + 255) / 256;
     pl.ko = (nb + 3) & ~3;
   }
-  if (sel && pl.nr > 1 && !pl.split && kch::decode_pick_keys(B, nb, topk, pl.nr, &pl.rb)) {
+  if (keys && sel && pl.nr > 1 && !pl.split &&
+      kch::decode_pick_keys(B, nb, topk, pl.nr, &pl.rb)) {
     pl.split = true;
     pl.nr = (nb + pl.rb - 1) / pl.rb;
     pl.ko = (nb + 3) & ~3;
@@ -1291,6 +1292,14 @@ DecodePlan decode_plan(int B, int nb, int nh, int hd, int topk, int ring_len, bo
   if (pl.ngrp > 1) off += a256((size_t)B * pl.ngrp * nh * 2 * 4);
   pl.bytes = off;
   return pl;
+}
+
+// The plan for a workspace of `room` bytes: one that holds the ranges' candidates
+// but not all logit keys (a small topk's are far fewer bytes) takes the former.
+DecodePlan decode_plan_in(size_t room, int B, int nb, int nh, int hd, int topk, int ring_len,
+                          bool sparse, bool one_range = false) {
+  const DecodePlan pl = decode_plan(B, nb, nh, hd, topk, ring_len, sparse, one_range);
+  return pl.bytes <= room ? pl : decode_plan(B, nb, nh, hd, topk, ring_len, sparse, one_range, false);
 }
 
 // Per-step counts of a device-driven decode step (decode_step.hip).
@@ -1361,7 +1370,7 @@ int kch_csa_decode(const void* q, const void* q_idx, const void* w_idx, const vo
   if (cI != 32 && cI != 64 && cI != 128)
     return fail(KCH_ERR_UNSUPPORTED, "%s: cI=%d not in {32,64,128}", fn, cI);
   if (B == 0) return KCH_OK;
-  const DecodePlan pl = decode_plan(B, nb, nh, hd, topk, ring_len, true);
+  const DecodePlan pl = decode_plan_in(ws_bytes, B, nb, nh, hd, topk, ring_len, true);
   if (!ws || ws_bytes < pl.bytes)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required", fn, pl.bytes);
   if ((uintptr_t)ws & 255) return fail(KCH_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
@@ -1447,7 +1456,7 @@ int kch_csa_decode_dyn(const void* q, long long ld_q, const void* q_idx, long lo
   if (ld_q < (long long)nh * hd || ld_qidx < (long long)nIh * cI || (w_idx && ld_w < nIh))
     return fail(KCH_ERR_INVALID, "%s: query row strides too small", fn);
   if (B == 0) return KCH_OK;
-  const DecodePlan pl = decode_plan(B, cap, nh, hd, topk, win, true, true);
+  const DecodePlan pl = decode_plan_in(ws_bytes, B, cap, nh, hd, topk, win, true, true);
   if (!ws || ws_bytes < pl.bytes)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required", fn, pl.bytes);
   if ((uintptr_t)ws & 255) return fail(KCH_ERR_INVALID, "%s: workspace must be 256-byte aligned", fn);
@@ -1571,7 +1580,8 @@ int kch_csa_decode_noalloc(const void* q, const void* q_idx, const void* w_idx,
     return fail(KCH_ERR_INVALID, "%s: bad sizes B=%d nb=%d nh=%d hd=%d topk=%d ring_len=%d", fn,
                 B, nb, nh, hd, topk, ring_len);
   if (B == 0) return KCH_OK;
-  const size_t need = decode_plan(B, nb, nh, hd, topk, ring_len, true).bytes;
+  const size_t need =
+      decode_plan_in(KCH_NOALLOC_SCRATCH_BYTES, B, nb, nh, hd, topk, ring_len, true).bytes;
   if (need > (size_t)KCH_NOALLOC_SCRATCH_BYTES)
     return fail(KCH_ERR_UNSUPPORTED,
                 "%s: B=%d nb=%d topk=%d ring_len=%d needs %zu bytes of scratch, more than the "

@@ -69,6 +69,17 @@ def test_noalloc_matches_workspace_entry_point(dev):
         np.testing.assert_array_equal(o_na.view(np.uint32), o_ws.view(np.uint32))
 
 
+def test_noalloc_where_all_logit_keys_do_not_fit(dev):
+    """110 sequences of 40000 blocks: their logit keys (17.6 MB) are beyond the
+    scratch, the ranges' top-8 candidates are not. The step takes the
+    candidates there, the workspace entry point the keys: the same selection,
+    and so the same attention, bit for bit."""
+    shape = (110, 40000, 64, 32, 8, 2, 16, 8, 4)
+    (o_ws, o_na), (i_ws, i_na) = _run("kch_csa_decode_noalloc", dev, *shape)
+    np.testing.assert_array_equal(i_na, i_ws)
+    np.testing.assert_array_equal(o_na.view(np.uint32), o_ws.view(np.uint32))
+
+
 def test_noalloc_refuses_sizes_beyond_its_scratch(dev):
     from kch import _lib
     lib = _lib.load()
