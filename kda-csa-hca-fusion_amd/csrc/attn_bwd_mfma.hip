@@ -1108,7 +1108,8 @@ bool attn_bwd_mfma_supported(const HcaBwdParams& p) {
 // (nb / 2 on average), the gather's with topk; whole backward, 8192 queries,
 // 16 heads of 128, window 128, tiles against gather: topk 512, nb 512 0.655 /
 // 0.852 ms, 1024 0.875 / 1.006, 2048 1.328 / 1.277, 4096 4.51 / 3.61; topk 128,
-// nb 512 0.657 / 0.635; topk 64, nb 512 0.704 / 0.631.
+// nb 512 0.657 / 0.635; topk 64, nb 512 0.704 / 0.631 (measured with the fp32
+// compression gradients that attn_bwd_finish.hip replaced; both sides share them).
 static bool attn_bwd_dense_rows(int nb, int topk) { return nb <= 3 * topk; }
 
 static size_t al256m(size_t x) { return (x + 255) & ~size_t(255); }
