@@ -437,7 +437,7 @@ static int check_attn_bwd(const char* fn, int B, int T, int nh, int c, int m, in
 
 size_t kch_hca_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win) {
   if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m2 < 1 || T % m2 || win < 0) return 0;
-  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, -1);
+  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, -1, 1);
 }
 
 int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
@@ -479,7 +479,9 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
 size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk) {
   if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m < 1 || T % m || win < 0 || topk < 0)
     return 0;
-  return kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk);
+  const size_t norm = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, 1);
+  const size_t raw = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, 0);
+  return norm > raw ? norm : raw;
 }
 
 int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
@@ -505,7 +507,7 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (int rc = check_bwd_rows(fn, "Cb", Cb, ldCb, c, cdt)) return rc;
   if (int rc = check_bwd_rows(fn, "Za", Za, ldZa, c, cdt)) return rc;
   if (int rc = check_bwd_rows(fn, "Zb", Zb, ldZb, c, cdt)) return rc;
-  const size_t need = kch_csa_attn_bwd_ws_bytes(B, T, nh, c, m, win, topk);
+  const size_t need = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, normalize != 0);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
                 ws ? ws_bytes : (size_t)0);

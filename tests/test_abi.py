@@ -92,6 +92,30 @@ def test_kda_backward_validation_and_workspace():
         assert lib.kch_kda_recurrent_bwd_ws_bytes(B, T, HV, K, V, code) == pad(ck) + pad(part)
 
 
+def _csa_bwd_needs(lib, B, T, nh, c, m, topk, win, normalize, slots=True, dsel=False):
+    """The workspace that kch_csa_attn_bwd says a call without one requires
+    (tensors stand for themselves: the call ends before any is read)."""
+    x = ctypes.c_void_p(4096)
+    rc = lib.kch_csa_attn_bwd(x, x, x, x, x, x, c, x, c, x, c, x, c, x, x, None, x, x, x, x, x, x, x, None,
+                              x if slots else None, x if dsel else None, 0, None, B, T, nh, c, m, topk,
+                              win, 1.0, normalize, 0, 0, 0, None, 0, None)
+    assert rc == 1
+    return int(re.search(rb"workspace of (\d+) bytes", lib.kch_last_error()).group(1))
+
+
+def test_csa_backward_workspace_holds_every_head_group():
+    """Head groups share one workspace, sized for the first: a last group of 16
+    or fewer heads needs no more than the whole ones before it (32 heads of 64
+    on raw rows, 16 on normalised ones)."""
+    from kch import _lib
+    lib = _lib.load()
+    for B, T, c, m, topk, win in ((1, 64, 64, 4, 4, 8), (2, 4096, 64, 4, 64, 128), (1, 1024, 128, 1, 8, 0)):
+        for normalize, most in ((0, 256 // (c // 8)), (1, 16)):
+            held = lib.kch_csa_attn_bwd_ws_bytes(B, T, most, c, m, win, topk)
+            for nh in range(1, most + 1):
+                assert _csa_bwd_needs(lib, B, T, nh, c, m, topk, win, normalize) <= held, (nh, normalize)
+
+
 def test_chunk_workspace_size_query():
     """kch_kda_chunk_ws_bytes: 0 where no workspace is used, else the sum of
     the six per-chunk records, each region padded to 256 bytes."""

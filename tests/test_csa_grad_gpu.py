@@ -69,6 +69,7 @@ CASES = [
     (1, 48, 2, 16, 4, 3, 5, True, False),      # c padded to 64
     (1, 64, 18, 128, 4, 6, 4, True, True),     # two head groups
     (2, 1040, 3, 64, 8, 16, 24, True, False),  # several query chunks per key tile
+    (1, 64, 37, 64, 4, 4, 8, True, False),     # raw rows: a group of 32 heads, then one of 5
 ]
 
 
