@@ -198,16 +198,16 @@ def _attn_bwd_qdtype(q, d_out, normalize=True):
     return torch.float32
 
 
-def _bwd_rows(dt, n, *xs):
-    """The rows of a backward's compression inputs ``[B, T, <= n]`` in ``dt``,
-    zero-padded to ``n`` channels, as alternating (tensor, row stride): views are
-    used in place when their rows lie 16-byte aligned at one stride."""
+def _bwd_rows(dev, dt, n, *xs):
+    """The rows of a backward's compression inputs ``[B, T, <= n]`` on ``dev`` in
+    ``dt``, zero-padded to ``n`` channels, as alternating (tensor, row stride):
+    views are used in place when their rows lie 16-byte aligned at one stride."""
     out = []
     for x in xs:
         if x is None:
             out += [None, n]
             continue
-        x = _pad_last(x.detach().to(dt), n)
+        x = _pad_last(x.detach().to(device=dev, dtype=dt), n)
         ld = x.stride(1)
         if not (x.stride(2) == 1 and ld >= n and ld * x.element_size() % 16 == 0
                 and (x.shape[0] == 1 or x.stride(0) == x.shape[1] * ld)
@@ -577,7 +577,7 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     hmax = _MAX_HEADS if normalize_qk else 256 // (cp // 8)
     one = nh <= hmax
     odt = cdt if one else f32
-    rows = _bwd_rows(cdt, cp, Ca, Cb, Za, Zb)
+    rows = _bwd_rows(dev, cdt, cp, Ca, Cb, Za, Zb)
     Car, Cbr, Zar, Zbr = rows[::2]
     if not normalize_qk:
         Car, Cbr, Zar, Zbr = (x.contiguous() for x in (Car, Cbr, Zar, Zbr))
@@ -673,13 +673,13 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
 
     qdt = _bwd_dtype((q_idx, w_idx), True)
     cdt = _bwd_dtype((K_idx, Z_idx), True)
-    rows = _bwd_rows(cdt, cIp, K_idx, Z_idx)
+    rows = _bwd_rows(dev, cdt, cIp, K_idx, Z_idx)
     Bf = _aligned(_pad_last(B_idx.detach().to(device=dev, dtype=f32), cIp))
     qf = q_idx.detach().to(qdt)
     if (cIp, nIp) != (cI, nIh):
         qf = F.pad(qf, (0, cIp - cI, 0, nIp - nIh))
     qf = _aligned(qf)
-    wf = _pad_last(w_idx.detach().to(qdt), nIp).contiguous()
+    wf = _pad_last(w_idx.detach().to(device=dev, dtype=qdt), nIp).contiguous()
     kc = torch.empty(B_, nb, cIp, device=dev, dtype=f32)
     raw = _compress(fn, rows[0], rows[2], Bf, m, out_raw=True, key=kc, normalize=bool(normalize_qk))
     if not normalize_qk:

@@ -69,7 +69,7 @@ def hca_core_grad(C, Z, q, B_pos, d_out, *, m2, sliding_window=0, sink_logits=No
     cdt = _bwd_dtype((C, Z, C_local_raw if win > 0 else None), True)
     one = nh <= _MAX_HEADS
     odt = cdt if one else f32
-    Cr, ldC, Zr, ldZ, lr, ldl = _bwd_rows(cdt, cp, C, Z, C_local_raw if win > 0 else None)
+    Cr, ldC, Zr, ldZ, lr, ldl = _bwd_rows(dev, cdt, cp, C, Z, C_local_raw if win > 0 else None)
     if lr is None:
         lr, ldl = Cr, ldC
     Bp = _aligned(prep(B_pos))

@@ -471,3 +471,29 @@ def test_attn_grad_at_tile_edges(dev, B, T, nh, c, m, topk, win, dtype):
     for b, i, j in zip(*np.nonzero(idx >= 0)):
         want[b, i, idx[b, i, j]] = ref["slot"][b, i, j]
     _check("dsel", dsel, want)
+
+
+def test_grads_move_inputs_to_the_first_ones_device(dev):
+    """The compression's other inputs, their biases and the indexer's weights may
+    lie on the host: they are copied to the first input's device, and the
+    gradients are those of device inputs, bit for bit."""
+    import kch
+    from kch.ops_csa import _bwd_rows, _ste_indexer_grads
+    torch.manual_seed(3)
+    B, T, nh, c, m, topk, nIh = 1, 24, 2, 64, 4, 3, 2
+    assert [x.device.type for x in _bwd_rows("meta", torch.float32, c, torch.zeros(B, T, c))[::2]] == ["meta"]
+    X = [torch.randn(B, T, c) for _ in range(4)]
+    q, W = torch.randn(B, T, nh, c), torch.randn(B, T, nh, c)
+    pos = [torch.randn(m, c) for _ in range(2)]
+    idx = torch.tensor(_selection(np.random.default_rng(3), B, T, m, topk))
+    on = lambda xs: [x.to(dev) for x in xs]  # noqa: E731
+    ref = kch.ops_csa.csa_attn_grad(*on(X), q.to(dev), *on(pos), idx.to(dev), W.to(dev), m=m)
+    got = kch.ops_csa.csa_attn_grad(X[0].to(dev), *X[1:], q, *pos, idx, W, m=m)
+    for k in ref:
+        assert got[k].is_cuda and torch.equal(got[k], ref[k]), k
+    K, Z, Bi = X[0], X[1], pos[0]
+    qi, w, slot = torch.randn(B, T, nIh, c), torch.randn(B, T, nIh), ref["slot"]
+    a = _ste_indexer_grads(*on((K, Z, qi, w, Bi)), idx.to(dev), slot, m=m, normalize_qk=True)
+    b = _ste_indexer_grads(K.to(dev), Z, qi.to(dev), w, Bi, idx.to(dev), slot, m=m, normalize_qk=True)
+    for x, y in zip(a, b):
+        assert y.is_cuda and torch.equal(x, y)
