@@ -1416,17 +1416,17 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(DecodeAttnParams p) {
 }
 
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, long long n, uint32_t v) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = v;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) p[i] = v;
 }
 
 }  // namespace
 
 // Fills n 32-bit words (a kernel rather than a memset node, so that a captured
-// graph replays it faithfully).
+// graph replays it faithfully). A launch takes fewer than 2^32 threads: past 2^28
+// words each thread fills more than one.
 hipError_t fill_u32(void* p, long long n, uint32_t v, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)min((n + 255) / 256, 1LL << 20)), dim3(256), 0, s,
                      static_cast<uint32_t*>(p), n, v);
   return hipGetLastError();
 }

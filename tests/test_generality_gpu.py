@@ -186,3 +186,14 @@ def test_hybrid_decoding_wide_odd_heads(dev):
     x = torch.from_numpy(rng.standard_normal((2, 44, cfg.d_model)).astype(np.float32)).to(
         dev, torch.bfloat16)
     decode_vs_oracle(dec, oracle, x, 40, "wide odd heads")
+
+
+def test_fill_of_more_words_than_a_launch_has_threads(dev):
+    """An indexer call without blocks writes -1 to every slot: here 2^32 + 2^21
+    words (17.2 GB), past the 2^32 - 1 threads that one launch can have."""
+    from kch import _lib
+    T, topk = 1 << 20, 2049
+    out = torch.zeros(T * topk, dtype=torch.int64, device=dev)
+    _lib.call("kch_csa_indexer_topk", _lib.ptr(out), None, None, _lib.ptr(out), 1, None, 1, T, 0, 1,
+              32, topk, 4, 0, 0, 0, 1.0, 0, 0, 0, _lib.stream_of(out))
+    assert not bool(out.ne(-1).any())
