@@ -30,7 +30,9 @@
 // attn_bwd_q_kernel   CSA over long contexts: one wave per query gathers only
 //   the selected rows, 32 a step, into its own LDS stage. Its bound is the L2
 //   gather of 512 bytes a row and pass (8.5 TB/s measured), the tile kernel's
-//   the matrix cores; see attn_bwd_dense_rows for where the line lies.
+//   the matrix cores; see attn_bwd_dense_rows for where the line lies. The
+//   slots' values go where they are asked for: slot by slot, or into the
+//   query's own row of dsel, which the wave clears first.
 // attn_bwd_k_kernel   one workgroup per 64 KG key rows (16 KG per wave, KG 1 or
 //   2, key fragments in registers) and chunk of queries; queries are taken in
 //   pairs: the pair's q and dout rows (32 rows of (query, head)) are staged in
@@ -667,6 +669,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
   const __amdgpu_buffer_rsrc_t rs_idx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int*>(has_idx ? p.idx + bt * p.topk : nullptr), 0, has_idx ? nsel * 4 : 0, 0x00020000);
   const bool idx16 = (nsel & 3) == 0;  // 16-byte index loads never straddle the end
+  float* const drow = p.dsel ? p.dsel + bt * p.nb : nullptr;
+  if (drow && !p.dsel_add) {
+    // the query's row of dsel, cleared while pass 1 runs
+    if ((p.nb & 3) == 0)
+      for (int j = 4 * lane; j < p.nb; j += 256) *reinterpret_cast<float4*>(drow + j) = make_float4(0.f, 0.f, 0.f, 0.f);
+    else
+      for (int j = lane; j < p.nb; j += 64) drow[j] = 0.f;
+  }
   const float sc = rq * p.scale * kLog2eF;  // raw score -> log2 units
 
   // the row indices of step m: selected or causal block, or window position
@@ -781,6 +791,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt) dq[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float psel = 0.f, dssel = 0.f;  // sums over the selected slots (gsum)
+  if (drow) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // its zeros are written before any value
   {
     typename W::Rows rr;
     Sel sl;
@@ -810,26 +821,39 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_q_kernel(HcaBwdParams p) {
         bh[e] = (bf16_t)dse[e];
         bl[e] = lo_of(dse[e]);
       }
+      if (32 * st < nsel_pad) {
+        if (p.gsum) {
+          // this head's p and ds sums over the selected rows (unused slots: 0)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            psel += pe[e];
+            dssel += dse[e];
+          }
+        }
+        if (drow || p.slot_grad) {
+          // sum over the heads of p ((dp - D) s + dp), the row's gradient dotted
+          // with the row; slot e of the lane group to its lane n = e
+          const int j = 32 * st + MW::row_sl(n & 7, q);
+          const int at = has_idx ? (int)__builtin_amdgcn_raw_buffer_load_b32(rs_idx, j * 4, 0, 0) : -1;
+          float mine = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float sraw = s8[e] > -INFINITY ? s8[e] * kLn2F : 0.f;  // scale qn.k
+            const float g = row16_sum(pe[e] * ((d8[e] - D) * sraw + d8[e]));
+            if (n == e) mine = g;
+          }
+          if (n < 8 && j < nsel && (unsigned)at < (unsigned)p.nb) {
+            // (no block is selected twice: one writer an element)
+            if (p.slot_grad) p.slot_grad[bt * p.topk + j] += mine;
+            if (drow) drow[at] = mine + (p.dsel_add ? drow[at] : 0.f);
+          }
+        }
+      }
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
         const bf16x8 vh = MqaWave<HD>::vt_frag(sth, to, tt);
         const bf16x8 vl = MqaWave<HD>::vt_frag(stl, to, tt);
         dq[tt] = mfma3(vh, vl, bh, bl, dq[tt]);
-      }
-      // the selected rows: sum over the heads of p ((dp - D) s + dp) (the row's
-      // gradient dotted with the row) per slot, and this head's p and ds sums
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int j = 32 * st + 16 * (e >> 2) + 4 * q + (e & 3);
-        const bool selk = j < nsel;
-        const float sraw = s8[e] > -INFINITY ? s8[e] * kLn2F : 0.f;  // scale qn.k
-        float g = selk ? pe[e] * ((d8[e] - D) * sraw + d8[e]) : 0.f;
-        g = row16_sum(g);
-        if (selk) {
-          psel += pe[e];
-          dssel += dse[e];
-        }
-        if (n == 0 && selk && p.slot_ws) p.slot_ws[bt * p.topk + j] = g;
       }
     }
   }
@@ -1126,8 +1150,8 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
   if (win > 0) z += al256m(BT * k.wnc * c * 4);         // window-row partials
   if (topk > 0) {
     z += al256m(BT * ((nb + 31) / 32) * 4);              // selection bitmap
-    z += al256m(BT * nb * 4);                            // dense slot gradients
-    if (!attn_bwd_dense_rows(nb, topk)) z += al256m(BT * topk * 4);  // per slot
+    // the tiled query pass's values by block, for the slots (at most 3 topk a query)
+    if (attn_bwd_dense_rows(nb, topk)) z += al256m(BT * nb * 4);
   }
   return z;
 }
@@ -1233,24 +1257,14 @@ hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStre
     const hipError_t e = sel_bitmap_launch(p.idx, sel, (long long)BT, p.topk, nw, s);
     if (e != hipSuccess) return e;
     p.sel = sel;
-    float* own = reinterpret_cast<float*>(take(BT * p.nb * 4));
-    if (!p.dsel && p.slot_grad) {
-      p.dsel = own;
+    if (tiled && p.slot_grad && !p.dsel) {
+      p.dsel = reinterpret_cast<float*>(take(BT * p.nb * 4));
       p.dsel_add = 0;
     }
-    if (p.dsel && !tiled) p.slot_ws = reinterpret_cast<float*>(take(BT * p.topk * 4));
   }
   hipError_t e = HD == 64 ? run_passes<64>(p, f, k, s) : run_passes<128>(p, f, k, s);
   if (e != hipSuccess) return e;
-  if (p.slot_ws) {
-    if (!p.dsel_add) {
-      e = fill_u32(p.dsel, (long long)BT * p.nb, 0u, s);
-      if (e != hipSuccess) return e;
-    }
-    e = ste_scatter_launch(p.idx, p.slot_ws, p.dsel, (long long)BT, p.topk, p.nb, s);
-    if (e != hipSuccess) return e;
-  }
-  if (p.slot_grad && p.idx) {
+  if (p.slot_grad && p.idx && tiled) {
     const long long ns = (long long)BT * p.topk;
     hipLaunchKernelGGL(slot_gather_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, s, p.idx, p.dsel,
                        p.slot_grad, ns, p.topk, p.nb);

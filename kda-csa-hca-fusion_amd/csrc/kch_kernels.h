@@ -132,7 +132,6 @@ struct HcaBwdParams {
   float scale;
   // set by the dispatch
   float* sink_part = nullptr;  // [B,T,nh] p_sink * D per query and head
-  float* slot_ws = nullptr;    // the gathering query pass's values per slot
   float* lse = nullptr;
   float* dval = nullptr;
   float* rq = nullptr;

@@ -116,6 +116,19 @@ def test_csa_backward_workspace_holds_every_head_group():
                 assert _csa_bwd_needs(lib, B, T, nh, c, m, topk, win, normalize) <= held, (nh, normalize)
 
 
+def test_csa_backward_workspace_of_long_sequences():
+    """Where a query selects few of its blocks, the selection costs the workspace
+    one bit a (query, block) and no value: 0.5 GiB at T 131072, m 4 (a dense
+    fp32 array would be 16). In tiles, at most three values a slot more."""
+    from kch import _lib
+    lib = _lib.load()
+    ws = lib.kch_csa_attn_bwd_ws_bytes
+    for T, topk in ((131072, 512), (32768, 64)):
+        assert ws(1, T, 16, 128, 4, 128, topk) - ws(1, T, 16, 128, 4, 128, 0) == T * (T // 4) // 8
+    for T, topk in ((4096, 512), (6144, 512)):
+        assert ws(1, T, 16, 128, 4, 128, topk) - ws(1, T, 16, 128, 4, 128, 0) <= T * (T // 32 + 3 * topk * 4)
+
+
 def test_chunk_workspace_size_query():
     """kch_kda_chunk_ws_bytes: 0 where no workspace is used, else the sum of
     the six per-chunk records, each region padded to 256 bytes."""
