@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define KCH_ABI_VERSION 22
+#define KCH_ABI_VERSION 23
 
 #define KCH_OK 0
 #define KCH_ERR_INVALID 1     /* bad pointer / shape / argument */
@@ -233,9 +233,13 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
  * dsel_add; gsum [B,T,c] or NULL: the sum over the selected slots of the
  * selected rows' gradients (written), which the full-softmax surrogate's dense
  * term (ops_csa.py:1050-1071) consumes. The window rows' gradient is added into
- * dCa.
+ * dCa. ws: kch_csa_attn_bwd_ws_bytes bytes hold a call of any kind.
  */
 size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk);
+/* the same for calls of one kind: normalize as given; slots = 1 with slot_grad
+ * and no dsel, which tiled rows (T/m <= 3 topk) take through a dense array */
+size_t kch_csa_attn_bwd_ws_bytes_for(int B, int T, int nh, int c, int m, int win, int topk,
+                                     int normalize, int slots);
 int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
                      const int* idx, const void* Ca, long long ldCa, const void* Cb, long long ldCb,
                      const void* Za, long long ldZa, const void* Zb, long long ldZb, const float* Ba,

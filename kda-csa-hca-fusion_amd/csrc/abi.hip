@@ -437,7 +437,7 @@ static int check_attn_bwd(const char* fn, int B, int T, int nh, int c, int m, in
 
 size_t kch_hca_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win) {
   if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m2 < 1 || T % m2 || win < 0) return 0;
-  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, -1, 1);
+  return kch::hca_bwd_ws_bytes(B, T, nh, c, m2, win, -1, 1, 0);
 }
 
 int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const float* raw,
@@ -476,11 +476,16 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   return hip_status(fn, kch::hca_bwd_dispatch(p, f, ws, (hipStream_t)stream));
 }
 
-size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk) {
+size_t kch_csa_attn_bwd_ws_bytes_for(int B, int T, int nh, int c, int m, int win, int topk, int normalize,
+                                     int slots) {
   if (B <= 0 || T <= 0 || nh < 1 || (c != 64 && c != 128) || m < 1 || T % m || win < 0 || topk < 0)
     return 0;
-  const size_t norm = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, 1);
-  const size_t raw = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, 0);
+  return kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, normalize != 0, slots != 0);
+}
+
+size_t kch_csa_attn_bwd_ws_bytes(int B, int T, int nh, int c, int m, int win, int topk) {
+  const size_t norm = kch_csa_attn_bwd_ws_bytes_for(B, T, nh, c, m, win, topk, 1, 1);
+  const size_t raw = kch_csa_attn_bwd_ws_bytes_for(B, T, nh, c, m, win, topk, 0, 1);
   return norm > raw ? norm : raw;
 }
 
@@ -507,7 +512,7 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (int rc = check_bwd_rows(fn, "Cb", Cb, ldCb, c, cdt)) return rc;
   if (int rc = check_bwd_rows(fn, "Za", Za, ldZa, c, cdt)) return rc;
   if (int rc = check_bwd_rows(fn, "Zb", Zb, ldZb, c, cdt)) return rc;
-  const size_t need = kch::hca_bwd_ws_bytes(B, T, nh, c, m, win, topk, normalize != 0);
+  const size_t need = kch_csa_attn_bwd_ws_bytes_for(B, T, nh, c, m, win, topk, normalize, slot_grad && !dsel);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
                 ws ? ws_bytes : (size_t)0);

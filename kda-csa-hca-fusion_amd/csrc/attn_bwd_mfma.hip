@@ -1138,7 +1138,7 @@ static bool attn_bwd_dense_rows(int nb, int topk) { return nb <= 3 * topk; }
 
 static size_t al256m(size_t x) { return (x + 255) & ~size_t(255); }
 
-size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
+size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk, bool slots) {
   const size_t BT = (size_t)B * T;
   const int nb = T / m2;
   const KeyPlan k = key_plan(B, T, nb, win);
@@ -1151,7 +1151,7 @@ size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk) {
   if (topk > 0) {
     z += al256m(BT * ((nb + 31) / 32) * 4);              // selection bitmap
     // the tiled query pass's values by block, for the slots (at most 3 topk a query)
-    if (attn_bwd_dense_rows(nb, topk)) z += al256m(BT * nb * 4);
+    if (slots && attn_bwd_dense_rows(nb, topk)) z += al256m(BT * nb * 4);
   }
   return z;
 }

@@ -529,18 +529,18 @@ static Tail tail(int B, int T, int nh, int c, int m2) {
 // The regions of the path that a call takes (attn_bwd_mfma_supported): a call on
 // raw rows is not asked for the MFMA path's, so that its last group of heads,
 // 16 or fewer, fits where its first, of 32, did.
-static size_t path_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize) {
-  if (normalize && nh <= 16) return attn_bwd_mfma_ws_bytes(B, T, c, m2, win, topk);
+static size_t path_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize, bool slots) {
+  if (normalize && nh <= 16) return attn_bwd_mfma_ws_bytes(B, T, c, m2, win, topk, slots);
   const Plan z = plan(B, T, T / m2, win, c);
   const size_t sel = topk > 0 ? al256((size_t)B * T * ((T / m2 + 31) / 32) * 4) : 0;
   return 3 * al256((size_t)B * T * nh * 4) + al256(z.part_b * 4) + al256(z.part_w * 4) + sel +
          al256((size_t)B * T * c * 4);
 }
 
-size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize) {
+size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize, bool slots) {
   const Tail t = tail(B, T, nh, c, m2);
-  return path_ws_bytes(B, T, nh, c, m2, win, topk < 0 ? 0 : topk, normalize) + (topk >= 0 ? 2 : 1) * t.terms + t.sink +
-         t.scratch;
+  return path_ws_bytes(B, T, nh, c, m2, win, topk < 0 ? 0 : topk, normalize, slots) + (topk >= 0 ? 2 : 1) * t.terms +
+         t.sink + t.scratch;
 }
 
 static hipError_t simt_dispatch(HcaBwdParams p, const BwdFinish& f, void* ws, hipStream_t stream) {
@@ -583,7 +583,8 @@ static hipError_t simt_dispatch(HcaBwdParams p, const BwdFinish& f, void* ws, hi
 hipError_t hca_bwd_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t stream) {
   const bool two = f.Cb != nullptr;
   const Tail t = tail(p.B, p.T, p.nh, p.c, p.m2);
-  char* w = static_cast<char*>(ws) + path_ws_bytes(p.B, p.T, p.nh, p.c, p.m2, p.win, p.topk, p.normalize);
+  char* w = static_cast<char*>(ws) +
+            path_ws_bytes(p.B, p.T, p.nh, p.c, p.m2, p.win, p.topk, p.normalize, p.slot_grad && !p.dsel);
   f.dBp = reinterpret_cast<float*>(w);
   w += t.terms;
   if (two) {

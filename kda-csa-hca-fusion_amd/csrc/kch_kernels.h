@@ -171,10 +171,11 @@ struct HcaBwdParams {
 };
 // MFMA attention backward (normalised queries and keys, c in {64, 128}, nh <= 16)
 bool attn_bwd_mfma_supported(const HcaBwdParams& p);
-size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk);
+// slots: the call has slot_grad and no dsel
+size_t attn_bwd_mfma_ws_bytes(int B, int T, int c, int m2, int win, int topk, bool slots);
 hipError_t attn_bwd_mfma_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t s);
 // topk < 0: HCA (single-branch compression)
-size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize);
+size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, int normalize, bool slots);
 hipError_t hca_bwd_dispatch(HcaBwdParams p, BwdFinish f, void* ws, hipStream_t stream);
 
 // The STE surrogate's backward for the indexer (ste_backward.hip), fp32

@@ -98,6 +98,7 @@ _QUERIES = {
     "kch_gen_attn_ws_bytes": (_SZ, [_I] * 8),
     "kch_hca_attn_bwd_ws_bytes": (_SZ, [_I] * 6),
     "kch_csa_attn_bwd_ws_bytes": (_SZ, [_I] * 7),
+    "kch_csa_attn_bwd_ws_bytes_for": (_SZ, [_I] * 9),
     "kch_csa_ste_bwd_ws_bytes": (_SZ, [_I] * 5),
     "kch_decode_ws_bytes": (_SZ, [_I] * 7),
     "kch_decode_dyn_ws_bytes": (_SZ, [_I] * 7),

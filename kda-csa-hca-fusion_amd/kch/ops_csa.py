@@ -600,7 +600,8 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     dsel = torch.empty(B_, T, nb, device=dev, dtype=f32) if _dense else None
     gsum = None
     dsink = None if sink is None else torch.empty(nh, device=dev, dtype=f32)
-    nbytes = _lib.load().kch_csa_attn_bwd_ws_bytes(B_, T, min(nh, hmax), cp, m, win, topk)
+    nbytes = _lib.load().kch_csa_attn_bwd_ws_bytes_for(B_, T, min(nh, hmax), cp, m, win, topk,
+                                                       int(bool(normalize_qk)), int(not _dense))
     ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
     total = None
     for h0 in range(0, nh, hmax):

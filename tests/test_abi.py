@@ -127,6 +127,11 @@ def test_csa_backward_workspace_of_long_sequences():
         assert ws(1, T, 16, 128, 4, 128, topk) - ws(1, T, 16, 128, 4, 128, 0) == T * (T // 4) // 8
     for T, topk in ((4096, 512), (6144, 512)):
         assert ws(1, T, 16, 128, 4, 128, topk) - ws(1, T, 16, 128, 4, 128, 0) <= T * (T // 32 + 3 * topk * 4)
+        # ... and none where dsel takes the values, or nobody
+        for dsel in (True, False):
+            need = _csa_bwd_needs(lib, 1, T, 16, 128, 4, topk, 128, 1, slots=False, dsel=dsel)
+            assert need - ws(1, T, 16, 128, 4, 128, 0) == T * (T // 4) // 8
+            assert need == lib.kch_csa_attn_bwd_ws_bytes_for(1, T, 16, 128, 4, 128, topk, 1, 0)
 
 
 def test_chunk_workspace_size_query():
