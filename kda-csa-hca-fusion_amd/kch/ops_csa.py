@@ -541,7 +541,8 @@ def _csa_core(Ca, Cb, Za, Zb, K_idx, Z_idx, q, q_idx, w_idx, Ba, Bb, B_idx, *, m
 
 
 def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
-                  sink_logits=None, normalize_qk=True, scale=None, want_gsum=False, _dense=False):
+                  sink_logits=None, normalize_qk=True, scale=None, want_gsum=False, _dense=False,
+                  _slots=True):
     """Gradients of the CSA attention (``ops_csa.py:869-1155``) with the selection
     ``idx`` ``[B,T,topk]`` (int32, -1 = unused) held fixed, on
     ``kch_csa_attn_bwd`` (fp32 arithmetic). Returns a dict with ``Ca, Cb, Za, Zb, q, Ba,
@@ -551,7 +552,8 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     rows' gradients over the slots. Channels are zero-padded to the kernel's
     size; more than 16 heads run as groups. ``_dense`` (internal,
     ``normalize_qk`` only): the slots' values as ``dsel`` ``[B,T,T/m]`` at their
-    blocks (0 at the others) in place of ``slot``."""
+    blocks (0 at the others) in place of ``slot``; ``_slots=False`` (internal):
+    neither."""
     fn = "csa_attn_grad"
     B_, T, c = Ca.shape
     nh = q.shape[2]
@@ -596,12 +598,12 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
     sink = None if sink_logits is None else sink_logits.detach().to(device=dev, dtype=f32).contiguous()
     dq = torch.empty_like(qf)
     # (zeros: the SIMT kernels add into it)
-    slot = None if _dense else torch.zeros(B_, T, topk, device=dev, dtype=f32)
+    slot = None if _dense or not _slots else torch.zeros(B_, T, topk, device=dev, dtype=f32)
     dsel = torch.empty(B_, T, nb, device=dev, dtype=f32) if _dense else None
     gsum = None
     dsink = None if sink is None else torch.empty(nh, device=dev, dtype=f32)
     nbytes = _lib.load().kch_csa_attn_bwd_ws_bytes_for(B_, T, min(nh, hmax), cp, m, win, topk,
-                                                       int(bool(normalize_qk)), int(not _dense))
+                                                       int(bool(normalize_qk)), int(slot is not None))
     ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
     total = None
     for h0 in range(0, nh, hmax):
@@ -632,7 +634,7 @@ def csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx, d_out, *, m, sliding_window=0,
            "Bb": dBb[:, :c].to(Bb.dtype)}
     if _dense:
         out["dsel"] = dsel
-    else:
+    elif _slots:
         out["slot"] = slot
     if gsum is not None:
         out["gsum"] = gsum[..., :c]
@@ -843,7 +845,7 @@ class _CsaCoreFunction(torch.autograd.Function):
         g = csa_attn_grad(Ca, Cb, Za, Zb, q, Ba, Bb, idx if idx.shape[-1] else None, d_out,
                           m=cfg["m"], sliding_window=cfg["sliding_window"], sink_logits=sink,
                           normalize_qk=cfg["normalize_qk"], scale=cfg["scale"], want_gsum=full,
-                          _dense=dense)
+                          _dense=dense, _slots=ste)
         dsel_extra = None
         if full:
             dsel_extra, extra = _full_softmax_grads(

@@ -497,3 +497,29 @@ def test_grads_move_inputs_to_the_first_ones_device(dev):
     b = _ste_indexer_grads(K.to(dev), Z, qi.to(dev), w, Bi, idx.to(dev), slot, m=m, normalize_qk=True)
     for x, y in zip(a, b):
         assert y.is_cuda and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("norm,m,topk", [(True, 4, 4), (True, 1, 4), (False, 4, 4)])  # in tiles, gathered, raw
+def test_core_backward_without_surrogate_computes_no_slots(dev, monkeypatch, norm, m, topk):
+    """``use_ste=False``: nothing reads the slots' values, so the kernel is given
+    no place for them; the gradients are those of a call that takes them."""
+    from kch import _lib
+    import kch
+    torch.manual_seed(topk + m)
+    B, T, nh, c, cI, nIh = 1, 48, 3, 64, 32, 2
+    x = [torch.randn(B, T, w, device=dev, requires_grad=True) for w in (c, c, c, c, cI, cI)]
+    q = torch.randn(B, T, nh, c, device=dev, requires_grad=True)
+    qi, w = torch.randn(B, T, nIh, cI, device=dev), torch.randn(B, T, nIh, device=dev)
+    pos = [torch.randn(m, n, device=dev) for n in (c, c, cI)]
+    kw = dict(m=m, topk=topk, sliding_window=5, normalize_qk=norm)
+    out, idx = kch.csa_core(*x, q, qi, w, *pos, return_indices=True, use_ste=False, **kw)
+    W = torch.randn_like(out)
+    seen, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (seen.append((name, a)), call(name, *a))[1])
+    got = torch.autograd.grad(out, [*x[:4], q], W)
+    args, = [a for name, a in seen if name == "kch_csa_attn_bwd"]
+    assert args[24] is None and args[25] is None  # slot_grad, dsel
+    ref = kch.ops_csa.csa_attn_grad(*x[:4], q, *pos[:2], idx, W, m=m, sliding_window=5,
+                                    normalize_qk=norm)
+    for g, name in zip(got, ("Ca", "Cb", "Za", "Zb", "q")):
+        assert torch.equal(g, ref[name]), name
