@@ -527,7 +527,7 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   p.topk = topk;
   p.sparse = 1;
   p.slot_grad = topk > 0 ? slot_grad : nullptr;
-  p.dsel = topk > 0 ? dsel : nullptr;
+  p.dsel = dsel;  // (topk = 0: zeros)
   p.dsel_add = dsel && dsel_add ? 1 : 0;
   p.gsum = gsum;
   p.normalize = normalize ? 1 : 0;

@@ -275,6 +275,31 @@ def test_attn_grad_sparse_edges(dev, topk, win):
         _check(name, g[name].cpu().numpy(), ref[name])
 
 
+@pytest.mark.parametrize("T,m,nh", [(16, 4, 2), (15, 1, 18)])  # rows of whole float4s or not; two head groups
+def test_attn_grad_dense_values_without_selection(dev, T, m, nh):
+    """With no selection the dense slot values are zeros, whatever their memory held."""
+    import kch
+    torch.manual_seed(T)
+    B, c = 2, 64
+    x = [torch.randn(B, T, c, device=dev) for _ in range(4)]
+    q, W = (torch.randn(B, T, nh, c, device=dev) for _ in range(2))
+    pos = [torch.randn(m, c, device=dev) for _ in range(2)]
+    empty, held = torch.empty, []
+
+    def poisoned(*a, **k):
+        t = empty(*a, **k)
+        if t.shape == (B, T, T // m):
+            held.append(t.fill_(float("nan")))
+        return t
+
+    torch.empty = poisoned
+    try:
+        g = kch.ops_csa.csa_attn_grad(*x, q, *pos, None, W, m=m, sliding_window=5, _dense=True)
+    finally:
+        torch.empty = empty
+    assert held and g["dsel"] is held[0] and not bool(g["dsel"].ne(0).any())
+
+
 @pytest.mark.parametrize("nIh,cI,norm", [(4, 64, True), (4, 64, False), (2, 32, True),
                                          (1, 128, False), (8, 64, True), (3, 48, False)])
 def test_ste_kernel_matches_dense_statement(dev, nIh, cI, norm):
