@@ -230,7 +230,7 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
  * surrogate (ops_csa.py:1033-1099) turns into the indexer's gradient; dsel
  * [B,T,T/m] or NULL (normalize = 1, nh <= 16): the same values at their blocks,
  * 0 at the others (the dsel of kch_csa_ste_bwd), added to what it holds with
- * dsel_add; gsum [B,T,c] or NULL: the sum over the selected slots of the
+ * dsel_add (then without slot_grad); gsum [B,T,c] or NULL: the sum over the selected slots of the
  * selected rows' gradients (written), which the full-softmax surrogate's dense
  * term (ops_csa.py:1050-1071) consumes. The window rows' gradient is added into
  * dCa. ws: kch_csa_attn_bwd_ws_bytes bytes hold a call of any kind.

@@ -503,6 +503,8 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (int rc = check_attn_bwd(fn, B, T, nh, c, m, win, scale, normalize, qdt, cdt)) return rc;
   if (dsel && (nh > 16 || !normalize))
     return fail(KCH_ERR_UNSUPPORTED, "%s: dsel needs normalize=1 and at most 16 heads a call (nh=%d)", fn, nh);
+  if (dsel && dsel_add && slot_grad)
+    return fail(KCH_ERR_UNSUPPORTED, "%s: slot_grad beside a dsel that is added to (its values hold earlier calls')", fn);
   if ((long long)B * T * topk >= (1LL << 39)) return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
   if (B == 0) return KCH_OK;
   if (!q || !d_out || !kc || !raw || !Ba || !Bb || !dq || !dCa || !dCb || !dZa || !dZb || !dBa || !dBb ||

@@ -92,14 +92,17 @@ def test_kda_backward_validation_and_workspace():
         assert lib.kch_kda_recurrent_bwd_ws_bytes(B, T, HV, K, V, code) == pad(ck) + pad(part)
 
 
-def _csa_bwd_needs(lib, B, T, nh, c, m, topk, win, normalize, slots=True, dsel=False):
-    """The workspace that kch_csa_attn_bwd says a call without one requires
-    (tensors stand for themselves: the call ends before any is read)."""
+def _csa_bwd_status(lib, B, T, nh, c, m, topk, win, normalize, slots=True, dsel=False, dsel_add=0):
+    """kch_csa_attn_bwd without a workspace: the call ends before any tensor is read."""
     x = ctypes.c_void_p(4096)
-    rc = lib.kch_csa_attn_bwd(x, x, x, x, x, x, c, x, c, x, c, x, c, x, x, None, x, x, x, x, x, x, x, None,
-                              x if slots else None, x if dsel else None, 0, None, B, T, nh, c, m, topk,
-                              win, 1.0, normalize, 0, 0, 0, None, 0, None)
-    assert rc == 1
+    return lib.kch_csa_attn_bwd(x, x, x, x, x, x, c, x, c, x, c, x, c, x, x, None, x, x, x, x, x, x, x,
+                                None, x if slots else None, x if dsel else None, dsel_add, None, B, T,
+                                nh, c, m, topk, win, 1.0, normalize, 0, 0, 0, None, 0, None)
+
+
+def _csa_bwd_needs(lib, *sizes, **kw):
+    """The workspace that kch_csa_attn_bwd says a call without one requires."""
+    assert _csa_bwd_status(lib, *sizes, **kw) == 1
     return int(re.search(rb"workspace of (\d+) bytes", lib.kch_last_error()).group(1))
 
 
@@ -114,6 +117,16 @@ def test_csa_backward_workspace_holds_every_head_group():
             held = lib.kch_csa_attn_bwd_ws_bytes(B, T, most, c, m, win, topk)
             for nh in range(1, most + 1):
                 assert _csa_bwd_needs(lib, B, T, nh, c, m, topk, win, normalize) <= held, (nh, normalize)
+
+
+def test_csa_backward_refuses_slots_beside_an_added_dsel():
+    """The slots would be read from a dsel that holds earlier calls' values too."""
+    from kch import _lib
+    lib = _lib.load()
+    assert _csa_bwd_status(lib, 1, 64, 16, 64, 4, 8, 8, 1, dsel=True, dsel_add=1) == 2
+    assert b"slot_grad" in lib.kch_last_error()
+    for kw in (dict(dsel=True), dict(slots=False, dsel=True, dsel_add=1), dict(dsel_add=1)):
+        assert _csa_bwd_needs(lib, 1, 64, 16, 64, 4, 8, 8, 1, **kw) > 0
 
 
 def test_csa_backward_workspace_of_long_sequences():
