@@ -401,12 +401,16 @@ int kch_gen_attn(const void* q, const void* kv, const long long* idx, const void
 
 // rows of c values of a backward's compression inputs (cdt, ld elements apart):
 // read and written 16 bytes at a time
-static int check_bwd_rows(const char* fn, const char* name, const void* p, long long ld, int c, int dt) {
+// (contiguous: the SIMT kernels' rows)
+static int check_bwd_rows(const char* fn, const char* name, const void* p, long long ld, int c, int dt, bool contiguous) {
   const long long es = dt == 0 ? 4 : 2;
   if (!p) return fail(KCH_ERR_INVALID, "%s: null tensor pointer (%s)", fn, name);
   if (ld < c) return fail(KCH_ERR_INVALID, "%s: %s rows of %d values lie %lld apart", fn, name, c, ld);
   if (((uintptr_t)p & 15) || (ld * es) % 16)
     return fail(KCH_ERR_INVALID, "%s: %s rows must be 16-byte aligned", fn, name);
+  if (contiguous && ld != c)
+    return fail(KCH_ERR_UNSUPPORTED, "%s: %s rows must be contiguous with raw rows or more than 16 heads (ld=%lld)", fn,
+                name, ld);
   return KCH_OK;
 }
 // gradients' storage: the inputs' or fp32
@@ -452,10 +456,10 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (B == 0) return KCH_OK;
   if (!q || !d_out || !kc || !raw || !B_pos || !dq || !dC || !dZ || !dB_pos)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
-  if (int rc = check_bwd_rows(fn, "C", C, ldC, c, cdt)) return rc;
-  if (int rc = check_bwd_rows(fn, "Z", Z, ldZ, c, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "C", C, ldC, c, cdt, nh > 16)) return rc;
+  if (int rc = check_bwd_rows(fn, "Z", Z, ldZ, c, cdt, nh > 16)) return rc;
   if (win > 0)
-    if (int rc = check_bwd_rows(fn, "window", lsrc, ld_l, c, cdt)) return rc;
+    if (int rc = check_bwd_rows(fn, "window", lsrc, ld_l, c, cdt, nh > 16)) return rc;
   const size_t need = kch_hca_attn_bwd_ws_bytes(B, T, nh, c, m2, win);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
@@ -510,10 +514,11 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (!q || !d_out || !kc || !raw || !Ba || !Bb || !dq || !dCa || !dCb || !dZa || !dZb || !dBa || !dBb ||
       (topk > 0 && !idx))
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
-  if (int rc = check_bwd_rows(fn, "Ca", Ca, ldCa, c, cdt)) return rc;
-  if (int rc = check_bwd_rows(fn, "Cb", Cb, ldCb, c, cdt)) return rc;
-  if (int rc = check_bwd_rows(fn, "Za", Za, ldZa, c, cdt)) return rc;
-  if (int rc = check_bwd_rows(fn, "Zb", Zb, ldZb, c, cdt)) return rc;
+  const bool simt = !normalize || nh > 16;
+  if (int rc = check_bwd_rows(fn, "Ca", Ca, ldCa, c, cdt, simt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Cb", Cb, ldCb, c, cdt, simt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Za", Za, ldZa, c, cdt, simt)) return rc;
+  if (int rc = check_bwd_rows(fn, "Zb", Zb, ldZb, c, cdt, simt)) return rc;
   const size_t need = kch_csa_attn_bwd_ws_bytes_for(B, T, nh, c, m, win, topk, normalize, slot_grad && !dsel);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,
@@ -568,8 +573,8 @@ int kch_csa_ste_bwd(const void* q_idx, const void* w_idx, const float* kc, const
   if (B == 0) return KCH_OK;
   if (!q_idx || !w_idx || !kc || !raw || !B_idx || !dsel || !dq_idx || !dw_idx || !dK_idx || !dZ_idx || !dB_idx)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
-  if (int rc = check_bwd_rows(fn, "K_idx", K_idx, ldK, cI, cdt)) return rc;
-  if (int rc = check_bwd_rows(fn, "Z_idx", Z_idx, ldZ, cI, cdt)) return rc;
+  if (int rc = check_bwd_rows(fn, "K_idx", K_idx, ldK, cI, cdt, false)) return rc;
+  if (int rc = check_bwd_rows(fn, "Z_idx", Z_idx, ldZ, cI, cdt, false)) return rc;
   const size_t need = kch_csa_ste_bwd_ws_bytes(B, T, nIh, cI, m);
   if (!ws || ws_bytes < need)
     return fail(KCH_ERR_INVALID, "%s: workspace of %zu bytes required, got %zu", fn, need,

@@ -546,7 +546,7 @@ size_t hca_bwd_ws_bytes(int B, int T, int nh, int c, int m2, int win, int topk, 
 static hipError_t simt_dispatch(HcaBwdParams p, const BwdFinish& f, void* ws, hipStream_t stream) {
   // the SIMT kernels read and write contiguous fp32 rows
   if (p.qdt != DT_F32 || f.cdt != DT_F32 || f.odt != DT_F32 || f.ldC != p.c || f.ldZ != p.c ||
-      (f.Cb && (f.ldCb != p.c || f.ldZb != p.c)) || p.dsel)
+      (f.Cb && (f.ldCb != p.c || f.ldZb != p.c)) || (p.win > 0 && f.ldl != p.c) || p.dsel)
     return hipErrorInvalidValue;
   p.C = static_cast<const float*>(f.C); p.Z = static_cast<const float*>(f.Z);
   p.Cb = static_cast<const float*>(f.Cb); p.Zb = static_cast<const float*>(f.Zb);

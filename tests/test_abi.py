@@ -129,6 +129,28 @@ def test_csa_backward_refuses_slots_beside_an_added_dsel():
         assert _csa_bwd_needs(lib, 1, 64, 16, 64, 4, 8, 8, 1, **kw) > 0
 
 
+def test_attention_backward_of_many_heads_takes_contiguous_rows_only():
+    """More than 16 heads a call run on kernels that read contiguous rows: a row
+    stride of its own is refused for each tensor, the window rows among them."""
+    from kch import _lib
+    lib = _lib.load()
+    x, c = ctypes.c_void_p(4096), 64
+    hca = lambda nh, win, ll, lc, lz: lib.kch_hca_attn_bwd(  # noqa: E731
+        x, x, x, x, x, ll, x, lc, x, lz, x, None, x, x, x, x, x, None, 1, 64, nh, c, 16, win, 1.0, 0, 0, 0,
+        None, 0, None)
+    for lds, name in (((c + 4, c, c), b"window"), ((c, c + 4, c), b"C"), ((c, c, 2 * c), b"Z")):
+        assert hca(17, 8, *lds) == 2 and name + b" rows must be contiguous" in lib.kch_last_error()
+        assert hca(16, 8, *lds) == 1 and b"workspace" in lib.kch_last_error()
+    assert hca(17, 0, c + 4, c, c) == 1 and b"workspace" in lib.kch_last_error()  # no window: not read
+    csa = lambda nh, norm, la, lb: lib.kch_csa_attn_bwd(  # noqa: E731
+        x, x, x, x, x, x, la, x, c, x, c, x, lb, x, x, None, x, x, x, x, x, x, x, None, None, None, 0, None,
+        1, 64, nh, c, 4, 8, 8, 1.0, norm, 0, 0, 0, None, 0, None)
+    for la, lb in ((c + 4, c), (c, c + 4)):
+        for nh, norm in ((17, 1), (4, 0)):
+            assert csa(nh, norm, la, lb) == 2 and b"contiguous" in lib.kch_last_error()
+        assert csa(16, 1, la, lb) == 1 and b"workspace" in lib.kch_last_error()
+
+
 def test_csa_backward_workspace_of_long_sequences():
     """Where a query selects few of its blocks, the selection costs the workspace
     one bit a (query, block) and no value: 0.5 GiB at T 131072, m 4 (a dense
