@@ -445,3 +445,36 @@ def test_append_one_matches_chunk_append(dev, kind, c, cI, dt, win):
                                        atol=0)
             assert torch.equal(k._prev[0], whole._prev[0]) and torch.equal(k._prev[1], whole._prev[1])
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind", ["csa", "hca"])
+def test_append_one_of_neighbouring_tensors(dev, kind):
+    """One sequence's projections as tensors of their own, 512 bytes each: the
+    allocator places them side by side, which does not make them one tensor. The
+    same cache as from slices of one projection, block ends included."""
+    import kch
+    torch.manual_seed(5)
+    c, m, win = 128, 2, 3
+    widths, n = ([c] * 4 + [c] * 2, 3) if kind == "csa" else ([c] * 2, 1)
+    pos = [0.1 * torch.randn(m, c, device=dev) for _ in range(n)]
+
+    def cache():
+        return (kch.CSADecodingCache(1, c, c, m, win, dev, torch.float32) if kind == "csa"
+                else kch.HCADecodingCache(1, c, m, win, dev, torch.float32))
+
+    a, b = cache(), cache()
+    torch.cuda.empty_cache()
+    beside = 0
+    for _ in range(5):
+        x = torch.randn(1, 1, sum(widths), device=dev)
+        a.append_step(*x.split(widths, -1), *pos)
+        own = [torch.empty(1, 1, w, device=dev) for w in widths]
+        for o, s in zip(own, x.split(widths, -1)):
+            o.copy_(s)
+        beside += all(u.data_ptr() + 512 == v.data_ptr() for u, v in zip(own, own[1:]))
+        b.append_step(*own, *pos)
+    if not beside:
+        pytest.skip("the allocator did not place the tensors side by side")
+    assert torch.equal(a.sw_buffer.raw(), b.sw_buffer.raw()) and torch.equal(a.C_comp, b.C_comp)
+    if kind == "csa":
+        assert torch.equal(a.K_IComp, b.K_IComp)
