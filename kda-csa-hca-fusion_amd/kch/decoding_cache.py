@@ -460,15 +460,14 @@ class CSADecodingCache:
             if fp is None or (C.rows is not None and C.rows.device != dev):
                 return None
             Ba, Bb, Bi = fp
+            C.ensure(nb, nb + 1)
+            K.ensure(nb, nb + 1)
+            cap = C.rows.shape[1]
+            if K.rows.shape[1] != cap:  # the kernel addresses both stores with one block stride
+                return None
             if self._prev_buf is None:
                 self._set_prev_buf(torch.empty(B, m, 2 * c, device=dev, dtype=dt))
             prev = self._prev_buf
-            C.ensure(nb, nb + 1)
-            K.ensure(nb, nb + 1)
-            cap = max(C.rows.shape[1], K.rows.shape[1])
-            # (the kernel addresses both stores with one block stride)
-            C.ensure(nb, cap)
-            K.ensure(nb, cap)
             if C.key_norm is None:
                 C.key_norm = self._normalize_qk
         if self._acc is None:

@@ -478,3 +478,33 @@ def test_append_one_of_neighbouring_tensors(dev, kind):
     assert torch.equal(a.sw_buffer.raw(), b.sw_buffer.raw()) and torch.equal(a.C_comp, b.C_comp)
     if kind == "csa":
         assert torch.equal(a.K_IComp, b.K_IComp)
+
+
+@pytest.mark.parametrize("c_cap,k_cap", [(10, 16), (16, 10), (11, 16)])
+def test_append_one_with_stores_of_different_capacity(dev, c_cap, k_cap):
+    """Block stores that differ in capacity (the append kernel takes one block
+    stride for both): the general path appends, the same cache as ever."""
+    import kch
+    torch.manual_seed(c_cap)
+    B, c, cI, m, n0 = 2, 64, 32, 2, 10
+    widths = [c] * 4 + [cI] * 2
+    P = torch.randn(B, (n0 + 3) * m, sum(widths), device=dev)
+    pos = [0.1 * torch.randn(m, w, device=dev) for w in (c, c, cI)]
+    a, b = (kch.CSADecodingCache(B, c, cI, m, 3, dev, torch.float32) for _ in range(2))
+    for k in (a, b):
+        k.append_step(*P[:, :n0 * m].split(widths, -1), *pos)
+    a.append_step(*P[:, n0 * m:].split(widths, -1), *pos)
+    for store, cap in ((b._C, c_cap), (b._K, k_cap)):
+        for name in ("rows", "keys", "inv"):
+            x = getattr(store, name)
+            if x is not None:
+                y = torch.empty(B, cap, *x.shape[2:], device=dev, dtype=x.dtype)
+                y[:, :n0] = x[:, :n0]
+                setattr(store, name, y)
+    for t in range(n0 * m, P.shape[1]):
+        b.append_step(*P[:, t:t + 1].split(widths, -1), *pos)
+    assert a.n_blocks == b.n_blocks == n0 + 3
+    torch.testing.assert_close(b.C_comp, a.C_comp, rtol=1e-5, atol=1e-6)
+    torch.testing.assert_close(b.K_IComp, a.K_IComp, rtol=1e-5, atol=1e-6)
+    for x, y in ((b._C.keys, a._C.keys), (b._K.inv, a._K.inv)):
+        torch.testing.assert_close(x[:, :n0 + 3], y[:, :n0 + 3], rtol=1e-2, atol=1e-3)
