@@ -70,11 +70,16 @@ __device__ __forceinline__ f32x4 mma4(float4 a, const float* b, f32x4 acc) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], acc, 0, 0, 0);
 }
 
-// The gate [a > 0] jumps at zero, and the two kernels sum a in different
-// orders: a score of unit rows that the matrix sum leaves at rounding level
-// (|qn.k| < kNearZero, about one in 10^5) is summed again in one fixed order,
-// CPL-channel chains joined by a balanced tree, so that both kernels take the
-// same side. (Raw rows keep the matrix sum.)
+// The gate [a > 0] jumps at zero. The two kernels sum a in the same order (the
+// same channels a step; exchanging the operands changes no bit: 0 of 512000
+// entries, half of them sums that cancel), so both take the same side. A score
+// of unit rows that the matrix sum leaves at rounding level (0 < |qn.k| <
+// kNearZero, about one in 10^5) is summed again in one fixed order, CPL-channel
+// chains joined by a balanced tree, so that its side does not depend on the
+// tiles' order of channels. A sum of exactly 0 stays: zero rows (a padded
+// sequence) have nothing else, and summing each of their pairs again took 2380
+// us where random rows take 420 (B2 T4096, 4 heads of 64, half of the queries
+// zero; whole indexer backward). Raw rows keep the matrix sum.
 constexpr float kNearZero = 2e-6f;
 
 // four consecutive stored values as fp32
@@ -112,12 +117,12 @@ __device__ __forceinline__ float tree_sq(const float* v) {
     return tree_sq<CPL, N / 2>(v) + tree_sq<CPL, N / 2>(v + N / 2 * CPL);
   }
 }
-// a[e] summed again where it is near zero; row(e): the query and key row of a[e]
+// a[e] summed again where it is near but not zero; row(e): the query and key row of a[e]
 template <int NIH, int CI, typename T, typename Rows>
 __device__ __forceinline__ void settle_zero(f32x4& a, int normalize, Rows rows) {
   unsigned near = 0;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) near |= fabsf(a[e]) < kNearZero ? 1u << e : 0u;
+  for (int e = 0; e < 4; ++e) near |= a[e] != 0.f && fabsf(a[e]) < kNearZero ? 1u << e : 0u;
   if (!normalize) return;
   while (near) {
     const int e = __builtin_ctz(near);

@@ -548,3 +548,83 @@ def test_core_backward_without_surrogate_computes_no_slots(dev, monkeypatch, nor
                                     normalize_qk=norm)
     for g, name in zip(got, ("Ca", "Cb", "Za", "Zb", "q")):
         assert torch.equal(g, ref[name]), name
+
+
+@pytest.mark.parametrize("norm,cI,nIh", [(True, 64, 1), (False, 64, 1), (False, 128, 1), (False, 64, 4)])
+def test_ste_kernels_gate_a_score_alike(dev, norm, cI, nIh):
+    """A score that is 0 but for its rounding (the second half of the channels
+    repeats the first's products, shuffled, with the other sign) opens the ReLU
+    gate of the query's gradient and of the key's, or of neither: per sequence,
+    query 1 sees block 0 with such scores and block 1 with negative ones, so its
+    gradient and block 0's are zero together, head for head of one."""
+    from kch.ops_csa import _ste_indexer_grads
+    g = torch.Generator().manual_seed(cI + nIh)
+    B, h = 2048, cI // 2
+    perm = torch.randperm(h, generator=g)
+    u, v = (torch.randn(B, h, generator=g) for _ in range(2))
+    q = torch.cat([u, u[:, perm]], 1)
+    K = torch.stack([torch.cat([v, -v[:, perm]], 1), -q], 1)
+    qi = torch.zeros(B, 2, nIh, cI)
+    qi[:, 1, 0] = q
+    w = torch.zeros(B, 2, nIh)
+    w[..., 0] = 1.0
+    idx = torch.tensor([[0, -1], [0, 1]], dtype=torch.int32).expand(B, 2, 2).contiguous()
+    slot = torch.tensor([[0.0, 0.0], [1.0, 0.0]]).expand(B, 2, 2).contiguous()
+    dK, _, dq, _, _ = _ste_indexer_grads(*(x.to(dev) for x in (K, torch.zeros_like(K), qi, w, torch.zeros(1, cI),
+                                                               idx, slot)), m=1, normalize_qk=norm)
+    in_q, in_k = dq[:, 1, 0].ne(0).any(-1), dK[:, 0].ne(0).any(-1)
+    assert 0 < int(in_q.sum()) < B and torch.equal(in_q, in_k)
+
+
+@pytest.mark.parametrize("zero", ["queries", "keys", "both"])
+def test_ste_zero_rows(dev, zero):
+    """Zero rows (a padded sequence): finite gradients against the dense statement,
+    and no time of their own (each of their pairs was once summed again, five
+    times the time of random rows)."""
+    from kch.ops_csa import _ste_indexer_grads, _ste_indexer_grads_dense
+    torch.manual_seed(7)
+
+    def inputs(B, T, m, topk, nIh, cI):
+        r = lambda *s: torch.randn(*s, device=dev)  # noqa: E731
+        K, Z, q, w, Bi = r(B, T, cI), r(B, T, cI), r(B, T, nIh, cI), r(B, T, nIh), 0.1 * r(m, cI)
+        score = torch.rand(B, T, T // m, device=dev)
+        t, n = torch.arange(T, device=dev), torch.arange(T // m, device=dev)
+        val, idx = score.masked_fill((t[:, None] + 1) // m <= n, -1.0).topk(topk, -1)
+        return [K, Z, q, w, Bi, torch.where(val >= 0, idx, -1).int(), r(B, T, topk) * (val >= 0)]
+
+    def pad(x):
+        K, q = x[0].clone(), x[2].clone()
+        if zero != "queries":
+            K[:, :K.shape[1] // 2] = 0
+        if zero != "keys":
+            q[:, q.shape[1] // 2:] = 0
+        return [K, x[1], q, *x[3:]]
+
+    x = pad(inputs(2, 128, 4, 8, 2, 64))
+    got = _ste_indexer_grads(*x, m=4, normalize_qk=True)
+    ref = _ste_indexer_grads_dense(*x, m=4, normalize_qk=True)
+    for i, name in ((1, "Z_idx"), (3, "w_idx"), (4, "B_idx")):
+        _check(name, got[i].cpu().numpy(), ref[i].cpu().numpy())
+    # (a zero row's own gradient is 1e12 times what reaches it: its scale)
+    for i, name in ((0, "K_idx"), (2, "q_idx")):
+        live = x[i].ne(0).any(-1)
+        if zero != "queries" and i == 0:
+            live[:, :64] = False
+        _check(name, got[i][live].cpu().numpy(), ref[i][live].cpu().numpy())
+        assert torch.isfinite(got[i]).all()
+
+    def time(x):
+        best = float("inf")
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(3):
+                _ste_indexer_grads(*x, m=4, normalize_qk=True)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    x = inputs(2, 4096, 4, 64, 4, 64)
+    plain, padded = time(x), time(pad(x))
+    assert padded < 1.8 * plain, (plain, padded)
