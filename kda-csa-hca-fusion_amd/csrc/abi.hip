@@ -1271,8 +1271,7 @@ DecodePlan decode_plan(int B, int nb, int nh, int hd, int topk, int ring_len, bo
     pl.nr = (nb + 255) / 256;
     pl.ko = (nb + 3) & ~3;
   }
-  if (keys && sel && pl.nr > 1 && !pl.split &&
-      kch::decode_pick_keys(B, nb, topk, pl.nr, &pl.rb)) {
+  if (keys && sel && pl.nr > 1 && !pl.split && kch::decode_pick_keys(B, nb, topk, &pl.rb)) {
     pl.split = true;
     pl.nr = (nb + pl.rb - 1) / pl.rb;
     pl.ko = (nb + 3) & ~3;

@@ -28,9 +28,9 @@
 // idx_merge_kernel   the top-k of the candidates of all ranges of a sequence
 //   (a global top-k lies in the union of the per-range top-ks), by the same
 //   estimate-gather-select over the candidates streamed from global memory;
-//   output sorted by value (logit desc, index asc). Up to KEYS_MAX blocks (and
-//   where the candidates would be as many bytes) it streams all logit keys of a
-//   score pass instead, and the ranges select nothing.
+//   output sorted by value (logit desc, index asc). Up to KEYS_MAX blocks
+//   (decode_pick_keys) it streams all logit keys of a score pass instead, and the
+//   ranges select nothing.
 // attn_kernel   joint-softmax MQA over a group of the attended rows of a
 //   sequence (selected or all compressed blocks, then the ring window): per
 //   wave and head M, L and the unnormalised o (MqaWave), merged across the
@@ -55,11 +55,19 @@ constexpr int MV_CAP = 4096;     // candidates the merge gathers at or above its
 // Blocks up to which the merge selects from all logit keys of a sequence
 // instead of from the ranges' top-k candidates (decode_pick_keys): a range's
 // own selection costs more than scoring it, while one workgroup streams a
-// sequence's keys at about 3 us per 8192. Step time of the two in us (candidates
-// / keys): B 16, 9000 blocks, top-512 55 / 46; 32769 blocks, top-64 60 / 56, top-512 83 /
-// 66; past this line only where the candidates are at least as many bytes:
-// B 4, 131073 blocks, top-512 126 / 107, but B 4, 65536, top-256 59 / 68 and B 1,
-// 131073, top-64 49 / 89.
+// sequence's keys at about 3 us per 8192. Step time of the two in us (keys /
+// candidates), top-64, 128, 256 and 512 at 16 heads of 128, 4 indexer heads of 64:
+//   B 1   8200 blocks  28 / 38   29 / 40   32 / 44   36 / 46
+//   B 1   32768        35 / 40   38 / 44   44 / 47   46 / 62
+//   B 1   40000        41 / 41   43 / 43   45 / 50   50 / 67
+//   B 4   32768        40 / 43   41 / 44   45 / 48   48 / 55
+//   B 4   40000        45 / 42   46 / 44   51 / 57   54 / 61
+//   B 16  32768        50 / 56   51 / 54   55 / 57   58 / 70
+//   B 16  40000        55 / 57   56 / 57   60 / 73   63 / 83
+// so a small batch's small top-k keeps the candidates past KEYS_FEW. At 65536
+// blocks the two are level up to top-256 and at top-512 (B 1 60 / 63, B 4 68 /
+// 68), and past it the keys' estimate misses too often.
+constexpr int KEYS_FEW = 32768;
 constexpr int KEYS_MAX = 40960;
 
 __device__ __forceinline__ uint32_t okey(float f) {
@@ -1461,13 +1469,18 @@ size_t decode_merge_lds(int topk) {
   return (size_t)merge_cap(topk) * 8 + (size_t)pow2_at_least(topk + 1) * 8 + 512 * 4 + 52 * 4;
 }
 
-bool decode_pick_keys(int B, int nb, int topk, int nr, int* rb) {
+bool decode_pick_keys(int B, int nb, int topk, int* rb) {
   if (nb <= RB_MAX || topk > MV_CAP / 2) return false;
-  if (nb > KEYS_MAX && 2LL * nr * topk < nb) return false;
-  // the merge's sampled estimate has to hold (sample_estimate's own terms)
+  if (nb > (B < 8 && topk < 256 ? KEYS_FEW : KEYS_MAX)) return false;
+  // The merge's sampled estimate has to hold (sample_estimate's own terms): it
+  // keeps the values down to the r-th of 256 sampled ones, r nb / 256 of them
+  // give or take a share of 1 / sqrt(r), and more than MV_CAP mean a radix
+  // select over the streamed keys, some 100 us (B 16, 32768 blocks, top-1024: a
+  // step of 161 us where most take 59 and the candidates 76): 2.5 deviations of
+  // room, a miss in about a hundred sequences at most.
   const float ex = (float)topk * 256.f / (float)nb;
-  const int r = (int)ceilf(ex + 3.f * sqrtf(ex) + 2.f);
-  if (2 * r > 256 || (float)r * (float)nb / 256.f * 1.25f > (float)MV_CAP) return false;
+  const float r = ceilf(ex + 3.f * sqrtf(ex) + 2.f);
+  if (2.f * r > 256.f || r * (float)nb / 256.f * (1.f + 2.5f / sqrtf(r)) > (float)MV_CAP) return false;
   // score ranges of about WG_TARGET workgroups over the batch
   const long long want = min((long long)RB_MAX, max(256LL, ((long long)B * nb + WG_TARGET - 1) / WG_TARGET));
   *rb = (int)((want + 15) & ~15LL);

@@ -91,7 +91,7 @@ struct DecodeIdxParams {
 // Whether the selection of a plan of nr > 1 ranges takes all logit keys of the
 // sequence from a score pass (in ranges of *rb blocks) instead of the ranges'
 // candidates.
-bool decode_pick_keys(int B, int nb, int topk, int nr, int* rb);
+bool decode_pick_keys(int B, int nb, int topk, int* rb);
 void decode_idx_plan(int B, int nb, int topk, int* rb, int* nr);
 int decode_range_max();  // most blocks one indexer range holds
 size_t decode_select_lds(int topk);

@@ -185,6 +185,26 @@ def test_chunk_workspace_size_query():
     assert lib.kch_kda_chunk_ws_bytes(B, T, 2, HV, K, V, 1) == expect
 
 
+def test_decode_plan_takes_keys_or_candidates():
+    """What the planned CSA step merges past 8192 blocks, by its workspace: all
+    logit keys (4 bytes a block) up to 40960 blocks, for a small selection of a
+    small batch up to 32768, and only where its estimate of the boundary leaves
+    room; else the ranges' top-k candidates (8 bytes each)."""
+    from kch import _lib
+    ws = _lib.load().kch_decode_ws_bytes
+    pad = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    for B, nb, topk, keys in ((1, 8193, 64, True), (16, 8200, 2048, True), (1, 32768, 64, True),
+                              (1, 32769, 255, False), (7, 40000, 128, False), (8, 40000, 128, True),
+                              (1, 40960, 256, True), (16, 40960, 512, True), (16, 40961, 512, False),
+                              (16, 32768, 1024, True), (16, 39000, 1024, False), (4, 131073, 512, False)):
+        region = ws(B, nb, 16, 128, topk, 128, 1) - ws(B, 1024, 16, 128, topk, 128, 1)
+        per = max(1024, 2 * topk)
+        r = max(-(-nb // 8192), min(-(-1024 // B), -(-nb // per)))
+        rb = (-(-nb // r) + 15) // 16 * 16
+        want = pad(B * ((nb + 3) // 4 * 4) * 4) if keys else pad(B * -(-nb // rb) * topk * 8)
+        assert region == want, (B, nb, topk, region, want)
+
+
 def test_hybrid_decoding_default_geometry_is_the_references():
     """``HybridDecoding()`` builds the reference's decode model
     (``run_decoding.py:642-656``)."""

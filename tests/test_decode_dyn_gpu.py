@@ -110,9 +110,12 @@ def test_csa_decode_dyn_matches_planned(dev, nb, topk, cap, m):
     (8193, 8, "random"),        # one block past the in-LDS selection
     (9000, 512, "equal"),       # every logit the same: the lowest indices win
     (8200, 2048, "random"),     # the largest selection merged from keys
-    (40960, 64, "random"),      # the last size merged from keys whatever the selection
+    (32768, 64, "random"),      # the last size merged from keys for a small selection of one sequence
+    (40960, 64, "random"),      # ranges and their candidates
+    (40960, 256, "random"),     # the last size merged from keys
     (40961, 64, "random"),      # ranges and their candidates
-    (40961, 1024, "random"),    # keys again: as many bytes as the candidates
+    (40961, 1024, "random"),
+    (39000, 1024, "random"),    # candidates: too many keys may pass the estimate
     (12000, 512, "sampled"),    # large logits where the estimate samples: it misses
 ])
 def test_csa_decode_selects_from_keys(dev, nb, topk, form):
