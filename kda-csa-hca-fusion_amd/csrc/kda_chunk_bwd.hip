@@ -34,10 +34,12 @@
 // Every operand that passes from one kernel to the next is split once, where
 // it is made, and lies in the workspace in the order the matrix instruction
 // reads it (Rec): a consumer's fragment is two 16-byte loads a lane, whole
-// 1 KB tiles, with no conversion, transpose or LDS staging. Between the two
-// products of a state kernel's chunk the state and v_n (dv_n) pass through
-// LDS as split planes; the transposed fragments that cb_grad_kernel reads are
-// taken from the same planes by transposing reads.
+// 1 KB tiles, with no conversion, transpose or LDS staging. The states S_n and
+// dS' alone stay fp32, in the same order (del multiplies them; a wave of
+// cb_grad_kernel splits each once, for its products). Between the two products
+// of a state kernel's chunk the state and v_n (dv_n) pass through LDS as split
+// planes; the transposed fragments that cb_grad_kernel reads are taken from the
+// planes by transposing reads, those of the states from a transpose in LDS.
 // The decay-weighted products (M, Aqk and their gradients) factor as
 // e^(G_i - G_a) e^(G_a - G_j) around token a = 31 and run on MFMA when every
 // gate of the chunk (channel tile) is <= 0 and every |G - G_a| <= 60 nats:
@@ -161,6 +163,24 @@ __device__ __forceinline__ void ft_store(bf16_t* m, int tile, int lane, const Sp
   *reinterpret_cast<bf16x8*>(p + 512) = s.lo;
 }
 
+// The same tiles in fp32 (as many bytes): columns d .. d + 3 of all lanes before
+// d + 4 .. d + 7.
+struct F8 {
+  f32x4 a, b;
+};
+
+__device__ __forceinline__ F8 ft_load_f32(__amdgpu_buffer_rsrc_t m, int off, int tile) {
+  const int v = 16 * (threadIdx.x & 63), so = 2 * (off + tile * kTile);
+  return {__builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(m, v, so, 0)),
+          __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(m, v + 1024, so, 0))};
+}
+
+__device__ __forceinline__ void ft_store_f32(bf16_t* m, int tile, int lane, f32x4 a, f32x4 b) {
+  float* p = reinterpret_cast<float*>(m + (size_t)tile * kTile) + 4 * lane;
+  *reinterpret_cast<f32x4*>(p) = a;
+  *reinterpret_cast<f32x4*>(p + 256) = b;
+}
+
 // Accumulator rows 16 tc + 4 kq + e, column r16 into a matrix whose rows are
 // the accumulator's columns (row tile tr) and whose contraction columns (nk
 // tiles of 32) are the accumulator's rows.
@@ -275,14 +295,14 @@ struct Rec {
   static constexpr int EL = XT + 2 * C * C;    // el       fp32 [K]
   static constexpr int FL = EL + 2 * K;        // per 64 channels: decay products factored (int)
   static constexpr int RS = FL + 128;
-  static constexpr int DSN = 0;                // dL/dS after the chunk, K x V
+  static constexpr int DSN = 0;                // dL/dS after the chunk, K x V, fp32
   static constexpr int DVN = U;                // dL/dv_n transposed, V x C
   static_assert(V <= 2 * C && RS % 128 == 0, "record layout");
 };
 
 struct CbWs {
   bf16_t* rec;  // [B*HV*NT][RS]
-  bf16_t* sn;   // [B*HV*NT] state at the start of each chunk, tiles K x V
+  bf16_t* sn;   // [B*HV*NT] state at the start of each chunk, fp32 tiles K x V
   bf16_t* vn;   // [B*HV*NT] v_n, tiles C x V
   float* part;  // [B,T,HV,3K+1] per-value-head partials (HV > H), else null
   int nt;
@@ -654,18 +674,27 @@ struct StateTile {
       }
   }
 
-  // the wave's own rows of the planes as fragment tiles K x V of the slice
-  static __device__ __forceinline__ void store_tiles(bf16_t* dst, const bf16_t* hi, const bf16_t* lo,
-                                                     int V, int v0) {
-    const int wv = wave_id();
+  // the wave's rows as fp32 fragment tiles K x V of the slice, transposed through
+  // its own 16 rows of LDS (row stride VS + 4: stores and loads free of conflicts)
+  static constexpr int LF = VS + 4;
+  static __device__ __forceinline__ void store_tiles(bf16_t* dst, const f32x4 (&S)[KT][VT], float* tile, int V,
+                                                     int v0) {
+    const int l = threadIdx.x & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
+    for (int kt = 0; kt < KT; ++kt) {
+      wave_lds_sync();  // the last reads are done
+#pragma unroll
+      for (int vt = 0; vt < VT; ++vt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tile[(4 * kq + e) * LF + 16 * vt + r16] = S[kt][vt][e];
+      wave_lds_sync();
 #pragma unroll
       for (int vk = 0; vk < VS / 32; ++vk) {
-        const int k0 = 16 * (wv * KT + kt);
-        const Sp x = {tr8(hi, LK, 32 * vk, k0), tr8(lo, LK, 32 * vk, k0)};
-        ft_store(dst, (wv * KT + kt) * (V / 32) + v0 / 32 + vk, threadIdx.x & 63, x);
+        const float* p = tile + r16 * LF + 32 * vk + 8 * kq;
+        ft_store_f32(dst, (wv * KT + kt) * (V / 32) + v0 / 32 + vk, l, *reinterpret_cast<const f32x4*>(p),
+                     *reinterpret_cast<const f32x4*>(p + 4));
       }
+    }
   }
 };
 
@@ -675,7 +704,7 @@ struct StateTile {
 // the chain of a chunk: two products with an LDS pass of split planes and a
 // barrier after each. A wave's share of W, Kd^T, U and el of chunk n + 1 is in
 // flight, in registers, through the whole of chunk n. At 64 heads of
-// 64 chunks 224 us (3.5 TB/s), where splitting fp32 operands in every consumer
+// 64 chunks 213 us (3.7 TB/s), where splitting fp32 operands in every consumer
 // and staging Kd through LDS took 456.
 // ---------------------------------------------------------------------------
 template <int K, int V, int VS>
@@ -684,6 +713,7 @@ __global__ __launch_bounds__(256, 1) void cb_fwd_kernel(KdaBwdParams p, CbWs w) 
   using ST = StateTile<K, VS>;
   constexpr int KT = ST::KT, VT = ST::VT, LK = ST::LK, LC = C + 8, KS = K / 32;
   __shared__ __attribute__((aligned(16))) bf16_t sS[2][VS * LK], sV[2][VS * LC];
+  __shared__ __attribute__((aligned(16))) float sT[4][16 * ST::LF];
   const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   int vs, bh;
   slice_of<V / VS>(vs, bh);
@@ -732,7 +762,7 @@ __global__ __launch_bounds__(256, 1) void cb_fwd_kernel(KdaBwdParams p, CbWs w) 
       *reinterpret_cast<bf16x4*>(&sV[0][o]) = x.hi;
       *reinterpret_cast<bf16x4*>(&sV[1][o]) = x.lo;
     }
-    ST::store_tiles(w.sn + ci * 2 * K * V, sS[0], sS[1], V, v0);
+    ST::store_tiles(w.sn + ci * 2 * K * V, S, sT[wv], V, v0);
     __syncthreads();
 #pragma unroll
     for (int vk = 0; vk < VS / 32; ++vk) {
@@ -770,7 +800,7 @@ __global__ __launch_bounds__(256, 1) void cb_fwd_kernel(KdaBwdParams p, CbWs w) 
 // reverse; the shape of cb_fwd_kernel with dS' as the state, the operands of
 // chunk n - 1 (and its dO rows, for the other of two LDS buffers) in flight
 // through chunk n. Bound by HBM (at K = V = 128, bf16: 128 KB read and 96 KB
-// written a chunk). 64 heads of 64 chunks: 314 us (2.9 TB/s; 683 with fp32
+// written a chunk). 64 heads of 64 chunks: 302 us (3.0 TB/s; 683 with fp32
 // operands, split by each wave and transposed through LDS).
 // ---------------------------------------------------------------------------
 template <int K, int V, int VS, typename InT>
@@ -780,6 +810,7 @@ __global__ __launch_bounds__(256, 1) void cb_bwd_kernel(KdaBwdParams p, CbWs w) 
   constexpr int KT = ST::KT, VT = ST::VT, LK = ST::LK, LC = C + 8, KS = K / 32, LV = VS + 8;
   constexpr int NP = kParts<InT>, NDO = C * VS / 8 / 256;
   __shared__ __attribute__((aligned(16))) bf16_t sD[2][VS * LK], sdV[2][VS * LC], sdO[2][NP][C * LV];
+  __shared__ __attribute__((aligned(16))) float sT[4][16 * ST::LF];
   const int tid = threadIdx.x, l = tid & 63, wv = wave_id(), r16 = l & 15, kq = l >> 4;
   int vs, bh;
   slice_of<V / VS>(vs, bh);
@@ -865,7 +896,7 @@ __global__ __launch_bounds__(256, 1) void cb_bwd_kernel(KdaBwdParams p, CbWs w) 
       *reinterpret_cast<bf16x4*>(&sdV[1][o]) = x.lo;
       ft_store_acc(rec + R::DVN, v0 / 16 + vt, 2, wv, x);
     }
-    ST::store_tiles(rec + R::DSN, sD[0], sD[1], V, v0);
+    ST::store_tiles(rec + R::DSN, D, sT[wv], V, v0);
     __syncthreads();
     // dS = el dS' + Qg^T dO - W^T dv_n
 #pragma unroll
@@ -919,7 +950,7 @@ __global__ __launch_bounds__(256, 1) void cb_bwd_kernel(KdaBwdParams p, CbWs w) 
 // tokens in accumulator order (lane kq: tokens 16 rt + 4 kq + e), which makes
 // those registers the operand as they stand. The row offsets
 // go through buffer addressing: as 64-bit lane addresses they spilled (805 us).
-// 4096 chunks: 494 us (2.9 TB/s), where fp32 operands split by every reader, two
+// 4096 chunks: 500 us (2.9 TB/s), where fp32 operands split by every reader, two
 // waves a SIMD of one workgroup and a load round trip per step took 1190.
 // ---------------------------------------------------------------------------
 template <int K, int V, typename InT>
@@ -1004,9 +1035,8 @@ __global__ __launch_bounds__(256, 2) void cb_grad_kernel(KdaBwdParams p, CbWs w)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, x.hi, acc, 0, 0, 0);
   };
 
-  // fp32 gradients also take the product of the low parts: what S and dS' lose
-  // in their two parts (del needs both) is then no more than the parts' products
-  // lost before
+  // fp32 gradients also take the product of the low parts (against float64 at
+  // K = V = 128: dq and dk 6.9e-6 -> 6.3e-6 of their norm, dg 1.4e-5 -> 9.9e-6)
   auto mmg = [](const Sp& a, const Sp& x, f32x4 acc) {
     if constexpr (SZ == 4) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.lo, x.lo, acc, 0, 0, 0);
     return mm3(a, x, acc);
@@ -1154,19 +1184,20 @@ __global__ __launch_bounds__(256, 2) void cb_grad_kernel(KdaBwdParams p, CbWs w)
     // (opaque, or the loop keeps every row's offset in a register of its own)
     asm volatile("" : "+v"(oq), "+v"(og), "+v"(od));
     uint32_t xg[4][4], xq[4][4], xk[4][4];
-    Sp b1 = ft_load(sn, 0, ctg * VS), b3 = ft_load(rec, R::DSN, ctg * VS);
+    F8 s1 = ft_load_f32(sn, 0, ctg * VS), s3 = ft_load_f32(rec, R::DSN, ctg * VS);
 #pragma unroll
     for (int ks = 0; ks < VS; ++ks) {
       decltype(do_load(0, 0, 0)) d[4];
-      Sp v[4], n1, n3;
+      Sp v[4];
+      F8 n1, n3;
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
         d[rt] = do_load(od, rt, ks);
         v[rt] = ft_load(vng, 0, rt * VS + ks);
       }
       if (ks + 1 < VS) {
-        n1 = ft_load(sn, 0, ctg * VS + ks + 1);
-        n3 = ft_load(rec, R::DSN, ctg * VS + ks + 1);
+        n1 = ft_load_f32(sn, 0, ctg * VS + ks + 1);
+        n3 = ft_load_f32(rec, R::DSN, ctg * VS + ks + 1);
       } else {
 #pragma unroll
         for (int rt = 0; rt < 4; ++rt)
@@ -1178,9 +1209,15 @@ __global__ __launch_bounds__(256, 2) void cb_grad_kernel(KdaBwdParams p, CbWs w)
           }
       }
       __builtin_amdgcn_sched_barrier(0);
+      float f1[8], f3[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        del += ((float)b1.hi[i] + (float)b1.lo[i]) * ((float)b3.hi[i] + (float)b3.lo[i]);
+      for (int i = 0; i < 4; ++i) {
+        f1[i] = s1.a[i]; f1[4 + i] = s1.b[i];
+        f3[i] = s3.a[i]; f3[4 + i] = s3.b[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) del += f1[i] * f3[i];
+      const Sp b1 = sp8(f1), b3 = sp8(f3);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
         x1[rt] = mma_do(do_split(d[rt]), b1, x1[rt]);
@@ -1188,8 +1225,8 @@ __global__ __launch_bounds__(256, 2) void cb_grad_kernel(KdaBwdParams p, CbWs w)
         x3[rt] = mmg(v[rt], b3, x3[rt]);
       }
       __builtin_amdgcn_sched_barrier(0);
-      b1 = n1;
-      b3 = n3;
+      s1 = n1;
+      s3 = n3;
     }
     del += __shfl_xor(del, 16);
     del += __shfl_xor(del, 32);

@@ -350,3 +350,29 @@ def test_chunk_bwd_tile_edges(dev, B, T, H, HV, K, V, exact):
     ts, s0t = _leaves(host, s0, dev, torch.float32, torch.float32)
     got = _hip_grads(kch.naive_chunk_kda, ts, s0t, w_o, w_s)
     _check(got, _ref(host, s0, w_o, w_s), 1e-4, label=f"{B} {T} {exact}")
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_chunk_bwd_state_gate_gradient_in_fp32(dev, dtype, K, V):
+    """The part of dg that the carried state has, sum_v S dS', keeps fp32 factors
+    whatever the inputs' type. With zero q, k, v, beta and g it is all of dg:
+    sum_v s0 ds at every token, here with the columns in pairs that cancel but
+    for 2^-10 of them. Against float64: the output's rounding, and 4e-6 for an
+    fp32 sum of V products up to about 4 (2^-24 each, random signs; factors of
+    16 significant bits would leave 6e-5)."""
+    import kch
+    torch.manual_seed(K)
+    B, T, H = 2, 100, 3
+    s0, ds, r = (torch.randn(B, H, K, V // 2, device=dev) for _ in range(3))
+    s0 = torch.stack([s0, s0], -1).flatten(-2).requires_grad_(True)
+    ds = torch.stack([ds, -ds * (1 + r / 1024)], -1).flatten(-2)
+    z = lambda *d: torch.zeros(B, T, H, *d, device=dev, dtype=dtype)  # noqa: E731
+    g = z(K).requires_grad_(True)
+    _, st = kch.naive_chunk_kda(z(K), z(K), z(V), g, z(), initial_state=s0, output_final_state=True)
+    dg, ds0 = torch.autograd.grad(st, [g, s0], ds)
+    assert torch.equal(ds0, ds)
+    ref = (s0.detach().double() * ds.double()).sum(-1)[:, None].expand(B, T, H, K)
+    ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    err = (dg.double() - ref).abs()
+    assert bool((err <= 4e-6 + ulp * ref.abs()).all()), float(err.max())
