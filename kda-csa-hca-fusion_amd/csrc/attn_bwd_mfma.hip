@@ -1129,11 +1129,12 @@ bool attn_bwd_mfma_supported(const HcaBwdParams& p) {
 
 // CSA: whether the query pass takes every visible block in tiles (true) or
 // gathers the selected rows. The tiles' cost grows with the visible blocks
-// (nb / 2 on average), the gather's with topk; whole backward, 8192 queries,
-// 16 heads of 128, window 128, tiles against gather: topk 512, nb 512 0.655 /
-// 0.852 ms, 1024 0.875 / 1.006, 2048 1.328 / 1.277, 4096 4.51 / 3.61; topk 128,
-// nb 512 0.657 / 0.635; topk 64, nb 512 0.704 / 0.631 (measured with the fp32
-// compression gradients that attn_bwd_finish.hip replaced; both sides share them).
+// (nb / 2 on average), the gather's with topk. Whole core backward with the
+// surrogate, about 8192 queries, 16 heads of 128, window 128, bf16, tiles /
+// gather in ms: topk 512, nb 1024 1.04 / 1.11, 1536 1.10 / 1.08, 2048 1.74 /
+// 1.62; topk 256, nb 512 0.69 / 0.73, 768 0.71 / 0.71, 1024 1.03 / 0.98; topk
+// 128, nb 256 0.54 / 0.57, 384 0.61 / 0.61, 512 0.68 / 0.67; topk 64, nb 128 0.48
+// / 0.51, 256 0.53 / 0.54, 512 0.68 / 0.64.
 static bool attn_bwd_dense_rows(int nb, int topk) { return nb <= 3 * topk; }
 
 static size_t al256m(size_t x) { return (x + 255) & ~size_t(255); }
