@@ -203,7 +203,8 @@ int kch_gen_attn(const void* q, const void* kv, const long long* idx, const void
  * The other tensors are fp32: kc / raw [B,T/m2,c] (the L2-normalised and the
  * raw compressed rows of C, Z, B_pos, from kch_compress), B_pos [m2,c], sink
  * [nh] or NULL. Outputs: dq; dC, dZ; dB_pos [m2,c]; dlocal (the window rows'
- * source gradient) or NULL to add it into dC; dsink [nh] or NULL. Coverage: c
+ * source gradient) or NULL to add it into dC; dsink [nh] or NULL (B = 0: the
+ * sums over the batch, dB_pos and dsink, are zeros). Coverage: c
  * in {64, 128}, nh <= 16 (c = 128) or 32 (c = 64), T a multiple of m2, T >= 1.
  * ws: 256-byte aligned, kch_hca_attn_bwd_ws_bytes bytes.
  */

@@ -420,6 +420,17 @@ static int check_bwd_types(const char* fn, int qdt, int cdt, int odt) {
     return fail(KCH_ERR_INVALID, "%s: cdt %d, odt %d (cdt 0 fp32, 1 bf16, 2 fp16; odt 0 or cdt)", fn, cdt, odt);
   return KCH_OK;
 }
+// An empty batch's sums over the batch: zeros.
+struct BatchSum {
+  float* p;
+  long long n;
+};
+static int zero_sums(const char* fn, std::initializer_list<BatchSum> sums, void* stream) {
+  for (const BatchSum& x : sums)
+    if (x.p)
+      if (int rc = hip_status(fn, kch::fill_u32(x.p, x.n, 0u, (hipStream_t)stream))) return rc;
+  return KCH_OK;
+}
 // what the HCA and the CSA attention backward check alike
 static int check_attn_bwd(const char* fn, int B, int T, int nh, int c, int m, int win, float scale, int normalize,
                           int qdt, int cdt) {
@@ -453,7 +464,7 @@ int kch_hca_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   const char* fn = "kch_hca_attn_bwd";
   if (int rc = check_bwd_types(fn, qdt, cdt, odt)) return rc;
   if (int rc = check_attn_bwd(fn, B, T, nh, c, m2, win, scale, 1, qdt, cdt)) return rc;
-  if (B == 0) return KCH_OK;
+  if (B == 0) return zero_sums(fn, {{dB_pos, (long long)m2 * c}, {dsink, nh}}, stream);
   if (!q || !d_out || !kc || !raw || !B_pos || !dq || !dC || !dZ || !dB_pos)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
   if (int rc = check_bwd_rows(fn, "C", C, ldC, c, cdt, nh > 16)) return rc;
@@ -510,7 +521,8 @@ int kch_csa_attn_bwd(const void* q, const void* d_out, const float* kc, const fl
   if (dsel && dsel_add && slot_grad)
     return fail(KCH_ERR_UNSUPPORTED, "%s: slot_grad beside a dsel that is added to (its values hold earlier calls')", fn);
   if ((long long)B * T * topk >= (1LL << 39)) return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
-  if (B == 0) return KCH_OK;
+  if (B == 0)
+    return zero_sums(fn, {{dBa, (long long)m * c}, {dBb, (long long)m * c}, {dsink, nh}}, stream);
   if (!q || !d_out || !kc || !raw || !Ba || !Bb || !dq || !dCa || !dCb || !dZa || !dZb || !dBa || !dBb ||
       (topk > 0 && !idx))
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
@@ -570,7 +582,7 @@ int kch_csa_ste_bwd(const void* q_idx, const void* w_idx, const float* kc, const
                 fn, nIh, cI);
   if (std::isnan(scale)) return fail(KCH_ERR_INVALID, "%s: scale is NaN", fn);
   if ((long long)B * T * (T / m) >= (1LL << 40)) return fail(KCH_ERR_UNSUPPORTED, "%s: too large", fn);
-  if (B == 0) return KCH_OK;
+  if (B == 0) return zero_sums(fn, {{dB_idx, (long long)m * cI}}, stream);
   if (!q_idx || !w_idx || !kc || !raw || !B_idx || !dsel || !dq_idx || !dw_idx || !dK_idx || !dZ_idx || !dB_idx)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);
   if (int rc = check_bwd_rows(fn, "K_idx", K_idx, ldK, cI, cdt, false)) return rc;

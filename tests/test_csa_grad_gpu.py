@@ -628,3 +628,26 @@ def test_ste_zero_rows(dev, zero):
     x = inputs(2, 4096, 4, 64, 4, 64)
     plain, padded = time(x), time(pad(x))
     assert padded < 1.8 * plain, (plain, padded)
+
+
+@pytest.mark.parametrize("kind,norm", [("csa", True), ("csa", False), ("hca", True)])
+def test_empty_batch_gives_zero_bias_and_sink_gradients(dev, monkeypatch, kind, norm):
+    """The gradients that sum over the batch (position biases, sink) of a batch of
+    no sequences are zeros, whatever the memory that they are given held."""
+    import kch
+    c, cI, nh, nIh, m, T = 64, 32, 2, 2, 4, 16
+    r = lambda *s: torch.randn(*s, device=dev, requires_grad=True)  # noqa: E731
+    sk = r(nh)
+    if kind == "csa":
+        pos = [r(m, n) for n in (c, c, cI)]
+        o = kch.csa_core(*[r(0, T, n) for n in (c, c, c, c, cI, cI)], r(0, T, nh, c), r(0, T, nIh, cI),
+                         r(0, T, nIh), *pos, m=m, topk=3, sliding_window=4, sink_logits=sk, use_ste=True,
+                         normalize_qk=norm)
+    else:
+        pos = [r(m, c)]
+        o = kch.hca_core(r(0, T, c), r(0, T, c), r(0, T, nh, c), *pos, m2=m, sliding_window=4, sink_logits=sk)
+    W, empty = torch.empty_like(o), torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: (lambda t: t.fill_(float("nan"))
+                                                         if t.is_floating_point() else t)(empty(*a, **k)))
+    for g in torch.autograd.grad(o, [*pos, sk], W):
+        assert not bool(g.ne(0).any())
