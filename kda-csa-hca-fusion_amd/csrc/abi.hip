@@ -287,6 +287,10 @@ int kch_kda_chunk_bwd(const void* q, const void* k, const void* v, const void* g
     return fail(KCH_ERR_INVALID, "%s: g_clamp_min or scale is NaN", fn);
   if ((long long)B * T * HV * (3 * K + 1) >= (1LL << 40) || (long long)T * HV * K >= (1LL << 31))
     return fail(KCH_ERR_UNSUPPORTED, "%s: tensors too large", fn);
+  // the kernels address the rows of a chunk with 32-bit byte offsets
+  const long long row = HV != H ? (3LL * K + 1) * 4 : (long long)(K > V ? K : V) * (dtype == KCH_DT_F32 ? 4 : 2);
+  if (64 * row * HV >= (1LL << 32))
+    return fail(KCH_ERR_UNSUPPORTED, "%s: 64 rows of HV=%d heads exceed 4 GiB", fn, HV);
   if (B == 0) return KCH_OK;
   if (!q || !k || !v || !g || !beta || !d_o || !dq || !dk || !dv || !dg || !dbeta)
     return fail(KCH_ERR_INVALID, "%s: null tensor pointer", fn);

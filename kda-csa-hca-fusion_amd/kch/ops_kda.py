@@ -233,7 +233,7 @@ def kda_recurrent_grad(q, k, v, g, beta, d_o, scale=None, initial_state=None, ds
     ``kch_kda_recurrent_bwd`` or, with ``chunked`` (the gradient of the chunk
     form with 64-token chunks, ``ops_kda.py:340-536``), on
     ``kch_kda_chunk_bwd`` where it covers the shape (fp32 / bf16 / fp16, K
-    padded to 64 or 128, V in {64, 128}). Returns ``(dq, dk, dv, dg, dbeta,
+    padded to 64 or 128, V in {64, 128}, 64 rows of all heads under 4 GiB). Returns ``(dq, dk, dv, dg, dbeta,
     ds0)``: the first five in the input dtype, ``ds0`` in the state dtype
     (fp32, fp64 for fp64 inputs) or ``None`` without an initial state. K is
     zero-padded to the kernel's next size; padded channels carry no
@@ -270,7 +270,9 @@ def kda_recurrent_grad(q, k, v, g, beta, d_o, scale=None, initial_state=None, ds
     ds0 = torch.empty(B, HV, Kp, V, device=q.device, dtype=st) if initial_state is not None \
         else None
     entry = "kch_kda_recurrent_bwd"
-    if chunked and code != 3 and Kp in (64, 128) and V in (64, 128):
+    # a chunk's rows, or its per-value-head partials, within 32-bit byte offsets
+    row = (3 * Kp + 1) * 4 if HV != H else max(Kp, V) * v.element_size()
+    if chunked and code != 3 and Kp in (64, 128) and V in (64, 128) and 64 * row * HV < 2 ** 32:
         entry = "kch_kda_chunk_bwd"
         q, k, v, g, beta, d_o = (_aligned(t) for t in (q, k, v, g, beta, d_o))
         nbytes = _lib.load().kch_kda_chunk_bwd_ws_bytes(B, T, H, HV, Kp, V, code)

@@ -7,6 +7,7 @@ import ctypes
 import os
 import re
 
+import pytest
 from conftest import REPO
 
 HEADER = os.path.join(REPO, "include", "kch.h")
@@ -167,6 +168,31 @@ def test_csa_backward_workspace_of_long_sequences():
             need = _csa_bwd_needs(lib, 1, T, 16, 128, 4, topk, 128, 1, slots=False, dsel=dsel)
             assert need - ws(1, T, 16, 128, 4, 128, 0) == T * (T // 4) // 8
             assert need == lib.kch_csa_attn_bwd_ws_bytes_for(1, T, 16, 128, 4, 128, topk, 1, 0)
+
+
+@pytest.mark.parametrize("H,HV,K,V,code,chunk", [
+    (131071, 131071, 128, 64, 0, True), (131072, 131072, 128, 64, 0, False),   # rows, fp32
+    (262143, 262143, 64, 128, 1, True), (262144, 262144, 64, 128, 1, False),   # bf16
+    (1, 43577, 128, 128, 1, True), (1, 43578, 128, 128, 1, False),             # partials, HV > H
+])
+def test_kda_chunk_backward_takes_rows_within_32_bit_offsets(monkeypatch, H, HV, K, V, code, chunk):
+    """A chunk's 64 rows of all heads (of the per-value-head partials, HV > H) are
+    addressed with 32-bit byte offsets; from 4 GiB on the entry refuses and the
+    gradient runs on the recurrence's kernel."""
+    import torch
+    from kch import _lib, ops_kda
+    lib = _lib.load()
+    x = ctypes.c_void_p(4096)
+    rc = lib.kch_kda_chunk_bwd(*[x] * 14, 1, 1, H, HV, K, V, 1.0, -10.0, code, None, 0, None)
+    assert (rc, b"4 GiB" in lib.kch_last_error()) == ((1, False) if chunk else (2, True))
+    seen = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: seen.append(name))
+    monkeypatch.setattr(_lib, "stream_of", lambda t: None)
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: torch.zeros(1))  # the workspace
+    dt = torch.float32 if code == 0 else torch.bfloat16
+    z = lambda *s: torch.zeros(1, dtype=dt).expand(1, 1, *s)  # noqa: E731
+    ops_kda.kda_recurrent_grad(z(H, K), z(H, K), z(HV, V), z(HV, K), z(HV), z(HV, V), chunked=True)
+    assert seen == ["kch_kda_chunk_bwd" if chunk else "kch_kda_recurrent_bwd"]
 
 
 def test_chunk_workspace_size_query():
