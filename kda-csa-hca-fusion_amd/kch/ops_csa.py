@@ -716,9 +716,8 @@ def _ste_indexer_grads(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, norma
 
 def _ste_indexer_grads_dense(K_idx, Z_idx, q_idx, w_idx, B_idx, idx, slot, *, m, normalize_qk,
                              dsel_extra=None):
-    """The same gradients for indexers wider than one wave per query
-    (``nIh * c_I > 512`` after padding), dense over the blocks with torch
-    operations."""
+    """The same gradients for indexers beyond ``kch_csa_ste_bwd``'s sizes
+    (``_ste_kernel_sizes``), dense over the blocks with torch operations."""
     leaves = [x.detach().requires_grad_(True) if x is not None else None
               for x in (K_idx, Z_idx, q_idx, w_idx, B_idx)]
     Kl, Zl, ql, wl, Bl = leaves
