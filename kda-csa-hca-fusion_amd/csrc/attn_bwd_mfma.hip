@@ -49,8 +49,8 @@
 // its own copy of every row and 16 keys per wave on three-MFMA products: HCA
 // B2 T8192 (64 blocks) query pass 254 -> 168 us, window keys 233 -> 105,
 // compressed keys 625 (32 workgroups) -> 62, splits of q and dout 68 -> 0; CSA
-// B2 T4096 top-512 (1024 blocks) query pass 565 -> 316, compressed keys 677 ->
-// 261, window keys 197 -> 73. (The window rows in two parts: 211, 150 and 349,
+// B2 T4096 top-512 (1024 blocks) query pass 565 -> 305, compressed keys 677 ->
+// 253, window keys 197 -> 71. (The window rows in two parts: 211, 150 and 349,
 // 114.)
 
 #include "attn_common.h"

@@ -33,8 +33,8 @@
 // Bound: the fp32 matrix rate (157 TFLOP/s), of 5 products over the visible
 // (query, head, block) triples. With one wave per query and 8 keys per thread
 // on the vector units (a shuffle reduction per pair) the two kernels took
-// 1002 + 921 us at B2 T4096, 4 heads of 64, 1024 blocks; now 186 + 105 us
-// (10.8 GFLOP of products: 37 TFLOP/s over the two, the causal imbalance of
+// 1002 + 921 us at B2 T4096, 4 heads of 64, 1024 blocks; now 178 + 108 us
+// (10.8 GFLOP of products: 38 TFLOP/s over the two, the causal imbalance of
 // the query kernel's workgroups and one exponential per lane being the rest).
 
 #include "attn_common.h"
