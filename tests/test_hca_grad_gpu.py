@@ -237,3 +237,32 @@ def test_core_grad_in_storage_type(dev, B, T, nh, c, m2, win, local, dtype, view
         r = ref.get(name)
         r = np.zeros((B, T, c)) if r is None else r
         _check(name, got[name].double().cpu().numpy(), r, 1e-4 + (ulp if half else 0.0))
+
+
+@pytest.mark.parametrize("win,local", [(7, False), (33, True), (0, False)])
+def test_attn_bwd_of_more_than_16_heads_a_call(dev, win, local):
+    """``kch_hca_attn_bwd`` with 20 heads of 64 in one call (the SIMT kernels, which
+    callers of the C entry reach; ``hca_core_grad`` runs groups of 16 on the MFMA
+    ones) against the fp64 oracle, the window rows' own gradient included."""
+    from kch import _lib
+    from kch.ops_csa import _compress
+    B, T, nh, c, m2 = 2, 96, 20, 64, 16
+    C, Z, q, Bp, sk, Cl, W = _make(T + win, B, T, nh, c, m2)
+    f = lambda x: torch.tensor(x, dtype=torch.float32, device=dev)  # noqa: E731
+    d = lambda x: x.double().cpu().numpy()  # noqa: E731
+    Ct, Zt, qt, Bt, st, Lt, Wt = (f(x) for x in (C, Z, q, Bp, sk, Cl, W))
+    ref = o_grad(d(Ct), d(Zt), d(qt), d(Bt), d(Wt), m2=m2, sliding_window=win, scale=0.9, sink_logits=d(st),
+                 C_local_raw=d(Lt) if local else None)
+    kc = torch.empty(B, T // m2, c, device=dev)
+    raw = _compress("test", Ct, Zt, Bt, m2, out_raw=True, key=kc, normalize=True)
+    out = {"q": qt, "C": Ct, "Z": Zt, "B_pos": Bt, "C_local_raw": Lt, "sink_logits": st}
+    out = {k: torch.full_like(v, float("nan")) for k, v in out.items()}
+    n = _lib.load().kch_hca_attn_bwd_ws_bytes(B, T, nh, c, m2, win)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    P = _lib.ptr
+    _lib.call("kch_hca_attn_bwd", P(qt), P(Wt), P(kc), P(raw), P(Lt if local else Ct), c, P(Ct), c, P(Zt), c,
+              P(Bt), P(st), P(out["q"]), P(out["C"]), P(out["Z"]), P(out["B_pos"]),
+              P(out["C_local_raw"]) if local else None, P(out["sink_logits"]), B, T, nh, c, m2, win, 0.9, 0,
+              0, 0, P(ws), n, _lib.stream_of(qt))
+    for name in ("q", "C", "Z", "B_pos", "sink_logits") + (("C_local_raw",) if local else ()):
+        _check(name, out[name].cpu().numpy(), ref[name], 1e-4)
