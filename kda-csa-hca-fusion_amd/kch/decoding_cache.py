@@ -225,8 +225,9 @@ def _alloc_acc(new, B, m):
 def _column_group(ts):
     """One ``[..., sum of widths]`` view over ``ts`` when they are adjacent column
     ranges of one tensor (the slices of one projection output), else None.
-    (Tensors of their own can lie side by side in memory too: the view has to end
-    inside the first one's storage.)"""
+    (Tensors of their own can lie side by side in memory too: ``as_strided`` refuses
+    a view that ends outside the first one's storage; asking for that storage's
+    size first costs a decode step 1 us.)"""
     t0 = ts[0]
     st = t0.stride()
     if st[-1] != 1:
@@ -237,10 +238,10 @@ def _column_group(ts):
         if t.dtype != dt or t.stride() != st or t.shape[:-1] != lead or t.data_ptr() != p + w * es:
             return None
         w += t.shape[-1]
-    end = t0.storage_offset() + sum((n - 1) * k for n, k in zip(lead, st)) + w
-    if end * es > t0.untyped_storage().nbytes():
+    try:
+        return t0.as_strided((*lead, w), st)
+    except RuntimeError:  # past the first one's storage
         return None
-    return t0.as_strided((*lead, w), st)
 
 
 # widths of the one-launch append: those of the bulk compression (the append
